@@ -130,7 +130,7 @@ static void potrf_panel_rec(gpl_ctx* c, hipStream_t s, Bucket& k, int64_t K0, in
         const int64_t kk = K0 / 64;
         {
             Prof p(c, "batch_potrf_diag", 0, 0, s);
-            potrf_diag3_f32_batched(s, L, N, kk, Dinv, k.d(BB_LDIAG), k.b[BB_INFO].as<int>(), nb, N2, N * 64, N, Dacc);
+            potrf_diag_f32_batched(s, L, N, kk, Dinv, k.d(BB_LDIAG), k.b[BB_INFO].as<int>(), nb, N2, N * 64, N, Dacc);
         }
         const int64_t M = N - (K0 + 64);
         if (M > 0) {

@@ -71,6 +71,7 @@ extern "C" int gpl_ctx_create(int32_t device, gpl_ctx** out) {
     if (e == hipSuccess) e = hipEventCreateWithFlags(&c->ev_d, hipEventDisableTiming);
     if (e == hipSuccess) e = hipMalloc((void**)&c->psync, kPanelSyncWords * sizeof(unsigned));
     if (e == hipSuccess) e = hipMemset(c->psync, 0, kPanelSyncWords * sizeof(unsigned));
+    if (e == hipSuccess) e = hipMalloc((void**)&c->dpub, kPanelMaxBlocks * 4096 * sizeof(double));
     if (e == hipSuccess) e = hipMalloc((void**)&c->tsync, kSolveSyncWords * sizeof(unsigned));
     if (e == hipSuccess) e = hipMemset(c->tsync, 0, kSolveSyncWords * sizeof(unsigned));
     if (const char* pw = getenv("GPL_PANEL_WAIT_POLLS")) c->pwait = (unsigned)strtoul(pw, nullptr, 10);
@@ -100,6 +101,7 @@ extern "C" void gpl_ctx_destroy(gpl_ctx* c) {
     hipEventDestroy(c->ev_h2);
     hipStreamDestroy(c->aux);
     if (c->psync) hipFree(c->psync);
+    if (c->dpub) hipFree(c->dpub);
     if (c->tsync) hipFree(c->tsync);
     hipStreamDestroy(c->side);
     hipStreamDestroy(c->stream);
@@ -253,12 +255,17 @@ int gpl::prepare_prog(const gpl_cf_term* terms, int32_t nterms, int64_t ncols, D
 // Outer row-panel height of the forward-substitution inverse (trtri_blocked
 // without scratch): 256 rows in 64-row steps.
 static const int kOuterNB = 256;
-// Outer panel width of the two-level right-looking Cholesky drivers: each panel
-// is factored in one launch (k_potrf_panel: 64-column blocks inside), then the
-// trailing matrix receives one rank-kPanelNB update.  512 columns measured 4 %
-// faster than 256 at n = 8192 (FP64 and mixed) and 3 % at n = 4096.
+// Outer block of the right-looking Cholesky drivers: its columns are factored by
+// panel launches (k_potrf_panel), then the trailing matrix receives one update of
+// that depth.  FP64: two launches of kPanelW = 256 columns, the second after an
+// update of its columns by the first (a launch keeps its blocks of 256 columns in
+// registers, and 512 columns in one launch are bound by its workgroups' products,
+// 131 us against 2 x 52 us for the chain); the update of the rest has depth 512,
+// as one of depth 256 costs 3 % of the n = 8192 step (15.2 ms against 15.6).  FP32
+// storage: one launch of 512 columns.
 static const int kPanelNB = 512;
-static_assert(kPanelNB / 64 <= kPanelMaxBlocks, "panel wider than the panel kernel's flags");
+static const int kPanelW = 64 * kPanelBlocksF64;
+static const int kPanelNB32 = 64 * kPanelBlocksF32;
 
 // X = L^-1 by recursive doubling from the 64x64 diagonal-block inverses Dinv.
 // At level b (b = 64, 128, ...) the b-blocks pair up: [[X11, 0], [L21, X22]]
@@ -420,14 +427,22 @@ struct InverseFork {
 // one launch, a workgroup per 64-row block (k_potrf_panel).
 static void potrf_panel(gpl_ctx* c, hipStream_t st, double* L, int64_t N, int64_t K0, int64_t W, double* Dinv,
                         double* ldiag, int* info, double* rhs) {
-    const int64_t nrb = (N - K0) / 64;
-    if (++c->pepoch == 0) c->pepoch = 1;
-    {
-        Prof p(c, "potrf_panel", (double)W * W * W / 3 + 2.0 * (N - K0 - W) * W * W, 8.0 * (N - K0) * W * 3, st);
-        potrf_panel_f64(st, L, N, K0, (int)(W / 64), nrb, Dinv, ldiag, info, c->psync, c->pepoch, c->pbase, c->pwait,
-                        rhs);
+    for (int64_t k0 = K0; k0 < K0 + W; k0 += kPanelW) {
+        const int64_t w = std::min<int64_t>(kPanelW, K0 + W - k0), k1 = k0 + w;
+        const int64_t nrb = (N - k0) / 64;
+        if (++c->pepoch == 0) c->pepoch = 1;
+        {
+            Prof p(c, "potrf_panel", (double)w * w * w / 3 + (double)(N - k1) * w * w, 8.0 * (N - k0) * w * 2, st);
+            potrf_panel_f64(st, L, N, k0, (int)(w / 64), nrb, Dinv, ldiag, info, c->psync, c->pepoch, c->pbase,
+                            c->dpub, c->pwait, rhs);
+        }
+        c->pbase += (unsigned)nrb;
+        if (k1 < K0 + W) {
+            Prof p(c, "syrk_update", 2.0 * (N - k1) * (K0 + W - k1) * w, 0, st);
+            const double* Q = L + k1 + k0 * N;
+            gemm2_f64(st, 0, 1, N - k1, K0 + W - k1, w, -1.0, Q, N, Q, N, 1.0, L + k1 * (N + 1), N, 0, 0);
+        }
     }
-    c->pbase += (unsigned)nrb;
 }
 
 // Two-level blocked right-looking Cholesky with one-panel look-ahead: after the
@@ -551,13 +566,13 @@ static void potrf32_blocked(gpl_ctx* c, float* L, int64_t N, double* Dinv, doubl
                             float* X = nullptr, float* Tm = nullptr) {
     hipStream_t s = c->stream, s2 = c->side;
     InverseFork<float> inv(c, L, Dinv, N, X, Tm);
-    potrf32_panel(c, s, L, N, 0, std::min<int64_t>(kPanelNB, N), Dinv, ldiag, info, Dacc);
-    inv.after_panel(std::min<int64_t>(kPanelNB, N));
-    for (int64_t K0 = 0; K0 < N; K0 += kPanelNB) {
-        const int64_t W = std::min<int64_t>(kPanelNB, N - K0);
+    potrf32_panel(c, s, L, N, 0, std::min<int64_t>(kPanelNB32, N), Dinv, ldiag, info, Dacc);
+    inv.after_panel(std::min<int64_t>(kPanelNB32, N));
+    for (int64_t K0 = 0; K0 < N; K0 += kPanelNB32) {
+        const int64_t W = std::min<int64_t>(kPanelNB32, N - K0);
         const int64_t K1 = K0 + W, R = N - K1;
         if (R <= 0) break;
-        const int64_t W1 = std::min<int64_t>(kPanelNB, R);
+        const int64_t W1 = std::min<int64_t>(kPanelNB32, R);
         const float* P = L + K1 + K0 * N;
         // the FP64 diagonal tiles of the next panel on the side stream, beside
         // its FP32 update (a few workgroups, latency-bound)

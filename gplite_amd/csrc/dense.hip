@@ -316,27 +316,39 @@ void gemm_mixed_f32f64f64(hipStream_t s, int ta, int tb, int64_t M, int64_t N, i
 }
 
 // ---------------------------------------------------------------------------
-// Diagonal block (64x64), FP64 arithmetic on FP64 or FP32 storage.
-// Thread (row i = t%64, wave w = t/64) keeps elements (i, 16w+q), q < 16, in
-// registers for the whole factorisation, which runs in four phases of 16
-// columns (one wave each, exchanging pivots by readlane) with a rank-16 update
-// of the waves to the right between phases.  The inverse
-// (written to Dinv, FP64) is then formed by 16x16 blocks: DPP forward
-// substitution inside the diagonal blocks, f64 MFMA for the block rows.
+// Cholesky of a 64-column block held in LDS, FP64.  The block is a trapezoid
+// S[col][row] (64 columns, row stride kTP): rows 0..63 the diagonal block and,
+// optionally, rows 64..127 a 64-row block below it, which leaves as
+// A_below L^-T in the same pass.
+//
+// It runs in four phases of 16 columns.  In a phase one wave per 64 rows keeps
+// its rows' 16 columns in registers, and beside them a copy of the phase's
+// 16x16 diagonal tile, one copy per 16-lane row.  Every wave factors that tile
+// for itself: the pivot and the multipliers of a column are then 16-lane row
+// broadcasts (v_mov_b64_dpp row_newbcast) of its own registers, so a column
+// costs no LDS round trip, no readlane and no exchange between waves, and the
+// rows below are solved by the same instructions.  The four waves then apply
+// the rank-16 update to the columns to the right on v_mfma_f64_16x16x4.
+//
+// Bound by the dependent FP64 chain of a column (rsq, two Newton steps, a
+// scale, one update).
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ double readlane_f64(double v, int lane) {
-    const long long b = __double_as_longlong(v);
-    const int lo = __builtin_amdgcn_readlane((int)(b & 0xffffffffLL), lane);
-    const int hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
-    return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
+constexpr int kPanelThreads = 512;
+constexpr int kTP = 144;  // row stride: 4 k-rows apart is 32 banks, so both halves of an MFMA operand read are conflict-free
 
-// 1/sqrt(d) for d > 0: hardware estimate refined by two Newton steps
-// y <- y (3 - d y^2) / 2 (each roughly doubles the correct bits), a short
-// dependent chain compared with a correctly rounded sqrt followed by a divide.
-// Non-positive or NaN d propagates NaN, which the pivot check reports.
+// 1/sqrt(d) for d > 0 from the hardware estimate y (good to 2^-24).  CUBIC: one
+// cubic step, y (1 + e/2 + 3e^2/8) with e = 1 - d y^2: four dependent operations,
+// of which only the last rounds at the result's size.  Otherwise two Newton
+// steps y (3 - d y^2) / 2, six operations (the FP32-storage forms: their factors
+// are rounded to FP32, and results stay bit for bit what they were).
+// Non-positive or NaN d gives NaN or a value the pivot check reports.
+template <bool CUBIC>
 __device__ __forceinline__ double rsqrt_f64(double d) {
     double y = __builtin_amdgcn_rsq(d);
+    if (CUBIC) {
+        const double e = fma(-(d * y), y, 1.0);
+        return fma(y * e, fma(e, 0.375, 0.5), y);
+    }
     const double h = 0.5 * d;
     y = y * fma(-h * y, y, 1.5);
     y = y * fma(-h * y, y, 1.5);
@@ -352,121 +364,156 @@ __device__ __forceinline__ double quad_bcast_f64(double v) {
     return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
 
-// One 64x64 diagonal block (block k of the N x N matrix A, leading dimension
-// ld) on one 256-thread workgroup: factor in place, Dinv + 4096k = the block's
-// inverse (when want_inv), ldiag[64k + i] = log L_ii, info = first failing row
-// + 1.  Dsrc (optional): the block's FP64 values (64x64 column-major) to factor
-// in place of A's.  IX: the block's values (FP64) are already in Xs
-// (Xs[col][row]), in place of either.  Lp, Xs (64 x 65), rinv, piv (64): workgroup LDS;
-// Lp[col][row] = L(row, col) (strictly lower after the factor), Xs[col][row] =
-// (L_kk^-1)(row, col).  MU (pcol: one LDS int): the waves to the right of
-// phase p apply its columns as rank-1 updates while wave p factors, following
-// a column counter in LDS, instead of one rank-16 update after a barrier.
-template <typename T, bool MU, bool IX = false>
-__device__ __forceinline__ void diag_block64(T* __restrict__ A, int64_t ld, int64_t k, double* __restrict__ Dinv,
-                                             double* __restrict__ ldiag, int* __restrict__ info, int want_inv,
-                                             const double* __restrict__ Dsrc, double (*Lp)[65], double (*Xs)[65],
-                                             double* rinv, double* piv, int* pcol = nullptr) {
-    // One 64x64 diagonal block per workgroup, FP64 arithmetic.  Wave w holds
-    // columns 16w..16w+15 of every row (lane = row).  Factor: four phases; in
-    // phase p wave p factors its 16 columns alone (pivots and multipliers are
-    // exchanged with readlane, no barrier), publishes them to LDS, and the
-    // waves to its right apply the rank-16 update.  Inverse: by 16x16 blocks
-    // (below).
-    T* blk = A + k * 64 * (ld + 1);
-    const int t = threadIdx.x, i = t & 63, w = t >> 6;
-    if (MU) {
-        if (t == 0) *pcol = 0;
-        __syncthreads();
+template <int LANE>
+__device__ __forceinline__ double row_bcast_f64(double v) {  // lane LANE of every 16-lane row
+    return __longlong_as_double(
+        __builtin_amdgcn_update_dpp((long long)0, __double_as_longlong(v), 0x150 | LANE, 0xf, 0xf, true));
+}
+
+// acc += (lane C of the 16-lane row of src) * m.  src needs two wait states
+// after the VALU instruction that wrote it (dpp_ready).
+template <int C>
+__device__ __forceinline__ void fmac_bcast_f64(double& acc, double src, double m) {
+    asm("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(src), "v"(m), "n"(C));
+}
+__device__ __forceinline__ void dpp_ready(double& v) { asm("s_nop 1" : "+v"(v)); }
+
+// Columns J..15 of a phase: d the 16x16 diagonal tile (lane % 16 = row), a this
+// lane's own row.  PIV: piv and rinv receive the pivot of column lane % 16 and
+// its 1/sqrt.  The updates
+// take their multipliers inside the multiply-add (4 cycles; a separate broadcast
+// costs another 6 per multiplier).
+template <int C>
+__device__ __forceinline__ void factor16_update(double (&a)[16], double (&d)[16], double nd, double l, double dl) {
+    if constexpr (C < 16) {
+        fmac_bcast_f64<C>(d[C], nd, dl);
+        fmac_bcast_f64<C>(a[C], nd, l);
+        factor16_update<C + 1>(a, d, nd, l, dl);
     }
-    double a[16];
-#pragma unroll
-    for (int q = 0; q < 16; ++q) {
-        const int c = 16 * w + q;
-        a[q] = (c <= i) ? (IX ? Xs[c][i] : Dsrc ? Dsrc[i + c * 64] : (double)blk[i + (int64_t)c * ld]) : 0.0;
-    }
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-        if (w == p) {
-            double myinv = 0.0, mypiv = 0.0;
-#pragma unroll
-            for (int jj = 0; jj < 16; ++jj) {
-                const int j = 16 * p + jj;
-                const double d = readlane_f64(a[jj], j);
-                const double inv = rsqrt_f64(d);
-                const double rt = d * inv;
-                const double l = (i > j) ? a[jj] * inv : ((i == j) ? rt : 0.0);
-                a[jj] = l;
-                myinv = (i == j) ? inv : myinv;
-                mypiv = (i == j) ? d : mypiv;
-                // rows above a column are cleared when that column is reached.
-                // Column j goes to LDS, which is also where the multipliers
-                // L(16p + cc, j) of the later columns are read from (one
-                // address for the whole wave); only the next pivot's column
-                // takes its multiplier by readlane, off the LDS round trip.
-                Lp[j][i] = l;
-                if (jj + 1 < 16) a[jj + 1] -= l * readlane_f64(l, j + 1);
-#pragma unroll
-                for (int cc = jj + 2; cc < 16; ++cc) a[cc] -= l * Lp[j][16 * p + cc];
-                // MU: every four columns, tell the waves to the right how many
-                // columns of L are in LDS (release: the columns land first)
-                if (MU && (jj & 3) == 3)
-                    __hip_atomic_store(pcol, j + 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
-            }
-            if (i >= 16 * p && i < 16 * p + 16) {
-                rinv[i] = myinv;
-                piv[i] = mypiv;
-            }
-        } else if (MU && w > p) {
-            // Pipelined: apply the rank-1 updates of phase p's columns to this
-            // wave's columns as they are published, four at a time, while wave p
-            // factors the next ones; no barrier between the phases, and the wave
-            // of the next phase starts right after the last four.  (Groups
-            // shrinking to single columns at the end of the phase, applied by a
-            // rolled loop, measured slower: 31 against 24 us per 64 columns.)
-#pragma unroll 1
-            for (int g = 0; g < 4; ++g) {
-                const int need = 16 * p + 4 * g + 4;
-                while (__hip_atomic_load(pcol, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) < need)
-                    __builtin_amdgcn_s_sleep(1);
-#pragma unroll
-                for (int jj = 0; jj < 4; ++jj) {
-                    const int j = need - 4 + jj;
-                    const double li = Lp[j][i];
-#pragma unroll
-                    for (int q = 0; q < 16; ++q) a[q] -= li * Lp[j][16 * w + q];
-                }
-            }
+}
+
+template <int J, bool PIV, bool CUBIC>
+__device__ __forceinline__ void factor16(double (&a)[16], double (&d)[16], int li, double& piv, double& rinv) {
+    if constexpr (J < 16) {
+        const double pv = row_bcast_f64<J>(d[J]);
+        const double inv = rsqrt_f64<CUBIC>(pv);
+        if (PIV) {
+            piv = (li == J) ? pv : piv;
+            rinv = (li == J) ? inv : rinv;
         }
-        if (!MU) __syncthreads();
-        if (!MU && w > p) {
-            double li[16];
+        double nd = d[J] * -inv;
+        d[J] *= inv;
+        a[J] *= inv;
+        dpp_ready(nd);
+        factor16_update<J + 1>(a, d, nd, a[J], d[J]);
+        factor16<J + 1, PIV, CUBIC>(a, d, li, piv, rinv);
+    }
+}
+
+// Tile (rt, ct) of the rank-16 update by phase p's columns (from j0):
+// S(r, c) -= sum_k L(r, j0 + k) L(c, j0 + k).  The product is formed transposed:
+// D lane (li, g) holds columns c = g + 4v of row r = li.  (The MFMA rounds like
+// sequential multiply-adds in k.)  SUM: the products are summed first and the
+// sum subtracted.
+template <bool SUM>
+__device__ __forceinline__ void trapezoid_tile(double (*S)[kTP], int j0, int rt, int ct, int li, int g) {
+    double ac[4], br[4], cv[4];
 #pragma unroll
-            for (int kk = 0; kk < 16; ++kk) li[kk] = Lp[16 * p + kk][i];
+    for (int k = 0; k < 4; ++k) {
+        ac[k] = S[j0 + 4 * k + g][16 * ct + li];
+        br[k] = S[j0 + 4 * k + g][16 * rt + li];
+    }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) cv[v] = S[16 * ct + g + 4 * v][16 * rt + li];
+    d4 acc;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) acc[v] = SUM ? 0.0 : cv[v];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        acc = __builtin_amdgcn_mfma_f64_16x16x4f64(SUM ? ac[k] : -ac[k], br[k], acc, 0, 0, 0);
+#pragma unroll
+    for (int v = 0; v < 4; ++v) S[16 * ct + g + 4 * v][16 * rt + li] = SUM ? cv[v] - acc[v] : acc[v];
+}
+
+// Factor of S by kPanelThreads threads (eight waves).  RT row tiles of 16 (4: the
+// diagonal block alone, its pivots and their 1/sqrt into piv[64], rinv[64]; 8:
+// with the block below).  After a
+// phase all waves update the next phase's columns, one tile each; the tiles
+// further right are updated by the waves of the other two SIMDs while the
+// factoring waves run the next phase.  Ends with a barrier.
+template <int RT, bool CUBIC, bool SUM>
+__device__ __forceinline__ void trapezoid_factor(double (*S)[kTP], double* piv, double* rinv) {
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int li = lane & 15, g = lane >> 4;
+#pragma unroll 1
+    for (int p = 0; p < 4; ++p) {
+        const int j0 = 16 * p;
+        if (w < RT / 4) {
+            const int row = 64 * w + lane;
+            double a[16], d[16], pv = 0.0, ri = 0.0;
 #pragma unroll
             for (int q = 0; q < 16; ++q) {
-                const int col = 16 * w + q;
-                double sum = 0.0;
-#pragma unroll
-                for (int kk = 0; kk < 16; ++kk) sum += li[kk] * Lp[16 * p + kk][col];
-                if (col <= i) a[q] -= sum;
+                d[q] = S[j0 + q][j0 + li];
+                a[q] = S[j0 + q][row];
             }
+            factor16<0, RT == 4, CUBIC>(a, d, li, pv, ri);
+#pragma unroll
+            for (int q = 0; q < 16; ++q) S[j0 + q][row] = (row < j0 + q) ? 0.0 : a[q];
+            if (RT == 4 && lane < 16) {
+                piv[j0 + lane] = pv;
+                rinv[j0 + lane] = ri;
+            }
+        } else if (p > 0 && (w & 2)) {
+            // waves 2, 3, 6, 7: the last phase's updates of the columns from tile p + 1
+            int u = (w & 1) + 2 * (w >> 2);
+#pragma unroll 1
+            for (int ct = p + 1; ct < 4; ++ct)
+#pragma unroll 1
+                for (int rt = ct; rt < RT; ++rt, ++u)
+                    if ((u & 3) == 0) trapezoid_tile<SUM>(S, j0 - 16, rt, ct, li, g);
+        }
+        __syncthreads();
+        if (p < 3) {
+            if (p + 1 + w < RT) trapezoid_tile<SUM>(S, j0, p + 1 + w, p + 1, li, g);
+            __syncthreads();
         }
     }
-    if (MU) __syncthreads();
+}
+
+// Blocks handed to other workgroups are stored with relaxed agent-scope atomics
+// (write-through), so publishing one needs no cache write-back: every wave waits
+// until its stores have been performed, then one thread sets the flag (0.9 us;
+// 3.5 us with a release fence in every wave).  Their readers take one acquire
+// fence after the flag and load plainly, so that the workgroups of an XCD share
+// the block in its L2 (loads that bypass it took 1.9 us instead of 0.7 us with 32
+// workgroups reading one block).
+template <typename T>
+__device__ __forceinline__ void put_shared(T* p, T v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// After trapezoid_factor<4>: the factor of diagonal block k to global memory
+// (blk, leading dimension ld; the upper triangle as zeros), ldiag[64k + i] =
+// log L_ii, info = first failing row + 1, and the block's inverse to Dinv (FP64,
+// 64x64 column-major) by 16x16 blocks: DPP substitution inside the diagonal
+// blocks, f64 MFMA for the block rows.  The inverse is left in rows 64..127 of
+// S, S[c][64 + r] = X(r, c).  rinv, piv: 64 doubles of LDS each.  SH: other
+// workgroups of the launch read Dinv (put_shared).
+template <typename T, bool SH = false>
+__device__ __forceinline__ void diag_finish(T* __restrict__ blk, int64_t ld, int64_t k, double* __restrict__ Dinv,
+                                            double* __restrict__ ldiag, int* __restrict__ info, double (*S)[kTP],
+                                            const double* rinv, const double* piv) {
+    const int t = threadIdx.x, i = t & 63, w = t >> 6;
 #pragma unroll
-    for (int q = 0; q < 16; ++q) {
-        const int c = 16 * w + q;
-        blk[i + (int64_t)c * ld] = (T)((c <= i) ? a[q] : 0.0);
-    }
-    if (t < 64) Lp[t][t] = 0.0;  // the substitution uses the strictly lower part
+    for (int q = 0; q < 8; ++q) blk[i + (int64_t)(8 * w + q) * ld] = (T)S[8 * w + q][i];
     __syncthreads();
     if (t < 64) {
+        S[t][t] = 0.0;  // the substitution uses the strictly lower part
         ldiag[k * 64 + t] = 0.5 * log(piv[t]);
         const unsigned long long bad = __ballot(!(piv[t] > 0.0));
         if (t == 0 && bad) atomicCAS(info, 0, (int)(k * 64 + __ffsll((long long)bad)));
     }
-    if (!want_inv) return;
+    __syncthreads();
     // Inverse by 16x16 blocks.  (1) Each wave inverts its diagonal block by
     // forward substitution, four lanes per column exchanging values by DPP (16
     // dependent steps).  (2) Block rows bi = 1..3 in turn, wave j < bi forming
@@ -475,7 +522,7 @@ __device__ __forceinline__ void diag_block64(T* __restrict__ A, int64_t ld, int6
     // g + 4v of column li), which is the A-operand layout of T^T with k = g + 4v,
     // so the product is taken as Y^T = T^T X_{bi,bi}^T without leaving registers.
     const int lane = t & 63, li = lane & 15, g = lane >> 4;
-    {
+    if (w < 4) {
         const int c = lane >> 2, q = lane & 3, base = 16 * w;
         double b[4];
 #pragma unroll
@@ -492,11 +539,11 @@ __device__ __forceinline__ void diag_block64(T* __restrict__ A, int64_t ld, int6
             }
             if (q == (kk & 3)) b[kr] = xk;
 #pragma unroll
-            for (int r = 0; r < 4; ++r) b[r] -= Lp[base + kk][base + 4 * r + q] * xk;
+            for (int r = 0; r < 4; ++r) b[r] -= S[base + kk][base + 4 * r + q] * xk;
         }
 #pragma unroll
-        for (int r = 0; r < 4; ++r) Xs[base + c][base + 4 * r + q] = b[r];
-        for (int r = q; r < base; r += 4) Xs[base + c][r] = 0.0;  // above the diagonal block
+        for (int r = 0; r < 4; ++r) S[base + c][64 + base + 4 * r + q] = b[r];
+        for (int r = q; r < base; r += 4) S[base + c][64 + r] = 0.0;  // above the diagonal block
     }
     __syncthreads();
 #pragma unroll
@@ -506,85 +553,101 @@ __device__ __forceinline__ void diag_block64(T* __restrict__ A, int64_t ld, int6
             d4 acc = d4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
             for (int kb = 0; kb < r0; kb += 4)  // X is zero above its diagonal blocks
-                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(Lp[kb + g][r0 + li], Xs[c0 + li][kb + g], acc, 0, 0, 0);
+                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(S[kb + g][r0 + li], S[c0 + li][64 + kb + g], acc, 0, 0, 0);
             d4 y = d4{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
             for (int v = 0; v < 4; ++v)
-                y = __builtin_amdgcn_mfma_f64_16x16x4f64(acc[v], Xs[r0 + g + 4 * v][r0 + li], y, 0, 0, 0);
+                y = __builtin_amdgcn_mfma_f64_16x16x4f64(acc[v], S[r0 + g + 4 * v][64 + r0 + li], y, 0, 0, 0);
 #pragma unroll
-            for (int v = 0; v < 4; ++v) Xs[c0 + g + 4 * v][r0 + li] = -y[v];
+            for (int v = 0; v < 4; ++v) S[c0 + g + 4 * v][64 + r0 + li] = -y[v];
         }
         __syncthreads();
     }
     double* D = Dinv + k * 64 * 64;
-    for (int e = t; e < 64 * 64; e += 256) D[(e & 63) + (e >> 6) * 64] = Xs[e >> 6][e & 63];
+    for (int e = t; e < 64 * 64; e += kPanelThreads) {
+        if (SH) put_shared(D + e, S[e >> 6][64 + (e & 63)]);
+        else D[e] = S[e >> 6][64 + (e & 63)];
+    }
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void k_potrf_diag3(T* __restrict__ A, int64_t ld, int64_t k,
-                                                     double* __restrict__ Dinv, double* __restrict__ ldiag,
-                                                     int* __restrict__ info, int want_inv, int64_t sA, int64_t sD,
-                                                     int64_t sL, const double* __restrict__ Dsrc) {
-    __shared__ double Lp[64][65];
-    __shared__ double Xs[64][65];
+// One 64x64 diagonal block per problem of a batch: FP32 storage, factored from
+// its FP64 tile (Dsrc, the layout of Dinv).
+__global__ __launch_bounds__(kPanelThreads) void k_potrf_diag(float* __restrict__ A, int64_t ld, int64_t k,
+                                                    double* __restrict__ Dinv, double* __restrict__ ldiag,
+                                                    int* __restrict__ info, int64_t sA, int64_t sD, int64_t sL,
+                                                    const double* __restrict__ Dsrc) {
+    __shared__ double S[64][kTP];
     __shared__ double rinv[64];
     __shared__ double piv[64];
-    A += blockIdx.x * sA;
-    Dinv += blockIdx.x * sD;
-    ldiag += blockIdx.x * sL;
-    info += blockIdx.x * ((sA != 0) ? 1 : 0);
-    // Dsrc (optional): the FP64 diagonal tiles (64x64 column-major, one per block
-    // row, same batch stride as Dinv) to factor in place of the stored tile of A
-    if (Dsrc) Dsrc += blockIdx.x * sD + k * 64 * 64;
-    diag_block64<T, false>(A, ld, k, Dinv, ldiag, info, want_inv, Dsrc, Lp, Xs, rinv, piv);
+    Dsrc += blockIdx.x * sD + k * 64 * 64;
+    for (int e = threadIdx.x; e < 64 * 64; e += kPanelThreads) S[e >> 6][e & 63] = Dsrc[e];
+    __syncthreads();
+    trapezoid_factor<4, false, true>(S, piv, rinv);
+    diag_finish(A + blockIdx.x * sA + k * 64 * (ld + 1), ld, k, Dinv + blockIdx.x * sD, ldiag + blockIdx.x * sL,
+                info + blockIdx.x, S, rinv, piv);
+}
+
+void potrf_diag_f32_batched(hipStream_t s, float* A, int64_t ld, int64_t k, double* Dinv, double* ldiag, int* info,
+                            int batch, int64_t sA, int64_t sD, int64_t sL, const double* Dacc) {
+    hipLaunchKernelGGL(k_potrf_diag, dim3((unsigned)batch), dim3(kPanelThreads), 0, s, A, ld, k, Dinv, ldiag, info, sA, sD, sL,
+                       Dacc);
 }
 
 // ---------------------------------------------------------------------------
-// One outer panel of the FP64 blocked Cholesky in a single launch: columns
-// [K0, K0 + 64nc), nc <= kPanelMaxBlocks column blocks, all rows from K0.  Workgroup rb owns
-// the 64-row block rb (rows K0 + 64rb ..) for the whole panel; for each column
-// block c it (1) waits for diagonal block c, (2) solves its block against the
-// block's inverse, L_{rb,c} = A_{rb,c} Dinv_c^T, and (3) subtracts
-// L_{rb,c} L_{c2,c}^T from its blocks in the later panel columns c2 <= rb,
-// reading L_{c2,c} once workgroup c2 has published it.  Workgroup c factors
-// diagonal block c (diag_block64) when its own updates are done.  The chain
-// per column block is then one diagonal factor, one 64x64 solve and one 64x64
-// update inside the workgroups, without the kernel boundaries of the separate
-// factor / panel-solve / panel-update launches.
+// One outer panel of the blocked Cholesky in a single launch: columns
+// [K0, K0 + 64nc), nc <= kPanelMaxBlocks column blocks, all rows from K0.
+// Workgroup rb owns the 64-row block rb (rows K0 + 64rb ..) for the whole
+// panel.  For each column block c < rb it
+//   (1) waits for the updated (not yet factored) diagonal block c,
+//   (2) factors it for itself together with its own block A_{rb,c}
+//       (trapezoid_factor), which leaves L_{rb,c},
+//   (3) subtracts L_{rb,c} L_{rb,c}^T from its own diagonal block (kept in
+//       registers) and L_{rb,c} L_{c2,c}^T from its blocks in the later panel
+//       columns, reading L_{c2,c} once workgroup c2 has published it.  The block
+//       of column c + 1 stays in LDS for the next step.
+// Workgroup c + 1 publishes its diagonal block right after its update by column
+// c, before it is factored: no factor, inverse or solve of another workgroup is
+// on the chain from one diagonal block to the next, only one 64-column
+// trapezoid factor, one 64x64 update, and the hand-over of a 64x64 block.  (With
+// one factor and inverse per block, handed to the workgroups below to multiply
+// by, the chain was 24-26 us per 64 columns.)  The diagonal block's own
+// workgroup stores its factor and inverse beside that chain.
+//
+// T = float (the mixed-precision form): A is FP32; the diagonal blocks come
+// from, and are published in, their FP64 copies Dpub = Dacc (64x64 column-major,
+// tile j at 4096j).  Block products are FP64 on the stored FP32 values with one
+// rounding to FP32 per stored result.  T = double: Dpub is workspace for the
+// panel's blocks 1 .. nc - 1 (tile c at 4096c); block 0 is read from A by every
+// workgroup, so its factor goes to tile 0 of Dpub first and the last workgroup
+// to report its read (or, for workgroup 0, that tile) copies it into A.
 //
 // rhs (optional, FP64 storage only): a vector b of N rows that leaves as
-// y = L^-1 b, the forward solve carried along: workgroup c stores
-// y_c = Dinv_c b_c with diagonal block c, and every workgroup below subtracts
-// L_{rb,c} y_c from its block of b after its block solve.  Only the backward
-// solve is then left to the caller.
+// y = L^-1 b, the forward solve carried along one column block behind:
+// workgroup c stores y_c = Dinv_c b_c and publishes it, every workgroup below
+// subtracts L_{rb,c} y_c from its block of b.
 //
 // Ordering: each workgroup takes a ticket (atomic counter) as its logical row
 // block, so block rb is held by a workgroup that started after those of every
 // lower block; all waits are on lower blocks, which have started and do not
-// wait on higher ones, so every wait ends.  Flags carry the launch's epoch
-// (release after the block's stores, acquire before its loads, agent scope).
+// wait on higher ones, so every wait ends.  Flags carry the launch's epoch.
 // A wait that outlasts maxpoll polls (2^20 by default: a second or more, far
 // beyond any legitimate wait) stores kPanelWaitTimeout in info and leaves the
 // kernel; the callers report it as a device error.
 //
-// sync (kPanelSyncWords words): [0, P) diagonal-block flags, [P, P + P^2)
-// flags of L_{c2,c} (P + P c2 + c), P = kPanelMaxBlocks, and the ticket counter
-// in the last word; base: tickets handed out before this launch.
+// sync (kPanelSyncWords words), P = kPanelMaxBlocks: [0, P) diagonal-block flags,
+// [P, P + P^2) flags of L_{c2,c} (P + P c2 + c), then P flags of y_c, the counter
+// of block 0's readers and the ticket counter; base: tickets handed out before
+// this launch (both counters advance by the grid size per launch).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ bool panel_wait(unsigned* f, unsigned epoch, int* info, int* s_ok, unsigned maxpoll) {
     if (threadIdx.x == 0) {
-        int ok = 1;
-        unsigned n = 0;
-        // poll with plain agent-scope loads, then one acquire fence (its cache
-        // invalidation once per wait rather than once per poll)
-        while (__hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != epoch) {
-            if (n++ >= maxpoll) {
-                ok = 0;
-                atomicCAS(info, 0, kPanelWaitTimeout);
-                break;
-            }
-            __builtin_amdgcn_s_sleep(2);
+        int ok = 0;
+        for (unsigned n = 0; n < maxpoll; ++n) {
+            ok = __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == epoch;
+            if (ok) break;
+            __builtin_amdgcn_s_sleep(1);
         }
+        if (!ok) atomicCAS(info, 0, kPanelWaitTimeout);
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         *s_ok = ok;
     }
@@ -592,263 +655,345 @@ __device__ __forceinline__ bool panel_wait(unsigned* f, unsigned epoch, int* inf
     return *s_ok != 0;
 }
 
-// Every wave makes its own stores visible at agent scope (the workgroup barrier
-// alone does not wait for other waves' stores), then one thread sets the flag.
+// the same for the flags f[stride * i], lo <= i < hi (hi - lo <= 64): one lane each
+__device__ __forceinline__ bool panel_wait_all(unsigned* f, int stride, int lo, int hi, unsigned epoch, int* info,
+                                               int* s_ok, unsigned maxpoll) {
+    if (threadIdx.x < 64) {
+        unsigned* fi = f + stride * (lo + ((int)threadIdx.x < hi - lo ? (int)threadIdx.x : 0));
+        int ok = 0;
+        for (unsigned n = 0; n < maxpoll; ++n) {
+            ok = !__ballot(__hip_atomic_load(fi, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != epoch);
+            if (ok) break;
+            __builtin_amdgcn_s_sleep(1);
+        }
+        if (!ok && threadIdx.x == 0) atomicCAS(info, 0, kPanelWaitTimeout);
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        if (threadIdx.x == 0) *s_ok = ok;
+    }
+    __syncthreads();
+    return *s_ok != 0;
+}
+
 __device__ __forceinline__ void panel_publish(unsigned* f, unsigned epoch) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (threadIdx.x == 0) __hip_atomic_store(f, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// S[k][r] = M(r, k) for a 64x64 block of a column-major matrix (leading dimension ld)
-template <typename T>
-__device__ __forceinline__ void blk_load(double (*S)[65], const T* M, int64_t ld) {
-    const int r = threadIdx.x & 63, kq = threadIdx.x >> 6;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) S[kq + 4 * j][r] = (double)M[r + (int64_t)(kq + 4 * j) * ld];
-}
-
-// the same block in two steps: its values into registers (a load that can be
-// issued early), then into S
-template <typename T>
-__device__ __forceinline__ void blk_fetch(T (&v)[16], const T* M, int64_t ld) {
-    const int r = threadIdx.x & 63, kq = threadIdx.x >> 6;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) v[j] = M[r + (int64_t)(kq + 4 * j) * ld];
-}
-
-template <typename T>
-__device__ __forceinline__ void blk_put(double (*S)[65], const T (&v)[16]) {
-    const int r = threadIdx.x & 63, kq = threadIdx.x >> 6;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) S[kq + 4 * j][r] = (double)v[j];
-}
-
-// M(r, k) = S[k][r] rounded to T; S keeps the rounded value (each thread
-// rewrites only the elements it stores)
-template <typename T>
-__device__ __forceinline__ void blk_store(T* M, int64_t ld, double (*S)[65]) {
-    const int r = threadIdx.x & 63, kq = threadIdx.x >> 6;
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-        const T v = (T)S[kq + 4 * j][r];
-        M[r + (int64_t)(kq + 4 * j) * ld] = v;
-        S[kq + 4 * j][r] = (double)v;
-    }
-}
-
-// M(r, k) = M(r, k) - S[k][r], formed in FP64 and rounded once to T.  All
-// loads are issued before the first store: interleaved, each load would wait
-// for the previous store (the compiler cannot rule out that two columns alias
-// for an arbitrary ld), sixteen global round trips in a row.
-template <typename T>
-__device__ __forceinline__ void blk_sub(T* M, int64_t ld, double (*S)[65]) {
-    const int r = threadIdx.x & 63, kq = threadIdx.x >> 6;
-    T v[16];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) v[j] = M[r + (int64_t)(kq + 4 * j) * ld];
-#pragma unroll
-    for (int j = 0; j < 16; ++j) M[r + (int64_t)(kq + 4 * j) * ld] = (T)((double)v[j] - S[kq + 4 * j][r]);
-}
-
-// C(r, j) = sum_k P(r, k) Q(j, k) with P, Q in LDS as [k][row]; wave w computes
-// the 32x32 quadrant (w / 2, w % 2) as 2 x 2 tiles of v_mfma_f64_16x16x4, then
-// (after a barrier) writes C to S as S[j][r] (SUB: subtracts it from S).
-// QG: Q is read from global memory instead, Qg (64x64 column-major, Q(j, k)
-// at Qg[j + 64k]).
-template <bool QG = false, bool SUB = false>
-__device__ __forceinline__ void blk_mm_nt(double (*P)[65], double (*Q)[65], double (*S)[65],
-                                          const double* __restrict__ Qg = nullptr) {
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int li = lane & 15, g = lane >> 4, r0 = 32 * (w >> 1), j0 = 32 * (w & 1);
-    d4 acc[2][2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
-#pragma unroll 4
-    for (int k0 = 0; k0 < 64; k0 += 4) {
-        double a[2], b[2];
-#pragma unroll
-        for (int i = 0; i < 2; ++i) a[i] = P[k0 + g][r0 + 16 * i + li];
-#pragma unroll
-        for (int j = 0; j < 2; ++j) b[j] = QG ? Qg[(j0 + 16 * j + li) + 64 * (k0 + g)] : Q[k0 + g][j0 + 16 * j + li];
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
-    }
-    __syncthreads();  // S may be P or Q
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                double& d = S[j0 + 16 * j + li][r0 + 16 * i + g + 4 * v];
-                d = SUB ? d - acc[i][j][v] : acc[i][j][v];
-            }
-    __syncthreads();
-}
-
-// b_rb -= L_{rb,c} y_c for the 64-row blocks bc (y_c) and brb, L_{rb,c} in S as S[k][r]
-__device__ __forceinline__ void rhs_update(const double* bc, double* brb, double (*S)[65], double* vb,
-                                           double* red) {
-    if (threadIdx.x < 64) vb[threadIdx.x] = bc[threadIdx.x];
-    __syncthreads();
+// sum_k M(e, k) y_k over a 64x64 block M (element (e, k) at M[e + k ld]), e < 64 in
+// threads t < 64; red: kPanelThreads doubles of LDS.  Ends with a barrier.
+__device__ __forceinline__ double blk_matvec(const double* M, int64_t ld, const double* y, double* red) {
     const int e = threadIdx.x & 63, pq = threadIdx.x >> 6;
     double sum = 0.0;
 #pragma unroll
-    for (int u = 0; u < 16; ++u) sum += S[16 * pq + u][e] * vb[16 * pq + u];
+    for (int u = 0; u < 8; ++u) sum += M[e + (int64_t)(8 * pq + u) * ld] * y[8 * pq + u];
     red[threadIdx.x] = sum;
     __syncthreads();
-    if (threadIdx.x < 64) brb[e] -= red[e] + red[e + 64] + red[e + 128] + red[e + 192];
+    sum = 0.0;
+    if (threadIdx.x < 64)
+#pragma unroll
+        for (int q = 0; q < 8; ++q) sum += red[e + 64 * q];
     __syncthreads();
+    return sum;
 }
 
-//
-// T = float (the mixed-precision form): A is FP32; Dacc holds FP64 copies of
-// the diagonal tiles (64x64 column-major, tile j at Dacc + 4096j), which the
-// diagonal factor reads instead of A's tiles and which receive the updates of
-// the diagonal blocks.  Block products are FP64 MFMA on the stored FP32 values
-// (exact products, FP64 sums) with one rounding to FP32 per stored result.
-template <typename T>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_potrf_panel(
-    T* __restrict__ A, int64_t ld, int64_t K0, int nc,
-                                                     double* __restrict__ Dinv, double* __restrict__ ldiag,
-                                                     int* __restrict__ info, unsigned* __restrict__ sync,
-                                                     unsigned epoch, unsigned base, double* __restrict__ Dacc,
-                                                     unsigned maxpoll, double* __restrict__ rhs) {
-    __shared__ double Ps[64][65];
-    __shared__ double Qs[64][65];
+// The lower 16x16 tiles of a 64x64 block over eight waves: tile u of wave w (two
+// tiles for waves 0 and 1) is (row, column) (diag_rt, diag_ct).
+__device__ __forceinline__ int diag_rt(int w, int u) { return u ? 3 : w < 1 ? 0 : w < 3 ? 1 : w < 6 ? 2 : 3; }
+__device__ __forceinline__ int diag_ct(int w, int u) { return u ? 2 + w : w < 1 ? 0 : w < 3 ? w - 1 : w < 6 ? w - 3 : w - 6; }
+
+template <typename T, int NC>
+__global__ __launch_bounds__(kPanelThreads) void k_potrf_panel(
+    T* A, int64_t ld, int64_t K0, int nc, double* Dinv, double* __restrict__ ldiag, int* __restrict__ info,
+    unsigned* __restrict__ sync, unsigned epoch, unsigned base, double* Dpub,
+    unsigned maxpoll, double* rhs) {
+    constexpr bool kF64 = sizeof(T) == 8;
+    constexpr int P = kPanelMaxBlocks;
+    __shared__ double S[64][kTP];
     __shared__ double rinv[64];
     __shared__ double piv[64];
-    __shared__ double red[256];
-    __shared__ double vb[64];
+    __shared__ double red[kPanelThreads];
     __shared__ unsigned s_id;
     __shared__ int s_ok;
-    __shared__ int s_col;
     if (threadIdx.x == 0) s_id = atomicAdd(&sync[kPanelSyncWords - 1], 1u) - base;
     __syncthreads();
-    const int rb = (int)s_id;
+    const int rb = __builtin_amdgcn_readfirstlane((int)s_id);
+    unsigned* const yflag = sync + P + P * P;
+    unsigned* const readers = yflag + P;
+    const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int li = lane & 15, g = lane >> 4, r64 = t & 63;
     const int64_t kb0 = K0 / 64;
-    T* Arow = A + K0 + 64 * (int64_t)rb;  // row block rb, column 0
-    // kNext: the owner of the next diagonal block keeps that block's last
-    // update in LDS (below).  FP64 storage only: with FP32 storage the
-    // registers it takes cost more than it saves (mixed-precision fits
-    // measured 10 % slower).
-    constexpr bool kNext = sizeof(T) == 8;
-    for (int c = 0; c < nc && c < rb; ++c) {
-        const int64_t kc = kb0 + c;
-        T* Ab = Arow + (K0 + 64 * c) * ld;  // A_{rb,c}
-        if (kNext && rb == c + 1 && rb < nc) {
-            // This workgroup factors diagonal block c + 1 next, and its only update
-            // left is that block's own.  A_{rb,c} and the diagonal block are
-            // final before the wait (their updates are this workgroup's own
-            // stores, made before the barriers since) and are staged into Ps
-            // and Qs while it waits; the solve reads Dinv_c straight from
-            // global memory, the update is subtracted in LDS, and the factor
-            // starts from Qs (FP64).  L_{rb,c} is published after the update
-            // (its stores have landed by then).
-            blk_load(Ps, Ab, ld);
-            blk_load(Qs, A + (kb0 + rb) * 64 * (ld + 1), ld);
-            if (!panel_wait(&sync[c], epoch, info, &s_ok, maxpoll)) return;
-            blk_mm_nt<true, false>(Ps, Ps, Ps, Dinv + kc * 4096);  // Ps[j][r] = L_{rb,c}(r, j)
-            blk_store(Ab, ld, Ps);
-            __syncthreads();
-            if (rhs) rhs_update(rhs + K0 + 64 * c, rhs + K0 + 64 * rb, Ps, vb, red);
-            blk_mm_nt<false, true>(Ps, Ps, Qs);  // Qs -= L_{rb,c} L_{rb,c}^T
-            panel_publish(&sync[kPanelMaxBlocks + kPanelMaxBlocks * rb + c], epoch);
-            continue;
+    T* const A0 = A + K0 + K0 * ld;           // the panel's first block
+    T* const Arow = A0 + 64 * (int64_t)rb;    // row block rb, column 0
+    if (!kF64) Dpub += kb0 * 4096;
+    // what column block c is solved with: FP64 storage, the diagonal block as
+    // published (block 0 is read from A); FP32 storage, its inverse
+    double dv[8];
+    auto diag_fetch = [&](int c) {
+        const bool ina = kF64 && c == 0;
+        const double* D = ina ? (const double*)A0 : kF64 ? Dpub + 4096 * c : Dinv + 4096 * (kb0 + c);
+        const int64_t ldd = ina ? ld : 64;
+#pragma unroll
+        for (int q = 0; q < 8; ++q) dv[q] = D[r64 + (int64_t)(w + 8 * q) * ldd];
+    };
+    auto diag_put = [&]() {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) S[w + 8 * q][r64] = dv[q];
+    };
+    // the last workgroup to report copies block 0's factor into A
+    auto report_read = [&]() {
+        if (!kF64) {  // (nothing is held back; the counter advances with the tickets)
+            if (t == 0) atomicAdd(readers, 1u);
+            return;
         }
-        // A_{rb,c} is final before the wait: its updates are this workgroup's own
-        // stores, made by the same threads (the blk_sub layout)
-        T pre[16];
-        blk_fetch(pre, Ab, ld);
-        if (!panel_wait(&sync[c], epoch, info, &s_ok, maxpoll)) return;
-        blk_load(Qs, Dinv + kc * 4096, 64);
-        blk_put(Ps, pre);
         __syncthreads();
-        blk_mm_nt(Ps, Qs, Ps);  // Ps[j][r] = L_{rb,c}(r, j)
-        blk_store(Ab, ld, Ps);  // (Ps now holds the stored values)
+        if (t == 0) {
+            const unsigned n = __hip_atomic_fetch_add(readers, 1u, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT) - base;
+            s_ok = n + 1 == gridDim.x;
+        }
         __syncthreads();
-        if (rhs) rhs_update(rhs + K0 + 64 * c, rhs + K0 + 64 * rb, Ps, vb, red);
-        if (rb < nc) panel_publish(&sync[kPanelMaxBlocks + kPanelMaxBlocks * rb + c], epoch);
-        for (int c2 = c + 1; c2 < nc && c2 <= rb; ++c2) {
-            if (c2 == rb) {
-                blk_mm_nt(Ps, Ps, Qs);  // the block's own diagonal block
-            } else {
-                if (!panel_wait(&sync[kPanelMaxBlocks + kPanelMaxBlocks * c2 + c], epoch, info, &s_ok, maxpoll)) return;
-                blk_load(Qs, A + K0 + 64 * c2 + (K0 + 64 * c) * ld, ld);  // L_{c2,c}
-                __syncthreads();
-                blk_mm_nt(Ps, Qs, Qs);
+        if (s_ok) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+#pragma unroll
+            for (int q = 0; q < 8; ++q) A0[r64 + (int64_t)(w + 8 * q) * ld] = (T)Dpub[r64 + 64 * (w + 8 * q)];
+        }
+    };
+    const int cend = rb < nc ? rb : nc;  // columns left of the own diagonal block
+    // The own blocks of columns c + 1 .. c + NC - 1 stay in registers as transposed
+    // 16x16 MFMA tiles until their column is reached: wave w has rows 16(w%4)..,
+    // columns 32(w/4).. of each (two tiles).  (Read and written back in global
+    // memory on every step, an update took 4 us against 1.7 us of products.)
+    const int r0 = 16 * (w & 3) + li, q0 = 32 * (w >> 2);
+    T own[NC - 1][2][4];
+    d4 dacc[2];
+    if (rb > 0) {
+#pragma unroll
+        for (int q = 0; q < 8; ++q) S[w + 8 * q][64 + r64] = (double)Arow[r64 + (int64_t)(w + 8 * q) * ld];
+        if (kF64) {
+            diag_fetch(0);
+            diag_put();
+        }
+#pragma unroll
+        for (int i = 0; i < NC - 1; ++i)
+            if (i + 1 < cend)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        own[i][j][v] = Arow[r0 + (int64_t)(64 * (i + 1) + q0 + 16 * j + g + 4 * v) * ld];
+        if (rb < nc) {  // the own diagonal block's lower tiles
+            const double* D = kF64 ? (const double*)(Arow + 64 * (int64_t)rb * ld) : Dpub + 4096 * rb;
+            const int64_t ldd = kF64 ? ld : 64;
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+                if (u < 1 || w < 2)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        dacc[u][v] = D[(16 * diag_rt(w, u) + li) + (int64_t)(16 * diag_ct(w, u) + g + 4 * v) * ldd];
+        }
+        report_read();
+        if (!kF64) {
+            if (!panel_wait(&sync[0], epoch, info, &s_ok, maxpoll)) return;
+            diag_fetch(0);
+            diag_put();
+        }
+    }
+#pragma unroll 1
+    for (int c = 0; c < cend; ++c) {
+        __syncthreads();
+        if constexpr (kF64) {
+            trapezoid_factor<8, true, false>(S, piv, rinv);
+        } else {
+            // L_{rb,c} = A_{rb,c} Dinv_c^T
+            d4 acc[2] = {d4{0.0, 0.0, 0.0, 0.0}, d4{0.0, 0.0, 0.0, 0.0}};
+#pragma unroll 8
+            for (int k0 = 0; k0 < 64; k0 += 4) {
+                const double b = S[k0 + g][64 + r0];
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+                    acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(S[k0 + g][q0 + 16 * j + li], b, acc[j], 0, 0, 0);
             }
-            if (Dacc && c2 == rb)
-                blk_sub(Dacc + (kb0 + c2) * 4096, 64, Qs);  // the FP64 copy the diagonal factor reads
-            else
-                blk_sub(Arow + (K0 + 64 * c2) * ld, ld, Qs);
             __syncthreads();
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) S[q0 + 16 * j + g + 4 * v][64 + r0] = acc[j][v];
+            __syncthreads();
+        }
+        // L_{rb,c} to global memory, rounded to T; LDS keeps the stored values
+        {
+            T* Ab = Arow + 64 * (int64_t)c * ld;
+#pragma unroll
+            for (int q = 0; q < 8; ++q) {
+                const T v = (T)S[w + 8 * q][64 + r64];
+                if (rb < nc) put_shared(Ab + r64 + (int64_t)(w + 8 * q) * ld, v);
+                else Ab[r64 + (int64_t)(w + 8 * q) * ld] = v;
+                if (!kF64) S[w + 8 * q][64 + r64] = (double)v;
+            }
+            if (!kF64) __syncthreads();
+        }
+        if (rb < nc) panel_publish(&sync[P + P * rb + c], epoch);
+        // the own diagonal block: D -= L_{rb,c} L_{rb,c}^T, lower tiles (here and
+        // below FP32 storage sums the products first, as its results always were)
+        auto diag_update = [&]() {
+            d4 old[2];
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                old[u] = dacc[u];
+                if (!kF64) dacc[u] = d4{0.0, 0.0, 0.0, 0.0};
+            }
+#pragma unroll 8
+            for (int k0 = 0; k0 < 64; k0 += 4) {
+                const double* Sk = &S[k0 + g][64 + li];
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+                    if (u < 1 || w < 2) {
+                        const double a = Sk[16 * diag_ct(w, u)];
+                        dacc[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(kF64 ? -a : a, Sk[16 * diag_rt(w, u)], dacc[u],
+                                                                       0, 0, 0);
+                    }
+            }
+            if (!kF64)
+#pragma unroll
+                for (int u = 0; u < 2; ++u) dacc[u] = old[u] - dacc[u];
+        };
+        if (rb == c + 1 && rb < nc) {
+            // the next diagonal block: published before it is factored
+            diag_update();
+            double* D = Dpub + 4096 * rb;
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+                if (u < 1 || w < 2)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) {
+                        const int row = 16 * diag_rt(w, u) + li, col = 16 * diag_ct(w, u) + g + 4 * v;
+                        if (kF64) put_shared(D + row + 64 * col, (double)dacc[u][v]);
+                        S[col][row] = dacc[u][v];
+                    }
+            if (kF64) panel_publish(&sync[rb], epoch);
+        }
+        // The own blocks of the later panel columns, nearest last: its result
+        // goes to LDS as the next step's block.  One wait for all of them; the
+        // next L_{c2,c} is loaded while the current one is multiplied.
+        if (cend - 1 > c) {
+            if (!panel_wait_all(sync + P + c, P, c + 1, cend, epoch, info, &s_ok, maxpoll)) return;
+            T lv[8];
+            auto fetch = [&](int c2) {
+                const T* Lc2 = A0 + 64 * (int64_t)c2 + 64 * (int64_t)c * ld;
+#pragma unroll
+                for (int q = 0; q < 8; ++q) lv[q] = Lc2[r64 + (int64_t)(w + 8 * q) * ld];
+            };
+            fetch(cend - 1);
+#pragma unroll
+            for (int i = NC - 2; i >= 0; --i) {
+                const int c2 = c + 1 + i;
+                if (c2 >= cend) continue;
+#pragma unroll
+                for (int q = 0; q < 8; ++q) S[w + 8 * q][r64] = (double)lv[q];
+                __syncthreads();
+                if (i > 0) fetch(c2 - 1);
+                d4 acc[2];
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) acc[j][v] = kF64 ? (double)own[i][j][v] : 0.0;
+#pragma unroll 8
+                for (int k0 = 0; k0 < 64; k0 += 4) {
+                    const double b = S[k0 + g][64 + r0];
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) {
+                        const double a = S[k0 + g][q0 + 16 * j + li];
+                        acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(kF64 ? -a : a, b, acc[j], 0, 0, 0);
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        own[i][j][v] = kF64 ? (T)acc[j][v] : (T)((double)own[i][j][v] - acc[j][v]);
+                if (i > 0) __syncthreads();  // the operand is free
+            }
+        }
+        if (c + 1 < cend) {
+            // the next diagonal block (published long before this workgroup gets
+            // here, unless it is the next but one): its load is covered by the
+            // update of the own diagonal block
+            if (!panel_wait(&sync[c + 1], epoch, info, &s_ok, maxpoll)) return;
+            diag_fetch(c + 1);
+            if (rb < nc) diag_update();
+            __syncthreads();  // S is no longer read
+            diag_put();
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) S[q0 + 16 * j + g + 4 * v][64 + r0] = (double)own[0][j][v];
+#pragma unroll
+            for (int i = 0; i + 1 < NC - 1; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) own[i][j][v] = own[i + 1][j][v];
+        }
+        if (rhs && c > 0) {
+            if (!panel_wait(&yflag[c - 1], epoch, info, &s_ok, maxpoll)) return;
+            const double u = blk_matvec((const double*)(Arow + 64 * (int64_t)(c - 1) * ld), ld, rhs + K0 + 64 * (c - 1), red);
+            if (t < 64) rhs[K0 + 64 * (int64_t)rb + t] -= u;
         }
     }
     if (rb < nc) {
-        // diagonal block rb with all its updates; with kNext in Qs: left there
-        // by the last column (rb > 0), or the stored block (no updates inside
-        // the panel)
-        const int c = rb;
-        const int64_t kc = kb0 + c;
-        if (kNext && rb == 0) {
-            blk_load(Qs, A + kc * 64 * (ld + 1), ld);
-            __syncthreads();
-        }
-        diag_block64<T, true, kNext>(A, ld, kc, Dinv, ldiag, info, 1, Dacc ? Dacc + kc * 4096 : nullptr, Ps, Qs, rinv,
-                                     piv, &s_col);
-        if (rhs) {  // y_c = L_cc^-1 b_c from the inverse left in Qs (Qs[k][e] = X(e, k))
-            double* bc = rhs + K0 + 64 * c;
-            if (threadIdx.x < 64) vb[threadIdx.x] = bc[threadIdx.x];
-            __syncthreads();
-            const int e = threadIdx.x & 63, pq = threadIdx.x >> 6;
-            double sum = 0.0;
+        // diagonal block rb with all its updates: in S (left there by the last
+        // column), or for rb = 0 as stored
+        const int64_t kc = kb0 + rb;
+        if (rb == 0) {
+            if (kF64) {
+                diag_fetch(0);
+                diag_put();
+            } else {
 #pragma unroll
-            for (int u = 0; u < 16; ++u) sum += Qs[16 * pq + u][e] * vb[16 * pq + u];
-            red[threadIdx.x] = sum;
-            __syncthreads();
-            if (threadIdx.x < 64) bc[threadIdx.x] = red[e] + red[e + 64] + red[e + 128] + red[e + 192];
+                for (int q = 0; q < 8; ++q) S[w + 8 * q][r64] = Dpub[r64 + 64 * (w + 8 * q)];
+            }
         }
-        panel_publish(&sync[c], epoch);
+        __syncthreads();
+        trapezoid_factor<4, kF64, false>(S, piv, rinv);
+        const bool hold = kF64 && rb == 0;  // A's block 0 may still be read
+        diag_finish<T, !kF64>(hold ? (T*)Dpub : Arow + 64 * (int64_t)rb * ld, hold ? 64 : ld, kc, Dinv, ldiag, info, S,
+                              rinv, piv);
+        if (!kF64) panel_publish(&sync[rb], epoch);
+        if (rb == 0) {
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+            report_read();
+        }
+        if (rhs) {  // y_c = L_cc^-1 b_c from the inverse left in S
+            double* bc = rhs + K0 + 64 * (int64_t)rb;
+            if (rb > 0) {
+                if (!panel_wait(&yflag[rb - 1], epoch, info, &s_ok, maxpoll)) return;
+                const double u = blk_matvec((const double*)(Arow + 64 * (int64_t)(rb - 1) * ld), ld, bc - 64, red);
+                if (t < 64) bc[t] -= u;
+                __syncthreads();
+            }
+            const double y = blk_matvec(&S[0][64], kTP, bc, red);
+            if (t < 64) put_shared(bc + t, y);
+            panel_publish(&yflag[rb], epoch);
+        }
+    } else if (rhs) {
+        if (!panel_wait(&yflag[nc - 1], epoch, info, &s_ok, maxpoll)) return;
+        const double u = blk_matvec((const double*)(Arow + 64 * (int64_t)(nc - 1) * ld), ld, rhs + K0 + 64 * (nc - 1), red);
+        if (t < 64) rhs[K0 + 64 * (int64_t)rb + t] -= u;
     }
 }
 
 void potrf_panel_f64(hipStream_t s, double* A, int64_t ld, int64_t K0, int nc, int64_t nrb, double* Dinv,
-                     double* ldiag, int* info, unsigned* sync, unsigned epoch, unsigned base, unsigned maxpoll,
-                     double* rhs) {
-    hipLaunchKernelGGL(k_potrf_panel<double>, dim3((unsigned)nrb), dim3(256), 0, s, A, ld, K0, nc, Dinv, ldiag, info,
-                       sync, epoch, base, (double*)nullptr, maxpoll, rhs);
+                     double* ldiag, int* info, unsigned* sync, unsigned epoch, unsigned base, double* Dpub,
+                     unsigned maxpoll, double* rhs) {
+    hipLaunchKernelGGL((k_potrf_panel<double, kPanelBlocksF64>), dim3((unsigned)nrb), dim3(kPanelThreads), 0, s, A, ld, K0, nc, Dinv, ldiag, info,
+                       sync, epoch, base, Dpub, maxpoll, rhs);
 }
 
 void potrf_panel_mixed(hipStream_t s, float* A, int64_t ld, int64_t K0, int nc, int64_t nrb, double* Dinv,
                        double* ldiag, int* info, unsigned* sync, unsigned epoch, unsigned base, double* Dacc,
                        unsigned maxpoll) {
-    hipLaunchKernelGGL(k_potrf_panel<float>, dim3((unsigned)nrb), dim3(256), 0, s, A, ld, K0, nc, Dinv, ldiag, info,
+    hipLaunchKernelGGL((k_potrf_panel<float, kPanelBlocksF32>), dim3((unsigned)nrb), dim3(kPanelThreads), 0, s, A, ld, K0, nc, Dinv, ldiag, info,
                        sync, epoch, base, Dacc, maxpoll, (double*)nullptr);
-}
-
-void potrf_diag3_f64(hipStream_t s, double* A, int64_t ld, int64_t k, double* Dinv, double* ldiag, int* info,
-                     int want_inv) {
-    hipLaunchKernelGGL(k_potrf_diag3<double>, dim3(1), dim3(256), 0, s, A, ld, k, Dinv, ldiag, info, want_inv,
-                       (int64_t)0, (int64_t)0, (int64_t)0, (const double*)nullptr);
-}
-
-void potrf_diag3_f32(hipStream_t s, float* A, int64_t ld, int64_t k, double* Dinv, double* ldiag, int* info,
-                     int want_inv, const double* Dacc) {
-    hipLaunchKernelGGL(k_potrf_diag3<float>, dim3(1), dim3(256), 0, s, A, ld, k, Dinv, ldiag, info, want_inv,
-                       (int64_t)0, (int64_t)0, (int64_t)0, Dacc);
-}
-
-// batch of problems, each with its own info slot (info[b])
-void potrf_diag3_f32_batched(hipStream_t s, float* A, int64_t ld, int64_t k, double* Dinv, double* ldiag, int* info,
-                             int batch, int64_t sA, int64_t sD, int64_t sL, const double* Dacc) {
-    hipLaunchKernelGGL(k_potrf_diag3<float>, dim3((unsigned)batch), dim3(256), 0, s, A, ld, k, Dinv, ldiag, info, 1,
-                       sA, sD, sL, Dacc);
 }
 
 // ---------------------------------------------------------------------------
@@ -1045,7 +1190,7 @@ __global__ __launch_bounds__(256) void k_trsv_persist(const double* __restrict__
     for (int u = 0; u < 16; ++u) s += dv[u] * sv[16 * p + u];
     red[t] = s;
     __syncthreads();
-    if (t < 64) x[64 * i + t] = red[t] + red[t + 64] + red[t + 128] + red[t + 192];
+    if (t < 64) put_shared(x + 64 * i + t, red[t] + red[t + 64] + red[t + 128] + red[t + 192]);
     panel_publish(&sync[i], epoch);
 }
 
@@ -1497,7 +1642,7 @@ void restore_factor_f64(hipStream_t s, double* L, int64_t n, int64_t N, const do
 }
 
 // Inverses of the 64x64 diagonal blocks of an existing lower-triangular factor
-// (the part of k_potrf_diag3 that follows the factorisation): Dinv + k*4096
+// (what diag_finish does after the factorisation): Dinv + k*4096
 // receives L_kk^-1 (column-major, ld 64, zeros above the diagonal) and
 // ldiag[64k + i] = log L_ii.  Lane t forward-substitutes column t.  A pivot
 // that is not positive (or NaN) sets info to its 1-based index if info is 0.

@@ -105,12 +105,6 @@ void trmv_lower_f32(hipStream_t s, const float* X, int64_t ld, int64_t N, const 
                     double* part, int nchunk);
 void colsumsq_f32(hipStream_t s, const float* A, int64_t ld, int64_t nrow, int64_t ncol, double* out, int lower);
 void rel_maxabs(hipStream_t s, const double* d, const double* u, int64_t n, double* out);
-// Factor the 64x64 diagonal block at A + k*64*(ld+1) in place (FP64 arithmetic); write its
-// inverse to Dinv + k*64*64 (FP64) and log(L_ii) to ldiag + k*64; info = first failing row + 1.
-void potrf_diag3_f64(hipStream_t s, double* A, int64_t ld, int64_t k, double* Dinv, double* ldiag, int* info,
-                     int want_inv);
-void potrf_diag3_f32(hipStream_t s, float* A, int64_t ld, int64_t k, double* Dinv, double* ldiag, int* info,
-                     int want_inv, const double* Dacc);
 // D_j -= P_j P_j^T in FP64 for ntiles consecutive diagonal tiles (FP32 panel P)
 void dacc_update(hipStream_t s, double* D, const float* P, int64_t ldp, int64_t ntiles, int64_t kdepth, int batch,
                  int64_t sD, int64_t sP);
@@ -148,17 +142,18 @@ void set_identity_f64(hipStream_t s, double* A, int64_t ld, int64_t N);
 // info value a panel factorisation stores when one of its device waits timed out
 constexpr int kPanelWaitTimeout = 0x7fffffff;
 // the single-launch panel: at most this many 64-column blocks, and its flag words
-constexpr int kPanelMaxBlocks = 16;
-constexpr int kPanelSyncWords = kPanelMaxBlocks + kPanelMaxBlocks * kPanelMaxBlocks + 1;
+constexpr int kPanelMaxBlocks = 8;
+constexpr int kPanelBlocksF64 = 4, kPanelBlocksF32 = 8;
+constexpr int kPanelSyncWords = 2 * kPanelMaxBlocks + kPanelMaxBlocks * kPanelMaxBlocks + 2;
 // one outer panel (nc <= kPanelMaxBlocks column blocks from column K0, nrb = (ld - K0) / 64
 // row blocks) of the FP64 blocked Cholesky in one launch; sync: kPanelSyncWords words
 // of the context (zero at creation), epoch: nonzero and new for every launch, base:
 // tickets handed out before (nrb per launch), maxpoll: polls before a wait
-// between workgroups gives up (kPanelWaitTimeout in info), rhs (optional): a
-// vector carried through the forward solve (leaves as L^-1 rhs on the panel's rows)
+// between workgroups gives up (kPanelWaitTimeout in info), Dpub: workspace of
+// kPanelMaxBlocks 64x64 blocks, rhs (optional): a vector carried through the forward solve (leaves as L^-1 rhs on the panel's rows)
 void potrf_panel_f64(hipStream_t s, double* A, int64_t ld, int64_t K0, int nc, int64_t nrb, double* Dinv,
-                     double* ldiag, int* info, unsigned* sync, unsigned epoch, unsigned base, unsigned maxpoll,
-                     double* rhs);
+                     double* ldiag, int* info, unsigned* sync, unsigned epoch, unsigned base, double* Dpub,
+                     unsigned maxpoll, double* rhs);
 // the blocked solves of trsv_lower_f64 (N / 64 <= kSolveMaxBlocks) in one launch
 // (b is left unchanged); sync: kSolveSyncWords words of the context (zero at
 // creation), epoch, base (N / 64 tickets per launch) and maxpoll as for the panel
@@ -294,7 +289,10 @@ void gemm_mixed_f32f64_batched(hipStream_t s, int ta, int tb, int64_t M, int64_t
 void gemm_mixed_f64f32_batched(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha,
                                const double* A, int64_t lda, const float* B, int64_t ldb, double beta, float* C,
                                int64_t ldc, int tiles, int batch, int64_t sA, int64_t sB, int64_t sC);
-void potrf_diag3_f32_batched(hipStream_t s, float* A, int64_t ld, int64_t k, double* Dinv, double* ldiag, int* info,
+// Factor the 64x64 diagonal block at A + k*64*(ld+1) of every problem from its FP64 tile
+// Dacc + k*64*64; its inverse goes to Dinv + k*64*64 (FP64), log(L_ii) to ldiag + k*64,
+// the first failing row + 1 to info[problem].
+void potrf_diag_f32_batched(hipStream_t s, float* A, int64_t ld, int64_t k, double* Dinv, double* ldiag, int* info,
                              int batch, int64_t sA, int64_t sD, int64_t sL, const double* Dacc);
 void set_identity_f32_batched(hipStream_t s, float* A, int64_t ld, int64_t N, int batch, int64_t sA);
 void trmv_lower_f32_batched(hipStream_t s, const float* X, int64_t ld, int64_t N, const double* b, double* y,

@@ -103,6 +103,7 @@ struct gpl_ctx {
     // environment variable GPL_PANEL_WAIT_POLLS overrides it, which tests use to
     // reach the timeout path)
     unsigned* psync = nullptr;
+    double* dpub = nullptr;  // its published diagonal blocks (kPanelMaxBlocks 64x64 blocks)
     unsigned pepoch = 0, pbase = 0;
     // the same for the single-launch triangular solve (kSolveSyncWords words; its
     // launches take their epochs from pepoch too)
