@@ -291,7 +291,7 @@ static void dbl_leaves(hipStream_t s, float* X, int64_t N, const double* Dinv, i
 }
 static void dbl_gemm(hipStream_t s, int64_t M, int64_t Nn, int64_t K, double alpha, const double* A, const double* B,
                      double* C, int64_t ld, int tiles, int64_t batch, int64_t step, double beta = 0.0) {
-    if (batch == 1) gemm2_f64(s, 0, 0, M, Nn, K, alpha, A, ld, B, ld, beta, C, ld, tiles, 0);
+    if (batch == 1) gemm2_f64(s, 0, 0, M, Nn, K, alpha, A, ld, B, ld, beta, C, ld, tiles);
     else gemm2_f64_batched(s, 0, 0, M, Nn, K, alpha, A, ld, B, ld, beta, C, ld, tiles, (int)batch, step, step, step);
 }
 static void dbl_gemm(hipStream_t s, int64_t M, int64_t Nn, int64_t K, double alpha, const float* A, const float* B,
@@ -440,7 +440,7 @@ static void potrf_panel(gpl_ctx* c, hipStream_t st, double* L, int64_t N, int64_
         if (k1 < K0 + W) {
             Prof p(c, "syrk_update", 2.0 * (N - k1) * (K0 + W - k1) * w, 0, st);
             const double* Q = L + k1 + k0 * N;
-            gemm2_f64(st, 0, 1, N - k1, K0 + W - k1, w, -1.0, Q, N, Q, N, 1.0, L + k1 * (N + 1), N, 0, 0);
+            gemm2_f64(st, 0, 1, N - k1, K0 + W - k1, w, -1.0, Q, N, Q, N, 1.0, L + k1 * (N + 1), N, 0);
         }
     }
 }
@@ -467,7 +467,7 @@ void gpl::potrf_blocked(gpl_ctx* c, double* L, int64_t N, double* Dinv, double* 
         const double* P = L + K1 + K0 * N;  // rows >= K1 of the factored panel
         {
             Prof p(c, "syrk_update", 2.0 * R * W1 * W, 8.0 * (2.0 * R * W1 + R * W), s);
-            gemm2_f64(s, 0, 1, R, W1, W, -1.0, P, N, P, N, 1.0, L + K1 * (N + 1), N, 0, 0);
+            gemm2_f64(s, 0, 1, R, W1, W, -1.0, P, N, P, N, 1.0, L + K1 * (N + 1), N, 0);
         }
         hipEventRecord(c->ev_a, s);
         potrf_panel(c, s, L, N, K1, W1, Dinv, ldiag, info, rhs);
@@ -478,7 +478,7 @@ void gpl::potrf_blocked(gpl_ctx* c, double* L, int64_t N, double* Dinv, double* 
             const double* P2 = L + (K1 + W1) + K0 * N;
             {
                 Prof p(c, "syrk_update", (double)R2 * R2 * W, 8.0 * ((double)R2 * R2 + 2.0 * R2 * W), s2);
-                gemm2_f64(s2, 0, 1, R2, R2, W, -1.0, P2, N, P2, N, 1.0, L + (K1 + W1) * (N + 1), N, 1, 0);
+                gemm2_f64(s2, 0, 1, R2, R2, W, -1.0, P2, N, P2, N, 1.0, L + (K1 + W1) * (N + 1), N, 1);
             }
             hipEventRecord(c->ev_p, s2);
             hipStreamWaitEvent(s, c->ev_p, 0);
@@ -494,12 +494,12 @@ static void trtri_panel(gpl_ctx* c, hipStream_t st, const double* L, const doubl
         const int64_t i = r0 / 64, Wc = r0 + 64;  // columns 0 .. r0+63 are non-zero
         {
             Prof p(c, "trtri_diag", 2.0 * 64 * 64 * Wc, 16.0 * 64 * Wc, st);
-            gemm2_f64(st, 0, 0, 64, Wc, 64, 1.0, Dinv + i * 64 * 64, 64, X + r0, N, 0.0, X + r0, N, 0, 0);
+            gemm2_f64(st, 0, 0, 64, Wc, 64, 1.0, Dinv + i * 64 * 64, 64, X + r0, N, 0.0, X + r0, N, 0);
         }
         const int64_t Mr = I0 + H - (r0 + 64);
         if (Mr > 0) {
             Prof p(c, "trtri_panel", 2.0 * Mr * Wc * 64, 16.0 * Mr * Wc, st);
-            gemm2_f64(st, 0, 0, Mr, Wc, 64, -1.0, L + (r0 + 64) + r0 * N, N, X + r0, N, 1.0, X + r0 + 64, N, 0, 0);
+            gemm2_f64(st, 0, 0, Mr, Wc, 64, -1.0, L + (r0 + 64) + r0 * N, N, X + r0, N, 1.0, X + r0 + 64, N, 0);
         }
     }
 }
@@ -524,7 +524,7 @@ void gpl::trtri_blocked(gpl_ctx* c, const double* L, const double* Dinv, int64_t
         const int64_t Wc = I0 + H;
         {
             Prof p(c, "trtri_update", 2.0 * H1 * Wc * H, 8.0 * (2.0 * H1 * Wc + Wc * H), s);
-            gemm2_f64(s, 0, 0, H1, Wc, H, -1.0, L + I1 + I0 * N, N, X + I0, N, 1.0, X + I1, N, 0, 0);
+            gemm2_f64(s, 0, 0, H1, Wc, H, -1.0, L + I1 + I0 * N, N, X + I0, N, 1.0, X + I1, N, 0);
         }
         hipEventRecord(c->ev_a, s);
         hipStreamWaitEvent(s2, c->ev_a, 0);
@@ -533,7 +533,7 @@ void gpl::trtri_blocked(gpl_ctx* c, const double* L, const double* Dinv, int64_t
         const int64_t R2 = R - H1;
         if (R2 > 0) {
             Prof p(c, "trtri_update", 2.0 * R2 * Wc * H, 8.0 * (2.0 * R2 * Wc + Wc * H), s);
-            gemm2_f64(s, 0, 0, R2, Wc, H, -1.0, L + (I1 + H1) + I0 * N, N, X + I0, N, 1.0, X + I1 + H1, N, 0, 0);
+            gemm2_f64(s, 0, 0, R2, Wc, H, -1.0, L + (I1 + H1) + I0 * N, N, X + I0, N, 1.0, X + I1 + H1, N, 0);
         }
         hipStreamWaitEvent(s, c->ev_p, 0);
     }
@@ -1526,7 +1526,7 @@ static int energy_grad_latent(gpl_model* m, double* grad) {
     double* Bi = m->d(B_BINV);
     {
         Prof p(c, "lauum", (double)N * N * N / 3, 8.0 * N * N);
-        gemm2_f64(s, 1, 0, N, N, N, 1.0, m->d(B_XINV), N, m->d(B_XINV), N, 0.0, Bi, N, 2, 0);
+        gemm2_f64(s, 1, 0, N, N, N, 1.0, m->d(B_XINV), N, m->d(B_XINV), N, 0.0, Bi, N, 2);
     }
     const double* sv = m->d(B_SV);
     double *u = nullptr, *t = nullptr;
@@ -1603,7 +1603,7 @@ extern "C" int gpl_energy_grad(gpl_model* m, double* grad) {
         }
         {
             Prof p(c, "lauum", (double)N * N * N / 3, 8.0 * N * N);
-            gemm2_f64(s, 1, 0, N, N, N, 1.0, m->d(B_XINV), N, m->d(B_XINV), N, 0.0, m->d(B_BINV), N, 2, 0);
+            gemm2_f64(s, 1, 0, N, N, N, 1.0, m->d(B_XINV), N, m->d(B_XINV), N, 0.0, m->d(B_BINV), N, 2);
         }
         Prof p(c, "grad", 0, 8.0 * N * (N + 64) / 2);
         launch_grad_tiles(s, m->b[B_PROG].as<DevProg>(), m->prog, m->d(B_F), n, N, m->d(B_BINV), N, 1.0 / s2,
@@ -1735,20 +1735,20 @@ int gpl::pred_on(gpl_ctx* c, gpl_model* m, const double* xt, int64_t mt, int32_t
             if (m->opts.precision == GPL_PREC_MIXED)
                 gemm_mixed_f32f64f64(s, 0, 0, N, M, N, 1.0, m->b[B_XINV].as<float>(), N, KtT, N, 0.0, A2, N, 3);
             else
-                gemm2_f64(s, 0, 0, N, M, N, 1.0, m->d(B_XINV), N, KtT, N, 0.0, A2, N, 3, 0);
+                gemm2_f64(s, 0, 0, N, M, N, 1.0, m->d(B_XINV), N, KtT, N, 0.0, A2, N, 3);
             KtT = A2;
         } else {
             for (int64_t i = 0; i < T; ++i) {
                 {
                     Prof p(c, "pred_trsm_diag", 2.0 * 64 * 64 * M, 16.0 * 64 * M);
                     gemm2_f64(s, 0, 0, 64, M, 64, 1.0, m->d(B_DINV) + i * 64 * 64, 64, KtT + i * 64, N, 0.0,
-                              KtT + i * 64, N, 0, 0);
+                              KtT + i * 64, N, 0);
                 }
                 if (i + 1 < T) {
                     const int64_t R = (T - 1 - i) * 64;
                     Prof p(c, "pred_trsm_update", 2.0 * R * M * 64, 16.0 * R * M);
                     gemm2_f64(s, 0, 0, R, M, 64, -1.0, m->d(B_L) + (i + 1) * 64 + i * 64 * N, N, KtT + i * 64, N,
-                              1.0, KtT + (i + 1) * 64, N, 0, 0);
+                              1.0, KtT + (i + 1) * 64, N, 0);
                 }
             }
         }
@@ -1809,14 +1809,14 @@ static int draw_on(gpl_ctx* c, gpl_model* m, const double* xt, int64_t mt, doubl
         if (m->opts.precision == GPL_PREC_MIXED)
             gemm_mixed_f32f64f64(s, 0, 0, N, M, N, 1.0, m->b[B_XINV].as<float>(), N, KtT, N, 0.0, A2, N, 3);
         else
-            gemm2_f64(s, 0, 0, N, M, N, 1.0, m->d(B_XINV), N, KtT, N, 0.0, A2, N, 3, 0);
+            gemm2_f64(s, 0, 0, N, M, N, 1.0, m->d(B_XINV), N, KtT, N, 0.0, A2, N, 3);
     } else {
         for (int64_t i = 0; i < T; ++i) {
             gemm2_f64(s, 0, 0, 64, M, 64, 1.0, m->d(B_DINV) + i * 64 * 64, 64, KtT + i * 64, N, 0.0, KtT + i * 64, N,
-                      0, 0);
+                      0);
             if (i + 1 < T)
                 gemm2_f64(s, 0, 0, (T - 1 - i) * 64, M, 64, -1.0, m->d(B_L) + (i + 1) * 64 + i * 64 * N, N,
-                          KtT + i * 64, N, 1.0, KtT + (i + 1) * 64, N, 0, 0);
+                          KtT + i * 64, N, 1.0, KtT + (i + 1) * 64, N, 0);
         }
         A2 = KtT;
     }
@@ -1824,7 +1824,7 @@ static int draw_on(gpl_ctx* c, gpl_model* m, const double* xt, int64_t mt, doubl
     launch_build_sym_f64(s, pd, *hp, Ft, mt, M, jitter, 0, 1.0, nullptr, Cv, M);
     {
         Prof p(c, "draw_cov", (double)M * M * N, 8.0 * N * M);
-        gemm2_f64(s, 1, 0, M, M, N, -1.0, A2, N, A2, N, 1.0, Cv, M, 1, 0);
+        gemm2_f64(s, 1, 0, M, M, N, -1.0, A2, N, A2, N, 1.0, Cv, M, 1);
     }
     HIP_TRY(hipMemsetAsync(info, 0, 64, s));
     potrf_blocked(c, Cv, M, Dv, ld, info);
@@ -1835,7 +1835,7 @@ static int draw_on(gpl_ctx* c, gpl_model* m, const double* xt, int64_t mt, doubl
     HIP_TRY(upload_2d(c, s, Zd, M, z, mt, draws, 20));
     {
         Prof p(c, "draw_trmm", (double)M * M * Dp, 8.0 * M * Dp * 2);
-        gemm2_f64(s, 0, 0, M, Dp, M, 1.0, Cv, M, Zd, M, 0.0, Wd, M, 3, 0);
+        gemm2_f64(s, 0, 0, M, Dp, M, 1.0, Cv, M, Zd, M, 0.0, Wd, M, 3);
     }
     std::vector<double> mean(mt);
     HIP_TRY(hipMemcpyAsync(mean.data(), vbuf, mt * 8, hipMemcpyDeviceToHost, s));
@@ -1883,7 +1883,7 @@ extern "C" int gpl_draw_prior(gpl_ctx* c, const gpl_cf_term* terms, int32_t nter
     HIP_TRY(hipMemcpyAsync(&inf, info, 4, hipMemcpyDeviceToHost, s));
     fill_f64(s, Zd, M * Dp, 0.0);
     HIP_TRY(upload_2d(c, s, Zd, M, z, mt, draws, 20));
-    gemm2_f64(s, 0, 0, M, Dp, M, 1.0, Cv, M, Zd, M, 0.0, Wd, M, 3, 0);
+    gemm2_f64(s, 0, 0, M, Dp, M, 1.0, Cv, M, Zd, M, 0.0, Wd, M, 3);
     HIP_TRY(download_2d(c, s, out, Wd, M, mt, draws, 21));
     HIP_TRY(hipStreamSynchronize(s));
     if (inf > 0) {

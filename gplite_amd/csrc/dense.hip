@@ -30,237 +30,269 @@ __device__ __forceinline__ void lower_tile(int64_t t, int64_t& ti, int64_t& tj) 
 }
 
 // ---------------------------------------------------------------------------
-// LDS-staged GEMM: BM x BM output tile per 256-thread workgroup (BM = 128 or 64),
-// 16-wide k chunks double-buffered in LDS as [k][m] (global -> registers for
-// chunk c+1 is issued before the MFMAs of chunk c and written to LDS after
-// them).  Each wave owns a (BM/2)^2 quadrant of v_mfma_f64_16x16x4 blocks.
-// M and N are multiples of 64; a 128 tile whose second half falls outside is
-// masked (zero loads, skipped stores).
+// FP64-compute GEMM, operands straight from global memory to registers.
+//
+// A workgroup of 2 x 2 waves; each wave owns a WT x WT block of C as 16x16 tiles
+// of v_mfma_f64_16x16x4 and loads its own operand fragments, PF - 1 chunks of 16
+// k ahead, into registers: no LDS, no barrier, so a wave never waits for another
+// and the loads of several chunks are in flight while one is multiplied.  The
+// waves of a workgroup share their operands through L1, the workgroups of an XCD
+// through its L2.  (The staged form this replaces, 64x64 or 128x128 tiles double
+// buffered in LDS, took about 1 us per 16-k chunk whatever the size, the load
+// latency and two barriers; measured alone, us staged -> here:
+// 512 x 256 x 256: 20.1 -> 7.1, 1024 x 512 x 512: 35.7 -> 18.5, 4096 x 512 x 512:
+// 60 -> 52, lower 7168, k = 512: 587 -> 507, X^T X at 8192: 3186 -> 2890.)
+//
+// Within a chunk lane (li, g) holds k = 4g + s of step s (s < 4), so an operand
+// that is contiguous in k is read as 32 bytes per lane and whole 128-byte lines
+// per 16 rows; one that is contiguous in m is read as pairs of rows (lane li: rows
+// 2li and 2li + 1, which belong to two tiles).  Sums run over k in one fixed order,
+// whatever the tile.
+// M, N and K are multiples of 64, operand addresses of 16 bytes.
+//
+// INP: C is one of the operands (a solve against a 64x64 inverse).  A workgroup
+// of 64x64 then covers the whole contraction of its rows (A = C, N = 64) or
+// columns (B = C, M = 64), and stores only after all of its waves have read.
 // ---------------------------------------------------------------------------
 template <typename T> struct vec2_of;
 template <> struct vec2_of<double> { typedef double2 type; };
 template <> struct vec2_of<float> { typedef float2 type; };
 
-// LDS tiles are [k][BM + 1]: the odd row stride keeps the eight lanes that
-// write one column's k values on distinct banks.
-template <int BM, int MCONT, typename T, int NT = 256>
-__device__ __forceinline__ void lds_gemm_load(const T* P, int64_t ld, int64_t base, int64_t lim, int64_t k0,
-                                              double2 (&r)[BM * 8 / NT]) {
+// row (column) of a WT-wide block that lane li of tile i holds
+template <bool KC, int NB>
+__device__ __forceinline__ int frag_row(int i, int li) {
+    return (KC || NB == 1) ? 16 * i + li : 32 * (i >> 1) + 2 * li + (i & 1);
+}
+
+// One chunk of an operand: p at the lane's element (its row of tile 0, k = 4g).
+template <bool KC, int NB, typename T>
+__device__ __forceinline__ void frag_load(T (&f)[NB][4], const T* p, int64_t ld) {
     typedef typename vec2_of<T>::type V2;
-    constexpr int AL = BM * 8 / NT;
-    const int t = threadIdx.x;
-    if (MCONT) {  // element (m, k) at P[m + k*ld]: pairs along m, 128-byte rows per 8 lanes
-        const int mp = (t % (BM / 2)) * 2, kq = t / (BM / 2), ks = NT / (BM / 2);
-        const bool ok = base + mp < lim;
+    if (KC) {
 #pragma unroll
-        for (int j = 0; j < AL; ++j) {
-            const int64_t k = k0 + kq + ks * j;
-            if (ok) {
-                const V2 v = *reinterpret_cast<const V2*>(P + base + mp + k * ld);
-                r[j] = double2{(double)v.x, (double)v.y};
-            } else {
-                r[j] = double2{0.0, 0.0};
-            }
+        for (int i = 0; i < NB; ++i) {
+            const V2* q = reinterpret_cast<const V2*>(p + 16 * i * ld);
+            const V2 a = q[0], b = q[1];
+            f[i][0] = a.x;
+            f[i][1] = a.y;
+            f[i][2] = b.x;
+            f[i][3] = b.y;
         }
-    } else {  // element (m, k) at P[k + m*ld]: 8 lanes read one column's 16 k contiguously
-        const int kq = t & 7, m = t >> 3;
+    } else if (NB == 1) {
 #pragma unroll
-        for (int j = 0; j < AL; ++j) {
-            const int64_t mm = base + m + (NT / 8) * j;
-            if (mm < lim) {
-                const V2 v = *reinterpret_cast<const V2*>(P + (k0 + 2 * kq) + mm * ld);
-                r[j] = double2{(double)v.x, (double)v.y};
-            } else {
-                r[j] = double2{0.0, 0.0};
-            }
-        }
-    }
-}
-
-template <int BM, int MCONT, int NT = 256>
-__device__ __forceinline__ void lds_gemm_store(double (*S)[BM + 1], const double2 (&r)[BM * 8 / NT]) {
-    constexpr int AL = BM * 8 / NT;
-    const int t = threadIdx.x;
-    if (MCONT) {
-        const int mp = (t % (BM / 2)) * 2, kq = t / (BM / 2), ks = NT / (BM / 2);
-#pragma unroll
-        for (int j = 0; j < AL; ++j) {
-            S[kq + ks * j][mp] = r[j].x;
-            S[kq + ks * j][mp + 1] = r[j].y;
-        }
+        for (int s = 0; s < 4; ++s) f[0][s] = p[s * ld];
     } else {
-        const int kq = t & 7, m = t >> 3;
 #pragma unroll
-        for (int j = 0; j < AL; ++j) {
-            S[2 * kq][m + (NT / 8) * j] = r[j].x;
-            S[2 * kq + 1][m + (NT / 8) * j] = r[j].y;
-        }
+        for (int i = 0; i < NB; i += 2)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const V2 a = *reinterpret_cast<const V2*>(p + 16 * i + s * ld);
+                f[i][s] = a.x;
+                f[i + 1 < NB ? i + 1 : i][s] = a.y;
+            }
     }
 }
 
-// C = beta*C + alpha*op(A) op(B), FP64 MFMA; A, B and C may be stored as float or double.
-// NW waves in a 2 x NW/2 grid each own a (BM/2) x (2BM/NW) block of 16x16 MFMA tiles.
-template <int TA, int TB, int BM, typename TAs, typename TBs, typename TCs, int NW = 4>
-__global__ __launch_bounds__(64 * NW) void k_gemm_lds(int64_t M, int64_t N, int64_t K, int64_t tilesM, double alpha,
-                                                      const TAs* A, int64_t lda, const TBs* B, int64_t ldb,
-                                                      double beta, TCs* C, int64_t ldc, int tiles, int64_t sA,
-                                                      int64_t sB, int64_t sC) {
-    constexpr int NT = 64 * NW, WCn = NW / 2, WTR = BM / 2, WTC = BM / WCn;
-    constexpr int NBR = WTR / 16, NBC = WTC / 16, AL = BM * 8 / NT;
-    static_assert(NBR >= 1 && NBC >= 1 && AL >= 1, "tile shape");
+// C = beta*C + alpha*op(A) op(B); A, B and C may be stored as float or double.
+template <int TA, int TB, int WT, int PF, bool INP, typename TAs, typename TBs, typename TCs>
+__global__ __launch_bounds__(256) void k_gemm_reg(int64_t M, int64_t N, int64_t K, int64_t tilesM, double alpha,
+                                                  const TAs* A, int64_t lda, const TBs* B, int64_t ldb, double beta,
+                                                  TCs* C, int64_t ldc, int tiles, int64_t sA, int64_t sB, int64_t sC) {
+    constexpr int NB = WT / 16, BM = 2 * WT;
+    constexpr bool KA = TA != 0, KB = TB == 0;  // contiguous in k
     A += blockIdx.y * sA;  // batch: one problem per grid row
     B += blockIdx.y * sB;
     C += blockIdx.y * sC;
-    __shared__ double As[2][16][BM + 1];
-    __shared__ double Bs[2][16][BM + 1];
-    // Contiguous tile ranges per XCD share operand panels in L2; with a
-    // k range that depends on the tile row (tiles == 2) or column (tiles == 4,
-    // whose columns are contiguous in the tile order) work per tile varies
-    // widely, so the hardware's round-robin placement is kept there to balance
-    // the XCDs.
+    // Contiguous tile ranges per XCD share operand panels in L2; with a k range
+    // that depends on the tile row (tiles == 2) or column (tiles == 4, whose
+    // columns are contiguous in the tile order) work per tile varies widely, so
+    // the hardware's round-robin placement is kept there to balance the XCDs.
     const int64_t bid = (tiles == 2 || tiles == 4) ? (int64_t)blockIdx.x : xcd_remap(blockIdx.x, gridDim.x);
     int64_t ti, tj;
     if (tiles == 0 || tiles == 3 || tiles == 4) {
         ti = bid % tilesM;
         tj = bid / tilesM;
-    } else {
+        if (tiles == 3) ti = tilesM - 1 - ti;  // the longest k ranges first
+    } else if (BM >= 64) {
         lower_tile(bid, ti, tj);
+    } else {  // the lower 64x64 tiles, 2 x 2 workgroups each
+        lower_tile(bid >> 2, ti, tj);
+        ti = 2 * ti + (bid & 1);
+        tj = 2 * tj + ((bid >> 1) & 1);
     }
-    const int64_t row0 = ti * BM, col0 = tj * BM;
-    const int64_t kbeg = (tiles == 2) ? ti * BM : (tiles == 4) ? tj * BM : 0;
-    const int64_t kend = (tiles == 3 && (ti + 1) * BM < K) ? (ti + 1) * BM : K;
-    const int64_t nch = kend > kbeg ? (kend - kbeg) / 16 : 0;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int li = lane & 15, g = lane >> 4;
-    const int wr = wave / WCn, wc = wave % WCn;
-
-    d4 acc[NBR][NBC];
+    const int64_t row0 = ti * BM + (w & 1) * WT, col0 = tj * BM + (w >> 1) * WT;
+    if (row0 >= M || col0 >= N) return;
+    if ((tiles == 1 || tiles == 2) && row0 / 64 < col0 / 64) return;  // above the diagonal tiles
+    const int64_t kbeg = (tiles == 2) ? row0 / 64 * 64 : (tiles == 4) ? col0 / 64 * 64 : 0;
+    const int64_t kend = (tiles == 3) ? (row0 / 64 + 1) * 64 < K ? (row0 / 64 + 1) * 64 : K : K;
+    const int nch = kend > kbeg ? (int)((kend - kbeg) / 16) : 0;
+    const int64_t ra = row0 + frag_row<KA, NB>(0, li), rb = col0 + frag_row<KB, NB>(0, li);
+    const TAs* pa = KA ? A + (kbeg + 4 * g) + ra * lda : A + ra + (kbeg + 4 * g) * lda;
+    const TBs* pb = KB ? B + (kbeg + 4 * g) + rb * ldb : B + rb + (kbeg + 4 * g) * ldb;
+    const int64_t stepa = KA ? 16 : 16 * lda, stepb = KB ? 16 : 16 * ldb;
+    d4 acc[NB][NB];
 #pragma unroll
-    for (int i = 0; i < NBR; ++i)
+    for (int i = 0; i < NB; ++i)
 #pragma unroll
-        for (int j = 0; j < NBC; ++j) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
-
-    auto chunk = [&](int buf) {
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            const int kk = 4 * g + s;
-            double a[NBR], b[NBC];
-#pragma unroll
-            for (int i = 0; i < NBR; ++i) a[i] = As[buf][kk][wr * WTR + i * 16 + li];
-#pragma unroll
-            for (int j = 0; j < NBC; ++j) b[j] = Bs[buf][kk][wc * WTC + j * 16 + li];
-#pragma unroll
-            for (int i = 0; i < NBR; ++i)
-#pragma unroll
-                for (int j = 0; j < NBC; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
-        }
+        for (int j = 0; j < NB; ++j) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
+    TAs fa[PF][NB][4];
+    TBs fb[PF][NB][4];
+    auto load = [&](int st) {
+        frag_load<KA, NB>(fa[st], pa, lda);
+        frag_load<KB, NB>(fb[st], pb, ldb);
+        pa += stepa;
+        pb += stepb;
     };
-    double2 ra[AL], rb[AL];
-    if (nch > 0) {
-        lds_gemm_load<BM, !TA, TAs, NT>(A, lda, row0, M, kbeg, ra);
-        lds_gemm_load<BM, TB, TBs, NT>(B, ldb, col0, N, kbeg, rb);
-        lds_gemm_store<BM, !TA, NT>(As[0], ra);
-        lds_gemm_store<BM, TB, NT>(Bs[0], rb);
-    }
-    __syncthreads();
-    for (int64_t c = 0; c < nch; ++c) {
-        const int buf = (int)(c & 1);
-        const bool more = c + 1 < nch;
-        if (more) {
-            lds_gemm_load<BM, !TA, TAs, NT>(A, lda, row0, M, kbeg + (c + 1) * 16, ra);
-            lds_gemm_load<BM, TB, TBs, NT>(B, ldb, col0, N, kbeg + (c + 1) * 16, rb);
+    // the tiles are formed transposed: D lane (li, g) holds columns g + 4v of row li
+    auto mult = [&](int st) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int i = 0; i < NB; ++i)
+#pragma unroll
+                for (int j = 0; j < NB; ++j)
+                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)fb[st][j][s], (double)fa[st][i][s],
+                                                                     acc[i][j], 0, 0, 0);
+    };
+#pragma unroll
+    for (int q = 0; q < PF - 1; ++q)
+        if (q < nch) load(q);
+    int c = 0;
+    for (; c + 2 * PF - 1 <= nch; c += PF)  // every load of this round exists
+#pragma unroll
+        for (int q = 0; q < PF; ++q) {
+            load((q + PF - 1) % PF);
+            mult(q);
         }
-        chunk(buf);
-        if (more) {
-            lds_gemm_store<BM, !TA, NT>(As[buf ^ 1], ra);
-            lds_gemm_store<BM, TB, NT>(Bs[buf ^ 1], rb);
+    for (; c < nch; c += PF)
+#pragma unroll
+        for (int q = 0; q < PF; ++q) {
+            if (c + q + PF - 1 < nch) load((q + PF - 1) % PF);
+            if (c + q < nch) mult(q);
         }
-        __syncthreads();
-    }
-    // v_mfma_f64_16x16x4 D layout: lane holds rows g, g+4, g+8, g+12 of column li.
-    // With beta != 0 every C value is loaded before the first store (a load
-    // placed after a store that may alias it waits for that store's round
-    // trip).  The eight-wave 128 tile pays for the registers with one wave per
-    // SIMD less and still comes out ahead (Cholesky trailing updates at
-    // n = 4096 and 8192); the FP32 GEMM, whose 128 tile measured slower with
-    // the same change, keeps the interleaved order.
-    TCs cv[NBR][NBC][4];
+    // With beta != 0 every C value is loaded before the first store (a load placed
+    // after a store that may alias it waits for that store's round trip).
+    typedef typename vec2_of<TCs>::type C2;
+    constexpr bool PAIR = !KA && NB > 1;  // rows 2li, 2li + 1 of tiles i, i + 1
+    constexpr int RI = PAIR ? 2 : 1;
+    TCs cv[NB][NB][4];
+    auto addr = [&](int i, int j, int v) {
+        return C + (row0 + frag_row<KA, NB>(i, li)) + (col0 + frag_row<KB, NB>(j, g + 4 * v)) * ldc;
+    };
     if (beta != 0.0) {
 #pragma unroll
-        for (int i = 0; i < NBR; ++i)
+        for (int i = 0; i < NB; i += RI)
 #pragma unroll
-            for (int j = 0; j < NBC; ++j) {
-                const int64_t rb0 = row0 + wr * WTR + i * 16, cb0 = col0 + wc * WTC + j * 16;
-                if (rb0 >= M || cb0 >= N) continue;
-                const TCs* p = C + (rb0 + g) + (cb0 + li) * ldc;
+            for (int j = 0; j < NB; ++j)
 #pragma unroll
-                for (int v = 0; v < 4; ++v) cv[i][j][v] = p[4 * v];
-            }
+                for (int v = 0; v < 4; ++v) {
+                    if (PAIR) {
+                        const C2 x = *reinterpret_cast<const C2*>(addr(i, j, v));
+                        cv[i][j][v] = x.x;
+                        cv[i + RI - 1][j][v] = x.y;
+                    } else {
+                        cv[i][j][v] = *addr(i, j, v);
+                    }
+                }
     }
+    if (INP) __syncthreads();
+    auto out = [&](int i, int j, int v) {
+        const double o = alpha * acc[i][j][v];
+        return (TCs)((beta == 0.0) ? o : beta * (double)cv[i][j][v] + o);
+    };
 #pragma unroll
-    for (int i = 0; i < NBR; ++i)
+    for (int i = 0; i < NB; i += RI)
 #pragma unroll
-        for (int j = 0; j < NBC; ++j) {
-            const int64_t rb0 = row0 + wr * WTR + i * 16, cb0 = col0 + wc * WTC + j * 16;
-            if (rb0 >= M || cb0 >= N) continue;
-            TCs* p = C + (rb0 + g) + (cb0 + li) * ldc;
+        for (int j = 0; j < NB; ++j)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                const double o = alpha * acc[i][j][v];
-                p[4 * v] = (TCs)((beta == 0.0) ? o : beta * (double)cv[i][j][v] + o);
+                if (PAIR) {
+                    C2 x;
+                    x.x = out(i, j, v);
+                    x.y = out(i + RI - 1, j, v);
+                    *reinterpret_cast<C2*>(addr(i, j, v)) = x;
+                } else {
+                    *addr(i, j, v) = out(i, j, v);
+                }
             }
-        }
 }
 
-template <int BM, typename TAs, typename TBs, typename TCs, int NW = 4>
-static void gemm_lds_launch(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha,
-                            const TAs* A, int64_t lda, const TBs* B, int64_t ldb, double beta, TCs* C,
-                            int64_t ldc, int tiles, int batch = 1, int64_t sA = 0, int64_t sB = 0,
-                            int64_t sC = 0) {
-    const int64_t tm = (M + BM - 1) / BM, tn = (N + BM - 1) / BM;
-    const int64_t nblk = (tiles == 0 || tiles == 3 || tiles == 4) ? tm * tn : tm * (tm + 1) / 2;
-    dim3 grid((unsigned)nblk, (unsigned)batch), block(64 * NW);
-#define GPL_GL(TAv, TBv)                                                                                      \
-    hipLaunchKernelGGL((k_gemm_lds<TAv, TBv, BM, TAs, TBs, TCs, NW>), grid, block, 0, s, M, N, K, tm, alpha, A, \
+template <int WT, int PF, bool INP, typename TAs, typename TBs, typename TCs>
+static void gemm_reg_launch(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha,
+                            const TAs* A, int64_t lda, const TBs* B, int64_t ldb, double beta, TCs* C, int64_t ldc,
+                            int tiles, int batch, int64_t sA, int64_t sB, int64_t sC) {
+    constexpr int BM = 2 * WT;
+    const int64_t tm = (M + BM - 1) / BM, tn = (N + BM - 1) / BM, t64 = M / 64;
+    const int64_t nblk = (tiles != 1 && tiles != 2) ? tm * tn : BM < 64 ? 4 * (t64 * (t64 + 1) / 2) : tm * (tm + 1) / 2;
+    dim3 grid((unsigned)nblk, (unsigned)batch), block(256);
+#define GPL_GR(TAv, TBv)                                                                                           \
+    hipLaunchKernelGGL((k_gemm_reg<TAv, TBv, WT, PF, INP, TAs, TBs, TCs>), grid, block, 0, s, M, N, K, tm, alpha, A, \
                        lda, B, ldb, beta, C, ldc, tiles, sA, sB, sC)
-    if (!ta && !tb) GPL_GL(0, 0);
-    else if (!ta && tb) GPL_GL(0, 1);
-    else if (ta && !tb) GPL_GL(1, 0);
-    else GPL_GL(1, 1);
-#undef GPL_GL
+    if (!ta && !tb) GPL_GR(0, 0);
+    else if (!ta && tb) GPL_GR(0, 1);
+    else if (ta && !tb) GPL_GR(1, 0);
+    else GPL_GR(1, 1);
+#undef GPL_GR
 }
 
-// Tile choice for FP64 storage.  Short inner dimensions (the panel and trailing
-// updates, k of 64 to 256) are bound by the chunk loop's load latency and want
-// the most workgroups: 64x64 tiles on four waves.  Long inner dimensions (B^-1 =
-// X^T X, prediction's L^-1 K_t^T, k = n) run faster on 128x128 tiles with eight
-// waves (half the operand reads per flop at the same occupancy): 57 against 46
-// TFLOP/s for X^T X at n = 8192.  bm = 64 or 128 forces the 64/4 or 128/8 form.
-static int pick_bm(int64_t M, int64_t N, int64_t K, int tiles, int batch = 1) {
-    const int64_t tm = (M + 127) / 128, tn = (N + 127) / 128;
-    const int64_t n128 = (tiles == 0 || tiles == 3 || tiles == 4) ? tm * tn : tm * (tm + 1) / 2;
-    return (K >= 1024 && n128 * batch >= 256) ? 128 : 64;
+// Wave tile by the number of 64x64 output tiles (all problems of the launch), t64,
+// and their number of 128x128 ones, t128; times staged LDS / 16 / 32 / 64 measured
+// alone, in us.  Fewer than 128: 16-wide waves (32x32 workgroups), so that a small
+// product spreads over the chip and its k loop is a quarter as long (512 x 256 x
+// 256: 20 / 7.0 / 12 / 37; X B at 512: 32 / 14 / 21 / 67; 128 tiles, 1024 x 512 x
+// 512: 36 / 20 / 22 / 68).  Else 32-wide ones (2048 x 512 x 512: 38 / 36 / 25 / 70;
+// lower 7168, k = 512: 558 / 769 / 458 / 496).  Long k with enough tiles to
+// fill the chip more than twice over: 64-wide ones, half the operand traffic per
+// flop (X B at 4096: 1562 / 2857 / 1278 / 1146; X^T X at 8192: 3213 / 9711 / 4902 /
+// 2943, at 3072: 423 / 542 / 297 / 377).  With both operands contiguous in k the
+// 32-wide waves are bound by their loads (37 TFLOP/s), so a product whose tiles
+// all have the same k range takes the 64-wide ones as soon as they fill the chip
+// once (1024 x 1024 x 32768 in four parts).
+template <typename TAs, typename TBs, typename TCs>
+static void gemm_any(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha, const TAs* A,
+                     int64_t lda, const TBs* B, int64_t ldb, double beta, TCs* C, int64_t ldc, int tiles, int batch,
+                     int64_t sA, int64_t sB, int64_t sC) {
+    if (M <= 0 || N <= 0 || batch <= 0) return;
+#define GPL_GA(WT, PF, INP) \
+    gemm_reg_launch<WT, PF, INP>(s, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tiles, batch, sA, sB, sC)
+    if ((const void*)A == (const void*)C || (const void*)B == (const void*)C) {
+        GPL_GA(32, 3, true);
+        return;
+    }
+    const bool low = tiles == 1 || tiles == 2;
+    const int64_t m = M / 64, n = N / 64, m2 = (m + 1) / 2, n2 = (n + 1) / 2;
+    const int64_t t64 = (low ? m * (m + 1) / 2 : m * n) * batch, t128 = (low ? m2 * (m2 + 1) / 2 : m2 * n2) * batch;
+    if (t64 < 128) GPL_GA(16, 4, false);
+    else if (K >= 1024 && t128 >= (ta && !tb && !tiles ? 256 : 600)) GPL_GA(64, 3, false);
+    else GPL_GA(32, 3, false);
+#undef GPL_GA
 }
 
 void gemm2_f64(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha, const double* A,
-               int64_t lda, const double* B, int64_t ldb, double beta, double* C, int64_t ldc, int tiles, int bm) {
-    if (M <= 0 || N <= 0) return;
-    if (bm == 0) bm = pick_bm(M, N, K, tiles);
-    if (bm == 128)
-        gemm_lds_launch<128, double, double, double, 8>(s, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tiles);
-    else gemm_lds_launch<64>(s, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tiles);
+               int64_t lda, const double* B, int64_t ldb, double beta, double* C, int64_t ldc, int tiles) {
+    gemm_any(s, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tiles, 1, 0, 0, 0);
 }
 
 // `batch` independent FP64 GEMMs (strides in elements), one grid row per problem
 void gemm2_f64_batched(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha, const double* A,
                        int64_t lda, const double* B, int64_t ldb, double beta, double* C, int64_t ldc, int tiles,
                        int batch, int64_t sA, int64_t sB, int64_t sC) {
-    if (M <= 0 || N <= 0 || batch <= 0) return;
-    if (pick_bm(M, N, K, tiles, batch) == 128)
-        gemm_lds_launch<128, double, double, double, 8>(s, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc,
-                                                        tiles, batch, sA, sB, sC);
-    else gemm_lds_launch<64>(s, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tiles, batch, sA, sB, sC);
+    gemm_any(s, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tiles, batch, sA, sB, sC);
+}
+
+// FP64-compute GEMMs on FP32 storage: A and C (panel solves of the batched form), A (prediction)
+void gemm_mixed_f32f64_batched(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha,
+                               const float* A, int64_t lda, const double* B, int64_t ldb, double beta, float* C,
+                               int64_t ldc, int tiles, int batch, int64_t sA, int64_t sB, int64_t sC) {
+    gemm_any(s, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tiles, batch, sA, sB, sC);
+}
+
+void gemm_mixed_f32f64f64(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha,
+                          const float* A, int64_t lda, const double* B, int64_t ldb, double beta, double* C,
+                          int64_t ldc, int tiles) {
+    gemm_any(s, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tiles, 1, 0, 0, 0);
 }
 
 // out[i] = sum over p < parts of W[p * stride + i], in order of p (deterministic)
@@ -275,44 +307,6 @@ __global__ void k_sum_parts(const double* __restrict__ W, int64_t stride, int pa
 
 void sum_parts_f64(hipStream_t s, const double* W, int64_t stride, int parts, int64_t n, double* out) {
     hipLaunchKernelGGL(k_sum_parts, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, W, stride, parts, n, out);
-}
-
-// FP64-compute GEMM on FP32 storage for A/C with an FP64 B (panel solves of the mixed path)
-void gemm_mixed_f32f64(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha, const float* A,
-                       int64_t lda, const double* B, int64_t ldb, double beta, float* C, int64_t ldc, int tiles) {
-    if (M <= 0 || N <= 0) return;
-    gemm_lds_launch<64>(s, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tiles);
-}
-
-// FP64 B on the left: C(float) = alpha * A(double) op B(float)
-void gemm_mixed_f64f32(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha,
-                       const double* A, int64_t lda, const float* B, int64_t ldb, double beta, float* C, int64_t ldc,
-                       int tiles) {
-    if (M <= 0 || N <= 0) return;
-    gemm_lds_launch<64>(s, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tiles);
-}
-
-void gemm_mixed_f32f64_batched(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha,
-                               const float* A, int64_t lda, const double* B, int64_t ldb, double beta, float* C,
-                               int64_t ldc, int tiles, int batch, int64_t sA, int64_t sB, int64_t sC) {
-    if (M <= 0 || N <= 0 || batch <= 0) return;
-    gemm_lds_launch<64>(s, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tiles, batch, sA, sB, sC);
-}
-
-void gemm_mixed_f64f32_batched(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha,
-                               const double* A, int64_t lda, const float* B, int64_t ldb, double beta, float* C,
-                               int64_t ldc, int tiles, int batch, int64_t sA, int64_t sB, int64_t sC) {
-    if (M <= 0 || N <= 0 || batch <= 0) return;
-    gemm_lds_launch<64>(s, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tiles, batch, sA, sB, sC);
-}
-
-void gemm_mixed_f32f64f64(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha,
-                          const float* A, int64_t lda, const double* B, int64_t ldb, double beta, double* C,
-                          int64_t ldc, int tiles) {
-    if (M <= 0 || N <= 0) return;
-    if (pick_bm(M, N, K, tiles) == 128)
-        gemm_lds_launch<128, float, double, double, 8>(s, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tiles);
-    else gemm_lds_launch<64>(s, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tiles);
 }
 
 // ---------------------------------------------------------------------------

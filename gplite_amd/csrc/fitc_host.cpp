@@ -115,11 +115,11 @@ static void fitc_predictive_matrix(gpl_fitc* f) {
     const int64_t Mz = f->Mz;
     trtri_blocked(c, f->d(F_G), f->d(F_DINVG), Mz, f->d(F_XG));
     double* Y = f->d(F_MM);  // Y = Lc^-1 H, then reused for M
-    gemm2_f64(s, 0, 0, Mz, Mz, Mz, 1.0, f->d(F_XG), Mz, f->d(F_H), Mz, 0.0, Y, Mz, 3, 0);
+    gemm2_f64(s, 0, 0, Mz, Mz, Mz, 1.0, f->d(F_XG), Mz, f->d(F_H), Mz, 0.0, Y, Mz, 3);
     hipMemcpyAsync(f->d(F_T1), f->d(F_H), Mz * Mz * 8, hipMemcpyDeviceToDevice, s);
-    gemm2_f64(s, 1, 0, Mz, Mz, Mz, -1.0, Y, Mz, Y, Mz, 1.0, f->d(F_T1), Mz, 0, 0);  // H - H G^-1 H
-    gemm2_f64(s, 0, 0, Mz, Mz, Mz, 1.0, f->d(F_XZ), Mz, f->d(F_T1), Mz, 0.0, f->d(F_XG), Mz, 3, 0);
-    gemm2_f64(s, 0, 1, Mz, Mz, Mz, 1.0, f->d(F_XG), Mz, f->d(F_XZ), Mz, 0.0, Y, Mz, 0, 0);
+    gemm2_f64(s, 1, 0, Mz, Mz, Mz, -1.0, Y, Mz, Y, Mz, 1.0, f->d(F_T1), Mz, 0);  // H - H G^-1 H
+    gemm2_f64(s, 0, 0, Mz, Mz, Mz, 1.0, f->d(F_XZ), Mz, f->d(F_T1), Mz, 0.0, f->d(F_XG), Mz, 3);
+    gemm2_f64(s, 0, 1, Mz, Mz, Mz, 1.0, f->d(F_XG), Mz, f->d(F_XZ), Mz, 0.0, Y, Mz, 0);
 }
 
 // One inversion-lemma solve for the current sites: S = D + V, G = Kz + K_zx S^-1 K_xz
@@ -135,7 +135,7 @@ static void fitc_lemma_step(gpl_fitc* f, int* flags) {
         Prof p(c, "fitc_syrk", 2.0 * Mz * Mz * N, 8.0 * N * Mz);
         const int P = fitc_split(f);
         if (P == 1) {
-            gemm2_f64(s, 1, 0, Mz, Mz, N, 1.0, f->d(F_W), N, f->d(F_W), N, 0.0, f->d(F_H), Mz, 0, 0);
+            gemm2_f64(s, 1, 0, Mz, Mz, N, 1.0, f->d(F_W), N, f->d(F_W), N, 0.0, f->d(F_H), Mz, 0);
         } else {
             const int64_t Kp = N / P;
             gemm2_f64_batched(s, 1, 0, Mz, Mz, Kp, 1.0, f->d(F_W), N, f->d(F_W), N, 0.0, f->d(F_SPLIT), Mz, 0, P, Kp,
@@ -167,7 +167,7 @@ static void fitc_q(gpl_fitc* f, double* out) {
     const int64_t N = f->N, Mz = f->Mz;
     trtri_blocked(c, f->d(F_G), f->d(F_DINVG), Mz, f->d(F_XG));
     Prof p(c, "fitc_q", (double)Mz * Mz * N, 16.0 * N * Mz);
-    gemm2_f64(s, 0, 0, Mz, N, Mz, 1.0, f->d(F_XG), Mz, f->d(F_UT), Mz, 0.0, f->d(F_W), Mz, 3, 0);
+    gemm2_f64(s, 0, 0, Mz, N, Mz, 1.0, f->d(F_XG), Mz, f->d(F_UT), Mz, 0.0, f->d(F_W), Mz, 3);
     colsumsq_f64(s, f->d(F_W), Mz, Mz, f->n, out, 0);
 }
 
@@ -300,7 +300,7 @@ static int fitc_run(gpl_fitc* f) {
     // D = diag K + jitter - colSums((Lz^-1 K_zx)^2)  (R/gp_fit.R:107-108); F_W holds Lz^-1 K_zx here
     {
         Prof p(c, "fitc_diag_trmm", (double)Mz * Mz * N, 16.0 * N * Mz);
-        gemm2_f64(s, 0, 0, Mz, N, Mz, 1.0, f->d(F_XZ), Mz, f->d(F_UT), Mz, 0.0, f->d(F_W), Mz, 3, 0);
+        gemm2_f64(s, 0, 0, Mz, N, Mz, 1.0, f->d(F_XZ), Mz, f->d(F_UT), Mz, 0.0, f->d(F_W), Mz, 3);
         colsumsq_f64(s, f->d(F_W), Mz, Mz, n, f->d(F_V1), 0);
     }
     launch_build_diag(s, pd, f->prog, f->d(F_F), N, f->d(F_F), N, n, f->d(F_V2));
@@ -469,7 +469,7 @@ extern "C" int gpl_fitc_pred(gpl_fitc* f, const double* xt, int64_t mt, int32_t 
     launch_features(s, xtd, mt, mt, (int)f->ncols, pd, f->prog, Ft, Mt);
     launch_build_cross(s, pd, f->prog, f->d(F_FZ), Mz, m, Mz, Ft, Mt, mt, Mt, KzT, Mz);
     // A_t = Lz^-1 K_zt (Kt_aux2); mean = A_t^T w
-    gemm2_f64(s, 0, 0, Mz, Mt, Mz, 1.0, f->d(F_XZ), Mz, KzT, Mz, 0.0, A2, Mz, 3, 0);
+    gemm2_f64(s, 0, 0, Mz, Mt, Mz, 1.0, f->d(F_XZ), Mz, KzT, Mz, 0.0, A2, Mz, 3);
     gemv_t_f64(s, A2, Mz, Mz, mt, f->d(F_WZ), vb);
     if (want_var) {
         // prior_var = colSums(K_zt * Kz^-1 K_zt) + Dt, Dt = diag K_tt - colSums(A_t^2)  (R/gp_pred.R:244-246,271)
@@ -477,14 +477,14 @@ extern "C" int gpl_fitc_pred(gpl_fitc* f, const double* xt, int64_t mt, int32_t 
         double* c2 = vb + 2 * Mt;
         double* kd = vb + 3 * Mt;
         double* red = vb + 4 * Mt;
-        gemm2_f64(s, 1, 0, Mz, Mt, Mz, 1.0, f->d(F_XZ), Mz, A2, Mz, 0.0, Yv, Mz, 0, 0);  // Kz^-1 K_zt = Lz^-T A_t
+        gemm2_f64(s, 1, 0, Mz, Mt, Mz, 1.0, f->d(F_XZ), Mz, A2, Mz, 0.0, Yv, Mz, 0);  // Kz^-1 K_zt = Lz^-T A_t
         coldot_f64(s, KzT, Yv, Mz, Mz, mt, c1);
         colsumsq_f64(s, A2, Mz, Mz, mt, c2, 0);
         launch_build_diag(s, pd, f->prog, Ft, Mt, Ft, Mt, mt, kd);
         vec_axpby(s, mt, 1.0, kd, -1.0, c2, c2);   // Dt
         vec_axpby(s, mt, 1.0, c1, 1.0, c2, c2);    // prior_var
         // var_reduction = colSums(A_t * (M A_t))  (R/gp_pred.R:278-280)
-        gemm2_f64(s, 0, 0, Mz, Mt, Mz, 1.0, f->d(F_MM), Mz, A2, Mz, 0.0, Yv, Mz, 0, 0);
+        gemm2_f64(s, 0, 0, Mz, Mt, Mz, 1.0, f->d(F_MM), Mz, A2, Mz, 0.0, Yv, Mz, 0);
         coldot_f64(s, A2, Yv, Mz, Mz, mt, red);
         vec_axpby(s, mt, 1.0, c2, -1.0, red, red);
         HIP_TRY(hipMemcpyAsync(var, red, mt * 8, hipMemcpyDeviceToHost, s));
@@ -523,7 +523,7 @@ extern "C" int gpl_fitc_draw(gpl_fitc* f, const double* xt, int64_t mt, double j
     if (mt * f->ncols > 0) HIP_TRY(hipMemcpyAsync(xtd, xt, mt * f->ncols * 8, hipMemcpyHostToDevice, s));
     launch_features(s, xtd, mt, mt, (int)f->ncols, pd, f->prog, Ft, Mt);
     launch_build_cross(s, pd, f->prog, f->d(F_FZ), Mz, m, Mz, Ft, Mt, mt, Mt, KzT, Mz);
-    gemm2_f64(s, 0, 0, Mz, Mt, Mz, 1.0, f->d(F_XZ), Mz, KzT, Mz, 0.0, A2, Mz, 3, 0);
+    gemm2_f64(s, 0, 0, Mz, Mt, Mz, 1.0, f->d(F_XZ), Mz, KzT, Mz, 0.0, A2, Mz, 3);
     gemv_t_f64(s, A2, Mz, Mz, mt, f->d(F_WZ), vb);
     // Dt = diag K_tt - colSums(A_t^2)
     double* dt = vb + Mt;
@@ -531,9 +531,9 @@ extern "C" int gpl_fitc_draw(gpl_fitc* f, const double* xt, int64_t mt, double j
     launch_build_diag(s, pd, f->prog, Ft, Mt, Ft, Mt, mt, vb + 2 * Mt);
     vec_axpby(s, mt, 1.0, vb + 2 * Mt, -1.0, dt, dt);
     // lower tiles of A_t^T A_t - A_t^T (M A_t), then the diagonal terms
-    gemm2_f64(s, 0, 0, Mz, Mt, Mz, 1.0, f->d(F_MM), Mz, A2, Mz, 0.0, Yv, Mz, 0, 0);
-    gemm2_f64(s, 1, 0, Mt, Mt, Mz, 1.0, A2, Mz, A2, Mz, 0.0, Cv, Mt, 1, 0);
-    gemm2_f64(s, 1, 0, Mt, Mt, Mz, -1.0, A2, Mz, Yv, Mz, 1.0, Cv, Mt, 1, 0);
+    gemm2_f64(s, 0, 0, Mz, Mt, Mz, 1.0, f->d(F_MM), Mz, A2, Mz, 0.0, Yv, Mz, 0);
+    gemm2_f64(s, 1, 0, Mt, Mt, Mz, 1.0, A2, Mz, A2, Mz, 0.0, Cv, Mt, 1);
+    gemm2_f64(s, 1, 0, Mt, Mt, Mz, -1.0, A2, Mz, Yv, Mz, 1.0, Cv, Mt, 1);
     add_diag_f64(s, Cv, Mt, mt, Mt, dt, jitter);
     HIP_TRY(hipMemsetAsync(info, 0, 64, s));
     potrf_blocked(c, Cv, Mt, Dv, ld, info);
@@ -541,7 +541,7 @@ extern "C" int gpl_fitc_draw(gpl_fitc* f, const double* xt, int64_t mt, double j
     HIP_TRY(hipMemcpyAsync(&inf, info, 4, hipMemcpyDeviceToHost, s));
     fill_f64(s, Zd, Mt * Dp, 0.0);
     HIP_TRY(upload_2d(c, s, Zd, Mt, z, mt, draws, 20));
-    gemm2_f64(s, 0, 0, Mt, Dp, Mt, 1.0, Cv, Mt, Zd, Mt, 0.0, Wd, Mt, 3, 0);
+    gemm2_f64(s, 0, 0, Mt, Dp, Mt, 1.0, Cv, Mt, Zd, Mt, 0.0, Wd, Mt, 3);
     std::vector<double> mean(mt);
     HIP_TRY(hipMemcpyAsync(mean.data(), vb, mt * 8, hipMemcpyDeviceToHost, s));
     HIP_TRY(download_2d(c, s, out, Wd, Mt, mt, draws, 21));
@@ -574,17 +574,17 @@ extern "C" int gpl_fitc_train_var(gpl_fitc* f, double* out) {
     double* X = (double*)c->buf(25, (size_t)Mz * Mz * 8);
     if (!A || !B || !v || !X) return fail(GPL_ERR_OOM, "device allocation failed");
     double *c2 = v, *kd = v + N, *c1 = v + 2 * N, *t1 = v + 3 * N, *q = v + 4 * N, *res = v + 5 * N;
-    gemm2_f64(s, 0, 0, Mz, N, Mz, 1.0, f->d(F_XZ), Mz, f->d(F_UT), Mz, 0.0, A, Mz, 3, 0);  // A = Lz^-1 K_zx
+    gemm2_f64(s, 0, 0, Mz, N, Mz, 1.0, f->d(F_XZ), Mz, f->d(F_UT), Mz, 0.0, A, Mz, 3);  // A = Lz^-1 K_zx
     colsumsq_f64(s, A, Mz, Mz, n, c2, 0);
     launch_build_diag(s, f->b[F_PROG].as<DevProg>(), f->prog, f->d(F_F), N, f->d(F_F), N, n, kd);
     vec_axpby(s, n, 1.0, kd, -1.0, c2, c2);  // Dt
-    gemm2_f64(s, 1, 0, Mz, N, Mz, 1.0, f->d(F_XZ), Mz, A, Mz, 0.0, B, Mz, 0, 0);  // Kz^-1 K_zx
+    gemm2_f64(s, 1, 0, Mz, N, Mz, 1.0, f->d(F_XZ), Mz, A, Mz, 0.0, B, Mz, 0);  // Kz^-1 K_zx
     coldot_f64(s, f->d(F_UT), B, Mz, Mz, n, c1);
     vec_axpby(s, n, 1.0, c1, 1.0, c2, c1);  // prior_var
-    gemm2_f64(s, 0, 0, Mz, N, Mz, 1.0, f->d(F_MM), Mz, A, Mz, 0.0, B, Mz, 0, 0);  // M A
+    gemm2_f64(s, 0, 0, Mz, N, Mz, 1.0, f->d(F_MM), Mz, A, Mz, 0.0, B, Mz, 0);  // M A
     coldot_f64(s, A, B, Mz, Mz, n, t1);
     trtri_blocked(c, f->d(F_G), f->d(F_DINVG), Mz, X);
-    gemm2_f64(s, 0, 0, Mz, N, Mz, 1.0, X, Mz, f->d(F_UT), Mz, 0.0, B, Mz, 3, 0);  // Lc^-1 K_zx
+    gemm2_f64(s, 0, 0, Mz, N, Mz, 1.0, X, Mz, f->d(F_UT), Mz, 0.0, B, Mz, 3);  // Lc^-1 K_zx
     colsumsq_f64(s, B, Mz, Mz, n, q, 0);
     fitc_train_var(s, n, c1, t1, c2, q, f->d(F_S), res);
     HIP_TRY(hipMemcpyAsync(out, res, n * 8, hipMemcpyDeviceToHost, s));

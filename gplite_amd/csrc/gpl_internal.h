@@ -79,20 +79,15 @@ void launch_grad_tiles_f32(hipStream_t s, const DevProg* prog, const DevProg& hp
 // 2 = lower tiles and k starts at the row tile (C = X^T X with X lower triangular),
 // 3 = full grid and k stops after the row tile (C = X B with X lower triangular),
 // 4 = full grid and k starts at the column tile (C = A X with X lower triangular).
-// bm: output tile edge (64 or 128; 0 = choose by grid size).
+// C may be A (N = 64) or B (M = 64), with tiles 0.
 void gemm2_f64(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha, const double* A,
-               int64_t lda, const double* B, int64_t ldb, double beta, double* C, int64_t ldc, int tiles, int bm);
+               int64_t lda, const double* B, int64_t ldb, double beta, double* C, int64_t ldc, int tiles);
 void gemm2_f64_batched(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha, const double* A,
                        int64_t lda, const double* B, int64_t ldb, double beta, double* C, int64_t ldc, int tiles,
                        int batch, int64_t sA, int64_t sB, int64_t sC);
 // out[i] = sum_p W[p * stride + i] for i < n (fixed order)
 void sum_parts_f64(hipStream_t s, const double* W, int64_t stride, int parts, int64_t n, double* out);
-// FP64 MFMA on FP32 storage: C(f32) = beta*C + alpha op(A(f32)) op(B(f64)) and the mirror case.
-void gemm_mixed_f32f64(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha, const float* A,
-                       int64_t lda, const double* B, int64_t ldb, double beta, float* C, int64_t ldc, int tiles);
-void gemm_mixed_f64f32(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha,
-                       const double* A, int64_t lda, const float* B, int64_t ldb, double beta, float* C, int64_t ldc,
-                       int tiles);
+// FP64 MFMA on an FP32 A
 void gemm_mixed_f32f64f64(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha,
                           const float* A, int64_t lda, const double* B, int64_t ldb, double beta, double* C,
                           int64_t ldc, int tiles);
@@ -285,9 +280,6 @@ void gemm_f32_batched2(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int6
 constexpr int kFoldInverse = 1;
 void gemm_mixed_f32f64_batched(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha,
                                const float* A, int64_t lda, const double* B, int64_t ldb, double beta, float* C,
-                               int64_t ldc, int tiles, int batch, int64_t sA, int64_t sB, int64_t sC);
-void gemm_mixed_f64f32_batched(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha,
-                               const double* A, int64_t lda, const float* B, int64_t ldb, double beta, float* C,
                                int64_t ldc, int tiles, int batch, int64_t sA, int64_t sB, int64_t sC);
 // Factor the 64x64 diagonal block at A + k*64*(ld+1) of every problem from its FP64 tile
 // Dacc + k*64*64; its inverse goes to Dinv + k*64*64 (FP64), log(L_ii) to ldiag + k*64,

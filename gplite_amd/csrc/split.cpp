@@ -34,10 +34,10 @@ void trsm_lower(hipStream_t s, const double* L, int64_t ld, const double* Dinv, 
                 int64_t M) {
     const int64_t T = N / 64;
     for (int64_t i = 0; i < T; ++i) {
-        gemm2_f64(s, 0, 0, 64, M, 64, 1.0, Dinv + i * 64 * 64, 64, B + i * 64, ldb, 0.0, B + i * 64, ldb, 0, 0);
+        gemm2_f64(s, 0, 0, 64, M, 64, 1.0, Dinv + i * 64 * 64, 64, B + i * 64, ldb, 0.0, B + i * 64, ldb, 0);
         if (i + 1 < T)
             gemm2_f64(s, 0, 0, (T - 1 - i) * 64, M, 64, -1.0, L + (i + 1) * 64 + i * 64 * ld, ld, B + i * 64, ldb, 1.0,
-                      B + (i + 1) * 64, ldb, 0, 0);
+                      B + (i + 1) * 64, ldb, 0);
     }
 }
 
@@ -180,7 +180,7 @@ int gpl::split_step(gpl_model* m, bool ep, double* logZ) {
     trsm_lower(s, L1, Ng, m->d(B_DINV), Ng, aux, Ng, Nb);
     double* Lk = m->d(B_LK);
     gather_sym_f64(s, K, N, bi, nb, bi, nb, nullptr, nullptr, 0, 1, Lk, Nb, Nb, Nb);
-    gemm2_f64(s, 1, 0, Nb, Nb, Ng, -1.0, aux, Ng, aux, Ng, 1.0, Lk, Nb, 1, 0);
+    gemm2_f64(s, 1, 0, Nb, Nb, Ng, -1.0, aux, Ng, aux, Ng, 1.0, Lk, Nb, 1);
     potrf_blocked(c, Lk, Nb, m->d(B_DK), m->d(B_LDK), info + 3);
     tril_f64(s, Lk, Nb, Nb);
     int fl[2];
@@ -200,7 +200,7 @@ int gpl::split_step(gpl_model* m, bool ep, double* logZ) {
     double* Tq = m->d(B_SPQ);
     double* Ac = m->d(B_AC);
     scale_rows_copy_f64(s, Lk, Nb, Nb, Nb, m->d(B_IV2), Tq);
-    gemm2_f64(s, 1, 0, Nb, Nb, Nb, 1.0, Lk, Nb, Tq, Nb, 0.0, Ac, Nb, 1, 0);
+    gemm2_f64(s, 1, 0, Nb, Nb, Nb, 1.0, Lk, Nb, Tq, Nb, 0.0, Ac, Nb, 1);
     fill_f64(s, t1, Nb, 0.0);
     add_diag_f64(s, Ac, Nb, nb, Nb, t1, 1.0);
     HIP_TRY(hipMemsetAsync(info + 2, 0, 4, s));
@@ -290,10 +290,10 @@ int gpl::split_step(gpl_model* m, bool ep, double* logZ) {
         colsumsq_f64(s, X1, Ng, Ng, Ng, t1, 1);  // [B1^-1]_ii
         double* G = m->d(B_SPG);
         double* H = m->d(B_SPH);
-        gemm2_f64(s, 1, 0, Nb, Ng, Ng, 1.0, aux, Ng, X1, Ng, 0.0, G, Nb, 0, 0);
+        gemm2_f64(s, 1, 0, Nb, Ng, Ng, 1.0, aux, Ng, X1, Ng, 0.0, G, Nb, 0);
         scale_rows_copy_f64(s, G, Nb, Nb, Ng, m->d(B_IV2), H);
         coldot_f64(s, G, H, Nb, Nb, Ng, t2);  // g^T V2^-1 g
-        gemm2_f64(s, 1, 0, Nb, Ng, Nb, 1.0, Lk, Nb, H, Nb, 0.0, G, Nb, 0, 0);
+        gemm2_f64(s, 1, 0, Nb, Ng, Nb, 1.0, Lk, Nb, H, Nb, 0.0, G, Nb, 0);
         trsm_lower(s, Ac, Nb, m->d(B_DA), Nb, G, Nb, Ng);
         colsumsq_f64(s, G, Nb, Nb, Ng, t3, 0);  // |A^-1/2 Lk^T V2^-1 g|^2
         vec_axpby(s, Ng, 1.0, t2, -1.0, t3, t2);
@@ -342,10 +342,10 @@ int gpl::split_var_reduction(gpl_ctx* c, gpl_model* m, const double* KtT, int64_
     trsm_lower(s, m->d(B_L), Ng, m->d(B_DINV), Ng, Q, Ng, M);
     colsumsq_f64(s, Q, Ng, Ng, M, red, 0);
     gather_rows_f64(s, KtT, N, bi, nb, Nb, M, nullptr, D, Nb);
-    gemm2_f64(s, 1, 0, Nb, M, Ng, -1.0, m->d(B_AUX), Ng, Q, Ng, 1.0, D, Nb, 0, 0);
+    gemm2_f64(s, 1, 0, Nb, M, Ng, -1.0, m->d(B_AUX), Ng, Q, Ng, 1.0, D, Nb, 0);
     scale_rows_copy_f64(s, D, Nb, Nb, M, m->d(B_IV2), E);
     coldot_f64(s, D, E, Nb, Nb, M, r1);
-    gemm2_f64(s, 1, 0, Nb, M, Nb, 1.0, m->d(B_LK), Nb, E, Nb, 0.0, Hh, Nb, 0, 0);
+    gemm2_f64(s, 1, 0, Nb, M, Nb, 1.0, m->d(B_LK), Nb, E, Nb, 0.0, Hh, Nb, 0);
     trsm_lower(s, m->d(B_AC), Nb, m->d(B_DA), Nb, Hh, Nb, M);
     colsumsq_f64(s, Hh, Nb, Nb, M, r2, 0);
     vec_axpby(s, M, 1.0, r1, -1.0, r2, r1);
