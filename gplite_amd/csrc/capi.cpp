@@ -74,6 +74,10 @@ extern "C" int gpl_ctx_create(int32_t device, gpl_ctx** out) {
     if (e == hipSuccess) e = hipMalloc((void**)&c->dpub, kPanelMaxBlocks * 4096 * sizeof(double));
     if (e == hipSuccess) e = hipMalloc((void**)&c->tsync, kSolveSyncWords * sizeof(unsigned));
     if (e == hipSuccess) e = hipMemset(c->tsync, 0, kSolveSyncWords * sizeof(unsigned));
+    if (e == hipSuccess) e = hipMalloc((void**)&c->msync, (kTrsmFlags + 64) * sizeof(unsigned));
+    if (e == hipSuccess) e = hipMemset(c->msync, 0, (kTrsmFlags + 64) * sizeof(unsigned));
+    if (e == hipSuccess) c->minfo = (int*)(c->msync + kTrsmFlags + 32);
+    if (e == hipSuccess) e = hipHostMalloc((void**)&c->stage, gpl_ctx::kStage * sizeof(double));
     if (const char* pw = getenv("GPL_PANEL_WAIT_POLLS")) c->pwait = (unsigned)strtoul(pw, nullptr, 10);
     if (e != hipSuccess) {
         delete c;
@@ -103,6 +107,8 @@ extern "C" void gpl_ctx_destroy(gpl_ctx* c) {
     if (c->psync) hipFree(c->psync);
     if (c->dpub) hipFree(c->dpub);
     if (c->tsync) hipFree(c->tsync);
+    if (c->msync) hipFree(c->msync);
+    if (c->stage) hipHostFree(c->stage);
     hipStreamDestroy(c->side);
     hipStreamDestroy(c->stream);
     delete c;
@@ -623,6 +629,22 @@ void gpl::trsv_lower(gpl_ctx* c, hipStream_t s, const double* L, int64_t ld, con
     if (++c->pepoch == 0) c->pepoch = 1;
     trsv_persist_f64(s, L, ld, Dinv, N, b, x, trans, c->tsync, c->pepoch, c->tbase, info, c->pwait);
     c->tbase += (unsigned)T;
+}
+
+void gpl::trsm_forward(gpl_ctx* c, hipStream_t s, const double* L, int64_t ld, const double* Dinv, int64_t N, double* B,
+                     int64_t ldb, int64_t M, const double* sv, int64_t n, int* info) {
+    const int64_t T = N / 64;
+    // columns per launch: as many as have flags (a model of more than 65536 row blocks, whose factor alone is
+    // 2^45 bytes, does not exist)
+    int64_t step = M;
+    while (step > 64 && T * (step / trsm_cols(N, step)) > kTrsmFlags) step = (step / 2 + 63) / 64 * 64;
+    for (int64_t j = 0; j < M; j += step) {
+        const int64_t m = std::min(step, M - j);
+        if (++c->pepoch == 0) c->pepoch = 1;
+        trsm_persist_f64(s, L, ld, Dinv, N, B + j * ldb, ldb, m, sv, n, c->msync, c->pepoch, c->mbase, info,
+                         c->pwait);
+        c->mbase += (unsigned)(T * (m / trsm_cols(N, m)));
+    }
 }
 
 // L^-1 S z in W1; then alpha = S L^-T W1.
@@ -1238,12 +1260,12 @@ static int fit_ep(gpl_model* m) {
             form_B_f64(s, m->d(B_K), m->d(B_L), N, n, N, m->d(B_SV));
         }
         potrf_blocked(c, m->d(B_L), N, m->d(B_DINV), m->d(B_LDIAG), flags, nullptr, nullptr, alpha_rhs(m, m->d(B_Z)));
+        trtri_blocked(c, m->d(B_L), m->d(B_DINV), N, m->d(B_XINV));
         solve_alpha_back(c, m, m->d(B_ALPHA));
         {
             Prof p(c, "symv", 2.0 * N * N, 8.0 * N * N / 2);
             symv_lt_f64(s, m->d(B_K), N, m->d(B_ALPHA), m->d(B_FMEAN), m->d(B_KMV), kmatvec_chunks(N), 1, 0, 0);
         }
-        trtri_blocked(c, m->d(B_L), m->d(B_DINV), N, m->d(B_XINV));
         colsumsq_f64(s, m->d(B_XINV), N, N, n, m->d(B_W3), 1);
         ep_post(s, n, m->d(B_V), m->d(B_Z), m->d(B_W3), m->d(B_CAVM), m->d(B_CAVV), m->d(B_LOGZS), m->d(B_FVAR),
                 m->d(B_TERM));
@@ -1651,7 +1673,7 @@ static size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 
 size_t gpl::pred_bufs_bytes(int64_t N, int64_t ncols, int64_t M) {
     return align256((size_t)M * std::max<int64_t>(ncols, 1) * 8) + align256((size_t)M * MAX_FEAT * 8) +
-           2 * align256((size_t)N * M * 8) + align256((size_t)M * 3 * 8);
+           2 * align256((size_t)N * M * 8) + align256(((size_t)M * 4 + 16) * 8);
 }
 
 PredBufs gpl::pred_bufs_carve(void* base, int64_t N, int64_t ncols, int64_t M) {
@@ -1682,6 +1704,14 @@ gpl_model* gpl::model_new(gpl_ctx* c) {
     return m;
 }
 
+// The status word a prediction brings back: a time-out of the solve's device waits
+// (cleared for the calls that follow).
+static int pred_status(gpl_ctx* c, double st) {
+    if (st == 0.0) return GPL_OK;
+    hipMemsetAsync(c->minfo, 0, sizeof(int), c->stream);
+    return gpl::wait_timeout_fail();
+}
+
 // Prediction on the streams of context c (which may differ from the context
 // that fitted the model: the model's device buffers are read-only here).
 int gpl::pred_on(gpl_ctx* c, gpl_model* m, const double* xt, int64_t mt, int32_t want_var, double* mean,
@@ -1706,8 +1736,11 @@ int gpl::pred_on(gpl_ctx* c, gpl_model* m, const double* xt, int64_t mt, int32_t
     double* xtd = pb ? pb->xt : (double*)c->buf(0, (size_t)mt * std::max<int64_t>(m->ncols, 1) * 8);
     double* Ft = pb ? pb->Ft : (double*)c->buf(1, (size_t)M * MAX_FEAT * 8);
     double* KtT = pb ? pb->KtT : (double*)c->buf(2, (size_t)N * M * 8);
-    double* vbuf = pb ? pb->v : (double*)c->buf(3, (size_t)M * 3 * 8);
+    double* vbuf = pb ? pb->v : (double*)c->buf(3, ((size_t)M * 4 + 16) * 8);
     if (!xtd || !Ft || !KtT || !vbuf) return fail(GPL_ERR_OOM, "device allocation failed");
+    // vbuf: the result, mean[mt] var[mt] and the solve's status, then K_tt's diagonal and the variance reduction
+    double* const kd = vbuf + 2 * M + 8;
+    double* const red = kd + M;
     if (mt * m->ncols > 0 && !(pb && pb->staged))
         HIP_TRY(hipMemcpyAsync(xtd, xt, mt * m->ncols * 8, hipMemcpyHostToDevice, s));
     launch_features(s, xtd, mt, mt, (int)m->ncols, pf, m->prog, Ft, M);
@@ -1719,16 +1752,15 @@ int gpl::pred_on(gpl_ctx* c, gpl_model* m, const double* xt, int64_t mt, int32_t
     if (want_var && m->split) {
         // var_reduction = K_t (K + V)^-1 K_t^T of the reference's C_lu branch (R/gp_pred.R:220-223)
         if (pb) return fail(GPL_ERR_UNSUPPORTED, "a fit with split sites (pseudo-variances <= 0) needs gpl_pred");
-        int r = split_var_reduction(c, m, KtT, M, vbuf + M);
+        int r = split_var_reduction(c, m, KtT, M, red);
         if (r) return r;
-        launch_build_diag(s, pd, *hp, Ft, M, Ft, M, mt, vbuf + 2 * M);
-        vec_axpby(s, mt, 1.0, vbuf + 2 * M, -1.0, vbuf + M, vbuf + M);
-        HIP_TRY(hipMemcpyAsync(var, vbuf + M, mt * 8, hipMemcpyDeviceToHost, s));
+        launch_build_diag(s, pd, *hp, Ft, M, Ft, M, mt, kd);
+        vec_axpby(s, mt, 1.0, kd, -1.0, red, red);
+        HIP_TRY(hipMemcpyAsync(var, red, mt * 8, hipMemcpyDeviceToHost, s));
     } else if (want_var) {
         // aux = C^-1 K_t^T = L^-1 (sv .* K_t^T)  (R/gp_pred.R:218)
-        scale_rows_f64(s, KtT, N, n, M, m->d(B_SV));
-        const int64_t T = N / 64;
         if (m->have_xinv) {
+            scale_rows_f64(s, KtT, N, n, M, m->d(B_SV));
             double* A2 = pb ? pb->A2 : (double*)c->buf(4, (size_t)N * M * 8);
             if (!A2) return fail(GPL_ERR_OOM, "device allocation failed");
             Prof p(c, "pred_trmm", (double)N * N * M, 8.0 * N * M * 2);
@@ -1738,24 +1770,25 @@ int gpl::pred_on(gpl_ctx* c, gpl_model* m, const double* xt, int64_t mt, int32_t
                 gemm2_f64(s, 0, 0, N, M, N, 1.0, m->d(B_XINV), N, KtT, N, 0.0, A2, N, 3);
             KtT = A2;
         } else {
-            for (int64_t i = 0; i < T; ++i) {
-                {
-                    Prof p(c, "pred_trsm_diag", 2.0 * 64 * 64 * M, 16.0 * 64 * M);
-                    gemm2_f64(s, 0, 0, 64, M, 64, 1.0, m->d(B_DINV) + i * 64 * 64, 64, KtT + i * 64, N, 0.0,
-                              KtT + i * 64, N, 0);
-                }
-                if (i + 1 < T) {
-                    const int64_t R = (T - 1 - i) * 64;
-                    Prof p(c, "pred_trsm_update", 2.0 * R * M * 64, 16.0 * R * M);
-                    gemm2_f64(s, 0, 0, R, M, 64, -1.0, m->d(B_L) + (i + 1) * 64 + i * 64 * N, N, KtT + i * 64, N,
-                              1.0, KtT + (i + 1) * 64, N, 0);
-                }
-            }
+            Prof p(c, "pred_trsm", (double)N * N * M, 4.0 * N * N + 16.0 * N * M);
+            trsm_forward(c, s, m->d(B_L), N, m->d(B_DINV), N, KtT, N, M, m->d(B_SV), n, c->minfo);
         }
-        colsumsq_f64(s, KtT, N, N, mt, vbuf + M, 0);
-        launch_build_diag(s, pd, *hp, Ft, M, Ft, M, mt, vbuf + 2 * M);
-        vec_axpby(s, mt, 1.0, vbuf + 2 * M, -1.0, vbuf + M, vbuf + M);
-        HIP_TRY(hipMemcpyAsync(var, vbuf + M, mt * 8, hipMemcpyDeviceToHost, s));
+        colsumsq_f64(s, KtT, N, N, mt, red, 0);
+        launch_build_diag(s, pd, *hp, Ft, M, Ft, M, mt, kd);
+        pred_finish(s, mt, kd, red, c->minfo, vbuf);
+        if (2 * mt + 1 <= gpl_ctx::kStage) {  // one copy through pinned memory
+            HIP_TRY(hipMemcpyAsync(c->stage, vbuf, (2 * mt + 1) * 8, hipMemcpyDeviceToHost, s));
+            HIP_TRY(hipStreamSynchronize(s));
+            memcpy(mean, c->stage, mt * 8);
+            memcpy(var, c->stage + mt, mt * 8);
+            return pred_status(c, c->stage[2 * mt]);
+        }
+        double st;
+        HIP_TRY(hipMemcpyAsync(var, vbuf + mt, mt * 8, hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipMemcpyAsync(&st, vbuf + 2 * mt, 8, hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipMemcpyAsync(mean, vbuf, mt * 8, hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipStreamSynchronize(s));
+        return pred_status(c, st);
     }
     HIP_TRY(hipMemcpyAsync(mean, vbuf, mt * 8, hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
@@ -1803,21 +1836,15 @@ static int draw_on(gpl_ctx* c, gpl_model* m, const double* xt, int64_t mt, doubl
     launch_features(s, xtd, mt, mt, (int)m->ncols, pf, m->prog, Ft, M);
     launch_build_cross(s, pd, *hp, m->d(B_F), N, n, N, Ft, M, mt, M, KtT, N);
     gemv_t_f64(s, KtT, N, N, mt, m->d(B_ALPHA), vbuf);
-    scale_rows_f64(s, KtT, N, n, M, m->d(B_SV));
-    const int64_t T = N / 64;
+    HIP_TRY(hipMemsetAsync(info, 0, 64, s));
     if (m->have_xinv) {
+        scale_rows_f64(s, KtT, N, n, M, m->d(B_SV));
         if (m->opts.precision == GPL_PREC_MIXED)
             gemm_mixed_f32f64f64(s, 0, 0, N, M, N, 1.0, m->b[B_XINV].as<float>(), N, KtT, N, 0.0, A2, N, 3);
         else
             gemm2_f64(s, 0, 0, N, M, N, 1.0, m->d(B_XINV), N, KtT, N, 0.0, A2, N, 3);
     } else {
-        for (int64_t i = 0; i < T; ++i) {
-            gemm2_f64(s, 0, 0, 64, M, 64, 1.0, m->d(B_DINV) + i * 64 * 64, 64, KtT + i * 64, N, 0.0, KtT + i * 64, N,
-                      0);
-            if (i + 1 < T)
-                gemm2_f64(s, 0, 0, (T - 1 - i) * 64, M, 64, -1.0, m->d(B_L) + (i + 1) * 64 + i * 64 * N, N,
-                          KtT + i * 64, N, 1.0, KtT + (i + 1) * 64, N, 0);
-        }
+        trsm_forward(c, s, m->d(B_L), N, m->d(B_DINV), N, KtT, N, M, m->d(B_SV), n, info);
         A2 = KtT;
     }
     // cov = K_tt + jitter I - aux^T aux over lower tiles (padding: identity), then its factor
@@ -1826,7 +1853,6 @@ static int draw_on(gpl_ctx* c, gpl_model* m, const double* xt, int64_t mt, doubl
         Prof p(c, "draw_cov", (double)M * M * N, 8.0 * N * M);
         gemm2_f64(s, 1, 0, M, M, N, -1.0, A2, N, A2, N, 1.0, Cv, M, 1);
     }
-    HIP_TRY(hipMemsetAsync(info, 0, 64, s));
     potrf_blocked(c, Cv, M, Dv, ld, info);
     int inf = 0;
     HIP_TRY(hipMemcpyAsync(&inf, info, 4, hipMemcpyDeviceToHost, s));
@@ -1841,6 +1867,7 @@ static int draw_on(gpl_ctx* c, gpl_model* m, const double* xt, int64_t mt, doubl
     HIP_TRY(hipMemcpyAsync(mean.data(), vbuf, mt * 8, hipMemcpyDeviceToHost, s));
     HIP_TRY(download_2d(c, s, out, Wd, M, mt, draws, 21));
     HIP_TRY(hipStreamSynchronize(s));
+    if (inf == kPanelWaitTimeout) return wait_timeout_fail();
     if (inf > 0) {
         set_minor(inf);
         return fail(GPL_ERR_NOT_PD, "predictive covariance: the leading minor of order " + std::to_string(inf) +

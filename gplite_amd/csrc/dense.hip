@@ -1198,6 +1198,190 @@ void trsv_persist_f64(hipStream_t s, const double* L, int64_t ld, const double* 
 }
 
 // ---------------------------------------------------------------------------
+// L Y = S B for many right-hand sides in one launch, in place (B: ldb x M, column
+// major, M a multiple of 64; S = diag(sv) on the first n rows, or none).  A
+// workgroup per 64-row block i and WN columns j, in ticket order of the row
+// blocks: it sums L_{ik} Y_{kj} over k < i as the blocks Y_{kj} are published
+// (operands straight from global memory, those of the next block loaded ahead),
+// forms Y_{ij} = Dinv_i (S_i B_{ij} - sum) and publishes it.  Every wait is on a
+// block of a lower ticket; the order of the sums is fixed.
+//
+// Bound by N/64 dependent blocks (a hand-over, one 64 x 64 x WN product and one
+// with the inverse each) for few columns, by its products for many.  In launches
+// of their own, two per 64 rows, the same steps took 7 us (13 before the products
+// lost their LDS staging) each: 1000 points on n = 4096 1.18 ms of the 1.47.
+//
+// sync: flags [0, T ncol) (i ncol + j), ncol = M / WN, the ticket counter at
+// sync[kTrsmFlags].
+// ---------------------------------------------------------------------------
+template <int WN>
+__global__ __launch_bounds__(256) void k_trsm_persist(const double* __restrict__ L, int64_t ld,
+                                                      const double* __restrict__ Dinv, double* B, int64_t ldb,
+                                                      int ncol, const double* __restrict__ sv, int64_t n,
+                                                      unsigned* __restrict__ sync, unsigned epoch, unsigned base,
+                                                      int* __restrict__ info, unsigned maxpoll) {
+    constexpr int NR = WN == 16 ? 1 : 2, NC = WN == 16 ? 1 : 2;  // 16x16 tiles of a wave
+    constexpr int RP = 66;
+    __shared__ double R[WN][RP];
+    __shared__ unsigned s_id;
+    __shared__ int s_ready;
+    const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+    if (t == 0) s_id = atomicAdd(&sync[kTrsmFlags], 1u) - base;
+    __syncthreads();
+    const int id = __builtin_amdgcn_readfirstlane((int)s_id), i = id / ncol, j = id % ncol;
+    const int li = lane & 15, g = lane >> 4;
+    // this wave's rows and columns of the 64 x WN block
+    const int r0 = WN == 16 ? 16 * w : 32 * (w & 1), c0 = WN == 16 ? 0 : 32 * (w >> 1);
+    const int ra = r0 + frag_row<false, NR>(0, li);
+    const double* pa = L + 64 * (int64_t)i + ra + 4 * g * ld;                // row ra of L_{i,0}, k = 4g
+    const double* pb = B + 4 * g + (WN * (int64_t)j + c0 + li) * ldb;        // column of Y_{0,j}, k = 4g
+    const double* pd = Dinv + 4096 * (int64_t)i + ra + 4 * g * 64;
+    double* pc = B + 64 * (int64_t)i + (WN * (int64_t)j) * ldb;
+    double bv[NR][NC][4];
+#pragma unroll
+    for (int a = 0; a < NR; ++a)
+#pragma unroll
+        for (int b = 0; b < NC; ++b)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int row = r0 + frag_row<false, NR>(a, li), col = c0 + 16 * b + g + 4 * v;
+                const int64_t gr = 64 * (int64_t)i + row;
+                bv[a][b][v] = pc[row + col * ldb] * (sv && gr < n ? sv[gr] : 1.0);
+            }
+    d4 acc[NR][NC];
+#pragma unroll
+    for (int a = 0; a < NR; ++a)
+#pragma unroll
+        for (int b = 0; b < NC; ++b) acc[a][b] = d4{0.0, 0.0, 0.0, 0.0};
+    double fa[2][4][NR][4], fb[2][4][NC][4];  // two 64-k blocks of each operand, in 16-k chunks
+    auto load_a = [&](int st, int k) {  // L_{ik}; for k = i the inverse of the diagonal block
+        const double* q = k < i ? pa + 64 * (int64_t)k * ld : pd;
+        const int64_t l = k < i ? ld : 64;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) frag_load<false, NR>(fa[st][c], q + 16 * c * l, l);
+    };
+    auto load_b = [&](int st, int k) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) frag_load<true, NC>(fb[st][c], pb + 64 * k + 16 * c, ldb);
+    };
+    auto mult = [&](int st) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+#pragma unroll
+                for (int a = 0; a < NR; ++a)
+#pragma unroll
+                    for (int b = 0; b < NC; ++b)
+                        acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(fb[st][c][b][s], fa[st][c][a][s], acc[a][b],
+                                                                         0, 0, 0);
+    };
+    load_a(0, 0);
+    int ready = 0;  // blocks below this one are published
+    bool have = false;
+    for (int k0 = 0; k0 < i; k0 += 2)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int k = k0 + u;
+            if (k >= i) break;
+            if (k >= ready) {
+                if (t < 64) {  // how many blocks from k on are published
+                    const int kk = k + lane < i ? k + lane : i - 1;
+                    unsigned long long miss = ~0ull;
+                    for (unsigned p = 0; p < maxpoll; ++p) {
+                        miss = __ballot(__hip_atomic_load(&sync[kk * ncol + j], __ATOMIC_RELAXED,
+                                                          __HIP_MEMORY_SCOPE_AGENT) != epoch);
+                        if (!(miss & 1)) break;
+                        __builtin_amdgcn_s_sleep(1);
+                    }
+                    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+                    const int cnt = miss ? __ffsll((long long)miss) - 1 : 64;
+                    if (t == 0) {
+                        s_ready = cnt ? (k + cnt < i ? k + cnt : i) : -1;
+                        if (!cnt) atomicCAS(info, 0, kPanelWaitTimeout);
+                    }
+                }
+                __syncthreads();
+                ready = __builtin_amdgcn_readfirstlane(s_ready);
+                __syncthreads();
+                if (ready < 0) return;
+            }
+            if (!have) load_b(u, k);
+            have = k + 1 < ready;
+            if (have) load_b(u ^ 1, k + 1);
+            load_a(u ^ 1, k + 1);
+            mult(u);
+        }
+    // R = S_i B_ij - sum, then Y_ij = Dinv_i R (the inverse's operand was loaded last)
+#pragma unroll
+    for (int a = 0; a < NR; ++a)
+#pragma unroll
+        for (int b = 0; b < NC; ++b)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                R[c0 + 16 * b + g + 4 * v][r0 + frag_row<false, NR>(a, li)] = bv[a][b][v] - acc[a][b][v];
+    __syncthreads();
+#pragma unroll
+    for (int a = 0; a < NR; ++a)
+#pragma unroll
+        for (int b = 0; b < NC; ++b) acc[a][b] = d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int b = 0; b < NC; ++b)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) fb[0][c][b][s] = R[c0 + 16 * b + li][16 * c + 4 * g + s];
+    if (i & 1) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int a = 0; a < NR; ++a)
+#pragma unroll
+                for (int s = 0; s < 4; ++s) fa[0][c][a][s] = fa[1][c][a][s];
+    }
+    mult(0);
+#pragma unroll
+    for (int a = 0; a < NR; ++a)
+#pragma unroll
+        for (int b = 0; b < NC; ++b)
+#pragma unroll
+            for (int v = 0; v < 4; ++v)
+                put_shared(pc + r0 + frag_row<false, NR>(a, li) + (c0 + 16 * b + g + 4 * v) * ldb, (double)acc[a][b][v]);
+    panel_publish(&sync[i * ncol + j], epoch);
+}
+
+// 16 columns a workgroup while the chain of row blocks is what takes the time (4 us
+// a block against 8 with 64 columns), 64 once the products are (a quarter of the
+// reads of L).  A whole prediction with 16 / 64, us: n = 640 m = 4096 265 / 274;
+// n = 2048 m = 1000 351 / 428, m = 2000 543 / 448; n = 4096 m = 500 582 / 608,
+// m = 1000 903 / 686.
+int trsm_cols(int64_t N, int64_t M) { return N * M <= 3000000 ? 16 : 64; }
+
+void trsm_persist_f64(hipStream_t s, const double* L, int64_t ld, const double* Dinv, int64_t N, double* B, int64_t ldb,
+                      int64_t M, const double* sv, int64_t n, unsigned* sync, unsigned epoch, unsigned base, int* info,
+                      unsigned maxpoll) {
+    const int wn = trsm_cols(N, M), ncol = (int)(M / wn);
+    const dim3 grid((unsigned)(N / 64 * ncol));
+    if (wn == 16)
+        hipLaunchKernelGGL(k_trsm_persist<16>, grid, dim3(256), 0, s, L, ld, Dinv, B, ldb, ncol, sv, n, sync, epoch,
+                           base, info, maxpoll);
+    else
+        hipLaunchKernelGGL(k_trsm_persist<64>, grid, dim3(256), 0, s, L, ld, Dinv, B, ldb, ncol, sv, n, sync, epoch,
+                           base, info, maxpoll);
+}
+
+__global__ void k_pred_finish(int64_t mt, const double* __restrict__ kd, const double* __restrict__ red,
+                              const int* __restrict__ info, double* __restrict__ out) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < mt) out[mt + i] = kd[i] - red[i];
+    if (i == 0) out[2 * mt] = (double)*info;
+}
+
+void pred_finish(hipStream_t s, int64_t mt, const double* kd, const double* red, const int* info, double* out) {
+    hipLaunchKernelGGL(k_pred_finish, dim3((unsigned)((mt + 255) / 256)), dim3(256), 0, s, mt, kd, red, info, out);
+}
+
+// ---------------------------------------------------------------------------
 // Triangular / symmetric matrix-vector products over lower tiles.  One
 // workgroup per 64-row output block, fixed summation order (deterministic).
 // ---------------------------------------------------------------------------

@@ -157,7 +157,16 @@ constexpr int kSolveSyncWords = kSolveMaxBlocks + 1;
 void trsv_persist_f64(hipStream_t s, const double* L, int64_t ld, const double* Dinv, int64_t N, const double* b,
                       double* x, int trans, unsigned* sync, unsigned epoch, unsigned base, int* info,
                       unsigned maxpoll);
-// the same on FP32 storage with the FP64 diagonal tiles Dacc (mixed precision)
+// L Y = diag(sv) B in place for M right-hand sides (multiples of 64) in one launch; sync: kTrsmFlags + 1 words
+// of the context, N / 64 * (M / trsm_cols(N, M)) <= kTrsmFlags flags and as many tickets per launch
+constexpr int kTrsmFlags = 65536;
+int trsm_cols(int64_t N, int64_t M);
+void trsm_persist_f64(hipStream_t s, const double* L, int64_t ld, const double* Dinv, int64_t N, double* B, int64_t ldb,
+                      int64_t M, const double* sv, int64_t n, unsigned* sync, unsigned epoch, unsigned base, int* info,
+                      unsigned maxpoll);
+// out[mt + i] = kd[i] - red[i], out[2 mt] = *info (the end of a prediction with variances)
+void pred_finish(hipStream_t s, int64_t mt, const double* kd, const double* red, const int* info, double* out);
+// the panel on FP32 storage with the FP64 diagonal tiles Dacc (mixed precision)
 void potrf_panel_mixed(hipStream_t s, float* A, int64_t ld, int64_t K0, int nc, int64_t nrb, double* Dinv,
                        double* ldiag, int* info, unsigned* sync, unsigned epoch, unsigned base, double* Dacc,
                        unsigned maxpoll);

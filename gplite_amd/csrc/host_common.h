@@ -40,6 +40,11 @@ void trtri_blocked(gpl_ctx* c, const double* L, const double* Dinv, int64_t N, d
 // if a device wait times out.
 void trsv_lower(gpl_ctx* c, hipStream_t s, const double* L, int64_t ld, const double* Dinv, int64_t N, double* b,
                 double* x, int trans, int* info);
+// L Y = diag(sv) B in place for M right-hand sides (sv: the first n rows, or null): the forward solve of a
+// prediction, in launches of at most kTrsmFlags blocks.  info receives kPanelWaitTimeout if a device wait
+// times out.
+void trsm_forward(gpl_ctx* c, hipStream_t s, const double* L, int64_t ld, const double* Dinv, int64_t N, double* B,
+                int64_t ldb, int64_t M, const double* sv, int64_t n, int* info);
 // the error reported for an info word of kPanelWaitTimeout
 int wait_timeout_fail();
 // probabilists' Gauss-Hermite nodes and weights normalised to sum 1 (R/quadrature.R:1-44)
@@ -109,6 +114,14 @@ struct gpl_ctx {
     // launches take their epochs from pepoch too)
     unsigned* tsync = nullptr;
     unsigned tbase = 0;
+    // and of the solve with many right-hand sides (kTrsmFlags + 1 words), with an
+    // info word for its time-outs
+    unsigned* msync = nullptr;
+    unsigned mbase = 0;
+    int* minfo = nullptr;
+    // pinned host memory that the results of a call cross in one copy
+    static constexpr int64_t kStage = 8200;
+    double* stage = nullptr;
     unsigned pwait = 1u << 20;
     bool prof = false;
     std::vector<ProfRec> pending;
