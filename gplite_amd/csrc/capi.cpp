@@ -258,9 +258,6 @@ int gpl::prepare_prog(const gpl_cf_term* terms, int32_t nterms, int64_t ncols, D
     return GPL_OK;
 }
 
-// Outer row-panel height of the forward-substitution inverse (trtri_blocked
-// without scratch): 256 rows in 64-row steps.
-static const int kOuterNB = 256;
 // Outer block of the right-looking Cholesky drivers: its columns are factored by
 // panel launches (k_potrf_panel), then the trailing matrix receives one update of
 // that depth.  FP64: two launches of kPanelW = 256 columns, the second after an
@@ -280,31 +277,50 @@ static const int kPanelNB32 = 64 * kPanelBlocksF32;
 // is two batched GEMMs (plus one more pair when the last is shorter): with
 // N/64 diagonal blocks the dependent chain is 2 log2(N/64) launches, against
 // two launches per 64 rows for forward substitution.  Both triangular operands
-// skip their zero tiles (tile modes 4 and 3).  T (N x N, ld N) holds the
-// products L21 X11 at the positions of X21.  FP64 (T = double) or FP32 storage
-// (float: FP32 MFMA with sums folded into FP64 every 64 k, FP64 leaves rounded).
+// skip their zero tiles.  The products T = L21 X11 lie in Tm (N x N, ld N) at the
+// positions of X21 or, without Tm (double only), transposed in X itself, at the
+// mirrored positions above its diagonal, which clear_upper_f64 sets to zero at the
+// end.  FP64 (T = double) or FP32 storage (float: FP32 MFMA with sums folded into
+// FP64 every 64 k, FP64 leaves rounded).
 //
 // The work splits at the top level bt = doubling_top(N): the inverse of the
 // diagonal block [0, bt) and T = L21 X11 below it (dbl_front) need only the
 // factor's first bt columns, so the blocked Cholesky can run them on the
 // context's third stream beside its remaining panels; the inverse of [bt, N)
 // and X21 = -X22 T (dbl_back) follow the factorization.
-static void dbl_leaves(hipStream_t s, double* X, int64_t N, const double* Dinv, int64_t c0, int64_t n) {
-    trtri_leaves_f64(s, X, N, Dinv, c0, n);
+static void dbl_leaves(hipStream_t s, double* X, int64_t N, const double* Dinv, int64_t c0, int64_t n, bool clear) {
+    trtri_leaves_f64(s, X, N, Dinv, c0, n, clear ? 1 : 0);
 }
-static void dbl_leaves(hipStream_t s, float* X, int64_t N, const double* Dinv, int64_t c0, int64_t n) {
+static void dbl_leaves(hipStream_t s, float* X, int64_t N, const double* Dinv, int64_t c0, int64_t n, bool) {
     trtri_leaves_f32_batched(s, X, N, Dinv, 1, 0, 0, c0, n);
 }
-static void dbl_gemm(hipStream_t s, int64_t M, int64_t Nn, int64_t K, double alpha, const double* A, const double* B,
-                     double* C, int64_t ld, int tiles, int64_t batch, int64_t step, double beta = 0.0) {
-    if (batch == 1) gemm2_f64(s, 0, 0, M, Nn, K, alpha, A, ld, B, ld, beta, C, ld, tiles);
-    else gemm2_f64_batched(s, 0, 0, M, Nn, K, alpha, A, ld, B, ld, beta, C, ld, tiles, (int)batch, step, step, step);
+static void dbl_gemm(hipStream_t s, int ta, int tb, int64_t M, int64_t Nn, int64_t K, double alpha, const double* A,
+                     const double* B, double* C, int64_t ld, int tiles, int64_t batch, int64_t step, double beta) {
+    gemm2_f64_batched(s, ta, tb, M, Nn, K, alpha, A, ld, B, ld, beta, C, ld, tiles, (int)batch, step, step, step);
 }
-static void dbl_gemm(hipStream_t s, int64_t M, int64_t Nn, int64_t K, double alpha, const float* A, const float* B,
-                     float* C, int64_t ld, int tiles, int64_t batch, int64_t step, double beta = 0.0) {
-    gemm_f32_batched(s, 0, 0, M, Nn, K, (float)alpha, A, ld, B, ld, (float)beta, C, ld, tiles, 0, (int)batch, step,
+static void dbl_gemm(hipStream_t s, int ta, int tb, int64_t M, int64_t Nn, int64_t K, double alpha, const float* A,
+                     const float* B, float* C, int64_t ld, int tiles, int64_t batch, int64_t step, double beta) {
+    gemm_f32_batched(s, ta, tb, M, Nn, K, (float)alpha, A, ld, B, ld, (float)beta, C, ld, tiles, 0, (int)batch, step,
                      step, step, kFoldInverse);
 }
+// T(i.., j..) = L21 X11 (r x b), X11 = X(j.., j..) lower triangular
+template <typename T>
+static void dbl_prod(hipStream_t s, int64_t r, int64_t b, const T* L, int64_t N, T* X, T* Tm, int64_t i, int64_t j,
+                     int64_t batch = 1, int64_t step = 0) {
+    const T *L21 = L + i + j * N, *X11 = X + j + j * N;
+    if (Tm) dbl_gemm(s, 0, 0, r, b, b, 1.0, L21, X11, Tm + i + j * N, N, 4, batch, step, 0.0);
+    else dbl_gemm(s, 1, 1, b, r, b, 1.0, X11, L21, X + j + i * N, N, 5, batch, step, 0.0);
+}
+// C = beta C - A T(i.., j..), C (M x n), K rows of T
+template <typename T>
+static void dbl_apply(hipStream_t s, int64_t M, int64_t n, int64_t K, const T* A, int64_t N, T* X, T* Tm, int64_t i,
+                      int64_t j, T* C, int tiles, int64_t batch = 1, int64_t step = 0, double beta = 0.0) {
+    const T* P = Tm ? Tm + i + j * N : X + j + i * N;
+    dbl_gemm(s, 0, Tm ? 0 : 1, M, n, K, -1.0, A, P, C, N, tiles, batch, step, beta);
+}
+
+static void dbl_clear(hipStream_t s, double* X, int64_t N) { clear_upper_f64(s, X, N); }
+static void dbl_clear(hipStream_t, float*, int64_t) {}
 
 // the leaves (columns r0 .. r0 + n) and the levels inside the diagonal block
 // [r0, r0 + n); r0 is 0 or bt, a multiple of 2b for every level run
@@ -314,27 +330,21 @@ static void dbl_levels(gpl_ctx* c, hipStream_t s, const T* L, const double* Dinv
     const bool f32 = sizeof(T) == 4;
     {
         Prof p(c, f32 ? "trtri_leaves_f32" : "trtri_leaves", 0, sizeof(T) * (double)N * n / 2, s);
-        dbl_leaves(s, X, N, Dinv, r0, n);
+        dbl_leaves(s, X, N, Dinv, r0, n, Tm != nullptr);
     }
-    const int64_t o0 = r0 * (N + 1);
-    L += o0;
-    X += o0;
-    Tm += o0;
     for (int64_t b = 64; b < n; b *= 2) {
         const int64_t full = n / (2 * b);  // pairs whose right block has b rows
         const int64_t r = std::min<int64_t>(b, n - full * 2 * b - b);  // rows of a last, shorter right block
         const int64_t step = 2 * b * (N + 1);
         Prof p(c, f32 ? "trtri_level_f32" : "trtri_level",
                2.0 * (double)b * b * b * full + (r > 0 ? (double)r * b * (b + r) : 0.0), 0, s);
-        if (full > 0) {
-            dbl_gemm(s, b, b, b, 1.0, L + b, X, Tm + b, N, 4, full, step);
-            dbl_gemm(s, b, b, b, -1.0, X + b * (N + 1), Tm + b, X + b, N, 3, full, step);
-        }
-        if (r > 0) {
-            const int64_t o = full * step;  // the last pair's top-left corner
-            dbl_gemm(s, r, b, b, 1.0, L + o + b, X + o, Tm + o + b, N, 4, 1, 0);
-            dbl_gemm(s, r, b, r, -1.0, X + o + b * (N + 1), Tm + o + b, X + o + b, N, 3, 1, 0);
-        }
+        auto pair = [&](int64_t j, int64_t rows, int64_t batch) {  // X11 at (j, j), X22 at (j + b, j + b)
+            const int64_t i = j + b;
+            dbl_prod(s, rows, b, L, N, X, Tm, i, j, batch, step);
+            dbl_apply(s, rows, b, rows, X + i * (N + 1), N, X, Tm, i, j, X + i + j * N, 3, batch, step);
+        };
+        if (full > 0) pair(r0, b, full);
+        if (r > 0) pair(r0 + full * 2 * b, r, 1);
     }
 }
 
@@ -342,14 +352,14 @@ template <typename T>
 static void dbl_front(gpl_ctx* c, hipStream_t s, const T* L, const double* Dinv, int64_t N, T* X, T* Tm, int64_t bt) {
     dbl_levels(c, s, L, Dinv, N, X, Tm, 0, bt);
     Prof p(c, sizeof(T) == 4 ? "trtri_level_f32" : "trtri_level", (double)(N - bt) * bt * bt, 0, s);
-    dbl_gemm(s, N - bt, bt, bt, 1.0, L + bt, X, Tm + bt, N, 4, 1, 0);
+    dbl_prod(s, N - bt, bt, L, N, X, Tm, bt, 0);
 }
 
 template <typename T>
 static void dbl_back(gpl_ctx* c, hipStream_t s, const T* L, const double* Dinv, int64_t N, T* X, T* Tm, int64_t bt) {
     dbl_levels(c, s, L, Dinv, N, X, Tm, bt, N - bt);
     Prof p(c, sizeof(T) == 4 ? "trtri_level_f32" : "trtri_level", (double)(N - bt) * (N - bt) * bt, 0, s);
-    dbl_gemm(s, N - bt, bt, N - bt, -1.0, X + bt * (N + 1), Tm + bt, X + bt, N, 3, 1, 0);
+    dbl_apply(s, N - bt, bt, N - bt, X + bt * (N + 1), N, X, Tm, bt, 0, X + bt, 3);
 }
 
 template <typename T>
@@ -401,31 +411,33 @@ struct InverseFork {
             hipStream_t a = c->aux;
             dbl_levels(c, a, L, Dinv, N, X, Tm, bt, h2);
             Prof p(c, sizeof(T) == 4 ? "trtri_level_f32" : "trtri_level", (double)r2 * h2 * h2 + (double)h2 * h2 * bt, 0, a);
-            dbl_gemm(a, r2, h2, h2, 1.0, L + bt2 + bt * N, X + bt * (N + 1), Tm + bt2 + bt * N, N, 4, 1, 0);
-            dbl_gemm(a, h2, bt, h2, -1.0, X + bt * (N + 1), Tm + bt, X + bt, N, 3, 1, 0);
+            dbl_prod(a, r2, h2, L, N, X, Tm, bt2, bt);
+            dbl_apply(a, h2, bt, h2, X + bt * (N + 1), N, X, Tm, bt, 0, X + bt, 3);
             hipEventRecord(c->ev_t, a);
             forked2 = true;
         }
     }
     void finish() {
         if (!X) return;
-        if (bt == 0) {
-            dbl_levels(c, c->stream, L, Dinv, N, X, Tm, 0, N);
-            return;
-        }
-        hipStreamWaitEvent(c->stream, c->ev_t, 0);
-        if (!forked2) {
-            dbl_back(c, c->stream, L, Dinv, N, X, Tm, bt);
-            return;
-        }
         hipStream_t s = c->stream;
-        const int64_t h2 = bt2 - bt, r2 = N - bt2;
-        dbl_levels(c, s, L, Dinv, N, X, Tm, bt2, r2);
-        Prof p(c, sizeof(T) == 4 ? "trtri_level_f32" : "trtri_level",
-               (double)r2 * r2 * h2 + 2.0 * r2 * h2 * bt + (double)r2 * r2 * bt, 0, s);
-        dbl_gemm(s, r2, h2, r2, -1.0, X + bt2 * (N + 1), Tm + bt2 + bt * N, X + bt2 + bt * N, N, 3, 1, 0);
-        dbl_gemm(s, r2, bt, h2, -1.0, X + bt2 + bt * N, Tm + bt, X + bt2, N, 0, 1, 0);
-        dbl_gemm(s, r2, bt, r2, -1.0, X + bt2 * (N + 1), Tm + bt2, X + bt2, N, 3, 1, 0, 1.0);
+        if (bt == 0) {
+            dbl_levels(c, s, L, Dinv, N, X, Tm, 0, N);
+            return;
+        }
+        hipStreamWaitEvent(s, c->ev_t, 0);
+        if (!forked2) {
+            dbl_back(c, s, L, Dinv, N, X, Tm, bt);
+        } else {
+            const int64_t h2 = bt2 - bt, r2 = N - bt2;
+            dbl_levels(c, s, L, Dinv, N, X, Tm, bt2, r2);
+            Prof p(c, sizeof(T) == 4 ? "trtri_level_f32" : "trtri_level",
+                   (double)r2 * r2 * h2 + 2.0 * r2 * h2 * bt + (double)r2 * r2 * bt, 0, s);
+            const T* C22 = X + bt2 * (N + 1);
+            dbl_apply(s, r2, h2, r2, C22, N, X, Tm, bt2, bt, X + bt2 + bt * N, 3);
+            dbl_apply(s, r2, bt, h2, X + bt2 + bt * N, N, X, Tm, bt, 0, X + bt2, 0);
+            dbl_apply(s, r2, bt, r2, C22, N, X, Tm, bt2, 0, X + bt2, 3, 1, 0, 1.0);
+        }
+        if (!Tm) dbl_clear(s, X, N);
     }
 };
 
@@ -493,56 +505,10 @@ void gpl::potrf_blocked(gpl_ctx* c, double* L, int64_t N, double* Dinv, double* 
     inv.finish();
 }
 
-// Rows [I0, I0+H) of X = L^-1: 64-row steps inside the panel, on stream st.
-static void trtri_panel(gpl_ctx* c, hipStream_t st, const double* L, const double* Dinv, int64_t N, int64_t I0,
-                        int64_t H, double* X) {
-    for (int64_t r0 = I0; r0 < I0 + H; r0 += 64) {
-        const int64_t i = r0 / 64, Wc = r0 + 64;  // columns 0 .. r0+63 are non-zero
-        {
-            Prof p(c, "trtri_diag", 2.0 * 64 * 64 * Wc, 16.0 * 64 * Wc, st);
-            gemm2_f64(st, 0, 0, 64, Wc, 64, 1.0, Dinv + i * 64 * 64, 64, X + r0, N, 0.0, X + r0, N, 0);
-        }
-        const int64_t Mr = I0 + H - (r0 + 64);
-        if (Mr > 0) {
-            Prof p(c, "trtri_panel", 2.0 * Mr * Wc * 64, 16.0 * Mr * Wc, st);
-            gemm2_f64(st, 0, 0, Mr, Wc, 64, -1.0, L + (r0 + 64) + r0 * N, N, X + r0, N, 1.0, X + r0 + 64, N, 0);
-        }
-    }
-}
-
-// X = L^-1 by blocked forward substitution against the identity, two levels with
-// look-ahead: the next row panel is updated first and solved on the side stream
-// while the main stream updates the remaining rows.  With scratch T (N x N) the
-// recursive doubling above runs instead.
+// X = L^-1 of a finished factor, with scratch T (N x N) or without
 void gpl::trtri_blocked(gpl_ctx* c, const double* L, const double* Dinv, int64_t N, double* X, double* T) {
-    if (T) {
-        trtri_doubling(c, c->stream, L, Dinv, N, X, T);
-        return;
-    }
-    hipStream_t s = c->stream, s2 = c->side;
-    set_identity_f64(s, X, N, N);
-    trtri_panel(c, s, L, Dinv, N, 0, std::min<int64_t>(kOuterNB, N), X);
-    for (int64_t I0 = 0; I0 < N; I0 += kOuterNB) {
-        const int64_t H = std::min<int64_t>(kOuterNB, N - I0);
-        const int64_t I1 = I0 + H, R = N - I1;
-        if (R <= 0) break;
-        const int64_t H1 = std::min<int64_t>(kOuterNB, R);
-        const int64_t Wc = I0 + H;
-        {
-            Prof p(c, "trtri_update", 2.0 * H1 * Wc * H, 8.0 * (2.0 * H1 * Wc + Wc * H), s);
-            gemm2_f64(s, 0, 0, H1, Wc, H, -1.0, L + I1 + I0 * N, N, X + I0, N, 1.0, X + I1, N, 0);
-        }
-        hipEventRecord(c->ev_a, s);
-        hipStreamWaitEvent(s2, c->ev_a, 0);
-        trtri_panel(c, s2, L, Dinv, N, I1, H1, X);
-        hipEventRecord(c->ev_p, s2);
-        const int64_t R2 = R - H1;
-        if (R2 > 0) {
-            Prof p(c, "trtri_update", 2.0 * R2 * Wc * H, 8.0 * (2.0 * R2 * Wc + Wc * H), s);
-            gemm2_f64(s, 0, 0, R2, Wc, H, -1.0, L + (I1 + H1) + I0 * N, N, X + I0, N, 1.0, X + I1 + H1, N, 0);
-        }
-        hipStreamWaitEvent(s, c->ev_p, 0);
-    }
+    trtri_doubling(c, c->stream, L, Dinv, N, X, T);
+    if (!T) clear_upper_f64(c->stream, X, N);
 }
 
 // ---------------------------------------------------------------------------
@@ -1259,8 +1225,9 @@ static int fit_ep(gpl_model* m) {
             Prof p(c, "form_B", 0, 16.0 * N * (N + 64) / 2);
             form_B_f64(s, m->d(B_K), m->d(B_L), N, n, N, m->d(B_SV));
         }
-        potrf_blocked(c, m->d(B_L), N, m->d(B_DINV), m->d(B_LDIAG), flags, nullptr, nullptr, alpha_rhs(m, m->d(B_Z)));
-        trtri_blocked(c, m->d(B_L), m->d(B_DINV), N, m->d(B_XINV));
+        // X = L^-1 for the posterior variances: its front half beside the factor, no scratch
+        potrf_blocked(c, m->d(B_L), N, m->d(B_DINV), m->d(B_LDIAG), flags, m->d(B_XINV), nullptr,
+                      alpha_rhs(m, m->d(B_Z)));
         solve_alpha_back(c, m, m->d(B_ALPHA));
         {
             Prof p(c, "symv", 2.0 * N * N, 8.0 * N * N / 2);

@@ -104,12 +104,12 @@ __global__ __launch_bounds__(256) void k_gemm_reg(int64_t M, int64_t N, int64_t 
     B += blockIdx.y * sB;
     C += blockIdx.y * sC;
     // Contiguous tile ranges per XCD share operand panels in L2; with a k range
-    // that depends on the tile row (tiles == 2) or column (tiles == 4, whose
+    // that depends on the tile row (tiles == 2, 5) or column (tiles == 4, whose
     // columns are contiguous in the tile order) work per tile varies widely, so
     // the hardware's round-robin placement is kept there to balance the XCDs.
-    const int64_t bid = (tiles == 2 || tiles == 4) ? (int64_t)blockIdx.x : xcd_remap(blockIdx.x, gridDim.x);
+    const int64_t bid = (tiles == 2 || tiles >= 4) ? (int64_t)blockIdx.x : xcd_remap(blockIdx.x, gridDim.x);
     int64_t ti, tj;
-    if (tiles == 0 || tiles == 3 || tiles == 4) {
+    if (tiles != 1 && tiles != 2) {
         ti = bid % tilesM;
         tj = bid / tilesM;
         if (tiles == 3) ti = tilesM - 1 - ti;  // the longest k ranges first
@@ -125,7 +125,7 @@ __global__ __launch_bounds__(256) void k_gemm_reg(int64_t M, int64_t N, int64_t 
     const int64_t row0 = ti * BM + (w & 1) * WT, col0 = tj * BM + (w >> 1) * WT;
     if (row0 >= M || col0 >= N) return;
     if ((tiles == 1 || tiles == 2) && row0 / 64 < col0 / 64) return;  // above the diagonal tiles
-    const int64_t kbeg = (tiles == 2) ? row0 / 64 * 64 : (tiles == 4) ? col0 / 64 * 64 : 0;
+    const int64_t kbeg = (tiles == 2 || tiles == 5) ? row0 / 64 * 64 : (tiles == 4) ? col0 / 64 * 64 : 0;
     const int64_t kend = (tiles == 3) ? (row0 / 64 + 1) * 64 < K ? (row0 / 64 + 1) * 64 : K : K;
     const int nch = kend > kbeg ? (int)((kend - kbeg) / 16) : 0;
     const int64_t ra = row0 + frag_row<KA, NB>(0, li), rb = col0 + frag_row<KB, NB>(0, li);
@@ -1709,35 +1709,30 @@ void colsumsq_f64(hipStream_t s, const double* A, int64_t ld, int64_t nrow, int6
 // ---------------------------------------------------------------------------
 // Elementwise helpers over lower tiles / vectors
 // ---------------------------------------------------------------------------
-// A = I over all T x T tiles: the triangular GEMM modes read whole tiles, so the
-// upper tiles of a triangular factor must hold zeros.
-__global__ void k_set_identity(double* __restrict__ A, int64_t ld, int64_t T) {
-    const int64_t ti = blockIdx.x % T, tj = blockIdx.x / T;
-    const int t = threadIdx.x, i = t & 63;
-    for (int c = t >> 6; c < 64; c += 4) {
-        const int64_t gi = ti * 64 + i, gj = tj * 64 + c;
-        A[gi + gj * ld] = (gi == gj) ? 1.0 : 0.0;
-    }
-}
-
-void set_identity_f64(hipStream_t s, double* A, int64_t ld, int64_t N) {
-    const int64_t T = N / 64;
-    hipLaunchKernelGGL(k_set_identity, dim3((unsigned)(T * T)), dim3(256), 0, s, A, ld, T);
-}
-
-// Column j = c0 + blockIdx.x of X (N x N, ld N): zero above its 64x64
-// diagonal block, the block's column from Dinv (64x64 column-major per block,
-// zero above its diagonal) on it; the rows below are left to the caller.
+// Column j = c0 + blockIdx.x of X (N x N, ld N): the block's column from Dinv
+// (64x64 column-major per block, zero above its diagonal) on its 64x64 diagonal
+// block and, with `clear`, zero above it; the rows below are left to the caller.
 __global__ __launch_bounds__(256) void k_trtri_leaves(double* __restrict__ X, int64_t N,
-                                                      const double* __restrict__ Dinv, int64_t c0) {
+                                                      const double* __restrict__ Dinv, int64_t c0, int clear) {
     const int64_t j = c0 + blockIdx.x, kb = j / 64, r0 = kb * 64;
     const double* D = Dinv + kb * 4096 + (j - r0) * 64;
-    for (int64_t i = threadIdx.x; i < r0 + 64; i += 256) X[i + j * N] = (i < r0) ? 0.0 : D[i - r0];
+    for (int64_t i = (clear ? 0 : r0) + threadIdx.x; i < r0 + 64; i += 256) X[i + j * N] = (i < r0) ? 0.0 : D[i - r0];
 }
 
-void trtri_leaves_f64(hipStream_t s, double* X, int64_t N, const double* Dinv, int64_t c0, int64_t ncols) {
+void trtri_leaves_f64(hipStream_t s, double* X, int64_t N, const double* Dinv, int64_t c0, int64_t ncols, int clear) {
     if (ncols <= 0) return;
-    hipLaunchKernelGGL(k_trtri_leaves, dim3((unsigned)ncols), dim3(256), 0, s, X, N, Dinv, c0);
+    hipLaunchKernelGGL(k_trtri_leaves, dim3((unsigned)ncols), dim3(256), 0, s, X, N, Dinv, c0, clear);
+}
+
+// zero above the 64x64 diagonal blocks of X (N x N, ld N)
+__global__ __launch_bounds__(256) void k_clear_upper(double* __restrict__ X, int64_t N) {
+    const int64_t j = 64 + blockIdx.x, r0 = j / 64 * 64;
+    for (int64_t i = threadIdx.x; i < r0; i += 256) X[i + j * N] = 0.0;
+}
+
+void clear_upper_f64(hipStream_t s, double* X, int64_t N) {
+    if (N <= 64) return;
+    hipLaunchKernelGGL(k_clear_upper, dim3((unsigned)(N - 64)), dim3(256), 0, s, X, N);
 }
 
 __global__ void k_fill(double* p, int64_t n, double v) {

@@ -78,7 +78,8 @@ void launch_grad_tiles_f32(hipStream_t s, const DevProg* prog, const DevProg& hp
 // ta/tb: operand stored transposed.  tiles: 0 = full grid, 1 = lower tiles of a square C,
 // 2 = lower tiles and k starts at the row tile (C = X^T X with X lower triangular),
 // 3 = full grid and k stops after the row tile (C = X B with X lower triangular),
-// 4 = full grid and k starts at the column tile (C = A X with X lower triangular).
+// 4 = full grid and k starts at the column tile (C = A X with X lower triangular),
+// 5 = full grid and k starts at the row tile (C = X^T B with X lower triangular).
 // C may be A (N = 64) or B (M = 64), with tiles 0.
 void gemm2_f64(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha, const double* A,
                int64_t lda, const double* B, int64_t ldb, double beta, double* C, int64_t ldc, int tiles);
@@ -133,7 +134,6 @@ void symv_lt_f64(hipStream_t s, const double* A, int64_t N, const double* v, dou
 // W = s B^-1 s - (t u^T + u t^T) in place over the lower tiles of B^-1 (t, u may be null)
 void form_wgrad_f64(hipStream_t s, double* B, int64_t N, int64_t n, const double* sv, const double* t,
                     const double* u);
-void set_identity_f64(hipStream_t s, double* A, int64_t ld, int64_t N);
 // info value a panel factorisation stores when one of its device waits timed out
 constexpr int kPanelWaitTimeout = 0x7fffffff;
 // the single-launch panel: at most this many 64-column blocks, and its flag words
@@ -172,7 +172,8 @@ void potrf_panel_mixed(hipStream_t s, float* A, int64_t ld, int64_t K0, int nc, 
                        unsigned maxpoll);
 // X (N x N, ld N), columns c0 .. c0 + ncols: zero above the 64x64 diagonal
 // blocks, the blocks from Dinv
-void trtri_leaves_f64(hipStream_t s, double* X, int64_t N, const double* Dinv, int64_t c0, int64_t ncols);
+void trtri_leaves_f64(hipStream_t s, double* X, int64_t N, const double* Dinv, int64_t c0, int64_t ncols, int clear);
+void clear_upper_f64(hipStream_t s, double* X, int64_t N);
 void trtri_leaves_f32_batched(hipStream_t s, float* X, int64_t N, const double* Dinv, int batch, int64_t sX,
                               int64_t sD, int64_t c0, int64_t ncols);
 // the top level of the recursive-doubling inverse: the largest 64 * 2^k below N (0 for N = 64)
