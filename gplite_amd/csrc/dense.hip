@@ -94,15 +94,23 @@ __device__ __forceinline__ void frag_load(T (&f)[NB][4], const T* p, int64_t ld)
 }
 
 // C = beta*C + alpha*op(A) op(B); A, B and C may be stored as float or double.
-template <int TA, int TB, int WT, int PF, bool INP, typename TAs, typename TBs, typename TCs>
+// KS: op(A) diag(ks) op(B), where the problems of the batch are consecutive ranges
+// of K of one contraction of length kall (the last may be shorter).
+template <int TA, int TB, int WT, int PF, bool INP, bool KS, typename TAs, typename TBs, typename TCs>
 __global__ __launch_bounds__(256) void k_gemm_reg(int64_t M, int64_t N, int64_t K, int64_t tilesM, double alpha,
                                                   const TAs* A, int64_t lda, const TBs* B, int64_t ldb, double beta,
-                                                  TCs* C, int64_t ldc, int tiles, int64_t sA, int64_t sB, int64_t sC) {
+                                                  TCs* C, int64_t ldc, int tiles, int64_t sA, int64_t sB, int64_t sC,
+                                                  const double* ks, int64_t kall) {
     constexpr int NB = WT / 16, BM = 2 * WT;
     constexpr bool KA = TA != 0, KB = TB == 0;  // contiguous in k
     A += blockIdx.y * sA;  // batch: one problem per grid row
     B += blockIdx.y * sB;
     C += blockIdx.y * sC;
+    if (KS) {
+        ks += blockIdx.y * K;
+        const int64_t left = kall - (int64_t)blockIdx.y * K;
+        K = left < K ? left : K;
+    }
     // Contiguous tile ranges per XCD share operand panels in L2; with a k range
     // that depends on the tile row (tiles == 2, 5) or column (tiles == 4, whose
     // columns are contiguous in the tile order) work per tile varies widely, so
@@ -139,14 +147,30 @@ __global__ __launch_bounds__(256) void k_gemm_reg(int64_t M, int64_t N, int64_t 
         for (int j = 0; j < NB; ++j) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
     TAs fa[PF][NB][4];
     TBs fb[PF][NB][4];
+    double2 fs[KS ? PF : 1][2];
+    const double* pk = KS ? ks + kbeg + 4 * g : nullptr;
     auto load = [&](int st) {
         frag_load<KA, NB>(fa[st], pa, lda);
         frag_load<KB, NB>(fb[st], pb, ldb);
+        if (KS) {
+            fs[st][0] = reinterpret_cast<const double2*>(pk)[0];
+            fs[st][1] = reinterpret_cast<const double2*>(pk)[1];
+            pk += 16;
+        }
         pa += stepa;
         pb += stepb;
     };
     // the tiles are formed transposed: D lane (li, g) holds columns g + 4v of row li
     auto mult = [&](int st) {
+        if (KS) {
+#pragma unroll
+            for (int j = 0; j < NB; ++j) {
+                fb[st][j][0] *= fs[st][0].x;
+                fb[st][j][1] *= fs[st][0].y;
+                fb[st][j][2] *= fs[st][1].x;
+                fb[st][j][3] *= fs[st][1].y;
+            }
+        }
 #pragma unroll
         for (int s = 0; s < 4; ++s)
 #pragma unroll
@@ -228,8 +252,8 @@ static void gemm_reg_launch(hipStream_t s, int ta, int tb, int64_t M, int64_t N,
     const int64_t nblk = (tiles != 1 && tiles != 2) ? tm * tn : BM < 64 ? 4 * (t64 * (t64 + 1) / 2) : tm * (tm + 1) / 2;
     dim3 grid((unsigned)nblk, (unsigned)batch), block(256);
 #define GPL_GR(TAv, TBv)                                                                                           \
-    hipLaunchKernelGGL((k_gemm_reg<TAv, TBv, WT, PF, INP, TAs, TBs, TCs>), grid, block, 0, s, M, N, K, tm, alpha, A, \
-                       lda, B, ldb, beta, C, ldc, tiles, sA, sB, sC)
+    hipLaunchKernelGGL((k_gemm_reg<TAv, TBv, WT, PF, INP, false, TAs, TBs, TCs>), grid, block, 0, s, M, N, K, tm,    \
+                       alpha, A, lda, B, ldb, beta, C, ldc, tiles, sA, sB, sC, (const double*)nullptr, (int64_t)0)
     if (!ta && !tb) GPL_GR(0, 0);
     else if (!ta && tb) GPL_GR(0, 1);
     else if (ta && !tb) GPL_GR(1, 0);
@@ -246,7 +270,8 @@ static void gemm_reg_launch(hipStream_t s, int ta, int tb, int64_t M, int64_t N,
 // lower 7168, k = 512: 558 / 769 / 458 / 496).  Long k with enough tiles to
 // fill the chip more than twice over: 64-wide ones, half the operand traffic per
 // flop (X B at 4096: 1562 / 2857 / 1278 / 1146; X^T X at 8192: 3213 / 9711 / 4902 /
-// 2943, at 3072: 423 / 542 / 297 / 377).  With both operands contiguous in k the
+// 2943, at 3072: 423 / 542 / 297 / 377; long is the mean range, half of K with a
+// triangular operand: X B with 1024 x 131072, 32 / 64: 2921 / 3155).  With both operands contiguous in k the
 // 32-wide waves are bound by their loads (37 TFLOP/s), so a product whose tiles
 // all have the same k range takes the 64-wide ones as soon as they fill the chip
 // once (1024 x 1024 x 32768 in four parts).
@@ -265,7 +290,7 @@ static void gemm_any(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_
     const int64_t m = M / 64, n = N / 64, m2 = (m + 1) / 2, n2 = (n + 1) / 2;
     const int64_t t64 = (low ? m * (m + 1) / 2 : m * n) * batch, t128 = (low ? m2 * (m2 + 1) / 2 : m2 * n2) * batch;
     if (t64 < 128) GPL_GA(16, 4, false);
-    else if (K >= 1024 && t128 >= (ta && !tb && !tiles ? 256 : 600)) GPL_GA(64, 3, false);
+    else if ((tiles >= 3 ? K / 2 : K) >= 1024 && t128 >= (ta && !tb && !tiles ? 256 : 600)) GPL_GA(64, 3, false);
     else GPL_GA(32, 3, false);
 #undef GPL_GA
 }
@@ -282,6 +307,18 @@ void gemm2_f64_batched(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int6
     gemm_any(s, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tiles, batch, sA, sB, sC);
 }
 
+// Lower 64x64 tiles of A diag(ks) A^T, A (M x K): `parts` partial products over kp
+// columns each, C + p * sC.  32-wide waves with three chunks in flight whatever the
+// size (M = 1024, K = 131072 in 64 parts: 2227 us, 64-wide 2330, 16-wide 5097;
+// M = 512 in 14 parts: 614, 1167, 1485).
+void gemm_gram_f64(hipStream_t s, int64_t M, int64_t K, const double* A, int64_t lda, const double* ks, int parts,
+                   int64_t kp, double* C, int64_t ldc, int64_t sC) {
+    const int64_t t = M / 64;
+    hipLaunchKernelGGL((k_gemm_reg<0, 1, 32, 4, false, true, double, double, double>),
+                       dim3((unsigned)(t * (t + 1) / 2), (unsigned)parts), dim3(256), 0, s, M, M, kp, t, 1.0, A, lda, A,
+                       lda, 0.0, C, ldc, 1, kp * lda, kp * lda, sC, ks, K);
+}
+
 // FP64-compute GEMMs on FP32 storage: A and C (panel solves of the batched form), A (prediction)
 void gemm_mixed_f32f64_batched(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha,
                                const float* A, int64_t lda, const double* B, int64_t ldb, double beta, float* C,
@@ -293,20 +330,6 @@ void gemm_mixed_f32f64f64(hipStream_t s, int ta, int tb, int64_t M, int64_t N, i
                           const float* A, int64_t lda, const double* B, int64_t ldb, double beta, double* C,
                           int64_t ldc, int tiles) {
     gemm_any(s, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tiles, 1, 0, 0, 0);
-}
-
-// out[i] = sum over p < parts of W[p * stride + i], in order of p (deterministic)
-__global__ void k_sum_parts(const double* __restrict__ W, int64_t stride, int parts, int64_t n,
-                            double* __restrict__ out) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    double acc = W[i];
-    for (int p = 1; p < parts; ++p) acc += W[p * stride + i];
-    out[i] = acc;
-}
-
-void sum_parts_f64(hipStream_t s, const double* W, int64_t stride, int parts, int64_t n, double* out) {
-    hipLaunchKernelGGL(k_sum_parts, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, W, stride, parts, n, out);
 }
 
 // ---------------------------------------------------------------------------

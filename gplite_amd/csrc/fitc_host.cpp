@@ -1,7 +1,12 @@
-// FITC (method_fitc) on the device: the n x m cross covariance K_xz stays
-// resident in both orientations, and every Newton step reduces to one
-// K_zx S^-1 K_xz product on MFMA, an m x m Cholesky and matrix-vector work
-// (kernels of its own: fitc.hip).
+// FITC (method_fitc) on the device, in whitened form: A = Lz^-1 K_zx (m x n,
+// Kz = Lz Lz^T) stays resident, and every Newton step reduces to one product
+// A S^-1 A^T on MFMA, an m x m Cholesky and three passes over A (kernels of their
+// own: fitc.hip).  With G = I + A S^-1 A^T the reference's Kz + K_zx S^-1 K_xz is
+// Lz G Lz^T: its leading minors have the same signs, its log-determinant is
+// log|Kz| + log|G|, and its inverse between K_xz and K_zx is G^-1 between A^T and A.
+// The rows of K_xz themselves are only needed while A is formed, a block of
+// columns at a time.  (Both orientations of K_xz resident, a scaled copy and six
+// passes took 16.2 ms of kernels at n = 131072, m = 1024 and 3.1 GB; now 1.5 GB.)
 //
 // Reference: R/gp_fit.R:101-123 (fit_laplace.method_fitc),
 // R/laplace.R:122-180 (laplace_iter.method_fitc, log-concave branch),
@@ -25,13 +30,13 @@ namespace {
 
 enum {
     F_PROG, F_X, F_F, F_ZX, F_FZ, F_Y, F_TR, F_OFF,
-    F_KZ, F_LZ, F_DINVZ, F_LDZ, F_XZ,           // Kz (kept), its factor, diagonal inverses, log pivots, Lz^-1
-    F_U, F_UT, F_W,                              // K_xz (N x Mz), K_zx (Mz x N), S^-1/2 K_xz
-    F_H, F_G, F_DINVG, F_LDG, F_XG, F_MM, F_T1,  // H = K_zx S^-1 K_xz, G = Kz + H -> Lc, Lc^-1, M, scratch
-    F_WZ,                                        // w = Lz^-1 K_zx alpha
-    F_D, F_Z, F_V, F_SV, F_S, F_RS, F_ZS, F_ALPHA, F_FMEAN, F_FOLD, F_V1, F_V2, F_V3, F_V4,
+    F_LZ, F_DINVZ, F_LDZ, F_XZ,  // Kz -> its factor Lz, diagonal inverses, log pivots, Lz^-1
+    F_A, F_W,                    // A = Lz^-1 K_zx (Mz x N), a block of columns (of K_zx, of Lc^-1 A)
+    F_G, F_DINVG, F_LDG, F_XG,   // G = I + A S^-1 A^T -> its factor Lc, Lc^-1
+    F_WZ,                        // w = A alpha = Lz^-1 K_zx alpha
+    F_D, F_Z, F_V, F_SV, F_S, F_SI, F_ZS, F_ALPHA, F_FMEAN, F_FOLD, F_V1, F_V2, F_V3, F_V4,
     F_FVAR, F_FVOLD, F_ZOLD, F_POLD, F_CAVM, F_CAVV, F_LOGZS, F_TERM, F_GH,  // EP state
-    F_Q1, F_Q2, F_SCAL, F_INFO, F_SPLIT,
+    F_Q1, F_Q2, F_SCAL, F_INFO, F_SPLIT, F_PART,
     F_COUNT
 };
 
@@ -58,36 +63,47 @@ struct gpl_fitc {
         if (!(fm)->b[idx].ensure(bytes)) return fail(GPL_ERR_OOM, "device allocation failed"); \
     } while (0)
 
-// K-split of the K_zx S^-1 K_xz product: with few m x m output tiles and a long
-// reduction over n, P partial products (rows split in P ranges) fill the chip and
-// are summed in a fixed order.
-static int fitc_split(const gpl_fitc* f) {
-    const int64_t tiles = (f->Mz / 64) * (f->Mz / 64);
-    int P = 1;
-    while (P < 16 && tiles * P < 1024 && (f->N / 64) % (2 * P) == 0 && f->N / (2 * P) >= 512) P *= 2;
-    return P;
+// Partial products of A S^-1 A^T over column ranges, summed in a fixed order: as
+// many as fill the chip with 64x64 output tiles four times over (2048 of them), at
+// least 256 columns each.  m = 1024, n = 131072: 7 / 15 / 30 parts 2.9 / 2.7 / 2.6 ms;
+// m = 128: 1 / 7 / 64 parts 4254 / 614 / 74 us.
+static int64_t fitc_part_cols(const gpl_fitc* f) {
+    const int64_t T = f->Mz / 64, tiles = T * (T + 1) / 2;
+    const int64_t P = std::max<int64_t>(1, std::min<int64_t>({2048 / tiles, 64, f->N / 256}));
+    return pad64((f->N + P - 1) / P);
+}
+static int fitc_parts(const gpl_fitc* f) {
+    const int64_t kp = fitc_part_cols(f);
+    return (int)((f->N + kp - 1) / kp);
+}
+
+// Columns of K_zx (of Lc^-1 A) formed at a time: 2^25 elements, four blocks at
+// m = 1024, n = 131072
+static int64_t fitc_block_cols(const gpl_fitc* f) {
+    return std::max<int64_t>(64, std::min<int64_t>(f->N, ((int64_t)1 << 25) / f->Mz / 64 * 64));
 }
 
 static int fitc_alloc(gpl_fitc* f) {
     const int64_t N = f->N, Mz = f->Mz;
-    const size_t vN = (size_t)N * 8, vM = (size_t)Mz * 8, mm = (size_t)Mz * Mz * 8, nm = (size_t)N * Mz * 8;
+    const size_t vN = (size_t)N * 8, vM = (size_t)Mz * 8, mm = (size_t)Mz * Mz * 8;
     FENSURE(f, F_PROG, sizeof(DevProg));
     FENSURE(f, F_X, (size_t)f->n * std::max<int64_t>(f->ncols, 1) * 8);
     FENSURE(f, F_ZX, (size_t)f->m * std::max<int64_t>(f->ncols, 1) * 8);
     FENSURE(f, F_F, (size_t)N * MAX_FEAT * 8);
     FENSURE(f, F_FZ, (size_t)Mz * MAX_FEAT * 8);
-    for (int i : {F_KZ, F_LZ, F_XZ, F_H, F_G, F_XG, F_MM, F_T1}) FENSURE(f, i, mm);
+    for (int i : {F_LZ, F_XZ, F_G, F_XG}) FENSURE(f, i, mm);
     for (int i : {F_DINVZ, F_DINVG}) FENSURE(f, i, (size_t)Mz * 64 * 8);
     for (int i : {F_LDZ, F_LDG, F_WZ, F_Q1, F_Q2}) FENSURE(f, i, vM);
-    for (int i : {F_U, F_UT, F_W}) FENSURE(f, i, nm);
-    for (int i : {F_Y, F_TR, F_OFF, F_D, F_Z, F_V, F_SV, F_S, F_RS, F_ZS, F_ALPHA, F_FMEAN, F_FOLD, F_V1, F_V2, F_V3,
+    FENSURE(f, F_A, (size_t)N * Mz * 8);
+    FENSURE(f, F_W, (size_t)fitc_block_cols(f) * Mz * 8);
+    for (int i : {F_Y, F_TR, F_OFF, F_D, F_Z, F_V, F_SV, F_S, F_SI, F_ZS, F_ALPHA, F_FMEAN, F_FOLD, F_V1, F_V2, F_V3,
                   F_V4, F_FVAR, F_FVOLD, F_ZOLD, F_POLD, F_CAVM, F_CAVV, F_LOGZS, F_TERM})
         FENSURE(f, i, vN);
     FENSURE(f, F_GH, 64 * 8);
     FENSURE(f, F_SCAL, 64 * 8);
     FENSURE(f, F_INFO, 64);
-    const int P = fitc_split(f);
-    if (P > 1) FENSURE(f, F_SPLIT, (size_t)P * Mz * Mz * 8);
+    FENSURE(f, F_SPLIT, fitc_parts(f) * mm);
+    FENSURE(f, F_PART, fitc_pass_parts(f->n) * vM);
     return GPL_OK;
 }
 
@@ -106,69 +122,44 @@ static int fitc_scalars(gpl_fitc* f, double* out, int k, int* flags) {
     return GPL_OK;
 }
 
-// M = A C^-1 A^T with A = Lz^-1 K_zx, the m x m matrix of the predictive
-// variance (inv_lemma_solve(C_inv, t(Kt_aux1), Kt_aux1), R/gp_pred.R:279):
-// A S^-1 A^T - (A S^-1 K_xz) G^-1 (K_zx S^-1 A^T) = Lz^-1 (H - H G^-1 H) Lz^-T.
-static void fitc_predictive_matrix(gpl_fitc* f) {
-    gpl_ctx* c = f->ctx;
-    hipStream_t s = c->stream;
-    const int64_t Mz = f->Mz;
-    trtri_blocked(c, f->d(F_G), f->d(F_DINVG), Mz, f->d(F_XG));
-    double* Y = f->d(F_MM);  // Y = Lc^-1 H, then reused for M
-    gemm2_f64(s, 0, 0, Mz, Mz, Mz, 1.0, f->d(F_XG), Mz, f->d(F_H), Mz, 0.0, Y, Mz, 3);
-    hipMemcpyAsync(f->d(F_T1), f->d(F_H), Mz * Mz * 8, hipMemcpyDeviceToDevice, s);
-    gemm2_f64(s, 1, 0, Mz, Mz, Mz, -1.0, Y, Mz, Y, Mz, 1.0, f->d(F_T1), Mz, 0);  // H - H G^-1 H
-    gemm2_f64(s, 0, 0, Mz, Mz, Mz, 1.0, f->d(F_XZ), Mz, f->d(F_T1), Mz, 0.0, f->d(F_XG), Mz, 3);
-    gemm2_f64(s, 0, 1, Mz, Mz, Mz, 1.0, f->d(F_XG), Mz, f->d(F_XZ), Mz, 0.0, Y, Mz, 0);
-}
-
-// One inversion-lemma solve for the current sites: S = D + V, G = Kz + K_zx S^-1 K_xz
-// and its factor, alpha = C^-1 z and the posterior mean K_f alpha into F_FMEAN
-// (R/laplace.R:134-141, R/ep.R:166-176).  flags[0] receives G's failing minor.
-static void fitc_lemma_step(gpl_fitc* f, int* flags) {
+// One inversion-lemma solve for the current sites: S = D + V, G = I + A S^-1 A^T
+// and its factor Lc, alpha = C^-1 z, w = A alpha and the posterior mean K_f alpha
+// into F_FMEAN (R/laplace.R:134-141, R/ep.R:166-176).  With `inverse` also Lc^-1,
+// its leading half beside the factor.  flags[0] receives G's failing minor.
+static void fitc_lemma_step(gpl_fitc* f, int* flags, bool inverse) {
     gpl_ctx* c = f->ctx;
     hipStream_t s = c->stream;
     const int64_t n = f->n, N = f->N, Mz = f->Mz;
-    fitc_site(s, n, N, f->d(F_D), f->d(F_V), f->d(F_Z), f->d(F_S), f->d(F_RS), f->d(F_ZS));
-    scale_rows_copy_f64(s, f->d(F_U), N, N, Mz, f->d(F_RS), f->d(F_W));
+    const double* A = f->d(F_A);
+    fitc_site(s, n, N, f->d(F_D), f->d(F_V), f->d(F_Z), f->d(F_S), f->d(F_SI), f->d(F_ZS));
     {
-        Prof p(c, "fitc_syrk", 2.0 * Mz * Mz * N, 8.0 * N * Mz);
-        const int P = fitc_split(f);
-        if (P == 1) {
-            gemm2_f64(s, 1, 0, Mz, Mz, N, 1.0, f->d(F_W), N, f->d(F_W), N, 0.0, f->d(F_H), Mz, 0);
-        } else {
-            const int64_t Kp = N / P;
-            gemm2_f64_batched(s, 1, 0, Mz, Mz, Kp, 1.0, f->d(F_W), N, f->d(F_W), N, 0.0, f->d(F_SPLIT), Mz, 0, P, Kp,
-                              Kp, Mz * Mz);
-            sum_parts_f64(s, f->d(F_SPLIT), Mz * Mz, P, Mz * Mz, f->d(F_H));
-        }
+        Prof p(c, "fitc_gram", (double)Mz * Mz * N, 8.0 * N * Mz);
+        const int P = fitc_parts(f);
+        gemm_gram_f64(s, Mz, N, A, Mz, f->d(F_SI), P, fitc_part_cols(f), f->d(F_SPLIT), Mz, Mz * Mz);
+        fitc_gram_sum(s, f->d(F_SPLIT), P, Mz, f->d(F_G));
     }
-    vec_axpby(s, Mz * Mz, 1.0, f->d(F_KZ), 1.0, f->d(F_H), f->d(F_G));
-    potrf_blocked(c, f->d(F_G), Mz, f->d(F_DINVG), f->d(F_LDG), flags);
-    Prof pv(c, "fitc_gemv", 0, 32.0 * N * Mz);
-    gemv_t_f64(s, f->d(F_U), N, N, Mz, f->d(F_ZS), f->d(F_Q1));
-    trsv_lower(c, s, f->d(F_G), Mz, f->d(F_DINVG), Mz, f->d(F_Q1), f->d(F_Q2), 0, flags);
-    trsv_lower(c, s, f->d(F_G), Mz, f->d(F_DINVG), Mz, f->d(F_Q2), f->d(F_Q1), 1, flags);
-    gemv_t_f64(s, f->d(F_UT), Mz, Mz, N, f->d(F_Q1), f->d(F_V1));
-    fitc_alpha(s, n, N, f->d(F_ZS), f->d(F_V1), f->d(F_S), f->d(F_ALPHA));
-    gemv_t_f64(s, f->d(F_U), N, N, Mz, f->d(F_ALPHA), f->d(F_Q1));
-    trsv_lower(c, s, f->d(F_LZ), Mz, f->d(F_DINVZ), Mz, f->d(F_Q1), f->d(F_Q2), 0, flags);
-    trsv_lower(c, s, f->d(F_LZ), Mz, f->d(F_DINVZ), Mz, f->d(F_Q2), f->d(F_Q1), 1, flags);
-    gemv_t_f64(s, f->d(F_UT), Mz, Mz, N, f->d(F_Q1), f->d(F_V2));
-    vec_mul(s, n, f->d(F_D), f->d(F_ALPHA), f->d(F_V3));
-    fill_f64(s, f->d(F_FMEAN), N, 0.0);
-    vec_axpby(s, n, 1.0, f->d(F_V2), 1.0, f->d(F_V3), f->d(F_FMEAN));
+    {
+        Prof p(c, "fitc_pass", 0, 8.0 * N * Mz);
+        fitc_combine(s, A, Mz, n, f->d(F_ZS), f->d(F_PART), f->d(F_Q1));
+    }
+    potrf_blocked(c, f->d(F_G), Mz, f->d(F_DINVG), f->d(F_LDG), flags, inverse ? f->d(F_XG) : nullptr, nullptr,
+                  f->d(F_Q1));
+    trsv_lower(c, s, f->d(F_G), Mz, f->d(F_DINVG), Mz, f->d(F_Q1), f->d(F_Q2), 1, flags);
+    Prof pv(c, "fitc_pass", 0, 16.0 * N * Mz);
+    fitc_alpha_pass(s, A, Mz, n, N, f->d(F_Q2), f->d(F_ZS), f->d(F_S), f->d(F_ALPHA), f->d(F_PART), f->d(F_WZ));
+    fitc_mean(s, A, Mz, n, N, f->d(F_WZ), f->d(F_D), f->d(F_ALPHA), f->d(F_FMEAN));
 }
 
-// q_i = |Lc^-1 u_i|^2 for the current G (into `out`), through Lc^-1 (F_XG) and F_W
+// q_i = |Lc^-1 a_i|^2 for the current G (into `out`), through F_W
 static void fitc_q(gpl_fitc* f, double* out) {
-    gpl_ctx* c = f->ctx;
-    hipStream_t s = c->stream;
-    const int64_t N = f->N, Mz = f->Mz;
-    trtri_blocked(c, f->d(F_G), f->d(F_DINVG), Mz, f->d(F_XG));
-    Prof p(c, "fitc_q", (double)Mz * Mz * N, 16.0 * N * Mz);
-    gemm2_f64(s, 0, 0, Mz, N, Mz, 1.0, f->d(F_XG), Mz, f->d(F_UT), Mz, 0.0, f->d(F_W), Mz, 3);
-    colsumsq_f64(s, f->d(F_W), Mz, Mz, f->n, out, 0);
+    hipStream_t s = f->ctx->stream;
+    const int64_t N = f->N, Mz = f->Mz, nb = fitc_block_cols(f);
+    Prof p(f->ctx, "fitc_q", (double)Mz * Mz * N, 16.0 * N * Mz);
+    for (int64_t c0 = 0; c0 < N; c0 += nb) {
+        const int64_t w = std::min(nb, N - c0);
+        gemm2_f64(s, 0, 0, Mz, w, Mz, 1.0, f->d(F_XG), Mz, f->d(F_A) + c0 * Mz, Mz, 0.0, f->d(F_W), Mz, 3);
+        colsumsq_f64(s, f->d(F_W), Mz, Mz, std::min(w, f->n - c0), out + c0, 0);
+    }
 }
 
 // Damped parallel EP over the FITC prior: ep.method_fitc (R/ep.R:332-370; its
@@ -217,7 +208,7 @@ static int fitc_ep_loop(gpl_fitc* f, const double* tr, const double* off) {
             return fail(GPL_ERR_UNSUPPORTED, "EP site variance <= 0: R/ep.R:186-270 is not on the device path");
         }
         if (fl[1] & 1) quad_ok = false;
-        fitc_lemma_step(f, flags);
+        fitc_lemma_step(f, flags, true);
         fitc_q(f, f->d(F_V1));
         fitc_ep_var(s, n, f->d(F_V), f->d(F_S), f->d(F_D), f->d(F_V1), f->d(F_FVAR));
         // per-site evidence terms (the binv argument only feeds an unused output here)
@@ -230,10 +221,9 @@ static int fitc_ep_loop(gpl_fitc* f, const double* tr, const double* off) {
         reduce_sum(s, f->d(F_V3), n, scd + 2);
         vec_log(s, n, f->d(F_S), f->d(F_V4));
         reduce_sum(s, f->d(F_V4), n, scd + 3);
-        reduce_sum(s, f->d(F_LDZ), Mz, scd + 4);
-        reduce_sum(s, f->d(F_LDG), Mz, scd + 5);
-        reduce_maxabsdiff(s, f->d(F_FOLD), f->d(F_FMEAN), n, scd + 6);
-        int r = fitc_scalars(f, sc, 7, fl);
+        reduce_sum(s, f->d(F_LDG), Mz, scd + 4);
+        reduce_maxabsdiff(s, f->d(F_FOLD), f->d(F_FMEAN), n, scd + 5);
+        int r = fitc_scalars(f, sc, 6, fl);
         if (r) return r;
         if (fl[0] == kPanelWaitTimeout) return wait_timeout_fail();
         if (fl[0] > 0) {
@@ -242,9 +232,9 @@ static int fitc_ep_loop(gpl_fitc* f, const double* tr, const double* off) {
                                             " of Kz + K_zx S^-1 K_xz is not positive");
         }
         // log Z_EP (R/ep.R:179-181); the site terms carry -1/2 log V, added back here
-        const double logdet = sc[3] - 2.0 * sc[4] + 2.0 * sc[5];
+        const double logdet = sc[3] + 2.0 * sc[4];
         f->logZ = sc[0] + 0.5 * sc[2] - 0.5 * logdet - 0.5 * sc[1];
-        diff_new = sc[6];
+        diff_new = sc[5];
         if (diff_new > diff_old) {
             damp = damp * damping;
             continue;
@@ -277,11 +267,9 @@ static int fitc_run(gpl_fitc* f) {
     int* flags = f->b[F_INFO].as<int>();
     int fl[2] = {0, 0};
     // Kz = K(z, z) + jitter I (padding: identity), its factor Lz and Lz^-1
-    fill_f64(s, f->d(F_KZ), Mz * Mz, 0.0);
-    launch_build_sym_f64(s, pd, f->prog, f->d(F_FZ), m, Mz, jitter, 0, 1.0, nullptr, f->d(F_KZ), Mz);
-    HIP_TRY(hipMemcpyAsync(f->d(F_LZ), f->d(F_KZ), Mz * Mz * 8, hipMemcpyDeviceToDevice, s));
+    launch_build_sym_f64(s, pd, f->prog, f->d(F_FZ), m, Mz, jitter, 0, 1.0, nullptr, f->d(F_LZ), Mz);
     HIP_TRY(hipMemsetAsync(flags, 0, 8, s));
-    potrf_blocked(c, f->d(F_LZ), Mz, f->d(F_DINVZ), f->d(F_LDZ), flags);
+    potrf_blocked(c, f->d(F_LZ), Mz, f->d(F_DINVZ), f->d(F_LDZ), flags, f->d(F_XZ));
     double sc[8];
     int r = fitc_scalars(f, sc, 1, fl);
     if (r) return r;
@@ -290,18 +278,19 @@ static int fitc_run(gpl_fitc* f) {
         set_minor(fl[0]);
         return fail(GPL_ERR_NOT_PD, "Kz: the leading minor of order " + std::to_string(fl[0]) + " is not positive");
     }
-    trtri_blocked(c, f->d(F_LZ), f->d(F_DINVZ), Mz, f->d(F_XZ));
-    // K_xz in both orientations (zero outside n x m)
+    // A = Lz^-1 K_zx (zero outside m x n), a block of K_zx's columns at a time;
+    // D = diag K + jitter - colSums(A^2)  (R/gp_fit.R:107-108)
     {
-        Prof p(c, "fitc_cross", 0, 16.0 * N * Mz);
-        launch_build_cross(s, pd, f->prog, f->d(F_F), N, n, N, f->d(F_FZ), Mz, m, Mz, f->d(F_U), N);
-        transpose_f64(s, f->d(F_U), N, N, Mz, f->d(F_UT), Mz);
-    }
-    // D = diag K + jitter - colSums((Lz^-1 K_zx)^2)  (R/gp_fit.R:107-108); F_W holds Lz^-1 K_zx here
-    {
-        Prof p(c, "fitc_diag_trmm", (double)Mz * Mz * N, 16.0 * N * Mz);
-        gemm2_f64(s, 0, 0, Mz, N, Mz, 1.0, f->d(F_XZ), Mz, f->d(F_UT), Mz, 0.0, f->d(F_W), Mz, 3);
-        colsumsq_f64(s, f->d(F_W), Mz, Mz, n, f->d(F_V1), 0);
+        Prof p(c, "fitc_whiten", (double)Mz * Mz * N, 32.0 * N * Mz);
+        const int64_t nb = fitc_block_cols(f);
+        for (int64_t c0 = 0; c0 < N; c0 += nb) {
+            const int64_t w = std::min(nb, N - c0);
+            double* A = f->d(F_A) + c0 * Mz;
+            launch_build_cross(s, pd, f->prog, f->d(F_FZ), Mz, m, Mz, f->d(F_F) + c0, N, std::min(w, n - c0), w,
+                               f->d(F_W), Mz);
+            gemm2_f64(s, 0, 0, Mz, w, Mz, 1.0, f->d(F_XZ), Mz, f->d(F_W), Mz, 0.0, A, Mz, 3);
+        }
+        colsumsq_f64(s, f->d(F_A), Mz, Mz, n, f->d(F_V1), 0);
     }
     launch_build_diag(s, pd, f->prog, f->d(F_F), N, f->d(F_F), N, n, f->d(F_V2));
     fitc_diag(s, n, N, f->d(F_V2), f->d(F_V1), jitter, f->d(F_D));
@@ -311,12 +300,6 @@ static int fitc_run(gpl_fitc* f) {
     if (f->opts.approx == GPL_APPROX_EP) {
         r = fitc_ep_loop(f, tr, off);
         if (r && r != GPL_ERR_NOCONV) return r;
-        gemv_t_f64(s, f->d(F_U), N, N, Mz, f->d(F_ALPHA), f->d(F_Q1));
-        trsv_lower_f64(s, f->d(F_LZ), Mz, f->d(F_DINVZ), Mz, f->d(F_Q1), f->d(F_WZ), 0);
-        {
-            Prof p(c, "fitc_pred_matrix", 0, 0);
-            fitc_predictive_matrix(f);
-        }
         HIP_TRY(hipStreamSynchronize(s));
         return r;
     }
@@ -334,7 +317,7 @@ static int fitc_run(gpl_fitc* f) {
             lik_pseudodata_la(s, f->lik.kind, f->lik.link, lik_par(f->lik), n, f->d(F_FOLD), f->d(F_Y), tr, off, f->d(F_Z),
                               f->d(F_V), f->d(F_SV), flags + 1, (f->opts.flags & GPL_FLAG_ANALYTIC_W) ? 1 : 0);
         // inversion lemma for C = K_xz Kz^-1 K_zx + S, S = D + V (R/linear_algebra.R:3-47)
-        fitc_lemma_step(f, flags);
+        fitc_lemma_step(f, flags, gauss);
         // log evidence (R/laplace.R:143-151): logdet C - log|V| from the lemma
         lik_loglik(s, f->lik.kind, f->lik.link, lik_par(f->lik), n, f->d(F_FMEAN), f->d(F_Y), tr, off,
                    f->d(F_V3));
@@ -345,9 +328,8 @@ static int fitc_run(gpl_fitc* f) {
         reduce_sum(s, f->d(F_V3), n, scd + 2);
         vec_log(s, n, f->d(F_S), f->d(F_V4));
         reduce_sum(s, f->d(F_V4), n, scd + 3);
-        reduce_sum(s, f->d(F_LDZ), Mz, scd + 4);
-        reduce_sum(s, f->d(F_LDG), Mz, scd + 5);
-        r = fitc_scalars(f, sc, 6, fl);
+        reduce_sum(s, f->d(F_LDG), Mz, scd + 4);
+        r = fitc_scalars(f, sc, 5, fl);
         if (r) return r;
         if (fl[1] & 6) {
             f->logZ = -INFINITY;
@@ -362,7 +344,7 @@ static int fitc_run(gpl_fitc* f) {
             return fail(GPL_ERR_NOT_PD, "inversion lemma: the leading minor of order " + std::to_string(fl[0]) +
                                             " of Kz + K_zx S^-1 K_xz is not positive");
         }
-        const double logdet = sc[3] - 2.0 * sc[4] + 2.0 * sc[5];
+        const double logdet = sc[3] + 2.0 * sc[4];
         const double log_post = sc[0] - 0.5 * sc[1];
         f->logZ = log_post + 0.5 * (sc[2] - logdet);
         HIP_TRY(hipMemcpyAsync(f->d(F_FOLD), f->d(F_FMEAN), N * 8, hipMemcpyDeviceToDevice, s));
@@ -372,13 +354,8 @@ static int fitc_run(gpl_fitc* f) {
     }
     if (it > maxiter) it = maxiter;
     f->iters = it;
-    // prediction state: w = Lz^-1 K_zx alpha and M (R/gp_pred.R:249-252,279)
-    gemv_t_f64(s, f->d(F_U), N, N, Mz, f->d(F_ALPHA), f->d(F_Q1));
-    trsv_lower_f64(s, f->d(F_LZ), Mz, f->d(F_DINVZ), Mz, f->d(F_Q1), f->d(F_WZ), 0);
-    {
-        Prof p(c, "fitc_pred_matrix", 0, 0);
-        fitc_predictive_matrix(f);
-    }
+    // prediction state: w (from the last step) and Lc^-1
+    if (!gauss) trtri_blocked(c, f->d(F_G), f->d(F_DINVG), Mz, f->d(F_XG));
     HIP_TRY(hipStreamSynchronize(s));
     if (maxiter > 1 && it == maxiter) {  // R/laplace.R:318-320 warns whenever the cap is reached
         fail(GPL_ERR_NOCONV, "Maximum number of iterations in Laplace reached, delta log post = " +
@@ -472,21 +449,19 @@ extern "C" int gpl_fitc_pred(gpl_fitc* f, const double* xt, int64_t mt, int32_t 
     gemm2_f64(s, 0, 0, Mz, Mt, Mz, 1.0, f->d(F_XZ), Mz, KzT, Mz, 0.0, A2, Mz, 3);
     gemv_t_f64(s, A2, Mz, Mz, mt, f->d(F_WZ), vb);
     if (want_var) {
-        // prior_var = colSums(K_zt * Kz^-1 K_zt) + Dt, Dt = diag K_tt - colSums(A_t^2)  (R/gp_pred.R:244-246,271)
-        double* c1 = vb + Mt;
-        double* c2 = vb + 2 * Mt;
-        double* kd = vb + 3 * Mt;
+        // prior_var = colSums(K_zt * Kz^-1 K_zt) + Dt with Dt = diag K_tt - colSums(A_t^2) is
+        // diag K_tt, and var_reduction = colSums(A_t * (M A_t)), M = A C^-1 A^T = I - G^-1, is
+        // colSums(A_t^2) - colSums((Lc^-1 A_t)^2)  (R/gp_pred.R:244-246,271,278-280)
+        double* c2 = vb + Mt;
+        double* kd = vb + 2 * Mt;
+        double* q = vb + 3 * Mt;
         double* red = vb + 4 * Mt;
-        gemm2_f64(s, 1, 0, Mz, Mt, Mz, 1.0, f->d(F_XZ), Mz, A2, Mz, 0.0, Yv, Mz, 0);  // Kz^-1 K_zt = Lz^-T A_t
-        coldot_f64(s, KzT, Yv, Mz, Mz, mt, c1);
         colsumsq_f64(s, A2, Mz, Mz, mt, c2, 0);
         launch_build_diag(s, pd, f->prog, Ft, Mt, Ft, Mt, mt, kd);
-        vec_axpby(s, mt, 1.0, kd, -1.0, c2, c2);   // Dt
-        vec_axpby(s, mt, 1.0, c1, 1.0, c2, c2);    // prior_var
-        // var_reduction = colSums(A_t * (M A_t))  (R/gp_pred.R:278-280)
-        gemm2_f64(s, 0, 0, Mz, Mt, Mz, 1.0, f->d(F_MM), Mz, A2, Mz, 0.0, Yv, Mz, 0);
-        coldot_f64(s, A2, Yv, Mz, Mz, mt, red);
-        vec_axpby(s, mt, 1.0, c2, -1.0, red, red);
+        vec_axpby(s, mt, 1.0, kd, -1.0, c2, c2);
+        gemm2_f64(s, 0, 0, Mz, Mt, Mz, 1.0, f->d(F_XG), Mz, A2, Mz, 0.0, Yv, Mz, 3);
+        colsumsq_f64(s, Yv, Mz, Mz, mt, q, 0);
+        vec_axpby(s, mt, 1.0, c2, 1.0, q, red);
         HIP_TRY(hipMemcpyAsync(var, red, mt * 8, hipMemcpyDeviceToHost, s));
     }
     HIP_TRY(hipMemcpyAsync(mean, vb, mt * 8, hipMemcpyDeviceToHost, s));
@@ -496,7 +471,7 @@ extern "C" int gpl_fitc_pred(gpl_fitc* f, const double* xt, int64_t mt, int32_t 
 
 // gp_draw_analytic.method_fitc with marginal = FALSE (R/gp_draw.R:126-140):
 // mean + chol(cov + jitter I) z, cov = A_t^T A_t + diag(Dt) - A_t^T M A_t
-// (R/gp_pred.R:258-268, train = FALSE).
+// (R/gp_pred.R:258-268, train = FALSE), = (Lc^-1 A_t)^T (Lc^-1 A_t) + diag(Dt).
 extern "C" int gpl_fitc_draw(gpl_fitc* f, const double* xt, int64_t mt, double jitter, const double* z,
                              int64_t draws, double* out) {
     if (!f || !xt || !z || !out || mt < 1 || draws < 1) return fail(GPL_ERR_ARG, "bad argument");
@@ -530,10 +505,9 @@ extern "C" int gpl_fitc_draw(gpl_fitc* f, const double* xt, int64_t mt, double j
     colsumsq_f64(s, A2, Mz, Mz, mt, dt, 0);
     launch_build_diag(s, pd, f->prog, Ft, Mt, Ft, Mt, mt, vb + 2 * Mt);
     vec_axpby(s, mt, 1.0, vb + 2 * Mt, -1.0, dt, dt);
-    // lower tiles of A_t^T A_t - A_t^T (M A_t), then the diagonal terms
-    gemm2_f64(s, 0, 0, Mz, Mt, Mz, 1.0, f->d(F_MM), Mz, A2, Mz, 0.0, Yv, Mz, 0);
-    gemm2_f64(s, 1, 0, Mt, Mt, Mz, 1.0, A2, Mz, A2, Mz, 0.0, Cv, Mt, 1);
-    gemm2_f64(s, 1, 0, Mt, Mt, Mz, -1.0, A2, Mz, Yv, Mz, 1.0, Cv, Mt, 1);
+    // lower tiles of the product, then the diagonal terms
+    gemm2_f64(s, 0, 0, Mz, Mt, Mz, 1.0, f->d(F_XG), Mz, A2, Mz, 0.0, Yv, Mz, 3);
+    gemm2_f64(s, 1, 0, Mt, Mt, Mz, 1.0, Yv, Mz, Yv, Mz, 0.0, Cv, Mt, 1);
     add_diag_f64(s, Cv, Mt, mt, Mt, dt, jitter);
     HIP_TRY(hipMemsetAsync(info, 0, 64, s));
     potrf_blocked(c, Cv, Mt, Dv, ld, info);
@@ -559,7 +533,7 @@ extern "C" int gpl_fitc_draw(gpl_fitc* f, const double* xt, int64_t mt, double j
 // Predictive variance at the training inputs with the FITC diagonal
 // (gp_pred_post.method_fitc, train = TRUE: R/gp_pred.R:270-285), the input of
 // loo_posteriors.approx_laplace (R/gp_loo.R:120-130).  With A = Lz^-1 K_zx,
-// Dt = diag K - colSums(A^2) and q_i = |Lc^-1 u_i|^2 the reference's three terms
+// Dt = diag K - colSums(A^2) and q_i = |Lc^-1 a_i|^2 the reference's three terms
 // are (A^T M A)_ii, 2 Dt_i q_i / S_i and Dt_i^2 [C^-1]_ii.
 extern "C" int gpl_fitc_train_var(gpl_fitc* f, double* out) {
     if (!f || !out) return fail(GPL_ERR_ARG, "NULL argument");
@@ -568,25 +542,15 @@ extern "C" int gpl_fitc_train_var(gpl_fitc* f, double* out) {
     HIP_TRY(hipSetDevice(c->device));
     hipStream_t s = c->stream;
     const int64_t n = f->n, N = f->N, Mz = f->Mz;
-    double* A = (double*)c->buf(22, (size_t)Mz * N * 8);
-    double* B = (double*)c->buf(23, (size_t)Mz * N * 8);
     double* v = (double*)c->buf(24, (size_t)N * 6 * 8);
-    double* X = (double*)c->buf(25, (size_t)Mz * Mz * 8);
-    if (!A || !B || !v || !X) return fail(GPL_ERR_OOM, "device allocation failed");
-    double *c2 = v, *kd = v + N, *c1 = v + 2 * N, *t1 = v + 3 * N, *q = v + 4 * N, *res = v + 5 * N;
-    gemm2_f64(s, 0, 0, Mz, N, Mz, 1.0, f->d(F_XZ), Mz, f->d(F_UT), Mz, 0.0, A, Mz, 3);  // A = Lz^-1 K_zx
-    colsumsq_f64(s, A, Mz, Mz, n, c2, 0);
+    if (!v) return fail(GPL_ERR_OOM, "device allocation failed");
+    double *c2 = v, *kd = v + N, *t1 = v + 2 * N, *q = v + 3 * N, *res = v + 4 * N;
+    colsumsq_f64(s, f->d(F_A), Mz, Mz, n, c2, 0);
     launch_build_diag(s, f->b[F_PROG].as<DevProg>(), f->prog, f->d(F_F), N, f->d(F_F), N, n, kd);
+    fitc_q(f, q);
+    vec_axpby(s, n, 1.0, c2, -1.0, q, t1);
     vec_axpby(s, n, 1.0, kd, -1.0, c2, c2);  // Dt
-    gemm2_f64(s, 1, 0, Mz, N, Mz, 1.0, f->d(F_XZ), Mz, A, Mz, 0.0, B, Mz, 0);  // Kz^-1 K_zx
-    coldot_f64(s, f->d(F_UT), B, Mz, Mz, n, c1);
-    vec_axpby(s, n, 1.0, c1, 1.0, c2, c1);  // prior_var
-    gemm2_f64(s, 0, 0, Mz, N, Mz, 1.0, f->d(F_MM), Mz, A, Mz, 0.0, B, Mz, 0);  // M A
-    coldot_f64(s, A, B, Mz, Mz, n, t1);
-    trtri_blocked(c, f->d(F_G), f->d(F_DINVG), Mz, X);
-    gemm2_f64(s, 0, 0, Mz, N, Mz, 1.0, X, Mz, f->d(F_UT), Mz, 0.0, B, Mz, 3);  // Lc^-1 K_zx
-    colsumsq_f64(s, B, Mz, Mz, n, q, 0);
-    fitc_train_var(s, n, c1, t1, c2, q, f->d(F_S), res);
+    fitc_train_var(s, n, kd, t1, c2, q, f->d(F_S), res);
     HIP_TRY(hipMemcpyAsync(out, res, n * 8, hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
     return GPL_OK;

@@ -86,8 +86,8 @@ void gemm2_f64(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, d
 void gemm2_f64_batched(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha, const double* A,
                        int64_t lda, const double* B, int64_t ldb, double beta, double* C, int64_t ldc, int tiles,
                        int batch, int64_t sA, int64_t sB, int64_t sC);
-// out[i] = sum_p W[p * stride + i] for i < n (fixed order)
-void sum_parts_f64(hipStream_t s, const double* W, int64_t stride, int parts, int64_t n, double* out);
+void gemm_gram_f64(hipStream_t s, int64_t M, int64_t K, const double* A, int64_t lda, const double* ks, int parts,
+                   int64_t kp, double* C, int64_t ldc, int64_t sC);
 // FP64 MFMA on an FP32 A
 void gemm_mixed_f32f64f64(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha,
                           const float* A, int64_t lda, const double* B, int64_t ldb, double beta, double* C,
@@ -229,11 +229,17 @@ void vec_recip(hipStream_t s, int64_t n, const double* a, double* out);
 
 // FITC (fitc.hip)
 void fitc_site(hipStream_t s, int64_t n, int64_t N, const double* D, const double* V, const double* z, double* S,
-               double* rs, double* zs);
+               double* si, double* zs);
 void scale_rows_copy_f64(hipStream_t s, const double* U, int64_t ld, int64_t nrow, int64_t ncol, const double* r,
                          double* W);
-void fitc_alpha(hipStream_t s, int64_t n, int64_t N, const double* zs, const double* u, const double* S,
-                double* alpha);
+void fitc_gram_sum(hipStream_t s, const double* parts, int P, int64_t Mz, double* G);
+// passes over A (Mz x N, ld Mz); part: fitc_pass_parts(n) * Mz doubles
+int fitc_pass_parts(int64_t n);
+void fitc_combine(hipStream_t s, const double* A, int64_t Mz, int64_t n, const double* coef, double* part, double* out);
+void fitc_alpha_pass(hipStream_t s, const double* A, int64_t Mz, int64_t n, int64_t N, const double* q, const double* zs,
+                     const double* S, double* alpha, double* part, double* out);
+void fitc_mean(hipStream_t s, const double* A, int64_t Mz, int64_t n, int64_t N, const double* w, const double* D,
+               const double* alpha, double* fmean);
 void coldot_f64(hipStream_t s, const double* A, const double* B, int64_t ld, int64_t nrow, int64_t ncol, double* out);
 void fitc_diag(hipStream_t s, int64_t n, int64_t N, const double* kd, const double* cs, double jitter, double* D);
 void vec_log(hipStream_t s, int64_t n, const double* a, double* out);
