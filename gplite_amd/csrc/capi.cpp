@@ -582,18 +582,18 @@ static void potrf32_blocked(gpl_ctx* c, float* L, int64_t N, double* Dinv, doubl
     inv.finish();
 }
 
-// alpha = sv .* L^-T L^-1 (sv .* z)   (R/laplace.R:29 with C = diag(sqrt V) L)
-// alpha = S B^-1 S z = S L^-T L^-1 S z with the factorization carrying the
-// forward solve: W1 = S z before potrf_blocked(..., rhs = W1), which leaves
 void gpl::trsv_lower(gpl_ctx* c, hipStream_t s, const double* L, int64_t ld, const double* Dinv, int64_t N, double* b,
-                     double* x, int trans, int* info) {
+                     double* x, int trans, int* info, const double* scale, int64_t n, double* scaled,
+                     const int* gate) {
     const int64_t T = N / 64;
     if (T > kSolveMaxBlocks) {
         trsv_lower_f64(s, L, ld, Dinv, N, b, x, trans);
+        if (scaled) vec_mul_pad(s, n, N, scale, x, scaled, gate);
         return;
     }
     if (++c->pepoch == 0) c->pepoch = 1;
-    trsv_persist_f64(s, L, ld, Dinv, N, b, x, trans, c->tsync, c->pepoch, c->tbase, info, c->pwait);
+    trsv_persist_f64(s, L, ld, Dinv, N, b, x, trans, c->tsync, c->pepoch, c->tbase, info, c->pwait, scale, n, scaled,
+                     gate);
     c->tbase += (unsigned)T;
 }
 
@@ -613,26 +613,14 @@ void gpl::trsm_forward(gpl_ctx* c, hipStream_t s, const double* L, int64_t ld, c
     }
 }
 
-// L^-1 S z in W1; then alpha = S L^-T W1.
-static double* alpha_rhs(gpl_model* m, const double* z) {
-    hipStream_t s = m->ctx->stream;
-    double* w1 = m->d(B_W1);
-    fill_f64(s, w1, m->N, 0.0);
-    vec_mul(s, m->n, m->d(B_SV), z, w1);
-    return w1;
-}
-
-static void solve_alpha_back(gpl_ctx* c, gpl_model* m, double* alpha) {
-    hipStream_t s = c->stream;
+// alpha = sv .* L^-T L^-1 (sv .* z) (R/laplace.R:29 with C = diag(sqrt V) L): the
+// factorization carries the forward solve (rhs = W1 = sv .* z, which the site
+// kernel leaves), so what is left is the transposed solve of W1.
+static void solve_alpha_back(gpl_ctx* c, gpl_model* m, const int* gate = nullptr) {
     const int64_t N = m->N;
-    double* w1 = m->d(B_W1);
-    double* w2 = m->d(B_W2);
-    {
-        Prof p(c, "trsv", 1.0 * N * N, 8.0 * N * N / 2);
-        trsv_lower(c, s, m->d(B_L), N, m->d(B_DINV), N, w1, w2, 1, m->b[B_INFO].as<int>());
-    }
-    fill_f64(s, alpha, N, 0.0);
-    vec_mul(s, m->n, m->d(B_SV), w2, alpha);
+    Prof p(c, "trsv", 1.0 * N * N, 8.0 * N * N / 2);
+    trsv_lower(c, c->stream, m->d(B_L), N, m->d(B_DINV), N, m->d(B_W1), m->d(B_W2), 1, m->b[B_INFO].as<int>(),
+               m->d(B_SV), m->n, m->d(B_ALPHA), gate);
 }
 
 int gpl::wait_timeout_fail() {
@@ -701,6 +689,15 @@ static int read_scalars(gpl_model* m, double* out, int k) {
 }
 
 // One Gaussian "Newton step" (exactly one: R/laplace.R:281-283).
+// What a finish kernel left in the context's pinned block: four scalars, two flags.
+static int read_finish(gpl_ctx* c, double* h, int* fl) {
+    HIP_TRY(hipStreamSynchronize(c->stream));
+    for (int k = 0; k < 4; ++k) h[k] = c->stage[k];
+    fl[0] = (int)c->stage[4];
+    fl[1] = (int)c->stage[5];
+    return GPL_OK;
+}
+
 static int fit_gaussian(gpl_model* m) {
     gpl_ctx* c = m->ctx;
     hipStream_t s = c->stream;
@@ -712,7 +709,7 @@ static int fit_gaussian(gpl_model* m) {
         launch_build_sym_f64(s, pd, m->prog, m->d(B_F), n, N, m->opts.jitter, 1, 1.0 / sigma, nullptr, m->d(B_L), N);
     }
     lik_pseudodata_la(s, GPL_LIK_GAUSSIAN, 0, sigma, n, nullptr, m->d(B_Y), nullptr, nullptr, m->d(B_Z), m->d(B_V),
-                      m->d(B_SV), m->b[B_INFO].as<int>() + 1);
+                      m->d(B_SV), m->b[B_INFO].as<int>() + 1, 0, N, m->d(B_W1));
     const bool inv = m->opts.flags & GPL_FLAG_INVERSE;
     if (inv) {
         // X = L^-1 with the factor; B^-1's buffer (which the gradient fills next)
@@ -721,36 +718,30 @@ static int fit_gaussian(gpl_model* m) {
         ENSURE(m, B_BINV, (size_t)N * N * 8);
     }
     potrf_blocked(c, m->d(B_L), N, m->d(B_DINV), m->d(B_LDIAG), m->b[B_INFO].as<int>(), inv ? m->d(B_XINV) : nullptr,
-                  inv ? m->d(B_BINV) : nullptr, inv ? nullptr : alpha_rhs(m, m->d(B_Z)));
+                  inv ? m->d(B_BINV) : nullptr, inv ? nullptr : m->d(B_W1));
     if (inv) {
         // alpha = S X^T X S z (S = 1/sigma)
         m->have_xinv = true;
         Prof p(c, "trmv", 4.0 * N * N / 2, 8.0 * N * N);
-        fill_f64(s, m->d(B_W1), N, 0.0);
-        vec_mul(s, n, m->d(B_SV), m->d(B_Z), m->d(B_W1));
         trmv_lower_f64_chunked(s, m->d(B_XINV), N, N, m->d(B_W1), m->d(B_W2), 0, m->d(B_KMV), kmatvec_chunks(N));
         trmv_lower_f64_chunked(s, m->d(B_XINV), N, N, m->d(B_W2), m->d(B_W1), 1, m->d(B_KMV), kmatvec_chunks(N));
-        fill_f64(s, m->d(B_ALPHA), N, 0.0);
-        vec_mul(s, n, m->d(B_SV), m->d(B_W1), m->d(B_ALPHA));
+        vec_mul_pad(s, n, N, m->d(B_SV), m->d(B_W1), m->d(B_ALPHA));
     } else {
-        solve_alpha_back(c, m, m->d(B_ALPHA));
+        solve_alpha_back(c, m);
     }
     {
         Prof p(c, "kmatvec", 0, 0);
         launch_kmatvec(s, pd, m->prog, m->d(B_F), n, N, m->opts.jitter, m->d(B_ALPHA), m->d(B_FMEAN), m->d(B_KMV),
                        kmatvec_chunks(N));
     }
-    lik_loglik(s, GPL_LIK_GAUSSIAN, 0, sigma, n, m->d(B_FMEAN), m->d(B_Y), nullptr,
-               m->has_offset ? m->d(B_OFF) : nullptr, m->d(B_W3));
-    double* sc = m->d(B_SCAL);
-    reduce_sum(s, m->d(B_W3), n, sc + 0);
-    reduce_dot(s, m->d(B_FMEAN), m->d(B_ALPHA), n, sc + 1);
-    reduce_sum(s, m->d(B_LDIAG), n, sc + 2);
-    int r = check_info(m);
+    laplace_finish(s, GPL_LIK_GAUSSIAN, 0, sigma, n, m->d(B_FMEAN), m->d(B_Y), nullptr,
+                   m->has_offset ? m->d(B_OFF) : nullptr, m->d(B_ALPHA), m->d(B_LDIAG), nullptr,
+                   m->b[B_INFO].as<int>(), c->stage);
+    double h[4];
+    int fl[2];
+    int r = read_finish(c, h, fl);
     if (r) return r;
-    double h[3];
-    r = read_scalars(m, h, 3);
-    if (r) return r;
+    if (fl[0] > 0) return pivot_fail(fl[0]);
     // log_lik - 1/2 f^T alpha - 1/2 (logdet C - logdet V), logdet C - logdet V = 2 sum log L_ii
     m->logZ = h[0] - 0.5 * h[1] - h[2];
     m->iters = 1;
@@ -900,30 +891,24 @@ static int fit_laplace(gpl_model* m) {
     double diff = INFINITY;
     int it = 0;
     for (it = 1; it <= maxiter; ++it) {
-        int* flags = m->b[B_INFO].as<int>();
-        hipMemsetAsync(flags, 0, 8, s);
+        int* flags = m->b[B_INFO].as<int>();  // zero here: the finish kernel clears them
         lik_pseudodata_la(s, m->lik.kind, m->lik.link, lik_par(m->lik), n, m->d(B_FOLD), m->d(B_Y), tr, off, m->d(B_Z),
-                          m->d(B_V), m->d(B_SV), flags + 1, (m->opts.flags & GPL_FLAG_ANALYTIC_W) ? 1 : 0);
+                          m->d(B_V), m->d(B_SV), flags + 1, (m->opts.flags & GPL_FLAG_ANALYTIC_W) ? 1 : 0, N, m->d(B_W1));
         {
             Prof p(c, "form_B", 0, 16.0 * N * (N + 64) / 2);
             form_B_f64(s, m->d(B_K), m->d(B_L), N, n, N, m->d(B_SV));
         }
-        potrf_blocked(c, m->d(B_L), N, m->d(B_DINV), m->d(B_LDIAG), flags, nullptr, nullptr, alpha_rhs(m, m->d(B_Z)));
-        solve_alpha_back(c, m, m->d(B_ALPHA));
+        potrf_blocked(c, m->d(B_L), N, m->d(B_DINV), m->d(B_LDIAG), flags, nullptr, nullptr, m->d(B_W1));
+        solve_alpha_back(c, m);
         {
             Prof p(c, "symv", 2.0 * N * N, 8.0 * N * N / 2);
             symv_lt_f64(s, m->d(B_K), N, m->d(B_ALPHA), m->d(B_FMEAN), m->d(B_KMV), kmatvec_chunks(N), 1, 0, 0);
         }
-        lik_loglik(s, m->lik.kind, m->lik.link, lik_par(m->lik), n, m->d(B_FMEAN), m->d(B_Y), tr, off, m->d(B_W3));
-        double* sc = m->d(B_SCAL);
-        reduce_sum(s, m->d(B_W3), n, sc + 0);
-        reduce_dot(s, m->d(B_FMEAN), m->d(B_ALPHA), n, sc + 1);
-        reduce_sum(s, m->d(B_LDIAG), n, sc + 2);
-        reduce_maxabsdiff(s, m->d(B_FOLD), m->d(B_FMEAN), n, sc + 3);
-        int fl[2];
-        HIP_TRY(hipMemcpyAsync(fl, flags, 8, hipMemcpyDeviceToHost, s));
+        laplace_finish(s, m->lik.kind, m->lik.link, lik_par(m->lik), n, m->d(B_FMEAN), m->d(B_Y), tr, off,
+                       m->d(B_ALPHA), m->d(B_LDIAG), m->d(B_FOLD), flags, c->stage);
         double h[4];
-        int r = read_scalars(m, h, 4);
+        int fl[2];
+        int r = read_finish(c, h, fl);
         if (r) return r;
         if (fl[1] & 2) {
             m->logZ = -INFINITY;
@@ -939,7 +924,9 @@ static int fit_laplace(gpl_model* m) {
                 HIP_TRY(hipMemcpyAsync(m->d(B_FMEAN), m->d(B_FOLD), N * 8, hipMemcpyDeviceToDevice, s));
                 break;
             }
-            reduce_maxabsdiff(s, m->d(B_FOLD), m->d(B_FMEAN), n, sc + 3);
+            reduce_maxabsdiff(s, m->d(B_FOLD), m->d(B_FMEAN), n, m->d(B_SCAL) + 3);
+            HIP_TRY(hipMemcpyAsync(m->d(B_FOLD), m->d(B_FMEAN), N * 8, hipMemcpyDeviceToDevice, s));
+            HIP_TRY(hipMemsetAsync(flags, 0, 8, s));
             r = read_scalars(m, h, 4);
             if (r) return r;
         } else {
@@ -948,7 +935,6 @@ static int fit_laplace(gpl_model* m) {
             m->logZ = h[0] - 0.5 * h[1] - h[2];
         }
         diff = h[3];
-        HIP_TRY(hipMemcpyAsync(m->d(B_FOLD), m->d(B_FMEAN), N * 8, hipMemcpyDeviceToDevice, s));
         if (diff < m->opts.tol) break;
     }
     if (it > maxiter) it = maxiter;
@@ -1177,30 +1163,45 @@ static int fit_ep(gpl_model* m) {
     bool quad_ok = true;
     int it;
     for (it = 1; it <= maxiter; ++it) {
-        int* flags = m->b[B_INFO].as<int>();
-        hipMemsetAsync(flags, 0, 8, s);
+        int* flags = m->b[B_INFO].as<int>();  // zero here: the finish kernel clears them
+        const int* gate = flags + 1;          // a flagged sweep leaves alpha, the means and the variances alone
         {
             Prof p(c, "ep_sites", 0, 0);
             ep_sites(s, m->lik.kind, m->lik.link, lik_par(m->lik), n, m->d(B_FOLD), m->d(B_FVOLD), m->d(B_ZOLD), m->d(B_POLD),
                      m->d(B_Y), tr, off, q, m->d(B_GH), m->d(B_GH) + 32, damp, m->d(B_Z), m->d(B_V), m->d(B_SV),
-                     m->d(B_LOGZS), m->d(B_CAVM), m->d(B_CAVV), flags + 1);
+                     m->d(B_LOGZS), m->d(B_CAVM), m->d(B_CAVV), flags + 1, N, m->d(B_W1));
         }
+        {
+            Prof p(c, "form_B", 0, 16.0 * N * (N + 64) / 2);
+            form_B_f64(s, m->d(B_K), m->d(B_L), N, n, N, m->d(B_SV));
+        }
+        // X = L^-1 for the posterior variances: its front half beside the factor, no scratch
+        potrf_blocked(c, m->d(B_L), N, m->d(B_DINV), m->d(B_LDIAG), flags, m->d(B_XINV), nullptr, m->d(B_W1));
+        solve_alpha_back(c, m, gate);
+        {
+            Prof p(c, "symv", 2.0 * N * N, 8.0 * N * N / 2);
+            symv_lt_f64(s, m->d(B_K), N, m->d(B_ALPHA), m->d(B_FMEAN), m->d(B_KMV), kmatvec_chunks(N), 1, 0, 0, gate);
+        }
+        colsumsq_f64(s, m->d(B_XINV), N, N, n, m->d(B_W3), 1);
+        ep_finish(s, n, m->d(B_V), m->d(B_Z), m->d(B_W3), m->d(B_CAVM), m->d(B_CAVV), m->d(B_LOGZS), m->d(B_ALPHA),
+                  m->d(B_LDIAG), m->d(B_FMEAN), m->d(B_FVAR), m->d(B_FOLD), m->d(B_FVOLD), m->d(B_ZOLD), m->d(B_POLD),
+                  diff_old, flags, c->stage);
+        double h[4];
         int fl[2];
-        HIP_TRY(hipMemcpyAsync(fl, flags, 8, hipMemcpyDeviceToHost, s));
-        HIP_TRY(hipStreamSynchronize(s));
+        int r = read_finish(c, h, fl);
+        if (r) return r;
         if (fl[1] & 2) {
             m->logZ = -INFINITY;
             m->iters = it;
             return fail(GPL_ERR_NAN, "NaN in EP site parameters (R/ep.R:30-32 returns log_evidence = -Inf)");
         }
         quad_ok = !(fl[1] & 1);  // the last sweep's flag decides (R/ep.R:326-328)
-        double* sc = m->d(B_SCAL);
-        double h[4];
         if (fl[1] & 4) {
             // some site variance <= 0: the split sweep of R/ep.R:50-138
             double lz = 0;
-            int r = split_step(m, true, &lz);
+            r = split_step(m, true, &lz);
             if (r) return r;
+            HIP_TRY(hipMemsetAsync(flags, 0, 8, s));
             if (m->no_posterior) {
                 // The reference returns fmean = Inf (R/ep.R:90-92): diff_new = Inf, so after an
                 // accepted sweep the sweep is rejected with more damping; on the first sweep it
@@ -1215,39 +1216,17 @@ static int fit_ep(gpl_model* m) {
                 damp = damp * damping;
                 continue;
             }
-            reduce_maxabsdiff(s, m->d(B_FOLD), m->d(B_FMEAN), n, sc + 3);
+            reduce_maxabsdiff(s, m->d(B_FOLD), m->d(B_FMEAN), n, m->d(B_SCAL) + 3);
             r = read_scalars(m, h, 4);
             if (r) return r;
             m->logZ = lz;
             m->have_xinv = false;
         } else {
-        {
-            Prof p(c, "form_B", 0, 16.0 * N * (N + 64) / 2);
-            form_B_f64(s, m->d(B_K), m->d(B_L), N, n, N, m->d(B_SV));
-        }
-        // X = L^-1 for the posterior variances: its front half beside the factor, no scratch
-        potrf_blocked(c, m->d(B_L), N, m->d(B_DINV), m->d(B_LDIAG), flags, m->d(B_XINV), nullptr,
-                      alpha_rhs(m, m->d(B_Z)));
-        solve_alpha_back(c, m, m->d(B_ALPHA));
-        {
-            Prof p(c, "symv", 2.0 * N * N, 8.0 * N * N / 2);
-            symv_lt_f64(s, m->d(B_K), N, m->d(B_ALPHA), m->d(B_FMEAN), m->d(B_KMV), kmatvec_chunks(N), 1, 0, 0);
-        }
-        colsumsq_f64(s, m->d(B_XINV), N, N, n, m->d(B_W3), 1);
-        ep_post(s, n, m->d(B_V), m->d(B_Z), m->d(B_W3), m->d(B_CAVM), m->d(B_CAVV), m->d(B_LOGZS), m->d(B_FVAR),
-                m->d(B_TERM));
-        reduce_sum(s, m->d(B_TERM), n, sc + 0);
-        reduce_dot(s, m->d(B_Z), m->d(B_ALPHA), n, sc + 1);
-        reduce_sum(s, m->d(B_LDIAG), n, sc + 2);
-        reduce_maxabsdiff(s, m->d(B_FOLD), m->d(B_FMEAN), n, sc + 3);
-        HIP_TRY(hipMemcpyAsync(fl, flags, 8, hipMemcpyDeviceToHost, s));
-        int r = read_scalars(m, h, 4);
-        if (r) return r;
-        if (fl[0] > 0) return pivot_fail(fl[0]);
-        m->split = false;
-        m->no_posterior = false;
-        m->have_xinv = true;
-        m->logZ = h[0] - h[2] - 0.5 * h[1];
+            if (fl[0] > 0) return pivot_fail(fl[0]);
+            m->split = false;
+            m->no_posterior = false;
+            m->have_xinv = true;
+            m->logZ = h[0] - h[2] - 0.5 * h[1];
         }
         diff_new = h[3];
         if (diff_new > diff_old) {
@@ -1255,10 +1234,12 @@ static int fit_ep(gpl_model* m) {
             continue;
         }
         damp = std::max(damp, dmin);
-        HIP_TRY(hipMemcpyAsync(m->d(B_FOLD), m->d(B_FMEAN), N * 8, hipMemcpyDeviceToDevice, s));
-        HIP_TRY(hipMemcpyAsync(m->d(B_FVOLD), m->d(B_FVAR), N * 8, hipMemcpyDeviceToDevice, s));
-        HIP_TRY(hipMemcpyAsync(m->d(B_ZOLD), m->d(B_Z), N * 8, hipMemcpyDeviceToDevice, s));
-        vec_recip(s, n, m->d(B_V), m->d(B_POLD));  // P_old = fit$P = 1 / V
+        if (fl[1] & 4) {  // else the finish kernel did this
+            HIP_TRY(hipMemcpyAsync(m->d(B_FOLD), m->d(B_FMEAN), N * 8, hipMemcpyDeviceToDevice, s));
+            HIP_TRY(hipMemcpyAsync(m->d(B_FVOLD), m->d(B_FVAR), N * 8, hipMemcpyDeviceToDevice, s));
+            HIP_TRY(hipMemcpyAsync(m->d(B_ZOLD), m->d(B_Z), N * 8, hipMemcpyDeviceToDevice, s));
+            vec_recip(s, n, m->d(B_V), m->d(B_POLD));  // P_old = fit$P = 1 / V
+        }
         diff_old = diff_new;
         if (diff_new < tol) break;
     }

@@ -1158,14 +1158,17 @@ void trsv_lower_f64(hipStream_t s, const double* L, int64_t ld, const double* Di
 // before the wait), forms x_i = Dinv_i b_i (Dinv_i^T b_i) and publishes x_i.
 // Every wait is on a block of a lower ticket, whose workgroup has started and
 // waits only on lower tickets, so every wait ends; the summation order is
-// fixed (deterministic).  sync: flags [0, T), the ticket counter at
-// sync[kSolveMaxBlocks].
+// fixed (deterministic).  With `scaled` the launch also leaves scale .* x there
+// (zero beyond n), unless the gate's flags say NaN or V <= 0.  sync: flags [0, T),
+// the ticket counter at sync[kSolveMaxBlocks].
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_trsv_persist(const double* __restrict__ L, int64_t ld,
                                                       const double* __restrict__ Dinv, int64_t T,
                                                       const double* __restrict__ b, double* __restrict__ x, int trans,
                                                       unsigned* __restrict__ sync, unsigned epoch, unsigned base,
-                                                      int* __restrict__ info, unsigned maxpoll) {
+                                                      int* __restrict__ info, unsigned maxpoll,
+                                                      const double* __restrict__ scale, int64_t n,
+                                                      double* __restrict__ scaled, const int* __restrict__ gate) {
     __shared__ double red[256];
     __shared__ double sv[64];
     __shared__ unsigned s_id;
@@ -1185,8 +1188,8 @@ __global__ __launch_bounds__(256) void k_trsv_persist(const double* __restrict__
     }
     const double bi = (t < 64) ? b[64 * i + t] : 0.0;
     double acc = 0.0;
-    for (int64_t n = 0; n < k; ++n) {
-        const int64_t j = trans ? T - 1 - n : n;  // the blocks solved before i, in their order
+    for (int64_t m = 0; m < k; ++m) {
+        const int64_t j = trans ? T - 1 - m : m;  // the blocks solved before i, in their order
         double lt[16];
 #pragma unroll
         for (int u = 0; u < 16; ++u) {
@@ -1207,17 +1210,19 @@ __global__ __launch_bounds__(256) void k_trsv_persist(const double* __restrict__
     for (int u = 0; u < 16; ++u) s += dv[u] * sv[16 * p + u];
     red[t] = s;
     __syncthreads();
-    if (t < 64) put_shared(x + 64 * i + t, red[t] + red[t + 64] + red[t + 128] + red[t + 192]);
+    const double xi = (t < 64) ? red[t] + red[t + 64] + red[t + 128] + red[t + 192] : 0.0;
+    if (t < 64) put_shared(x + 64 * i + t, xi);
     panel_publish(&sync[i], epoch);
+    if (scaled && t < 64 && !(gate && (*gate & 6))) scaled[64 * i + t] = 64 * i + t < n ? scale[64 * i + t] * xi : 0.0;
 }
 
 void trsv_persist_f64(hipStream_t s, const double* L, int64_t ld, const double* Dinv, int64_t N, const double* b,
                       double* x, int trans, unsigned* sync, unsigned epoch, unsigned base, int* info,
-                      unsigned maxpoll) {
+                      unsigned maxpoll, const double* scale, int64_t n, double* scaled, const int* gate) {
     const int64_t T = N / 64;
     if (T <= 0) return;
     hipLaunchKernelGGL(k_trsv_persist, dim3((unsigned)T), dim3(256), 0, s, L, ld, Dinv, T, b, x, trans, sync, epoch,
-                       base, info, maxpoll);
+                       base, info, maxpoll, scale, n, scaled, gate);
 }
 
 // ---------------------------------------------------------------------------
@@ -1607,7 +1612,9 @@ __global__ __launch_bounds__(256) void k_symv2(const double* __restrict__ A, int
 
 // y[i] = sum of the row-role slots CJ <= I and the column-role slots RI >= I of
 // output block i (I = its super-tile row), in that order
-__global__ void k_symv2_sum(const double* __restrict__ part, int64_t T, int G, double* __restrict__ y, int64_t sV) {
+__global__ void k_symv2_sum(const double* __restrict__ part, int64_t T, int G, double* __restrict__ y, int64_t sV,
+                            const int* __restrict__ gate) {
+    if (gate && (*gate & 6)) return;
     const int64_t b = blockIdx.y, S = (T + G - 1) / G, N = T * 64;
     part += b * 2 * S * N;
     y += b * sV;
@@ -1635,7 +1642,7 @@ __global__ void k_chunk_sum(const double* __restrict__ part, int64_t N, int nchu
 // part: batch * symv_slots(N, batch) * N doubles (nchunk is not used)
 void chunk_sum_f64(hipStream_t s, const double* part, int64_t N, int nchunk, double* y, int batch, int64_t sV);
 void symv_lt_f64(hipStream_t s, const double* A, int64_t N, const double* v, double* y, double* part, int nchunk,
-                 int batch, int64_t sA, int64_t sV) {
+                 int batch, int64_t sA, int64_t sV, const int* gate) {
     (void)nchunk;
     const int64_t T = N / 64;
     const int G = symv_group(batch);
@@ -1644,7 +1651,7 @@ void symv_lt_f64(hipStream_t s, const double* A, int64_t N, const double* v, dou
     if (G == 4) hipLaunchKernelGGL(k_symv2<4>, grid, dim3(256), 0, s, A, N, T, v, part, sA, sV);
     else hipLaunchKernelGGL(k_symv2<2>, grid, dim3(256), 0, s, A, N, T, v, part, sA, sV);
     hipLaunchKernelGGL(k_symv2_sum, dim3((unsigned)((N + 255) / 256), (unsigned)batch), dim3(256), 0, s, part, T, G, y,
-                       sV);
+                       sV, gate);
 }
 
 // y[b][i] = sum_c part[b][c][i] (fixed order)

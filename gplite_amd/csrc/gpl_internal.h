@@ -130,7 +130,7 @@ void chunk_sum_f64(hipStream_t s, const double* part, int64_t N, int nchunk, dou
 // batch * symv_slots(N, batch) * N doubles; nchunk is not used)
 int symv_slots(int64_t N, int batch);
 void symv_lt_f64(hipStream_t s, const double* A, int64_t N, const double* v, double* y, double* part, int nchunk,
-                 int batch, int64_t sA, int64_t sV);
+                 int batch, int64_t sA, int64_t sV, const int* gate = nullptr);
 // W = s B^-1 s - (t u^T + u t^T) in place over the lower tiles of B^-1 (t, u may be null)
 void form_wgrad_f64(hipStream_t s, double* B, int64_t N, int64_t n, const double* sv, const double* t,
                     const double* u);
@@ -156,7 +156,7 @@ constexpr int kSolveMaxBlocks = 4096;
 constexpr int kSolveSyncWords = kSolveMaxBlocks + 1;
 void trsv_persist_f64(hipStream_t s, const double* L, int64_t ld, const double* Dinv, int64_t N, const double* b,
                       double* x, int trans, unsigned* sync, unsigned epoch, unsigned base, int* info,
-                      unsigned maxpoll);
+                      unsigned maxpoll, const double* scale, int64_t n, double* scaled, const int* gate);
 // L Y = diag(sv) B in place for M right-hand sides (multiples of 64) in one launch; sync: kTrsmFlags + 1 words
 // of the context, N / 64 * (M / trsm_cols(N, M)) <= kTrsmFlags flags and as many tickets per launch
 constexpr int kTrsmFlags = 65536;
@@ -203,10 +203,11 @@ void reduce_cols(hipStream_t s, const double* part, int64_t rows, int64_t ld, in
                  double* out);  // out[c] = sum_r part[r*ld + c]
 
 // Likelihood kernels (lik.hip)
-// exact != 0: the exact curvature in place of the reference's forward difference
+// exact != 0: the exact curvature in place of the reference's forward difference; rhs (N
+// long, or none) receives sv .* z
 void lik_pseudodata_la(hipStream_t s, int lik, int link, double sigma, int64_t n, const double* f,
                        const double* y, const double* trials, const double* offset, double* z,
-                       double* V, double* sv, int* bad, int exact = 0);
+                       double* V, double* sv, int* bad, int exact = 0, int64_t N = 0, double* rhs = nullptr);
 // Laplace gradient vectors at the mode: u = d log p / d f, s2 = 1/2 V_i (1 - B^-1_ii) d3_i
 void lik_la_grad_vectors(hipStream_t s, int lik, int link, double par, int64_t n, int64_t N, const double* f,
                          const double* y, const double* trials, const double* offset, const double* V,
@@ -218,13 +219,22 @@ void ep_sites(hipStream_t s, int lik, int link, double par, int64_t n, const dou
               const double* z_old, const double* P_old, const double* y, const double* trials,
               const double* offset, int q, const double* gh_x, const double* gh_w, double damping,
               double* z, double* V, double* sv, double* logZs, double* cav_m, double* cav_v,
-              int* nan_flag);
+              int* nan_flag, int64_t N = 0, double* rhs = nullptr);
+void laplace_finish(hipStream_t s, int lik, int link, double par, int64_t n, const double* f, const double* y,
+                    const double* trials, const double* offset, const double* alpha, const double* ldiag, double* fold,
+                    int* flags, double* host);
+void ep_finish(hipStream_t s, int64_t n, const double* V, const double* z, const double* binv_diag, const double* cav_m,
+               const double* cav_v, const double* logZs, const double* alpha, const double* ldiag, const double* f,
+               double* fvar, double* fold, double* fvold, double* zold, double* pold, double diff_old, int* flags,
+               double* host);
 void ep_post(hipStream_t s, int64_t n, const double* V, const double* z, const double* binv_diag,
              const double* cav_m, const double* cav_v, const double* logZs, double* fvar,
              double* term);
 void vec_axpby(hipStream_t s, int64_t n, double a, const double* x, double b, const double* y,
                double* out);
 void vec_mul(hipStream_t s, int64_t n, const double* a, const double* b, double* out);
+void vec_mul_pad(hipStream_t s, int64_t n, int64_t N, const double* a, const double* b, double* out,
+                 const int* gate = nullptr);
 void vec_recip(hipStream_t s, int64_t n, const double* a, double* out);
 
 // FITC (fitc.hip)

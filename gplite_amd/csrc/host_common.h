@@ -37,9 +37,11 @@ void trtri_blocked(gpl_ctx* c, const double* L, const double* Dinv, int64_t N, d
 // Blocked triangular solve with one vector (trsv_lower_f64's arguments, b left
 // unchanged): one launch on the context's solve flags when N / 64 <=
 // kSolveMaxBlocks, else one launch per block.  info receives kPanelWaitTimeout
-// if a device wait times out.
+// if a device wait times out.  With `scaled` also scaled = scale .* x (n entries,
+// zero on the padding) unless *gate (if any) flags NaN or V <= 0.
 void trsv_lower(gpl_ctx* c, hipStream_t s, const double* L, int64_t ld, const double* Dinv, int64_t N, double* b,
-                double* x, int trans, int* info);
+                double* x, int trans, int* info, const double* scale = nullptr, int64_t n = 0,
+                double* scaled = nullptr, const int* gate = nullptr);
 // L Y = diag(sv) B in place for M right-hand sides (sv: the first n rows, or null): the forward solve of a
 // prediction, in launches of at most kTrsmFlags blocks.  info receives kPanelWaitTimeout if a device wait
 // times out.
