@@ -71,6 +71,7 @@ def _sig(lib):
         "gpl_profile_reset": (C.c_int, [_vp]),
         "gpl_profile_read": (C.c_int, [_vp, i32, C.c_char_p, _dp, C.POINTER(i64), _dp, _dp]),
         "gpl_opts_default": (None, [C.POINTER(Opts)]),
+        "gpl_col_scales": (None, [_dp, i64, i64, _dp, _dp]),
         "gpl_grad_len": (i32, [C.POINTER(CfTerm), i32, i32]),
         "gpl_cf_sexp": (C.c_int, [_vp, _dp, i64, _dp, i64, i64, _dp, i64, C.c_double, i32, _dp]),
         "gpl_cf_matern32": (C.c_int, [_vp, _dp, i64, _dp, i64, i64, _dp, i64, C.c_double, i32, _dp]),

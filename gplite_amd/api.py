@@ -111,6 +111,12 @@ class Cf:
         x = _as_matrix(x)
         if self.vars is not None:
             x = x[:, _col_index(x, self.vars)]
+        if L._lib is not None and x.size >= 4096 and x.shape[0] > 1 and x.shape[1] > 1 and x.flags.c_contiguous:
+            # numpy's sums over the rows in the same order, without its n x d temporaries
+            # (131072 x 8: 4.0 ms there, 0.3 here; below 4096 numbers the calls cost the same)
+            self.means, self.scales = np.empty(x.shape[1]), np.empty(x.shape[1])
+            L._lib.gpl_col_scales(L.dptr(x), x.shape[0], x.shape[1], L.dptr(self.means), L.dptr(self.scales))
+            return
         self.means = x.mean(axis=0)
         self.scales = x.std(axis=0, ddof=1) if x.shape[0] > 1 else np.ones(x.shape[1])
 

@@ -25,7 +25,7 @@ namespace {
 
 enum {
     BB_X, BB_XOFF, BB_N, BB_PROG, BB_F, BB_Y, BB_SV, BB_SCAL, BB_SIG, BB_WSC, BB_IDX, BB_RHS, BB_U, BB_R, BB_D, BB_T1,
-    BB_KU, BB_ALPHA, BB_L, BB_X32, BB_BI, BB_DINV, BB_LDIAG, BB_INFO, BB_PART, BB_KMV, BB_RED, BB_CORR, BB_DACC, BB_B64, BB_RELMAX, BB_COUNT
+    BB_KU, BB_ALPHA, BB_L, BB_X32, BB_BI, BB_DINV, BB_LDIAG, BB_PART, BB_KMV, BB_RED, BB_CORR, BB_DACC, BB_B64, BB_COUNT
 };
 
 struct Bucket {
@@ -35,6 +35,8 @@ struct Bucket {
     int bm = 0;       // GEMM tile edge (0 = heuristic)
     int nbo = 256;    // outer panel width
     int nchunk = 1;
+    int* info = nullptr;    // per problem, in the batch's status block: failing minor
+    double* rel = nullptr;  // the last refinement correction, then the one before
     DevBuf b[BB_COUNT];
     double* d(int i) const { return b[i].as<double>(); }
     float* f(int i) const { return b[i].as<float>(); }
@@ -62,6 +64,8 @@ struct gpl_batch {
     std::vector<int> bucket_of;  // problem -> bucket index
     std::vector<int> pos_in;     // problem -> position in its bucket
     DevBuf res_logz, res_grad;
+    DevBuf stat;  // every bucket's corrections (two doubles per problem), then every bucket's info words
+    size_t stat_bytes() const { return (size_t)nprob * 20; }
     std::vector<hipGraph_t> graph;      // one per lane
     std::vector<hipGraphExec_t> exec;   // one per lane (null: lane without buckets)
     std::vector<Lane> lanes;
@@ -74,6 +78,7 @@ struct gpl_batch {
         for (auto* b : buckets) delete b;
         res_logz.free_();
         res_grad.free_();
+        stat.free_();
         for (auto e : exec)
             if (e) hipGraphExecDestroy(e);
         for (auto g : graph)
@@ -130,7 +135,7 @@ static void potrf_panel_rec(gpl_ctx* c, hipStream_t s, Bucket& k, int64_t K0, in
         const int64_t kk = K0 / 64;
         {
             Prof p(c, "batch_potrf_diag", 0, 0, s);
-            potrf_diag_f32_batched(s, L, N, kk, Dinv, k.d(BB_LDIAG), k.b[BB_INFO].as<int>(), nb, N2, N * 64, N, Dacc);
+            potrf_diag_f32_batched(s, L, N, kk, Dinv, k.d(BB_LDIAG), k.info, nb, N2, N * 64, N, Dacc);
         }
         const int64_t M = N - (K0 + 64);
         if (M > 0) {
@@ -285,8 +290,8 @@ static void bucket_pipeline(gpl_batch* B, Bucket& k, Lane& ln) {
         }
         vec_axpby(s2, NV, 1.0, dd, 1.0, u, u);
         // the last two corrections relative to the solution: their ratio is the contraction
-        if (it == sweeps - 2) seg_relmax(s2, dd, u, nvec, N, k.d(BB_RELMAX) + nb, nb);
-        if (it == sweeps - 1) seg_relmax(s2, dd, u, nvec, N, k.d(BB_RELMAX), nb);
+        if (it == sweeps - 2) seg_relmax(s2, dd, u, nvec, N, k.rel + nb, nb);
+        if (it == sweeps - 1) seg_relmax(s2, dd, u, nvec, N, k.rel, nb);
         {  // r = S y - B u with the FP64 copy of B
             Prof p(c, "batch_symv_b64", 2.0 * nb * N * N, 0, s2);
             symv_lt_f64(s2, k.d(BB_B64), N, u, Ku, k.d(BB_KMV), k.nchunk, nb, N2, N);
@@ -476,10 +481,10 @@ extern "C" int gpl_batch_create(gpl_ctx* c, int32_t nprob, const gpl_cf_term* te
                   k->b[BB_F].ensure((size_t)nb * N * MAX_FEAT * 8) && k->b[BB_SCAL].ensure(nb * 8) &&
                   k->b[BB_SIG].ensure(nb * 8) && k->b[BB_WSC].ensure(nb * 8) && k->b[BB_IDX].ensure(nb * 4) &&
                   k->b[BB_L].ensure(mat32) && k->b[BB_X32].ensure(mat32) && k->b[BB_BI].ensure(mat32) &&
-                  k->b[BB_B64].ensure(mat32 * 2) && k->b[BB_RELMAX].ensure((size_t)nb * 16) &&
+                  k->b[BB_B64].ensure(mat32 * 2) &&
                   k->b[BB_DINV].ensure((size_t)nb * N * 64 * 8) && k->b[BB_DACC].ensure((size_t)nb * N * 64 * 8) &&
                   k->b[BB_LDIAG].ensure(vec) &&
-                  k->b[BB_INFO].ensure(nb * 4 + 64) && k->b[BB_PART].ensure((size_t)nb * T * (T + 1) / 2 * 8 * std::max(1, B->hp.ngrad)) &&
+                  k->b[BB_PART].ensure((size_t)nb * T * (T + 1) / 2 * 8 * std::max(1, B->hp.ngrad)) &&
                   k->b[BB_KMV].ensure((size_t)nb * std::max(k->nchunk, symv_slots(N, nb)) * N * 8) &&
                   k->b[BB_RED].ensure((size_t)nb * red_stride(B) * 8) &&
                   k->b[BB_CORR].ensure((size_t)nb * T * (T + 1) / 2 * 8);
@@ -502,9 +507,20 @@ extern "C" int gpl_batch_create(gpl_ctx* c, int32_t nprob, const gpl_cf_term* te
         HIP_TRY(hipMemcpyAsync(k->b[BB_Y].p, ys.data(), ys.size() * 8, hipMemcpyHostToDevice, s));
         HIP_TRY(hipStreamSynchronize(s));
     }
-    if (!B->res_logz.ensure((size_t)nprob * 8) || !B->res_grad.ensure((size_t)nprob * B->ng * 8)) {
+    if (!B->res_logz.ensure((size_t)nprob * 8) || !B->res_grad.ensure((size_t)nprob * B->ng * 8) ||
+        !B->stat.ensure(B->stat_bytes() + 64)) {
         delete B;
         return fail(GPL_ERR_OOM, "device allocation failed for the batch");
+    }
+    {
+        double* rel = B->stat.as<double>();
+        int* info = (int*)(rel + 2 * nprob);
+        for (auto* k : B->buckets) {
+            k->rel = rel;
+            k->info = info;
+            rel += 2 * k->idx.size();
+            info += k->idx.size();
+        }
     }
     // lanes: up to sixteen stream pairs; buckets go to the least-loaded lane,
     // largest estimated time first (GEMM work plus a fixed cost per 64-row
@@ -580,9 +596,8 @@ extern "C" int gpl_batch_set_params(gpl_batch* B, const gpl_cf_term* terms, cons
 }
 
 static void reset_flags(gpl_batch* B, hipStream_t s) {
-    // outside any graph: status words are cleared with plain memsets before a pass
-    for (auto* k : B->buckets) hipMemsetAsync(k->b[BB_RELMAX].p, 0, k->idx.size() * 16, s);
-    for (auto* k : B->buckets) hipMemsetAsync(k->b[BB_INFO].p, 0, k->idx.size() * 4, s);
+    // outside any graph: status words are cleared with a plain memset before a pass
+    hipMemsetAsync(B->stat.p, 0, B->stat_bytes(), s);
 }
 
 // One graph per lane, captured on the lane's stream (its look-ahead side stream
@@ -644,10 +659,26 @@ static int batch_pass(gpl_batch* B, bool eager, double* log_evidence, double* gr
         int r = run_once(B);
         if (r) return r;
     }
-    if (log_evidence)
-        HIP_TRY(hipMemcpyAsync(log_evidence, B->res_logz.p, (size_t)B->nprob * 8, hipMemcpyDeviceToHost, s));
-    if (grad) HIP_TRY(hipMemcpyAsync(grad, B->res_grad.p, (size_t)B->nprob * B->ng * 8, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    // results and status words: through the pinned block with one wait (they are a
+    // few kilobytes; two copies per bucket with a wait each were 1 ms of a pass over
+    // 32 buckets)
+    const size_t nbytes = (size_t)B->nprob * 8, sbytes = B->stat_bytes();
+    std::vector<char> stat(sbytes);
+    if (sbytes + 8 + nbytes * (1 + B->ng) <= gpl_ctx::kStage * 8) {
+        char* st = (char*)B->ctx->stage;
+        HIP_TRY(hipMemcpyAsync(st, B->stat.p, sbytes, hipMemcpyDeviceToHost, s));
+        st += (sbytes + 7) / 8 * 8;
+        if (log_evidence) HIP_TRY(hipMemcpyAsync(st, B->res_logz.p, nbytes, hipMemcpyDeviceToHost, s));
+        if (grad) HIP_TRY(hipMemcpyAsync(st + nbytes, B->res_grad.p, nbytes * B->ng, hipMemcpyDeviceToHost, s));
+        HIP_TRY(hipStreamSynchronize(s));
+        memcpy(stat.data(), B->ctx->stage, sbytes);
+        if (log_evidence) memcpy(log_evidence, st, nbytes);
+        if (grad) memcpy(grad, st + nbytes, nbytes * B->ng);
+    } else {
+        HIP_TRY(read_back(B->ctx, stat.data(), B->stat.p, sbytes));
+        if (log_evidence) HIP_TRY(read_back(B->ctx, log_evidence, B->res_logz.p, nbytes));
+        if (grad) HIP_TRY(read_back(B->ctx, grad, B->res_grad.p, nbytes * B->ng));
+    }
     // Non-PD pivots, and refinements whose last correction stays above 1e-8 of the
     // solution (cond(B) too large for the FP32 inverse factor with the pass's fixed
     // sweep count): those problems get log_evidence = -Inf and NaN gradients, the
@@ -659,10 +690,11 @@ static int batch_pass(gpl_batch* B, bool eager, double* log_evidence, double* gr
     B->refine_rel.assign(B->nprob, 0.0);
     for (auto* k : B->buckets) {
         const size_t nb = k->idx.size();
+        const char* base = stat.data();
         std::vector<int> info(nb);
         std::vector<double> rr(2 * nb);
-        HIP_TRY(hipMemcpy(info.data(), k->b[BB_INFO].p, nb * 4, hipMemcpyDeviceToHost));
-        HIP_TRY(hipMemcpy(rr.data(), k->b[BB_RELMAX].p, nb * 16, hipMemcpyDeviceToHost));
+        memcpy(info.data(), base + ((char*)k->info - B->stat.as<char>()), nb * 4);
+        memcpy(rr.data(), base + ((char*)k->rel - B->stat.as<char>()), nb * 16);
         for (size_t q = 0; q < nb; ++q) {
             const int pidx = k->idx[q];
             B->refine_rel[pidx] = rr[q];

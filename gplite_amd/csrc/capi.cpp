@@ -48,6 +48,77 @@ void set_minor(int64_t minor) { g_minor = minor; }
 extern "C" const char* gpl_last_error(void) { return g_err.c_str(); }
 extern "C" int64_t gpl_last_error_minor(void) { return g_minor; }
 
+// ---------------------------------------------------------------------------
+// device blocks of freed models
+// ---------------------------------------------------------------------------
+static std::mutex g_pools_mu;
+static std::vector<BlockPool*> g_pools;
+
+BlockPool::BlockPool(size_t cap_bytes) : cap(cap_bytes) {
+    std::lock_guard<std::mutex> lk(g_pools_mu);
+    g_pools.push_back(this);
+}
+BlockPool::~BlockPool() {
+    {
+        std::lock_guard<std::mutex> lk(g_pools_mu);
+        g_pools.erase(std::find(g_pools.begin(), g_pools.end(), this));
+    }
+    clear();
+}
+void* BlockPool::take(size_t bytes, size_t* sz) {
+    if (bytes < kMin) return nullptr;
+    std::lock_guard<std::mutex> lk(mu);
+    int best = -1;
+    for (int i = 0; i < (int)blocks.size(); ++i)
+        if (blocks[i].sz >= bytes && blocks[i].sz <= bytes + bytes / 4 && (best < 0 || blocks[i].sz < blocks[best].sz))
+            best = i;
+    if (best < 0) return nullptr;
+    void* p = blocks[best].p;
+    *sz = blocks[best].sz;
+    total -= *sz;
+    blocks.erase(blocks.begin() + best);
+    return p;
+}
+void BlockPool::put(void* p, size_t sz) {
+    std::lock_guard<std::mutex> lk(mu);
+    if (sz < kMin || sz > cap) {
+        hipFree(p);
+        return;
+    }
+    while (total + sz > cap) {  // the oldest first
+        total -= blocks.front().sz;
+        hipFree(blocks.front().p);
+        blocks.erase(blocks.begin());
+    }
+    blocks.push_back({p, sz, frees});
+    total += sz;
+}
+void BlockPool::age() {
+    std::lock_guard<std::mutex> lk(mu);
+    ++frees;
+    while (!blocks.empty() && frees - blocks.front().born > kKeep) {
+        total -= blocks.front().sz;
+        hipFree(blocks.front().p);
+        blocks.erase(blocks.begin());
+    }
+}
+void BlockPool::clear() {
+    std::lock_guard<std::mutex> lk(mu);
+    for (auto& b : blocks) hipFree(b.p);
+    blocks.clear();
+    total = 0;
+}
+hipError_t dev_malloc(void** p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e == hipSuccess) return e;
+    {
+        std::lock_guard<std::mutex> lk(g_pools_mu);
+        for (auto* b : g_pools) b->clear();
+    }
+    (void)hipGetLastError();
+    return hipMalloc(p, bytes);
+}
+
 extern "C" int gpl_ctx_create(int32_t device, gpl_ctx** out) {
     if (!out) return fail(GPL_ERR_ARG, "out is NULL");
     int count = 0;
@@ -78,6 +149,10 @@ extern "C" int gpl_ctx_create(int32_t device, gpl_ctx** out) {
     if (e == hipSuccess) e = hipMemset(c->msync, 0, (kTrsmFlags + 64) * sizeof(unsigned));
     if (e == hipSuccess) c->minfo = (int*)(c->msync + kTrsmFlags + 32);
     if (e == hipSuccess) e = hipHostMalloc((void**)&c->stage, gpl_ctx::kStage * sizeof(double));
+    if (e == hipSuccess) e = hipHostMalloc((void**)&c->up, gpl_ctx::kStage * sizeof(double));
+    size_t mfree = 0, mtotal = 0;
+    if (e == hipSuccess) e = hipMemGetInfo(&mfree, &mtotal);
+    if (e == hipSuccess) c->blocks = new BlockPool(t_ctx_for_server ? 0 : mtotal / 32);
     if (const char* pw = getenv("GPL_PANEL_WAIT_POLLS")) c->pwait = (unsigned)strtoul(pw, nullptr, 10);
     if (e != hipSuccess) {
         delete c;
@@ -109,6 +184,8 @@ extern "C" void gpl_ctx_destroy(gpl_ctx* c) {
     if (c->tsync) hipFree(c->tsync);
     if (c->msync) hipFree(c->msync);
     if (c->stage) hipHostFree(c->stage);
+    if (c->up) hipHostFree(c->up);
+    delete c->blocks;
     hipStreamDestroy(c->side);
     hipStreamDestroy(c->stream);
     delete c;
@@ -180,6 +257,32 @@ static int term_ngrad(const gpl_cf_term& t) {
         case GPL_CF_NN: return 3;
         case GPL_CF_PERIODIC: return 2 + t.n_lscale;
         default: return 1 + t.n_lscale;
+    }
+}
+
+// W columns at x (row stride d): their sums stay in registers
+template <int W>
+static void col_scales(const double* x, int64_t n, int64_t d, double* means, double* scales) {
+#pragma clang fp contract(off)
+    double m[W], v[W];
+    for (int j = 0; j < W; ++j) m[j] = x[j], v[j] = 0.0;
+    for (int64_t i = 1; i < n; ++i)
+        for (int j = 0; j < W; ++j) m[j] += x[i * d + j];
+    for (int j = 0; j < W; ++j) m[j] /= (double)n;
+    for (int64_t i = 0; i < n; ++i)
+        for (int j = 0; j < W; ++j) {
+            const double e = x[i * d + j] - m[j];
+            v[j] += e * e;
+        }
+    for (int j = 0; j < W; ++j) means[j] = m[j], scales[j] = std::sqrt(v[j] / (double)(n - 1));
+}
+
+extern "C" void gpl_col_scales(const double* x, int64_t n, int64_t d, double* means, double* scales) {
+    for (int64_t j = 0; j < d;) {
+        const int w = d - j >= 8 ? 8 : d - j >= 4 ? 4 : d - j >= 2 ? 2 : 1;
+        (w == 8 ? col_scales<8> : w == 4 ? col_scales<4> : w == 2 ? col_scales<2> : col_scales<1>)(x + j, n, d, means + j,
+                                                                                                 scales + j);
+        j += w;
     }
 }
 
@@ -636,8 +739,7 @@ static int pivot_fail(int info) {
 
 static int check_info(gpl_model* m) {
     int info = 0;
-    HIP_TRY(hipMemcpyAsync(&info, m->b[B_INFO].p, sizeof(int), hipMemcpyDeviceToHost, m->ctx->stream));
-    HIP_TRY(hipStreamSynchronize(m->ctx->stream));
+    HIP_TRY(read_back(m->ctx, &info, m->b[B_INFO].p, sizeof(int)));
     if (info > 0) return pivot_fail(info);
     return GPL_OK;
 }
@@ -677,14 +779,13 @@ static int alloc_model(gpl_model* m, int64_t n, int64_t ncols, bool need_k, bool
 static int upload_vec(gpl_model* m, int idx, const double* h, int64_t n) {
     hipStream_t s = m->ctx->stream;
     fill_f64(s, m->d(idx), m->N, 0.0);
-    if (h) HIP_TRY(hipMemcpyAsync(m->d(idx), h, n * 8, hipMemcpyHostToDevice, s));
+    if (h) HIP_TRY(upload(m->ctx, s, m->d(idx), h, n * 8));
     return GPL_OK;
 }
 
 // Read small device scalars (one synchronisation).
 static int read_scalars(gpl_model* m, double* out, int k) {
-    HIP_TRY(hipMemcpyAsync(out, m->d(B_SCAL), k * 8, hipMemcpyDeviceToHost, m->ctx->stream));
-    HIP_TRY(hipStreamSynchronize(m->ctx->stream));
+    HIP_TRY(read_back(m->ctx, out, m->d(B_SCAL), k * 8));
     return GPL_OK;
 }
 
@@ -840,8 +941,7 @@ static int fit_gaussian_mixed(gpl_model* m) {
         vec_axpby(s, n, 1.0, rhs, -1.0, t1, r);
         rel_maxabs(s, d, u, n, m->d(B_SCAL) + 8);
         double h;
-        HIP_TRY(hipMemcpyAsync(&h, m->d(B_SCAL) + 8, 8, hipMemcpyDeviceToHost, s));
-        HIP_TRY(hipStreamSynchronize(s));
+        HIP_TRY(read_back(c, &h, m->d(B_SCAL) + 8, 8));
         rel = h;
         if (rel < kRefineStop) break;
         if (refine_diverging(it, rel, prev)) break;
@@ -986,8 +1086,7 @@ static int refine_alpha_mixed(gpl_model* m, int maxref, int nch) {
         vec_axpby(s, n, 1.0, rhs, -1.0, t1, r);
         rel_maxabs(s, d, u, n, m->d(B_SCAL) + 8);
         double h;
-        HIP_TRY(hipMemcpyAsync(&h, m->d(B_SCAL) + 8, 8, hipMemcpyDeviceToHost, s));
-        HIP_TRY(hipStreamSynchronize(s));
+        HIP_TRY(read_back(c, &h, m->d(B_SCAL) + 8, 8));
         rel = h;
         if (rel < kRefineStop) break;
         if (refine_diverging(k, rel, prev)) break;
@@ -1420,11 +1519,11 @@ extern "C" int gpl_fit(gpl_ctx* c, const gpl_cf_term* terms, int32_t nterms, con
     m->split = m->no_posterior = m->restored = false;
     hipStream_t s = c->stream;
     HIP_TRY(hipMemcpyAsync(m->b[B_PROG].p, &m->prog, sizeof(DevProg), hipMemcpyHostToDevice, s));
-    if (n * ncols > 0) HIP_TRY(hipMemcpyAsync(m->d(B_X), x, n * ncols * 8, hipMemcpyHostToDevice, s));
+    if (n * ncols > 0) HIP_TRY(upload(c, s, m->d(B_X), x, n * ncols * 8));
     launch_features(s, m->d(B_X), n, n, (int)ncols, m->b[B_PROG].as<DevProg>(), m->prog, m->d(B_F), m->N);
     upload_vec(m, B_Y, y, n);
-    upload_vec(m, B_TR, trials, n);
-    upload_vec(m, B_OFF, offset, n);
+    if (trials) upload_vec(m, B_TR, trials, n);  // read only with has_trials, has_offset
+    if (offset) upload_vec(m, B_OFF, offset, n);
     hipMemsetAsync(m->b[B_INFO].p, 0, 64, s);
     m->refit_fp64 = false;
     m->refine_iters_done = 0;
@@ -1532,8 +1631,7 @@ static int energy_grad_latent(gpl_model* m, double* grad) {
     double* sc = m->d(B_SCAL);
     reduce_cols(s, m->d(B_PART), ntiles, ng, ng, sc);
     std::vector<double> h(ng > 0 ? ng : 1);
-    HIP_TRY(hipMemcpyAsync(h.data(), sc, ng * 8, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    HIP_TRY(read_back(c, h.data(), sc, ng * 8));
     for (int p = 0; p < ng; ++p) grad[p] = -0.5 * h[p];
     return GPL_OK;
 }
@@ -1587,8 +1685,7 @@ extern "C" int gpl_energy_grad(gpl_model* m, double* grad) {
     else colsumsq_f64(s, m->d(B_XINV), N, N, n, m->d(B_W3), 1);
     reduce_sum(s, m->d(B_W3), n, sc + ng + 1);
     std::vector<double> h(ng + 2);
-    HIP_TRY(hipMemcpyAsync(h.data(), sc, (ng + 2) * 8, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    HIP_TRY(read_back(c, h.data(), sc, (ng + 2) * 8));
     for (int p = 0; p < ng; ++p) grad[p] = -0.5 * h[p];
     // sigma: -1/2 tr((a a^T - Ky^-1) 2 sigma^2 I) = -sigma^2 a^T a + tr(B^-1)
     grad[ng] = -s2 * h[ng] + h[ng + 1];
@@ -1919,8 +2016,7 @@ extern "C" int gpl_model_vector(gpl_model* m, int32_t which, double* out) {
     }
     std::lock_guard<std::mutex> lk(m->ctx->mu);
     HIP_TRY(hipSetDevice(m->ctx->device));
-    HIP_TRY(hipMemcpyAsync(out, m->d(idx), m->n * 8, hipMemcpyDeviceToHost, m->ctx->stream));
-    HIP_TRY(hipStreamSynchronize(m->ctx->stream));
+    HIP_TRY(read_back(m->ctx, out, m->d(idx), m->n * 8));
     return GPL_OK;
 }
 
@@ -2049,8 +2145,11 @@ extern "C" int gpl_model_info(gpl_model* m, int64_t* n, int32_t* iters, double* 
 
 extern "C" void gpl_model_free(gpl_model* m) {
     if (!m) return;
-    hipSetDevice(m->ctx->device);
-    hipStreamSynchronize(m->ctx->stream);
+    gpl_ctx* c = m->ctx;
+    hipSetDevice(c->device);
+    for (hipStream_t st : {c->stream, c->side, c->aux}) hipStreamSynchronize(st);
+    for (auto& x : m->b) x.give(c->blocks);
+    c->blocks->age();
     delete m;
 }
 

@@ -60,7 +60,7 @@ struct gpl_fitc {
 
 #define FENSURE(fm, idx, bytes)                                                               \
     do {                                                                                      \
-        if (!(fm)->b[idx].ensure(bytes)) return fail(GPL_ERR_OOM, "device allocation failed"); \
+        if (!(fm)->b[idx].ensure(bytes, (fm)->ctx->blocks)) return fail(GPL_ERR_OOM, "device allocation failed"); \
     } while (0)
 
 // Partial products of A S^-1 A^T over column ranges, summed in a fixed order: as
@@ -110,15 +110,18 @@ static int fitc_alloc(gpl_fitc* f) {
 static int fitc_upload(gpl_fitc* f, int idx, const double* h) {
     hipStream_t s = f->ctx->stream;
     fill_f64(s, f->d(idx), f->N, 0.0);
-    if (h) HIP_TRY(hipMemcpyAsync(f->d(idx), h, f->n * 8, hipMemcpyHostToDevice, s));
+    if (h) HIP_TRY(upload(f->ctx, s, f->d(idx), h, f->n * 8));
     return GPL_OK;
 }
 
 static int fitc_scalars(gpl_fitc* f, double* out, int k, int* flags) {
     hipStream_t s = f->ctx->stream;
-    HIP_TRY(hipMemcpyAsync(out, f->d(F_SCAL), k * 8, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipMemcpyAsync(flags, f->b[F_INFO].p, 8, hipMemcpyDeviceToHost, s));
+    double* st = f->ctx->stage;
+    HIP_TRY(hipMemcpyAsync(st, f->d(F_SCAL), k * 8, hipMemcpyDeviceToHost, s));
+    HIP_TRY(hipMemcpyAsync(st + k, f->b[F_INFO].p, 8, hipMemcpyDeviceToHost, s));
     HIP_TRY(hipStreamSynchronize(s));
+    memcpy(out, st, k * 8);
+    memcpy(flags, st + k, 8);
     return GPL_OK;
 }
 
@@ -402,8 +405,8 @@ extern "C" int gpl_fitc_fit(gpl_ctx* c, const gpl_cf_term* terms, int32_t nterms
     hipStream_t s = c->stream;
     auto setup = [&]() -> int {
         HIP_TRY(hipMemcpyAsync(f->b[F_PROG].p, &f->prog, sizeof(DevProg), hipMemcpyHostToDevice, s));
-        if (n * ncols > 0) HIP_TRY(hipMemcpyAsync(f->d(F_X), x, n * ncols * 8, hipMemcpyHostToDevice, s));
-        if (m * ncols > 0) HIP_TRY(hipMemcpyAsync(f->d(F_ZX), z, m * ncols * 8, hipMemcpyHostToDevice, s));
+        if (n * ncols > 0) HIP_TRY(upload(c, s, f->d(F_X), x, n * ncols * 8));
+        if (m * ncols > 0) HIP_TRY(upload(c, s, f->d(F_ZX), z, m * ncols * 8));
         const DevProg* pd = f->b[F_PROG].as<DevProg>();
         launch_features(s, f->d(F_X), n, n, (int)ncols, pd, f->prog, f->d(F_F), f->N);
         launch_features(s, f->d(F_ZX), m, m, (int)ncols, pd, f->prog, f->d(F_FZ), f->Mz);
@@ -462,10 +465,9 @@ extern "C" int gpl_fitc_pred(gpl_fitc* f, const double* xt, int64_t mt, int32_t 
         gemm2_f64(s, 0, 0, Mz, Mt, Mz, 1.0, f->d(F_XG), Mz, A2, Mz, 0.0, Yv, Mz, 3);
         colsumsq_f64(s, Yv, Mz, Mz, mt, q, 0);
         vec_axpby(s, mt, 1.0, c2, 1.0, q, red);
-        HIP_TRY(hipMemcpyAsync(var, red, mt * 8, hipMemcpyDeviceToHost, s));
+        HIP_TRY(read_back(c, var, red, mt * 8));
     }
-    HIP_TRY(hipMemcpyAsync(mean, vb, mt * 8, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
+    HIP_TRY(read_back(c, mean, vb, mt * 8));
     return GPL_OK;
 }
 
@@ -572,8 +574,7 @@ extern "C" int gpl_fitc_vector(gpl_fitc* f, int32_t which, double* out) {
     }
     std::lock_guard<std::mutex> lk(f->ctx->mu);
     HIP_TRY(hipSetDevice(f->ctx->device));
-    HIP_TRY(hipMemcpyAsync(out, f->d(idx), f->n * 8, hipMemcpyDeviceToHost, f->ctx->stream));
-    HIP_TRY(hipStreamSynchronize(f->ctx->stream));
+    HIP_TRY(read_back(f->ctx, out, f->d(idx), f->n * 8));
     return GPL_OK;
 }
 
@@ -588,7 +589,10 @@ extern "C" int gpl_fitc_info(gpl_fitc* f, int64_t* n, int64_t* m, int32_t* iters
 
 extern "C" void gpl_fitc_free(gpl_fitc* f) {
     if (!f) return;
-    hipSetDevice(f->ctx->device);
-    hipStreamSynchronize(f->ctx->stream);
+    gpl_ctx* c = f->ctx;
+    hipSetDevice(c->device);
+    for (hipStream_t st : {c->stream, c->side, c->aux}) hipStreamSynchronize(st);
+    for (auto& x : f->b) x.give(c->blocks);
+    c->blocks->age();
     delete f;
 }

@@ -47,7 +47,7 @@ struct gpl_model {
 
 #define ENSURE(m, idx, bytes)                                                             \
     do {                                                                                  \
-        if (!(m)->b[idx].ensure(bytes)) return fail(GPL_ERR_OOM, "device allocation failed"); \
+        if (!(m)->b[idx].ensure(bytes, (m)->ctx->blocks)) return fail(GPL_ERR_OOM, "device allocation failed"); \
     } while (0)
 
 

@@ -446,6 +446,10 @@ static void worker_main(gpl_server* s, int w) {
     }
 }
 
+// The server's budget covers the device memory of its models, and it keeps spare
+// ones itself: its contexts keep no blocks of freed models.
+thread_local bool gpl::t_ctx_for_server = false;
+
 extern "C" int gpl_server_create(int32_t device, int32_t n_workers, int64_t mem_budget_bytes, gpl_server** out) {
     if (!out || n_workers < 1 || n_workers > 16 || mem_budget_bytes <= 0)
         return fail(GPL_ERR_ARG, "need 1..16 workers and a positive memory budget");
@@ -454,7 +458,9 @@ extern "C" int gpl_server_create(int32_t device, int32_t n_workers, int64_t mem_
     s->budget = (size_t)mem_budget_bytes;
     for (int w = 0; w < n_workers; ++w) {
         gpl_ctx* c = nullptr;
+        gpl::t_ctx_for_server = true;
         int r = gpl_ctx_create(device, &c);
+        gpl::t_ctx_for_server = false;
         if (r) {
             for (auto* cc : s->ctxs) gpl_ctx_destroy(cc);
             delete s;

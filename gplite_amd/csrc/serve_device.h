@@ -11,6 +11,7 @@
 #include "../../include/gplite_amd.h"
 
 namespace gpl {
+extern thread_local bool t_ctx_for_server;  // gpl_ctx_create is called by a server (set in serve.cpp)
 
 int fail(int code, const std::string& msg);
 

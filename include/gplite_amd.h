@@ -70,6 +70,10 @@ typedef struct gpl_cf_term {
  * followed by the likelihood's parameters (Gaussian: sigma). */
 int32_t gpl_grad_len(const gpl_cf_term* terms, int32_t nterms, int32_t lik_kind);
 
+/* Column means and standard deviations (divisor n - 1) of the row-major n x d
+ * host matrix x, n >= 2 (R/cf.R:836-845); sums run over the rows in order. */
+void gpl_col_scales(const double* x, int64_t n, int64_t d, double* means, double* scales);
+
 /* ---- likelihood and options -------------------------------------------- */
 enum { GPL_LIK_GAUSSIAN = 0, GPL_LIK_BERNOULLI = 1, GPL_LIK_BINOMIAL = 2, GPL_LIK_POISSON = 3, GPL_LIK_BETABINOM = 4 };
 enum { GPL_LINK_IDENTITY = 0, GPL_LINK_LOGIT = 1, GPL_LINK_PROBIT = 2, GPL_LINK_LOG = 3 };
