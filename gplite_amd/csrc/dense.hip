@@ -1021,63 +1021,74 @@ void potrf_panel_mixed(hipStream_t s, float* A, int64_t ld, int64_t K0, int nc, 
 // blocks that are factored carry no FP32 accumulation error.
 // D: first tile to update (64x64 column-major tiles, consecutive), P: the panel
 // rows of that tile (leading dimension ldp), kdepth: panel width (multiple of 64).
+//
+// A wave per lower 16x16 tile (ten per block; the strictly upper ones are never
+// read), straight from global memory with 64 k loaded ahead: bound by its chain of
+// kdepth / 4 matrix instructions, 0.11 us per 16 k.  (A workgroup per block that
+// staged 16 k at a time in LDS took a load latency and two barriers for each, about
+// 1 us: depth 64 / 128 / 256 / 512 on eight blocks 7.7 / 12 / 18.5 / 36 us.)
+// The sums run over k in order and are subtracted at the end.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_dacc_update(double* __restrict__ D, const float* __restrict__ P, int64_t ldp,
-                                                     int64_t kdepth, int64_t sD, int64_t sP) {
-    // D_j -= P_j P_j^T on v_mfma_f64_16x16x4f64: each wave owns a 32x32 quadrant
-    // (2x2 blocks of 16x16); P_j is staged 16 k at a time in LDS as FP64.
-    // f64 16x16x4 layouts: A lane l -> A[l%16][k=l/16], B lane l -> B[k=l/16][l%16],
-    // D item v of lane l -> row l/16 + 4v, column l%16.
-    D += blockIdx.y * sD + (int64_t)blockIdx.x * 64 * 64;
-    P += blockIdx.y * sP + (int64_t)blockIdx.x * 64;
-    __shared__ double Ps[16][64 + 2];
-    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-    const int wr = w >> 1, wc = w & 1;
+                                                     int64_t kdepth, int64_t nwaves, int64_t sD, int64_t sP) {
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t id = (int64_t)blockIdx.x * 4 + w;
+    if (id >= nwaves) return;
+    const int64_t j = id / 10;
+    const int u = (int)(id - 10 * j);
+    const int rt = u < 1 ? 0 : u < 3 ? 1 : u < 6 ? 2 : 3, ct = u - rt * (rt + 1) / 2;
+    D += blockIdx.y * sD + j * 64 * 64;
+    P += blockIdx.y * sP + j * 64;
     const int l16 = lane & 15, lk = lane >> 4;
-    typedef double d4 __attribute__((ext_vector_type(4)));
-    d4 acc[2][2];
+    // lane (l16, lk) of the (transposed) product holds columns lk + 4v of row l16
+    double* d = D + (16 * rt + l16) + (16 * ct + lk) * 64;
+    double old[4];
 #pragma unroll
-    for (int bi = 0; bi < 2; ++bi)
+    for (int v = 0; v < 4; ++v) old[v] = d[4 * v * 64];
+    const float* pr = P + 16 * rt + l16 + lk * ldp;
+    const float* pc = P + 16 * ct + l16 + lk * ldp;
+    float r[2][16], c[2][16];
+    auto load = [&](int st) {
 #pragma unroll
-        for (int bj = 0; bj < 2; ++bj) acc[bi][bj] = d4{0.0, 0.0, 0.0, 0.0};
-    for (int64_t k0 = 0; k0 < kdepth; k0 += 16) {
-        __syncthreads();
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int kk = (t >> 6) + 4 * q;
-            Ps[kk][lane] = (double)P[lane + (k0 + kk) * ldp];
+        for (int q = 0; q < 16; ++q) {
+            r[st][q] = pr[4 * q * ldp];
+            c[st][q] = pc[4 * q * ldp];
         }
-        __syncthreads();
+        pr += 64 * ldp;
+        pc += 64 * ldp;
+    };
+    d4 acc = d4{0.0, 0.0, 0.0, 0.0};
+    auto mult = [&](int st) {
 #pragma unroll
-        for (int ks = 0; ks < 16; ks += 4) {
-            double a[2], b[2];
-#pragma unroll
-            for (int bi = 0; bi < 2; ++bi) a[bi] = Ps[ks + lk][32 * wr + 16 * bi + l16];
-#pragma unroll
-            for (int bj = 0; bj < 2; ++bj) b[bj] = Ps[ks + lk][32 * wc + 16 * bj + l16];
-#pragma unroll
-            for (int bi = 0; bi < 2; ++bi)
-#pragma unroll
-                for (int bj = 0; bj < 2; ++bj)
-                    acc[bi][bj] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[bi], b[bj], acc[bi][bj], 0, 0, 0);
-        }
+        for (int q = 0; q < 16; ++q)
+            acc = __builtin_amdgcn_mfma_f64_16x16x4f64((double)c[st][q], (double)r[st][q], acc, 0, 0, 0);
+    };
+    const int nch = (int)(kdepth / 64);
+    load(0);
+    int q = 0;
+    for (; q + 2 < nch; q += 2) {
+        load(1);
+        mult(0);
+        load(0);
+        mult(1);
+    }
+    if (q + 1 < nch) {
+        load(1);
+        mult(0);
+        mult(1);
+    } else {
+        mult(0);
     }
 #pragma unroll
-    for (int bi = 0; bi < 2; ++bi)
-#pragma unroll
-        for (int bj = 0; bj < 2; ++bj)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int row = 32 * wr + 16 * bi + lk + 4 * v, col = 32 * wc + 16 * bj + l16;
-                D[row + col * 64] -= acc[bi][bj][v];
-            }
+    for (int v = 0; v < 4; ++v) d[4 * v * 64] = old[v] - acc[v];
 }
 
 void dacc_update(hipStream_t s, double* D, const float* P, int64_t ldp, int64_t ntiles, int64_t kdepth, int batch,
                  int64_t sD, int64_t sP) {
-    if (ntiles <= 0 || batch <= 0) return;
-    hipLaunchKernelGGL(k_dacc_update, dim3((unsigned)ntiles, (unsigned)batch), dim3(256), 0, s, D, P, ldp, kdepth, sD,
-                       sP);
+    if (ntiles <= 0 || batch <= 0 || kdepth <= 0) return;
+    const int64_t nwaves = 10 * ntiles;
+    hipLaunchKernelGGL(k_dacc_update, dim3((unsigned)((nwaves + 3) / 4), (unsigned)batch), dim3(256), 0, s, D, P, ldp,
+                       kdepth, nwaves, sD, sP);
 }
 
 // ---------------------------------------------------------------------------
