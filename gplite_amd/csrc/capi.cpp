@@ -148,6 +148,7 @@ extern "C" int gpl_ctx_create(int32_t device, gpl_ctx** out) {
     if (e == hipSuccess) e = hipMalloc((void**)&c->msync, (kTrsmFlags + 64) * sizeof(unsigned));
     if (e == hipSuccess) e = hipMemset(c->msync, 0, (kTrsmFlags + 64) * sizeof(unsigned));
     if (e == hipSuccess) c->minfo = (int*)(c->msync + kTrsmFlags + 32);
+    if (e == hipSuccess) c->fin = c->msync + kTrsmFlags + 48;
     if (e == hipSuccess) e = hipHostMalloc((void**)&c->stage, gpl_ctx::kStage * sizeof(double));
     if (e == hipSuccess) e = hipHostMalloc((void**)&c->up, gpl_ctx::kStage * sizeof(double));
     size_t mfree = 0, mtotal = 0;
@@ -837,7 +838,7 @@ static int fit_gaussian(gpl_model* m) {
     }
     laplace_finish(s, GPL_LIK_GAUSSIAN, 0, sigma, n, m->d(B_FMEAN), m->d(B_Y), nullptr,
                    m->has_offset ? m->d(B_OFF) : nullptr, m->d(B_ALPHA), m->d(B_LDIAG), nullptr,
-                   m->b[B_INFO].as<int>(), c->stage);
+                   m->b[B_INFO].as<int>(), m->d(B_TERM), c->fin, c->stage);
     double h[4];
     int fl[2];
     int r = read_finish(c, h, fl);
@@ -1005,7 +1006,7 @@ static int fit_laplace(gpl_model* m) {
             symv_lt_f64(s, m->d(B_K), N, m->d(B_ALPHA), m->d(B_FMEAN), m->d(B_KMV), kmatvec_chunks(N), 1, 0, 0);
         }
         laplace_finish(s, m->lik.kind, m->lik.link, lik_par(m->lik), n, m->d(B_FMEAN), m->d(B_Y), tr, off,
-                       m->d(B_ALPHA), m->d(B_LDIAG), m->d(B_FOLD), flags, c->stage);
+                       m->d(B_ALPHA), m->d(B_LDIAG), m->d(B_FOLD), flags, m->d(B_TERM), c->fin, c->stage);
         double h[4];
         int fl[2];
         int r = read_finish(c, h, fl);
@@ -1284,7 +1285,7 @@ static int fit_ep(gpl_model* m) {
         colsumsq_f64(s, m->d(B_XINV), N, N, n, m->d(B_W3), 1);
         ep_finish(s, n, m->d(B_V), m->d(B_Z), m->d(B_W3), m->d(B_CAVM), m->d(B_CAVV), m->d(B_LOGZS), m->d(B_ALPHA),
                   m->d(B_LDIAG), m->d(B_FMEAN), m->d(B_FVAR), m->d(B_FOLD), m->d(B_FVOLD), m->d(B_ZOLD), m->d(B_POLD),
-                  diff_old, flags, c->stage);
+                  diff_old, flags, m->d(B_TERM), c->fin, c->stage);
         double h[4];
         int fl[2];
         int r = read_finish(c, h, fl);

@@ -220,13 +220,14 @@ void ep_sites(hipStream_t s, int lik, int link, double par, int64_t n, const dou
               const double* offset, int q, const double* gh_x, const double* gh_w, double damping,
               double* z, double* V, double* sv, double* logZs, double* cav_m, double* cav_v,
               int* nan_flag, int64_t N = 0, double* rhs = nullptr);
+// part: (n + 255) / 256 * 4 doubles (512 at most); counter: a device word that is zero between launches
 void laplace_finish(hipStream_t s, int lik, int link, double par, int64_t n, const double* f, const double* y,
                     const double* trials, const double* offset, const double* alpha, const double* ldiag, double* fold,
-                    int* flags, double* host);
+                    int* flags, double* part, unsigned* counter, double* host);
 void ep_finish(hipStream_t s, int64_t n, const double* V, const double* z, const double* binv_diag, const double* cav_m,
                const double* cav_v, const double* logZs, const double* alpha, const double* ldiag, const double* f,
                double* fvar, double* fold, double* fvold, double* zold, double* pold, double diff_old, int* flags,
-               double* host);
+               double* part, unsigned* counter, double* host);
 void ep_post(hipStream_t s, int64_t n, const double* V, const double* z, const double* binv_diag,
              const double* cav_m, const double* cav_v, const double* logZs, double* fvar,
              double* term);

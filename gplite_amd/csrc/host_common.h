@@ -152,6 +152,7 @@ struct gpl_ctx {
     unsigned* msync = nullptr;
     unsigned mbase = 0;
     int* minfo = nullptr;
+    unsigned* fin = nullptr;  // counter of the step-ending kernels' workgroups (zero between launches)
     // pinned host memory: results on their way to the caller (`stage`), inputs on
     // theirs to the device (`up`, filled from upos; a call that needs it from the
     // start again waits for the stream)

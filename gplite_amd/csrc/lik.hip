@@ -6,6 +6,8 @@
 // R/gp_loo.R:136-144).
 #include "gpl_internal.h"
 
+#include <algorithm>
+
 #include <cmath>
 
 namespace gpl {
@@ -385,18 +387,23 @@ void vec_mul_pad(hipStream_t s, int64_t n, int64_t N, const double* a, const dou
 }
 
 // ---------------------------------------------------------------------------
-// The end of a Newton step, an EP sweep or a Gaussian fit, in one workgroup: the
+// The end of a Newton step, an EP sweep or a Gaussian fit in one launch: the
 // scalars that the host decides on, straight into pinned host memory with the
 // step's flags (which are cleared for the next one), and the state that the next
 // step starts from.  A launch costs 4.5 us on the stream and a copy to the host
-// about 20, against 3 us of work here: a Newton step at n = 500 took nine of the
-// former and three of the latter after its last product, 110 us of 400.
-// Fixed order: per thread, then a tree over the wave, then the waves in order.
+// about 20: a Newton step at n = 500 took nine of the former and three of the
+// latter after its last product, 110 us of 400.  A thread per point up to 128
+// workgroups, as the log likelihoods are hundreds of instructions (one workgroup
+// took 75 us for 4096 of them, this 9): each leaves its partial sums, and the one
+// that arrives last adds them in order, so the result does not depend on it.
 // ---------------------------------------------------------------------------
+constexpr int kFinishMaxBlocks = 128;
+static int finish_blocks(int64_t n) { return (int)std::max<int64_t>(1, std::min<int64_t>(kFinishMaxBlocks, (n + 255) / 256)); }
+
 __device__ __forceinline__ double nan_max(double a, double b) { return (b > a || isnan(b)) ? b : a; }
 
-// s[0..2] sums, s[3] a maximum that keeps NaN; on return thread-independent
-__device__ __forceinline__ void finish_reduce(double (&s)[4], double (*red)[4]) {
+// s[0..2] sums, s[3] a maximum that keeps NaN, over the workgroup's 256 threads
+__device__ __forceinline__ void finish_block_reduce(double (&s)[4], double (*red)[4]) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
@@ -404,32 +411,71 @@ __device__ __forceinline__ void finish_reduce(double (&s)[4], double (*red)[4]) 
         for (int k = 0; k < 3; ++k) s[k] += __shfl_xor(s[k], o, 64);
         s[3] = nan_max(s[3], __shfl_xor(s[3], o, 64));
     }
+    __syncthreads();
     if (lane == 0)
 #pragma unroll
         for (int k = 0; k < 4; ++k) red[w][k] = s[k];
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < 4; ++k) s[k] = red[0][k];
-    for (int v = 1; v < 16; ++v) {
+#pragma unroll
+    for (int v = 1; v < 4; ++v) {
 #pragma unroll
         for (int k = 0; k < 3; ++k) s[k] += red[v][k];
         s[3] = nan_max(s[3], red[v][3]);
     }
 }
 
+// The workgroups' sums to part (4 doubles each); true in the last to arrive, with
+// the totals in s.  counter: zero before the launch and after it.
+__device__ __forceinline__ bool finish_combine(double (&s)[4], double (*red)[4], double* part, unsigned* counter) {
+    __shared__ int s_last;
+    finish_block_reduce(s, red);
+    if (gridDim.x == 1) return true;
+    if (threadIdx.x == 0) {
+        // write-through stores, waited for before the counter is
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            __hip_atomic_store(part + 4 * blockIdx.x + k, s[k], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        s_last = atomicInc(counter, gridDim.x - 1) == gridDim.x - 1;
+        if (s_last) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    }
+    __syncthreads();
+    if (!s_last) return false;
+    s[0] = s[1] = s[2] = s[3] = 0.0;
+    if (threadIdx.x < gridDim.x)
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            s[k] = __hip_atomic_load(part + 4 * threadIdx.x + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    finish_block_reduce(s, red);
+    return true;
+}
+
+// by the last workgroup, every other having read the flags
+__device__ __forceinline__ void finish_report(const double (&s)[4], int* flags, double* host) {
+    if (threadIdx.x > 0) return;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) host[k] = s[k];
+    host[4] = flags[0];
+    host[5] = flags[1];
+    flags[0] = flags[1] = 0;
+}
+
 // host: sum log lik, f . alpha, sum ldiag, max |fold - f|, flags[0], flags[1].  fold
 // (if any) = f unless the pseudo-data were flagged.
-__global__ __launch_bounds__(1024) void k_laplace_finish(int lik, int link, double par, int64_t n,
-                                                         const double* __restrict__ f, const double* __restrict__ y,
-                                                         const double* __restrict__ trials,
-                                                         const double* __restrict__ offset,
-                                                         const double* __restrict__ alpha,
-                                                         const double* __restrict__ ldiag, double* __restrict__ fold,
-                                                         int* __restrict__ flags, double* __restrict__ host) {
-    __shared__ double red[16][4];
-    const int f0 = flags[0], f1 = flags[1];
+__global__ __launch_bounds__(256) void k_laplace_finish(int lik, int link, double par, int64_t n,
+                                                        const double* __restrict__ f, const double* __restrict__ y,
+                                                        const double* __restrict__ trials,
+                                                        const double* __restrict__ offset,
+                                                        const double* __restrict__ alpha,
+                                                        const double* __restrict__ ldiag, double* __restrict__ fold,
+                                                        int* flags, double* __restrict__ part,
+                                                        unsigned* __restrict__ counter, double* __restrict__ host) {
+    __shared__ double red[4][4];
+    const int f1 = flags[1];
     double s[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int64_t i = threadIdx.x; i < n; i += 1024) {
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
         const double fi = f[i];
         s[0] += d_loglik(lik, link, par, fi + (offset ? offset[i] : 0.0), y[i], trials ? trials[i] : 1.0);
         s[1] += fi * alpha[i];
@@ -439,42 +485,33 @@ __global__ __launch_bounds__(1024) void k_laplace_finish(int lik, int link, doub
             if (!(f1 & 6)) fold[i] = fi;
         }
     }
-    finish_reduce(s, red);
-    if (threadIdx.x > 0) return;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) host[k] = s[k];
-    host[4] = f0;
-    host[5] = f1;
-    flags[0] = flags[1] = 0;
+    if (finish_combine(s, red, part, counter)) finish_report(s, flags, host);
 }
 
 void laplace_finish(hipStream_t s, int lik, int link, double par, int64_t n, const double* f, const double* y,
                     const double* trials, const double* offset, const double* alpha, const double* ldiag, double* fold,
-                    int* flags, double* host) {
-    hipLaunchKernelGGL(k_laplace_finish, dim3(1), dim3(1024), 0, s, lik, link, par, n, f, y, trials, offset, alpha,
-                       ldiag, fold, flags, host);
+                    int* flags, double* part, unsigned* counter, double* host) {
+    hipLaunchKernelGGL(k_laplace_finish, dim3(finish_blocks(n)), dim3(256), 0, s, lik, link, par, n, f, y, trials,
+                       offset, alpha, ldiag, fold, flags, part, counter, host);
 }
 
 // host: sum of the evidence terms, z . alpha, sum ldiag, max |fold - f|, flags.  The
 // variances fvar = V (1 - diag B^-1) (k_ep_post) and, if the sweep is accepted (its
 // change does not exceed diff_old), the next one's old state; neither if flagged.
-__global__ __launch_bounds__(1024) void k_ep_finish(int64_t n, const double* __restrict__ V,
-                                                    const double* __restrict__ z,
-                                                    const double* __restrict__ binv_diag,
-                                                    const double* __restrict__ cav_m,
-                                                    const double* __restrict__ cav_v,
-                                                    const double* __restrict__ logZs,
-                                                    const double* __restrict__ alpha,
-                                                    const double* __restrict__ ldiag, const double* __restrict__ f,
-                                                    double* __restrict__ fvar, double* __restrict__ fold,
-                                                    double* __restrict__ fvold, double* __restrict__ zold,
-                                                    double* __restrict__ pold, double diff_old,
-                                                    int* __restrict__ flags, double* __restrict__ host) {
-    __shared__ double red[16][4];
-    const int f0 = flags[0], f1 = flags[1];
-    const bool bad = f1 & 6;
+__global__ __launch_bounds__(256) void k_ep_finish(int64_t n, const double* __restrict__ V,
+                                                   const double* __restrict__ z, const double* __restrict__ binv_diag,
+                                                   const double* __restrict__ cav_m, const double* __restrict__ cav_v,
+                                                   const double* __restrict__ logZs, const double* __restrict__ alpha,
+                                                   const double* __restrict__ ldiag, const double* __restrict__ f,
+                                                   double* __restrict__ fvar, double* __restrict__ fold,
+                                                   double* __restrict__ fvold, double* __restrict__ zold,
+                                                   double* __restrict__ pold, double diff_old, int* flags,
+                                                   double* __restrict__ part, unsigned* __restrict__ counter,
+                                                   double* __restrict__ host) {
+    __shared__ double red[4][4];
+    const bool bad = flags[1] & 6;
     double s[4] = {0.0, 0.0, 0.0, 0.0};
-    for (int64_t i = threadIdx.x; i < n; i += 1024) {
+    for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
         const double Vi = V[i], zi = z[i], cv = cav_v[i] + Vi, dz = cav_m[i] - zi;
         s[0] += logZs[i] + 0.5 * log(cv) + 0.5 * dz * dz / cv - 0.5 * log(Vi);
         s[1] += zi * alpha[i];
@@ -482,28 +519,23 @@ __global__ __launch_bounds__(1024) void k_ep_finish(int64_t n, const double* __r
         s[3] = nan_max(s[3], fabs(fold[i] - f[i]));
         if (!bad) fvar[i] = Vi * (1.0 - binv_diag[i]);
     }
-    finish_reduce(s, red);
+    if (!finish_combine(s, red, part, counter)) return;
     if (!bad && !(s[3] > diff_old))
-        for (int64_t i = threadIdx.x; i < n; i += 1024) {
+        for (int64_t i = threadIdx.x; i < n; i += 256) {
             fold[i] = f[i];
-            fvold[i] = fvar[i];
+            fvold[i] = V[i] * (1.0 - binv_diag[i]);
             zold[i] = z[i];
             pold[i] = 1.0 / V[i];
         }
-    if (threadIdx.x > 0) return;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) host[k] = s[k];
-    host[4] = f0;
-    host[5] = f1;
-    flags[0] = flags[1] = 0;
+    finish_report(s, flags, host);
 }
 
 void ep_finish(hipStream_t s, int64_t n, const double* V, const double* z, const double* binv_diag, const double* cav_m,
                const double* cav_v, const double* logZs, const double* alpha, const double* ldiag, const double* f,
                double* fvar, double* fold, double* fvold, double* zold, double* pold, double diff_old, int* flags,
-               double* host) {
-    hipLaunchKernelGGL(k_ep_finish, dim3(1), dim3(1024), 0, s, n, V, z, binv_diag, cav_m, cav_v, logZs, alpha, ldiag,
-                       f, fvar, fold, fvold, zold, pold, diff_old, flags, host);
+               double* part, unsigned* counter, double* host) {
+    hipLaunchKernelGGL(k_ep_finish, dim3(finish_blocks(n)), dim3(256), 0, s, n, V, z, binv_diag, cav_m, cav_v, logZs,
+                       alpha, ldiag, f, fvar, fold, fvold, zold, pold, diff_old, flags, part, counter, host);
 }
 
 __global__ __launch_bounds__(256) void k_reduce_cols(const double* __restrict__ part, int64_t rows, int64_t ld,
