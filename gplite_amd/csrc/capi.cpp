@@ -143,11 +143,17 @@ extern "C" int gpl_ctx_create(int32_t device, gpl_ctx** out) {
     if (e == hipSuccess) e = hipMalloc((void**)&c->psync, kPanelSyncWords * sizeof(unsigned));
     if (e == hipSuccess) e = hipMemset(c->psync, 0, kPanelSyncWords * sizeof(unsigned));
     if (e == hipSuccess) e = hipMalloc((void**)&c->dpub, kPanelMaxBlocks * 4096 * sizeof(double));
-    if (e == hipSuccess) e = hipMalloc((void**)&c->tsync, kSolveSyncWords * sizeof(unsigned));
-    if (e == hipSuccess) e = hipMemset(c->tsync, 0, kSolveSyncWords * sizeof(unsigned));
+    if (e == hipSuccess) e = hipMalloc((void**)&c->tpub[0], 2 * 64 * kSolveMaxBlocks * sizeof(double));
+    if (e == hipSuccess) {
+        c->tpub[1] = c->tpub[0] + 64 * kSolveMaxBlocks;
+        double unsolved;
+        memcpy(&unsolved, &kUnsolved, 8);
+        fill_f64(c->stream, c->tpub[0], 2 * 64 * kSolveMaxBlocks, unsolved);
+    }
     if (e == hipSuccess) e = hipMalloc((void**)&c->msync, (kTrsmFlags + 64) * sizeof(unsigned));
     if (e == hipSuccess) e = hipMemset(c->msync, 0, (kTrsmFlags + 64) * sizeof(unsigned));
     if (e == hipSuccess) c->minfo = (int*)(c->msync + kTrsmFlags + 32);
+    if (e == hipSuccess) c->tticket = c->msync + kTrsmFlags + 40;
     if (e == hipSuccess) c->fin = c->msync + kTrsmFlags + 48;
     if (e == hipSuccess) e = hipHostMalloc((void**)&c->stage, gpl_ctx::kStage * sizeof(double));
     if (e == hipSuccess) e = hipHostMalloc((void**)&c->up, gpl_ctx::kStage * sizeof(double));
@@ -182,7 +188,7 @@ extern "C" void gpl_ctx_destroy(gpl_ctx* c) {
     hipStreamDestroy(c->aux);
     if (c->psync) hipFree(c->psync);
     if (c->dpub) hipFree(c->dpub);
-    if (c->tsync) hipFree(c->tsync);
+    if (c->tpub[0]) hipFree(c->tpub[0]);
     if (c->msync) hipFree(c->msync);
     if (c->stage) hipHostFree(c->stage);
     if (c->up) hipHostFree(c->up);
@@ -686,18 +692,20 @@ static void potrf32_blocked(gpl_ctx* c, float* L, int64_t N, double* Dinv, doubl
     inv.finish();
 }
 
-void gpl::trsv_lower(gpl_ctx* c, hipStream_t s, const double* L, int64_t ld, const double* Dinv, int64_t N, double* b,
-                     double* x, int trans, int* info, const double* scale, int64_t n, double* scaled,
-                     const int* gate) {
+void gpl::trsv_back(gpl_ctx* c, hipStream_t s, const double* L, int64_t ld, const double* Dinv, int64_t N, double* b,
+                    double* x, int* info, const double* scale, int64_t n, double* scaled, const int* gate) {
     const int64_t T = N / 64;
     if (T > kSolveMaxBlocks) {
-        trsv_lower_f64(s, L, ld, Dinv, N, b, x, trans);
+        trsv_lower_f64(s, L, ld, Dinv, N, b, x, 1);
         if (scaled) vec_mul_pad(s, n, N, scale, x, scaled, gate);
         return;
     }
-    if (++c->pepoch == 0) c->pepoch = 1;
-    trsv_persist_f64(s, L, ld, Dinv, N, b, x, trans, c->tsync, c->pepoch, c->tbase, info, c->pwait, scale, n, scaled,
-                     gate);
+    const int cur = c->tcur;
+    trsv_persist_f64(s, L, ld, Dinv, N, b, x, c->tpub[cur], c->tpub[1 - cur], c->tdirty[1 - cur], c->tticket,
+                     c->tbase, info, c->pwait, scale, n, scaled, gate);
+    c->tdirty[cur] = T;
+    c->tdirty[1 - cur] = 0;
+    c->tcur = 1 - cur;
     c->tbase += (unsigned)T;
 }
 
@@ -723,8 +731,8 @@ void gpl::trsm_forward(gpl_ctx* c, hipStream_t s, const double* L, int64_t ld, c
 static void solve_alpha_back(gpl_ctx* c, gpl_model* m, const int* gate = nullptr) {
     const int64_t N = m->N;
     Prof p(c, "trsv", 1.0 * N * N, 8.0 * N * N / 2);
-    trsv_lower(c, c->stream, m->d(B_L), N, m->d(B_DINV), N, m->d(B_W1), m->d(B_W2), 1, m->b[B_INFO].as<int>(),
-               m->d(B_SV), m->n, m->d(B_ALPHA), gate);
+    trsv_back(c, c->stream, m->d(B_L), N, m->d(B_DINV), N, m->d(B_W1), m->d(B_W2), m->b[B_INFO].as<int>(),
+              m->d(B_SV), m->n, m->d(B_ALPHA), gate);
 }
 
 int gpl::wait_timeout_fail() {

@@ -1163,77 +1163,115 @@ void trsv_lower_f64(hipStream_t s, const double* L, int64_t ld, const double* Di
 }
 
 // ---------------------------------------------------------------------------
-// The same solves in one launch: workgroup k (ticket order) owns block i = k
-// (forward) or T - 1 - k (transposed).  It subtracts the products with the
-// blocks it depends on as each is published (the tile values are loaded
-// before the wait), forms x_i = Dinv_i b_i (Dinv_i^T b_i) and publishes x_i.
-// Every wait is on a block of a lower ticket, whose workgroup has started and
-// waits only on lower tickets, so every wait ends; the summation order is
-// fixed (deterministic).  With `scaled` the launch also leaves scale .* x there
-// (zero beyond n), unless the gate's flags say NaN or V <= 0.  sync: flags [0, T),
-// the ticket counter at sync[kSolveMaxBlocks].
+// The transposed solve L^T x = b in one launch: workgroup k (ticket order) owns
+// block i = T - 1 - k and waits only on blocks of lower tickets, whose workgroups
+// have started, so every wait ends; the summation order is fixed.
+//
+// Bound by the chain from block to block.  So (1) a solved block is handed over as
+// data alone: the 64 values lie in `pub`, which holds a signalling NaN that no
+// arithmetic returns (kUnsolved) until they are stored, and every wave of a consumer
+// polls the values it multiplies, one per lane, with no flag, fence or barrier in
+// between; (2) a wave keeps 16 rows, lane (li, p) the row li and the columns 16p ..
+// 16p + 15 of it, whose multipliers are then 16-lane row broadcasts of the polled
+// register (v_fmac_f64_dpp row_newbcast), and only the product with Dinv_i needs an
+// exchange between the waves.  1.25 us per block: n = 4096 82 us, 1200 26, 500 12.
+// (With a flag per block, a fence and LDS reductions 2.9: 188, 55, 22.  With Dinv_i
+// L_{i,i-1} formed beforehand, so that the last block's values meet one product
+// instead of two: 85, 34, 21, as its operands' cold loads stand in front of the
+// chain.)  pub: N doubles, all kUnsolved; the launch sets the first 64 nreset
+// of `reset`, the other of the context's two such arrays, back for the next one.
+// With `scaled` the launch also leaves scale .* x there (zero beyond n), unless the
+// gate's flags say NaN or V <= 0.  ticket: one word.
 // ---------------------------------------------------------------------------
+template <int C = 0>
+__device__ __forceinline__ void fmac16(double (&acc)[2], double src, const double (&m)[16]) {
+    if constexpr (C < 16) {
+        fmac_bcast_f64<C>(acc[C & 1], src, m[C]);
+        fmac16<C + 1>(acc, src, m);
+    }
+}
+
+// this lane's value of a published block; a wave that has timed out waits no more
+__device__ __forceinline__ double take_solved(const double* p, bool& ok, unsigned maxpoll) {
+    unsigned long long v = 0;
+    if (ok) {
+        ok = false;
+        for (unsigned n = 0; n < maxpoll; ++n) {
+            v = __hip_atomic_load(reinterpret_cast<const unsigned long long*>(p), __ATOMIC_RELAXED,
+                                  __HIP_MEMORY_SCOPE_AGENT);
+            ok = !__ballot(v == kUnsolved);
+            if (ok) break;
+            __builtin_amdgcn_s_sleep(1);
+        }
+    }
+    double d = __longlong_as_double((long long)v);
+    dpp_ready(d);
+    return d;
+}
+
 __global__ __launch_bounds__(256) void k_trsv_persist(const double* __restrict__ L, int64_t ld,
                                                       const double* __restrict__ Dinv, int64_t T,
-                                                      const double* __restrict__ b, double* __restrict__ x, int trans,
-                                                      unsigned* __restrict__ sync, unsigned epoch, unsigned base,
+                                                      const double* __restrict__ b, double* __restrict__ x,
+                                                      double* pub, double* __restrict__ reset, int64_t nreset,
+                                                      unsigned* __restrict__ ticket, unsigned base,
                                                       int* __restrict__ info, unsigned maxpoll,
                                                       const double* __restrict__ scale, int64_t n,
                                                       double* __restrict__ scaled, const int* __restrict__ gate) {
-    __shared__ double red[256];
     __shared__ double sv[64];
     __shared__ unsigned s_id;
-    __shared__ int s_ok;
-    const int t = threadIdx.x, e = t & 63, p = t >> 6;
-    if (t == 0) s_id = atomicAdd(&sync[kSolveMaxBlocks], 1u) - base;
+    const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+    if (t == 0) s_id = atomicAdd(ticket, 1u) - base;
     __syncthreads();
-    const int64_t k = s_id;
-    const int64_t i = trans ? T - 1 - k : k;
-    // Dinv_i and b_i do not depend on the waits: loaded first, off the chain
+    const int64_t k = __builtin_amdgcn_readfirstlane((int)s_id);
+    const int64_t i = T - 1 - k;
+    for (int64_t q = k; q < nreset; q += T)
+        if (t < 64) reinterpret_cast<unsigned long long*>(reset)[64 * q + t] = kUnsolved;
+    const int li = lane & 15, p = lane >> 4, row = 16 * w + li;
     const double* D = Dinv + i * 64 * 64;
     double dv[16];
 #pragma unroll
-    for (int u = 0; u < 16; ++u) {
-        const int c = 16 * p + u;
-        dv[u] = trans ? D[c + e * 64] : D[e + c * 64];
-    }
-    const double bi = (t < 64) ? b[64 * i + t] : 0.0;
-    double acc = 0.0;
+    for (int u = 0; u < 16; ++u) dv[u] = D[(16 * p + u) + row * 64];
+    const double bi = b[64 * i + row];
+    bool ok = true;
+    double acc[2] = {0.0, 0.0};
     for (int64_t m = 0; m < k; ++m) {
-        const int64_t j = trans ? T - 1 - m : m;  // the blocks solved before i, in their order
+        const int64_t j = T - 1 - m;  // the blocks solved before i, in their order
         double lt[16];
 #pragma unroll
-        for (int u = 0; u < 16; ++u) {
-            const int r = 16 * p + u;
-            // forward: L(64i + e, 64j + r); transposed: L(64j + r, 64i + e)
-            lt[u] = trans ? L[(64 * j + r) + (64 * i + e) * ld] : L[(64 * i + e) + (64 * j + r) * ld];
-        }
-        if (!panel_wait(&sync[j], epoch, info, &s_ok, maxpoll)) return;
-#pragma unroll
-        for (int u = 0; u < 16; ++u) acc += lt[u] * x[64 * j + 16 * p + u];
+        for (int u = 0; u < 16; ++u) lt[u] = L[(64 * j + 16 * p + u) + (64 * i + row) * ld];
+        const double xv = take_solved(pub + 64 * j + lane, ok, maxpoll);
+        fmac16(acc, xv, lt);
     }
-    red[t] = acc;
+    double s = acc[0] + acc[1];
+    s += __shfl_xor(s, 16, 64);
+    s += __shfl_xor(s, 32, 64);
+    if (p == 0) sv[row] = bi - s;
     __syncthreads();
-    if (t < 64) sv[t] = bi - (red[t] + red[t + 64] + red[t + 128] + red[t + 192]);
-    __syncthreads();
-    double s = 0.0;
-#pragma unroll
-    for (int u = 0; u < 16; ++u) s += dv[u] * sv[16 * p + u];
-    red[t] = s;
-    __syncthreads();
-    const double xi = (t < 64) ? red[t] + red[t + 64] + red[t + 128] + red[t + 192] : 0.0;
-    if (t < 64) put_shared(x + 64 * i + t, xi);
-    panel_publish(&sync[i], epoch);
-    if (scaled && t < 64 && !(gate && (*gate & 6))) scaled[64 * i + t] = 64 * i + t < n ? scale[64 * i + t] * xi : 0.0;
+    double rv = sv[lane];
+    dpp_ready(rv);
+    double out[2] = {0.0, 0.0};
+    fmac16(out, rv, dv);
+    double xi = out[0] + out[1];
+    xi += __shfl_xor(xi, 16, 64);
+    xi += __shfl_xor(xi, 32, 64);
+    if (!ok) {  // nothing is published, so the blocks that wait for this one time out too
+        if (lane == 0) atomicCAS(info, 0, kPanelWaitTimeout);
+        return;
+    }
+    if (p != 0) return;
+    put_shared(pub + 64 * i + row, xi);
+    x[64 * i + row] = xi;
+    if (scaled && !(gate && (*gate & 6))) scaled[64 * i + row] = 64 * i + row < n ? scale[64 * i + row] * xi : 0.0;
 }
 
 void trsv_persist_f64(hipStream_t s, const double* L, int64_t ld, const double* Dinv, int64_t N, const double* b,
-                      double* x, int trans, unsigned* sync, unsigned epoch, unsigned base, int* info,
-                      unsigned maxpoll, const double* scale, int64_t n, double* scaled, const int* gate) {
+                      double* x, double* pub, double* reset, int64_t nreset, unsigned* ticket,
+                      unsigned base, int* info, unsigned maxpoll, const double* scale, int64_t n, double* scaled,
+                      const int* gate) {
     const int64_t T = N / 64;
     if (T <= 0) return;
-    hipLaunchKernelGGL(k_trsv_persist, dim3((unsigned)T), dim3(256), 0, s, L, ld, Dinv, T, b, x, trans, sync, epoch,
-                       base, info, maxpoll, scale, n, scaled, gate);
+    hipLaunchKernelGGL(k_trsv_persist, dim3((unsigned)T), dim3(256), 0, s, L, ld, Dinv, T, b, x, pub, reset,
+                           nreset, ticket, base, info, maxpoll, scale, n, scaled, gate);
 }
 
 // ---------------------------------------------------------------------------

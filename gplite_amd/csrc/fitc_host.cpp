@@ -147,7 +147,7 @@ static void fitc_lemma_step(gpl_fitc* f, int* flags, bool inverse) {
     }
     potrf_blocked(c, f->d(F_G), Mz, f->d(F_DINVG), f->d(F_LDG), flags, inverse ? f->d(F_XG) : nullptr, nullptr,
                   f->d(F_Q1));
-    trsv_lower(c, s, f->d(F_G), Mz, f->d(F_DINVG), Mz, f->d(F_Q1), f->d(F_Q2), 1, flags);
+    trsv_back(c, s, f->d(F_G), Mz, f->d(F_DINVG), Mz, f->d(F_Q1), f->d(F_Q2), flags);
     Prof pv(c, "fitc_pass", 0, 16.0 * N * Mz);
     fitc_alpha_pass(s, A, Mz, n, N, f->d(F_Q2), f->d(F_ZS), f->d(F_S), f->d(F_ALPHA), f->d(F_PART), f->d(F_WZ));
     fitc_mean(s, A, Mz, n, N, f->d(F_WZ), f->d(F_D), f->d(F_ALPHA), f->d(F_FMEAN));

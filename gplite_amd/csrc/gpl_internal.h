@@ -149,14 +149,16 @@ constexpr int kPanelSyncWords = 2 * kPanelMaxBlocks + kPanelMaxBlocks * kPanelMa
 void potrf_panel_f64(hipStream_t s, double* A, int64_t ld, int64_t K0, int nc, int64_t nrb, double* Dinv,
                      double* ldiag, int* info, unsigned* sync, unsigned epoch, unsigned base, double* Dpub,
                      unsigned maxpoll, double* rhs);
-// the blocked solves of trsv_lower_f64 (N / 64 <= kSolveMaxBlocks) in one launch
-// (b is left unchanged); sync: kSolveSyncWords words of the context (zero at
-// creation), epoch, base (N / 64 tickets per launch) and maxpoll as for the panel
+// trsv_lower_f64's transposed solve (N / 64 <= kSolveMaxBlocks) in one launch
+// (b is left unchanged); pub, reset: the context's two arrays of 64 kSolveMaxBlocks
+// doubles, pub all kUnsolved, reset so again up to block nreset; ticket, base (N / 64
+// tickets per launch) and maxpoll as for the panel
 constexpr int kSolveMaxBlocks = 4096;
-constexpr int kSolveSyncWords = kSolveMaxBlocks + 1;
+constexpr unsigned long long kUnsolved = 0x7ff0dead5eed0001ull;  // a signalling NaN
 void trsv_persist_f64(hipStream_t s, const double* L, int64_t ld, const double* Dinv, int64_t N, const double* b,
-                      double* x, int trans, unsigned* sync, unsigned epoch, unsigned base, int* info,
-                      unsigned maxpoll, const double* scale, int64_t n, double* scaled, const int* gate);
+                      double* x, double* pub, double* reset, int64_t nreset, unsigned* ticket,
+                      unsigned base, int* info, unsigned maxpoll, const double* scale, int64_t n, double* scaled,
+                      const int* gate);
 // L Y = diag(sv) B in place for M right-hand sides (multiples of 64) in one launch; sync: kTrsmFlags + 1 words
 // of the context, N / 64 * (M / trsm_cols(N, M)) <= kTrsmFlags flags and as many tickets per launch
 constexpr int kTrsmFlags = 65536;

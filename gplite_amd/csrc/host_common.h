@@ -36,14 +36,14 @@ int prepare_prog(const gpl_cf_term* terms, int32_t nterms, int64_t ncols, DevPro
 void potrf_blocked(gpl_ctx* c, double* L, int64_t N, double* Dinv, double* ldiag, int* info, double* X = nullptr,
                    double* Tm = nullptr, double* rhs = nullptr);
 void trtri_blocked(gpl_ctx* c, const double* L, const double* Dinv, int64_t N, double* X, double* T = nullptr);
-// Blocked triangular solve with one vector (trsv_lower_f64's arguments, b left
-// unchanged): one launch on the context's solve flags when N / 64 <=
-// kSolveMaxBlocks, else one launch per block.  info receives kPanelWaitTimeout
-// if a device wait times out.  With `scaled` also scaled = scale .* x (n entries,
-// zero on the padding) unless *gate (if any) flags NaN or V <= 0.
-void trsv_lower(gpl_ctx* c, hipStream_t s, const double* L, int64_t ld, const double* Dinv, int64_t N, double* b,
-                double* x, int trans, int* info, const double* scale = nullptr, int64_t n = 0,
-                double* scaled = nullptr, const int* gate = nullptr);
+// L^T x = b with one vector (trsv_lower_f64's arguments, b left unchanged): one
+// launch when N / 64 <= kSolveMaxBlocks, else one per block.  info receives
+// kPanelWaitTimeout if a device wait times out.  With `scaled` also scaled =
+// scale .* x (n entries, zero on the padding) unless *gate (if any) flags NaN or
+// V <= 0.
+void trsv_back(gpl_ctx* c, hipStream_t s, const double* L, int64_t ld, const double* Dinv, int64_t N, double* b,
+               double* x, int* info, const double* scale = nullptr, int64_t n = 0, double* scaled = nullptr,
+               const int* gate = nullptr);
 // L Y = diag(sv) B in place for M right-hand sides (sv: the first n rows, or null): the forward solve of a
 // prediction, in launches of at most kTrsmFlags blocks.  info receives kPanelWaitTimeout if a device wait
 // times out.
@@ -143,10 +143,13 @@ struct gpl_ctx {
     unsigned* psync = nullptr;
     double* dpub = nullptr;  // its published diagonal blocks (kPanelMaxBlocks 64x64 blocks)
     unsigned pepoch = 0, pbase = 0;
-    // the same for the single-launch triangular solve (kSolveSyncWords words; its
-    // launches take their epochs from pepoch too)
-    unsigned* tsync = nullptr;
+    // the single-launch triangular solve: its ticket word, and the two arrays that
+    // its launches publish in by turns (every launch clears what the last one left)
+    unsigned* tticket = nullptr;
     unsigned tbase = 0;
+    double* tpub[2] = {nullptr, nullptr};
+    int64_t tdirty[2] = {0, 0};  // blocks of each that are not cleared
+    int tcur = 0;
     // and of the solve with many right-hand sides (kTrsmFlags + 1 words), with an
     // info word for its time-outs
     unsigned* msync = nullptr;
