@@ -380,6 +380,12 @@ static const int kPanelNB = 512;
 static const int kPanelW = 64 * kPanelBlocksF64;
 static const int kPanelNB32 = 64 * kPanelBlocksF32;
 
+// Up to this many rows left the whole trailing update runs on the main stream as one
+// launch: its part beside the next panel is then shorter than the 12 us that the two
+// events cost (factor and gradient at n = 1507: 1172 us with them, 1145 without; a
+// limit of 1536 gives the same).
+static const int64_t kInlineRows = 1024;
+
 // X = L^-1 by recursive doubling from the 64x64 diagonal-block inverses Dinv.
 // At level b (b = 64, 128, ...) the b-blocks pair up: [[X11, 0], [L21, X22]]
 // with X11 and X22 already inverted has the inverse [[X11, 0], [X21, X22]],
@@ -593,6 +599,15 @@ void gpl::potrf_blocked(gpl_ctx* c, double* L, int64_t N, double* Dinv, double* 
         if (R <= 0) break;
         const int64_t W1 = std::min<int64_t>(kPanelNB, R);
         const double* P = L + K1 + K0 * N;  // rows >= K1 of the factored panel
+        if (R <= kInlineRows) {
+            {
+                Prof p(c, "syrk_update", (double)R * R * W, 8.0 * ((double)R * R + 2.0 * R * W), s);
+                gemm2_f64(s, 0, 1, R, R, W, -1.0, P, N, P, N, 1.0, L + K1 * (N + 1), N, 1);
+            }
+            potrf_panel(c, s, L, N, K1, W1, Dinv, ldiag, info, rhs);
+            inv.after_panel(K1 + W1);
+            continue;
+        }
         {
             Prof p(c, "syrk_update", 2.0 * R * W1 * W, 8.0 * (2.0 * R * W1 + R * W), s);
             gemm2_f64(s, 0, 1, R, W1, W, -1.0, P, N, P, N, 1.0, L + K1 * (N + 1), N, 0);
