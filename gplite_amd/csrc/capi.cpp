@@ -715,18 +715,25 @@ void gpl::trsv_back(gpl_ctx* c, hipStream_t s, const double* L, int64_t ld, cons
         if (scaled) vec_mul_pad(s, n, N, scale, x, scaled, gate);
         return;
     }
-    const int cur = c->tcur;
-    trsv_persist_f64(s, L, ld, Dinv, N, b, x, c->tpub[cur], c->tpub[1 - cur], c->tdirty[1 - cur], c->tticket,
-                     c->tbase, info, c->pwait, scale, n, scaled, gate);
-    c->tdirty[cur] = T;
-    c->tdirty[1 - cur] = 0;
-    c->tcur = 1 - cur;
+    double *pub, *reset;
+    int64_t nreset;
+    c->next_pub(T, &pub, &reset, &nreset);
+    trsv_persist_f64(s, L, ld, Dinv, N, b, x, pub, reset, nreset, c->tticket, c->tbase, info, c->pwait, scale, n, scaled,
+                     gate);
     c->tbase += (unsigned)T;
 }
 
 void gpl::trsm_forward(gpl_ctx* c, hipStream_t s, const double* L, int64_t ld, const double* Dinv, int64_t N, double* B,
-                     int64_t ldb, int64_t M, const double* sv, int64_t n, int* info) {
+                     int64_t ldb, int64_t M, int64_t mt, const double* sv, int64_t n, int* info) {
     const int64_t T = N / 64;
+    if (mt <= kTrsmFew && mt * T <= kTrsmFewBlocks) {
+        double *pub, *reset;
+        int64_t nreset;
+        c->next_pub(mt * T, &pub, &reset, &nreset);
+        trsm_few_f64(s, L, ld, Dinv, N, B, ldb, (int)mt, sv, n, pub, reset, nreset, c->tticket, c->tbase, info, c->pwait);
+        c->tbase += (unsigned)(mt * T);
+        return;
+    }
     // columns per launch: as many as have flags (a model of more than 65536 row blocks, whose factor alone is
     // 2^45 bytes, does not exist)
     int64_t step = M;
@@ -1840,7 +1847,7 @@ int gpl::pred_on(gpl_ctx* c, gpl_model* m, const double* xt, int64_t mt, int32_t
             KtT = A2;
         } else {
             Prof p(c, "pred_trsm", (double)N * N * M, 4.0 * N * N + 16.0 * N * M);
-            trsm_forward(c, s, m->d(B_L), N, m->d(B_DINV), N, KtT, N, M, m->d(B_SV), n, c->minfo);
+            trsm_forward(c, s, m->d(B_L), N, m->d(B_DINV), N, KtT, N, M, mt, m->d(B_SV), n, c->minfo);
         }
         colsumsq_f64(s, KtT, N, N, mt, red, 0);
         launch_build_diag(s, pd, *hp, Ft, M, Ft, M, mt, kd);
@@ -1913,7 +1920,7 @@ static int draw_on(gpl_ctx* c, gpl_model* m, const double* xt, int64_t mt, doubl
         else
             gemm2_f64(s, 0, 0, N, M, N, 1.0, m->d(B_XINV), N, KtT, N, 0.0, A2, N, 3);
     } else {
-        trsm_forward(c, s, m->d(B_L), N, m->d(B_DINV), N, KtT, N, M, m->d(B_SV), n, info);
+        trsm_forward(c, s, m->d(B_L), N, m->d(B_DINV), N, KtT, N, M, mt, m->d(B_SV), n, info);
         A2 = KtT;
     }
     // cov = K_tt + jitter I - aux^T aux over lower tiles (padding: identity), then its factor

@@ -159,6 +159,17 @@ void trsv_persist_f64(hipStream_t s, const double* L, int64_t ld, const double* 
                       double* x, double* pub, double* reset, int64_t nreset, unsigned* ticket,
                       unsigned base, int* info, unsigned maxpoll, const double* scale, int64_t n, double* scaled,
                       const int* gate);
+// L Y = diag(sv) B in place for the first ncol columns, in one launch; pub .. maxpoll
+// as above (ncol N / 64 tickets).  Up to kTrsmFew columns of kTrsmFewBlocks blocks in
+// all: beyond, every column reading L for itself costs more than the shorter chain
+// gives.  A whole prediction here / with 16 columns a workgroup, us: n = 640 1 point
+// 67 / 79, 64 86 / 90, 100 93 / 92; n = 1000 1 70 / 100, 64 106 / 115, 100 120 / 118;
+// n = 2048 1 96 / 161, 32 133 / 170, 64 171 / 177; n = 4000 1 145 / 295, 32 260 / 305,
+// 48 324 / 307.
+constexpr int kTrsmFew = 64, kTrsmFewBlocks = 2048;
+void trsm_few_f64(hipStream_t s, const double* L, int64_t ld, const double* Dinv, int64_t N, double* B, int64_t ldb,
+                  int ncol, const double* sv, int64_t n, double* pub, double* reset, int64_t nreset, unsigned* ticket,
+                  unsigned base, int* info, unsigned maxpoll);
 // L Y = diag(sv) B in place for M right-hand sides (multiples of 64) in one launch; sync: kTrsmFlags + 1 words
 // of the context, N / 64 * (M / trsm_cols(N, M)) <= kTrsmFlags flags and as many tickets per launch
 constexpr int kTrsmFlags = 65536;

@@ -44,11 +44,11 @@ void trtri_blocked(gpl_ctx* c, const double* L, const double* Dinv, int64_t N, d
 void trsv_back(gpl_ctx* c, hipStream_t s, const double* L, int64_t ld, const double* Dinv, int64_t N, double* b,
                double* x, int* info, const double* scale = nullptr, int64_t n = 0, double* scaled = nullptr,
                const int* gate = nullptr);
-// L Y = diag(sv) B in place for M right-hand sides (sv: the first n rows, or null): the forward solve of a
+// L Y = diag(sv) B in place for M right-hand sides (of which the first mt are not padding) (sv: the first n rows, or null): the forward solve of a
 // prediction, in launches of at most kTrsmFlags blocks.  info receives kPanelWaitTimeout if a device wait
 // times out.
 void trsm_forward(gpl_ctx* c, hipStream_t s, const double* L, int64_t ld, const double* Dinv, int64_t N, double* B,
-                int64_t ldb, int64_t M, const double* sv, int64_t n, int* info);
+                int64_t ldb, int64_t M, int64_t mt, const double* sv, int64_t n, int* info);
 // the error reported for an info word of kPanelWaitTimeout
 int wait_timeout_fail();
 // probabilists' Gauss-Hermite nodes and weights normalised to sum 1 (R/quadrature.R:1-44)
@@ -143,8 +143,8 @@ struct gpl_ctx {
     unsigned* psync = nullptr;
     double* dpub = nullptr;  // its published diagonal blocks (kPanelMaxBlocks 64x64 blocks)
     unsigned pepoch = 0, pbase = 0;
-    // the single-launch triangular solve: its ticket word, and the two arrays that
-    // its launches publish in by turns (every launch clears what the last one left)
+    // the single-launch triangular solves with one or a few vectors: their ticket word,
+    // and the two arrays that the launches publish in by turns (every launch clears what the last one left)
     unsigned* tticket = nullptr;
     unsigned tbase = 0;
     double* tpub[2] = {nullptr, nullptr};
@@ -174,6 +174,16 @@ struct gpl_ctx {
     std::vector<size_t> scratch_sz;
     std::mutex mu;
 
+    // the array that a launch of nblocks blocks publishes in, and the other, of which
+    // it clears the first `nreset` blocks
+    void next_pub(int64_t nblocks, double** pub, double** reset, int64_t* nreset) {
+        *pub = tpub[tcur];
+        *reset = tpub[1 - tcur];
+        *nreset = tdirty[1 - tcur];
+        tdirty[tcur] = nblocks;
+        tdirty[1 - tcur] = 0;
+        tcur = 1 - tcur;
+    }
     hipEvent_t ev() {
         if (!pool.empty()) {
             hipEvent_t e = pool.back();
