@@ -1814,7 +1814,10 @@ int gpl::pred_on(gpl_ctx* c, gpl_model* m, const double* xt, int64_t mt, int32_t
     double* KtT = pb ? pb->KtT : (double*)c->buf(2, (size_t)N * M * 8);
     double* vbuf = pb ? pb->v : (double*)c->buf(3, ((size_t)M * 4 + 16) * 8);
     if (!xtd || !Ft || !KtT || !vbuf) return fail(GPL_ERR_OOM, "device allocation failed");
-    // vbuf: the result, mean[mt] var[mt] and the solve's status, then K_tt's diagonal and the variance reduction
+    // the result, mean[mt] var[mt] and the solve's status, in pinned memory if it fits; in vbuf
+    // else, and after it K_tt's diagonal and the variance reduction
+    const bool pinned = 2 * mt + 1 <= gpl_ctx::kStage;
+    double* const out = pinned ? c->stage : vbuf;
     double* const kd = vbuf + 2 * M + 8;
     double* const red = kd + M;
     if (mt * m->ncols > 0 && !(pb && pb->staged))
@@ -1824,15 +1827,14 @@ int gpl::pred_on(gpl_ctx* c, gpl_model* m, const double* xt, int64_t mt, int32_t
         Prof p(c, "pred_cross", 0, 8.0 * N * M);
         launch_build_cross(s, pd, *hp, m->d(B_F), N, n, N, Ft, M, mt, M, KtT, N);
     }
-    gemv_t_f64(s, KtT, N, N, mt, m->d(B_ALPHA), vbuf);
+    launch_pred_mean(s, pd, Ft, M, KtT, N, mt, m->d(B_ALPHA), out, want_var ? kd : nullptr);
     if (want_var && m->split) {
         // var_reduction = K_t (K + V)^-1 K_t^T of the reference's C_lu branch (R/gp_pred.R:220-223)
         if (pb) return fail(GPL_ERR_UNSUPPORTED, "a fit with split sites (pseudo-variances <= 0) needs gpl_pred");
         int r = split_var_reduction(c, m, KtT, M, red);
         if (r) return r;
-        launch_build_diag(s, pd, *hp, Ft, M, Ft, M, mt, kd);
-        vec_axpby(s, mt, 1.0, kd, -1.0, red, red);
-        HIP_TRY(hipMemcpyAsync(var, red, mt * 8, hipMemcpyDeviceToHost, s));
+        vec_axpby(s, mt, 1.0, kd, -1.0, red, out + mt);
+        fill_f64(s, out + 2 * mt, 1, 0.0);
     } else if (want_var) {
         // aux = C^-1 K_t^T = L^-1 (sv .* K_t^T)  (R/gp_pred.R:218)
         if (m->have_xinv) {
@@ -1849,26 +1851,21 @@ int gpl::pred_on(gpl_ctx* c, gpl_model* m, const double* xt, int64_t mt, int32_t
             Prof p(c, "pred_trsm", (double)N * N * M, 4.0 * N * N + 16.0 * N * M);
             trsm_forward(c, s, m->d(B_L), N, m->d(B_DINV), N, KtT, N, M, mt, m->d(B_SV), n, c->minfo);
         }
-        colsumsq_f64(s, KtT, N, N, mt, red, 0);
-        launch_build_diag(s, pd, *hp, Ft, M, Ft, M, mt, kd);
-        pred_finish(s, mt, kd, red, c->minfo, vbuf);
-        if (2 * mt + 1 <= gpl_ctx::kStage) {  // one copy through pinned memory
-            HIP_TRY(hipMemcpyAsync(c->stage, vbuf, (2 * mt + 1) * 8, hipMemcpyDeviceToHost, s));
-            HIP_TRY(hipStreamSynchronize(s));
-            memcpy(mean, c->stage, mt * 8);
-            memcpy(var, c->stage + mt, mt * 8);
-            return pred_status(c, c->stage[2 * mt]);
-        }
-        double st;
-        HIP_TRY(hipMemcpyAsync(var, vbuf + mt, mt * 8, hipMemcpyDeviceToHost, s));
-        HIP_TRY(hipMemcpyAsync(&st, vbuf + 2 * mt, 8, hipMemcpyDeviceToHost, s));
-        HIP_TRY(hipMemcpyAsync(mean, vbuf, mt * 8, hipMemcpyDeviceToHost, s));
-        HIP_TRY(hipStreamSynchronize(s));
-        return pred_status(c, st);
+        launch_pred_var(s, KtT, N, mt, kd, c->minfo, out + mt);
     }
-    HIP_TRY(hipMemcpyAsync(mean, vbuf, mt * 8, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    return GPL_OK;
+    if (pinned) {
+        HIP_TRY(hipStreamSynchronize(s));
+        memcpy(mean, out, mt * 8);
+        if (!want_var) return GPL_OK;
+        memcpy(var, out + mt, mt * 8);
+        return pred_status(c, out[2 * mt]);
+    }
+    HIP_TRY(read_back(c, mean, out, mt * 8));
+    if (!want_var) return GPL_OK;
+    double st;
+    HIP_TRY(read_back(c, var, out + mt, mt * 8));
+    HIP_TRY(read_back(c, &st, out + 2 * mt, 8));
+    return pred_status(c, st);
 }
 
 // Latent posterior draws at mt test points (R/gp_draw.R:107-124, method_full,

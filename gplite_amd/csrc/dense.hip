@@ -1547,17 +1547,6 @@ void trsm_persist_f64(hipStream_t s, const double* L, int64_t ld, const double* 
                            base, info, maxpoll);
 }
 
-__global__ void k_pred_finish(int64_t mt, const double* __restrict__ kd, const double* __restrict__ red,
-                              const int* __restrict__ info, double* __restrict__ out) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < mt) out[mt + i] = kd[i] - red[i];
-    if (i == 0) out[2 * mt] = (double)*info;
-}
-
-void pred_finish(hipStream_t s, int64_t mt, const double* kd, const double* red, const int* info, double* out) {
-    hipLaunchKernelGGL(k_pred_finish, dim3((unsigned)((mt + 255) / 256)), dim3(256), 0, s, mt, kd, red, info, out);
-}
-
 // ---------------------------------------------------------------------------
 // Triangular / symmetric matrix-vector products over lower tiles.  One
 // workgroup per 64-row output block, fixed summation order (deterministic).

@@ -60,6 +60,10 @@ void launch_build_cross(hipStream_t s, const DevProg* prog, const DevProg& hp, c
 // out[i] = k(Fa_i, Fb_i), i < n
 void launch_build_diag(hipStream_t s, const DevProg* prog, const DevProg& hp, const double* Fa,
                        int64_t lda_f, const double* Fb, int64_t ldb_f, int64_t n, double* out);
+void launch_pred_mean(hipStream_t s, const DevProg* prog, const double* Ft, int64_t ldf, const double* K, int64_t N,
+                      int64_t mt, const double* alpha, double* mean, double* kd);
+void launch_pred_var(hipStream_t s, const double* Y, int64_t N, int64_t mt, const double* kd, const int* info,
+                     double* out);
 // y = (K + jitter I) v  (matrix-free FP64, recomputes K from F). part: N*nchunk scratch.
 void launch_kmatvec(hipStream_t s, const DevProg* prog, const DevProg& hp, const double* F,
                     int64_t n, int64_t N, double jitter, const double* v, double* y, double* part,
@@ -177,8 +181,6 @@ int trsm_cols(int64_t N, int64_t M);
 void trsm_persist_f64(hipStream_t s, const double* L, int64_t ld, const double* Dinv, int64_t N, double* B, int64_t ldb,
                       int64_t M, const double* sv, int64_t n, unsigned* sync, unsigned epoch, unsigned base, int* info,
                       unsigned maxpoll);
-// out[mt + i] = kd[i] - red[i], out[2 mt] = *info (the end of a prediction with variances)
-void pred_finish(hipStream_t s, int64_t mt, const double* kd, const double* red, const int* info, double* out);
 // the panel on FP32 storage with the FP64 diagonal tiles Dacc (mixed precision)
 void potrf_panel_mixed(hipStream_t s, float* A, int64_t ld, int64_t K0, int nc, int64_t nrb, double* Dinv,
                        double* ldiag, int* info, unsigned* sync, unsigned epoch, unsigned base, double* Dacc,
