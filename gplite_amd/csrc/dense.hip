@@ -390,27 +390,33 @@ __device__ __forceinline__ double row_bcast_f64(double v) {  // lane LANE of eve
 // acc += (lane C of the 16-lane row of src) * m.  src needs two wait states
 // after the VALU instruction that wrote it (dpp_ready).
 template <int C>
+__device__ __forceinline__ void fnmac_bcast_f64(double& acc, double src, double m) {  // acc -= the same
+    asm("v_fmac_f64_dpp %0, %1, -%2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(src), "v"(m), "n"(C));
+}
+template <int C>
 __device__ __forceinline__ void fmac_bcast_f64(double& acc, double src, double m) {
     asm("v_fmac_f64_dpp %0, %1, %2 row_newbcast:%3 row_mask:0xf bank_mask:0xf" : "+v"(acc) : "v"(src), "v"(m), "n"(C));
 }
 __device__ __forceinline__ void dpp_ready(double& v) { asm("s_nop 1" : "+v"(v)); }
 
 // Columns J..15 of a phase: d the 16x16 diagonal tile (lane % 16 = row), a this
-// lane's own row.  PIV: piv and rinv receive the pivot of column lane % 16 and
-// its 1/sqrt.  The updates
+// lane's own row, whose columns go to out (row stride kTP) as they are done (rows above
+// the tile's diagonal leave what is not read).  PIV: piv and rinv receive the pivot of
+// column lane % 16 and its 1/sqrt.  The updates
 // take their multipliers inside the multiply-add (4 cycles; a separate broadcast
 // costs another 6 per multiplier).
 template <int C>
-__device__ __forceinline__ void factor16_update(double (&a)[16], double (&d)[16], double nd, double l, double dl) {
+__device__ __forceinline__ void factor16_update(double (&a)[16], double (&d)[16], double l, double dl) {
     if constexpr (C < 16) {
-        fmac_bcast_f64<C>(d[C], nd, dl);
-        fmac_bcast_f64<C>(a[C], nd, l);
-        factor16_update<C + 1>(a, d, nd, l, dl);
+        fnmac_bcast_f64<C>(d[C], dl, dl);
+        fnmac_bcast_f64<C>(a[C], dl, l);
+        factor16_update<C + 1>(a, d, l, dl);
     }
 }
 
 template <int J, bool PIV, bool CUBIC>
-__device__ __forceinline__ void factor16(double (&a)[16], double (&d)[16], int li, double& piv, double& rinv) {
+__device__ __forceinline__ void factor16(double (&a)[16], double (&d)[16], int li, double& piv, double& rinv,
+                                         double* out) {
     if constexpr (J < 16) {
         const double pv = row_bcast_f64<J>(d[J]);
         const double inv = rsqrt_f64<CUBIC>(pv);
@@ -418,12 +424,12 @@ __device__ __forceinline__ void factor16(double (&a)[16], double (&d)[16], int l
             piv = (li == J) ? pv : piv;
             rinv = (li == J) ? inv : rinv;
         }
-        double nd = d[J] * -inv;
         d[J] *= inv;
         a[J] *= inv;
-        dpp_ready(nd);
-        factor16_update<J + 1>(a, d, nd, a[J], d[J]);
-        factor16<J + 1, PIV, CUBIC>(a, d, li, piv, rinv);
+        out[J * kTP] = a[J];
+        dpp_ready(d[J]);
+        factor16_update<J + 1>(a, d, a[J], d[J]);
+        factor16<J + 1, PIV, CUBIC>(a, d, li, piv, rinv, out);
     }
 }
 
@@ -473,9 +479,7 @@ __device__ __forceinline__ void trapezoid_factor(double (*S)[kTP], double* piv, 
                 d[q] = S[j0 + q][j0 + li];
                 a[q] = S[j0 + q][row];
             }
-            factor16<0, RT == 4, CUBIC>(a, d, li, pv, ri);
-#pragma unroll
-            for (int q = 0; q < 16; ++q) S[j0 + q][row] = (row < j0 + q) ? 0.0 : a[q];
+            factor16<0, RT == 4, CUBIC>(a, d, li, pv, ri, &S[j0][row]);
             if (RT == 4 && lane < 16) {
                 piv[j0 + lane] = pv;
                 rinv[j0 + lane] = ri;
@@ -522,7 +526,11 @@ __device__ __forceinline__ void diag_finish(T* __restrict__ blk, int64_t ld, int
                                             const double* rinv, const double* piv) {
     const int t = threadIdx.x, i = t & 63, w = t >> 6;
 #pragma unroll
-    for (int q = 0; q < 8; ++q) blk[i + (int64_t)(8 * w + q) * ld] = (T)S[8 * w + q][i];
+    for (int q = 0; q < 8; ++q) {
+        const int c = 8 * w + q;
+        if (i < c) S[c][i] = 0.0;  // what the factorization left above the diagonal
+        blk[i + (int64_t)c * ld] = (i < c) ? (T)0 : (T)S[c][i];
+    }
     __syncthreads();
     if (t < 64) {
         S[t][t] = 0.0;  // the substitution uses the strictly lower part
