@@ -352,6 +352,7 @@ void gemm_mixed_f32f64f64(hipStream_t s, int ta, int tb, int64_t M, int64_t N, i
 // ---------------------------------------------------------------------------
 constexpr int kPanelThreads = 512;
 constexpr int kTP = 144;  // row stride: 4 k-rows apart is 32 banks, so both halves of an MFMA operand read are conflict-free
+static_assert(kTP >= 128 + 16, "trapezoid_factor parks a tile's rows in the padding");
 
 // 1/sqrt(d) for d > 0 from the hardware estimate y (good to 2^-24).  CUBIC: one
 // cubic step, y (1 + e/2 + 3e^2/8) with e = 1 - d y^2: four dependent operations,
@@ -479,7 +480,10 @@ __device__ __forceinline__ void trapezoid_factor(double (*S)[kTP], double* piv, 
                 d[q] = S[j0 + q][j0 + li];
                 a[q] = S[j0 + q][row];
             }
-            factor16<0, RT == 4, CUBIC>(a, d, li, pv, ri, &S[j0][row]);
+            // The other factoring wave may still be loading the diagonal tile, and with a
+            // block below nobody reads that tile's factor: its rows go to the padding.
+            const int orow = (RT == 8 && row >> 4 == p) ? 128 + li : row;
+            factor16<0, RT == 4, CUBIC>(a, d, li, pv, ri, &S[j0][orow]);
             if (RT == 4 && lane < 16) {
                 piv[j0 + lane] = pv;
                 rinv[j0 + lane] = ri;

@@ -51,3 +51,15 @@ def test_failing_minor_is_reported(k, precision):
                  precision=precision)
     assert e.value.code == L.GPL_ERR_NOT_PD
     assert e.value.minor == k + 1
+
+
+@pytest.mark.parametrize("n", [576, 960, 2049])
+def test_factor_has_the_same_bits_every_time(n):
+    # the waves of a panel's workgroups read each other's columns of one LDS block while they factor it
+    x, y, _ = _problem(n)
+    gp = G.gp_init(G.cf_sexp(lscale=0.3), G.lik_gaussian(sigma=0.1))
+    want = None
+    for _ in range(150):
+        a = G.gp_fit(gp, x, y).fit.alpha
+        want = a if want is None else want
+        np.testing.assert_array_equal(a, want)
