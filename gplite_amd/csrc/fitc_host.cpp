@@ -136,7 +136,7 @@ static void fitc_lemma_step(gpl_fitc* f, int* flags, bool inverse) {
     const double* A = f->d(F_A);
     fitc_site(s, n, N, f->d(F_D), f->d(F_V), f->d(F_Z), f->d(F_S), f->d(F_SI), f->d(F_ZS));
     {
-        Prof p(c, "fitc_gram", (double)Mz * Mz * N, 8.0 * N * Mz);
+        Prof p(c, "fitc_syrk", (double)Mz * Mz * N, 8.0 * N * Mz);
         const int P = fitc_parts(f);
         gemm_gram_f64(s, Mz, N, A, Mz, f->d(F_SI), P, fitc_part_cols(f), f->d(F_SPLIT), Mz, Mz * Mz);
         fitc_gram_sum(s, f->d(F_SPLIT), P, Mz, f->d(F_G));
