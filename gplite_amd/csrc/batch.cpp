@@ -141,8 +141,7 @@ static void potrf_panel_rec(gpl_ctx* c, hipStream_t s, Bucket& k, int64_t K0, in
         if (M > 0) {
             float* L21 = L + (K0 + 64) + K0 * N;
             Prof p(c, "batch_trsm_f64", 2.0 * nb * M * 64 * 64, 0, s);
-            gemm_mixed_f32f64_batched(s, 0, 1, M, 64, 64, 1.0, L21, N, Dinv + kk * 64 * 64, 64, 0.0, L21, N, 0, nb, N2,
-                                      N * 64, N2);
+            panel_solve_f32_batched(s, L21, N, M, Dinv + kk * 64 * 64, nb, N2, N * 64);
         }
         return;
     }

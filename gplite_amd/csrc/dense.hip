@@ -319,13 +319,7 @@ void gemm_gram_f64(hipStream_t s, int64_t M, int64_t K, const double* A, int64_t
                        lda, 0.0, C, ldc, 1, kp * lda, kp * lda, sC, ks, K);
 }
 
-// FP64-compute GEMMs on FP32 storage: A and C (panel solves of the batched form), A (prediction)
-void gemm_mixed_f32f64_batched(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha,
-                               const float* A, int64_t lda, const double* B, int64_t ldb, double beta, float* C,
-                               int64_t ldc, int tiles, int batch, int64_t sA, int64_t sB, int64_t sC) {
-    gemm_any(s, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tiles, batch, sA, sB, sC);
-}
-
+// FP64-compute GEMM on FP32 storage of A (prediction)
 void gemm_mixed_f32f64f64(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha,
                           const float* A, int64_t lda, const double* B, int64_t ldb, double beta, double* C,
                           int64_t ldc, int tiles) {
@@ -620,6 +614,62 @@ void potrf_diag_f32_batched(hipStream_t s, float* A, int64_t ld, int64_t k, doub
                             int batch, int64_t sA, int64_t sD, int64_t sL, const double* Dacc) {
     hipLaunchKernelGGL(k_potrf_diag, dim3((unsigned)batch), dim3(kPanelThreads), 0, s, A, ld, k, Dinv, ldiag, info, sA, sD, sL,
                        Dacc);
+}
+
+// The rows below a diagonal block of a batch's factorization: A = A Dinv^T in place, A (M x
+// 64, FP32), Dinv the block's inverse (FP64, lower triangular), FP64 products with one
+// rounding.  A wave per 16 rows, all of its operand loaded at once; Dinv's lower tiles go
+// to LDS once per workgroup and its zero tiles are skipped.
+// Bound by A's traffic for many rows, by one load latency and 40 matrix instructions for few.
+// (As a general product in place, a wave with 32 rows and half of the columns loading two
+// chunks ahead: 112 us for 16 problems of up to 8128 rows beside the other streams' products,
+// 47 here; 6.1 and 4.5 in a batch of 64 .. 2048 points.)
+__global__ __launch_bounds__(256) void k_panel_solve(float* __restrict__ A, int64_t ld,
+                                                     const double* __restrict__ Dinv, int64_t sA, int64_t sD) {
+    constexpr int LP = 68;  // 4 rows of k are 32 banks apart: both halves of an operand read are conflict-free
+    __shared__ double S[64][LP];
+    A += blockIdx.y * sA + 64 * (int64_t)blockIdx.x;
+    Dinv += blockIdx.y * sD;
+    const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+    const int li = lane & 15, g = lane >> 4;
+    float* p = A + 16 * w + li;
+    float a[4][4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) a[q][s] = p[(16 * q + 4 * g + s) * ld];
+    double d[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {  // column w + 4u: rows from its 16-block down
+        const int k = w + 4 * u;
+        d[u] = lane >= (k & ~15) ? Dinv[lane + 64 * k] : 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < 16; ++u) S[w + 4 * u][lane] = d[u];
+    __syncthreads();
+    // lane (li, g) of the (transposed) product holds columns g + 4v of row li; the
+    // sums run over k in the order of the other products (k = 4g + s of each 16 in step s)
+    d4 acc[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[j] = d4{0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int j = q; j < 4; ++j)
+                acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(S[16 * q + 4 * g + s][16 * j + li], (double)a[q][s],
+                                                              acc[j], 0, 0, 0);
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) p[(16 * j + g + 4 * v) * ld] = (float)acc[j][v];
+}
+
+void panel_solve_f32_batched(hipStream_t s, float* A, int64_t ld, int64_t M, const double* Dinv, int batch, int64_t sA,
+                             int64_t sD) {
+    if (M <= 0 || batch <= 0) return;
+    hipLaunchKernelGGL(k_panel_solve, dim3((unsigned)(M / 64), (unsigned)batch), dim3(256), 0, s, A, ld, Dinv, sA, sD);
 }
 
 // ---------------------------------------------------------------------------

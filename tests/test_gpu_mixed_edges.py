@@ -44,3 +44,12 @@ def test_batch_of_all_sizes():
     ps = [_problem(n) for n in SIZES + [513, 64]]
     e, _ = GPBatch([_gp()] * len(ps), [p[0] for p in ps], [p[1] for p in ps]).energy_grad(include_prior=False)
     assert np.all(np.abs(e - [p[3] for p in ps]) <= [p[4] for p in ps])
+
+
+# the solves of the rows below a diagonal block: none, one and several row blocks, the last one padded or whole
+@pytest.mark.parametrize("n", [65, 128, 129, 192, 321, 1025])
+@pytest.mark.parametrize("copies", [1, 3])
+def test_batched_panel_solve(n, copies):
+    x, y, _, e, tol = _problem(n)
+    got, _ = GPBatch([_gp()] * copies, [x] * copies, [y] * copies).energy_grad(include_prior=False)
+    assert np.all(np.abs(got - e) <= tol)
