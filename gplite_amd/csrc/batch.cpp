@@ -133,16 +133,8 @@ static void potrf_panel_rec(gpl_ctx* c, hipStream_t s, Bucket& k, int64_t K0, in
     double* Dacc = k.d(BB_DACC);
     if (W == 64) {
         const int64_t kk = K0 / 64;
-        {
-            Prof p(c, "batch_potrf_diag", 0, 0, s);
-            potrf_diag_f32_batched(s, L, N, kk, Dinv, k.d(BB_LDIAG), k.info, nb, N2, N * 64, N, Dacc);
-        }
-        const int64_t M = N - (K0 + 64);
-        if (M > 0) {
-            float* L21 = L + (K0 + 64) + K0 * N;
-            Prof p(c, "batch_trsm_f64", 2.0 * nb * M * 64 * 64, 0, s);
-            panel_solve_f32_batched(s, L21, N, M, Dinv + kk * 64 * 64, nb, N2, N * 64);
-        }
+        Prof p(c, "batch_trsm_f64", 2.0 * nb * (N - K0 - 64) * 64 * 64, 0, s);
+        potrf_step_f32_batched(s, L, N, kk, N - K0 - 64, Dinv, k.d(BB_LDIAG), k.info, nb, N2, N * 64, N, Dacc);
         return;
     }
     const int64_t h = (W / 128) * 64, W2 = W - h, M = N - (K0 + h);

@@ -517,21 +517,21 @@ __device__ __forceinline__ void put_shared(T* p, T v) {
 // 64x64 column-major) by 16x16 blocks: DPP substitution inside the diagonal
 // blocks, f64 MFMA for the block rows.  The inverse is left in rows 64..127 of
 // S, S[c][64 + r] = X(r, c).  rinv, piv: 64 doubles of LDS each.  SH: other
-// workgroups of the launch read Dinv (put_shared).
+// workgroups of the launch read Dinv (put_shared).  Without `put` nothing is stored.
 template <typename T, bool SH = false>
 __device__ __forceinline__ void diag_finish(T* __restrict__ blk, int64_t ld, int64_t k, double* __restrict__ Dinv,
                                             double* __restrict__ ldiag, int* __restrict__ info, double (*S)[kTP],
-                                            const double* rinv, const double* piv) {
+                                            const double* rinv, const double* piv, bool put = true) {
     const int t = threadIdx.x, i = t & 63, w = t >> 6;
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
         const int c = 8 * w + q;
         if (i < c) S[c][i] = 0.0;  // what the factorization left above the diagonal
-        blk[i + (int64_t)c * ld] = (i < c) ? (T)0 : (T)S[c][i];
+        if (put) blk[i + (int64_t)c * ld] = (i < c) ? (T)0 : (T)S[c][i];
     }
     __syncthreads();
-    if (t < 64) {
-        S[t][t] = 0.0;  // the substitution uses the strictly lower part
+    if (t < 64) S[t][t] = 0.0;  // the substitution uses the strictly lower part
+    if (put && t < 64) {
         ldiag[k * 64 + t] = 0.5 * log(piv[t]);
         const unsigned long long bad = __ballot(!(piv[t] > 0.0));
         if (t == 0 && bad) atomicCAS(info, 0, (int)(k * 64 + __ffsll((long long)bad)));
@@ -586,6 +586,7 @@ __device__ __forceinline__ void diag_finish(T* __restrict__ blk, int64_t ld, int
         }
         __syncthreads();
     }
+    if (!put) return;
     double* D = Dinv + k * 64 * 64;
     for (int e = t; e < 64 * 64; e += kPanelThreads) {
         if (SH) put_shared(D + e, S[e >> 6][64 + (e & 63)]);
@@ -594,7 +595,10 @@ __device__ __forceinline__ void diag_finish(T* __restrict__ blk, int64_t ld, int
 }
 
 // One 64x64 diagonal block per problem of a batch: FP32 storage, factored from
-// its FP64 tile (Dsrc, the layout of Dinv).
+// its FP64 tile (Dsrc, the layout of Dinv).  SOLVE: with the rows below it, A = A Dinv^T;
+// then every 64-row block below has a workgroup, which factors the block for itself (the
+// first stores it), and the solve's launch and load latency leave the chain.
+template <bool SOLVE>
 __global__ __launch_bounds__(kPanelThreads) void k_potrf_diag(float* __restrict__ A, int64_t ld, int64_t k,
                                                     double* __restrict__ Dinv, double* __restrict__ ldiag,
                                                     int* __restrict__ info, int64_t sA, int64_t sD, int64_t sL,
@@ -602,18 +606,39 @@ __global__ __launch_bounds__(kPanelThreads) void k_potrf_diag(float* __restrict_
     __shared__ double S[64][kTP];
     __shared__ double rinv[64];
     __shared__ double piv[64];
-    Dsrc += blockIdx.x * sD + k * 64 * 64;
+    const int64_t pr = blockIdx.y;
+    Dsrc += pr * sD + k * 64 * 64;
+    A += pr * sA + k * 64 * (ld + 1);
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int li = lane & 15, g = lane >> 4;
+    float* const p = A + 64 * ((int64_t)blockIdx.x + 1) + 16 * (w & 3) + li;  // wave w: rows 16 (w % 4) .. of its block
+    float a[4][4];
+    if (SOLVE)
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) a[q][s] = p[(16 * q + 4 * g + s) * ld];
     for (int e = threadIdx.x; e < 64 * 64; e += kPanelThreads) S[e >> 6][e & 63] = Dsrc[e];
     __syncthreads();
     trapezoid_factor<4, false, true>(S, piv, rinv);
-    diag_finish(A + blockIdx.x * sA + k * 64 * (ld + 1), ld, k, Dinv + blockIdx.x * sD, ldiag + blockIdx.x * sL,
-                info + blockIdx.x, S, rinv, piv);
-}
-
-void potrf_diag_f32_batched(hipStream_t s, float* A, int64_t ld, int64_t k, double* Dinv, double* ldiag, int* info,
-                            int batch, int64_t sA, int64_t sD, int64_t sL, const double* Dacc) {
-    hipLaunchKernelGGL(k_potrf_diag, dim3((unsigned)batch), dim3(kPanelThreads), 0, s, A, ld, k, Dinv, ldiag, info, sA, sD, sL,
-                       Dacc);
+    diag_finish(A, ld, k, Dinv + pr * sD, ldiag + pr * sL, info + pr, S, rinv, piv, !SOLVE || blockIdx.x == 0);
+    if (!SOLVE) return;
+    // as k_panel_solve; waves 0 - 3 the 16 columns of tiles 0 and 3, the others of 1 and 2
+    d4 acc[2] = {d4{0.0, 0.0, 0.0, 0.0}, d4{0.0, 0.0, 0.0, 0.0}};
+    const int j0 = w < 4 ? 0 : 1, j1 = 3 - j0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const double* X = &S[16 * q + 4 * g + s][64 + li];
+            if (q <= j0) acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(X[16 * j0], (double)a[q][s], acc[0], 0, 0, 0);
+            if (q <= j1) acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(X[16 * j1], (double)a[q][s], acc[1], 0, 0, 0);
+        }
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+        p[(16 * j0 + g + 4 * v) * ld] = (float)acc[0][v];
+        p[(16 * j1 + g + 4 * v) * ld] = (float)acc[1][v];
+    }
 }
 
 // The rows below a diagonal block of a batch's factorization: A = A Dinv^T in place, A (M x
@@ -666,10 +691,23 @@ __global__ __launch_bounds__(256) void k_panel_solve(float* __restrict__ A, int6
         for (int v = 0; v < 4; ++v) p[(16 * j + g + 4 * v) * ld] = (float)acc[j][v];
 }
 
-void panel_solve_f32_batched(hipStream_t s, float* A, int64_t ld, int64_t M, const double* Dinv, int batch, int64_t sA,
-                             int64_t sD) {
-    if (M <= 0 || batch <= 0) return;
-    hipLaunchKernelGGL(k_panel_solve, dim3((unsigned)(M / 64), (unsigned)batch), dim3(256), 0, s, A, ld, Dinv, sA, sD);
+// Up to this many row blocks, a workgroup to a CU, the two are one launch (a batch of 128, 64 ..
+// 2048 points: 21.3 ms as two, 20.5 with any line from 64 to 1024; one of 2048 problems: 62.6, and
+// 62.3 with a line at 256, 63.0 at 512, 63.7 at 4096, as the factors are then repeated on a full chip).
+static const int64_t kStepFused = 256;
+void potrf_step_f32_batched(hipStream_t s, float* A, int64_t ld, int64_t k, int64_t M, double* Dinv, double* ldiag,
+                            int* info, int batch, int64_t sA, int64_t sD, int64_t sL, const double* Dacc) {
+    if (batch <= 0) return;
+    if (M > 0 && M / 64 * batch <= kStepFused) {
+        hipLaunchKernelGGL(k_potrf_diag<true>, dim3((unsigned)(M / 64), (unsigned)batch), dim3(kPanelThreads), 0, s, A, ld,
+                           k, Dinv, ldiag, info, sA, sD, sL, Dacc);
+        return;
+    }
+    hipLaunchKernelGGL(k_potrf_diag<false>, dim3(1, (unsigned)batch), dim3(kPanelThreads), 0, s, A, ld, k, Dinv, ldiag,
+                       info, sA, sD, sL, Dacc);
+    if (M > 0)
+        hipLaunchKernelGGL(k_panel_solve, dim3((unsigned)(M / 64), (unsigned)batch), dim3(256), 0, s,
+                           A + (k + 1) * 64 + k * 64 * ld, ld, Dinv + k * 64 * 64, sA, sD);
 }
 
 // ---------------------------------------------------------------------------

@@ -320,14 +320,12 @@ void gemm_f32_batched2(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int6
 // FP64 folding in the GEMMs of L^-1 and B^-1 = X^T X (they feed the gradient and
 // the predictive variance, not the log evidence)
 constexpr int kFoldInverse = 1;
-// A = A Dinv^T in place (M x 64, M a multiple of 64; Dinv: the 64x64 inverse of the diagonal block above it)
-void panel_solve_f32_batched(hipStream_t s, float* A, int64_t ld, int64_t M, const double* Dinv, int batch, int64_t sA,
-                             int64_t sD);
 // Factor the 64x64 diagonal block at A + k*64*(ld+1) of every problem from its FP64 tile
 // Dacc + k*64*64; its inverse goes to Dinv + k*64*64 (FP64), log(L_ii) to ldiag + k*64,
-// the first failing row + 1 to info[problem].
-void potrf_diag_f32_batched(hipStream_t s, float* A, int64_t ld, int64_t k, double* Dinv, double* ldiag, int* info,
-                             int batch, int64_t sA, int64_t sD, int64_t sL, const double* Dacc);
+// the first failing row + 1 to info[problem].  The M rows below it (a multiple of 64) are
+// multiplied by the inverse's transpose.
+void potrf_step_f32_batched(hipStream_t s, float* A, int64_t ld, int64_t k, int64_t M, double* Dinv, double* ldiag,
+                            int* info, int batch, int64_t sA, int64_t sD, int64_t sL, const double* Dacc);
 void set_identity_f32_batched(hipStream_t s, float* A, int64_t ld, int64_t N, int batch, int64_t sA);
 void trmv_lower_f32_batched(hipStream_t s, const float* X, int64_t ld, int64_t N, const double* b, double* y,
                             int trans, int batch, int64_t sX, int64_t sv, double* part, int nchunk);

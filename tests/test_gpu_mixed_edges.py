@@ -53,3 +53,11 @@ def test_batched_panel_solve(n, copies):
     x, y, _, e, tol = _problem(n)
     got, _ = GPBatch([_gp()] * copies, [x] * copies, [y] * copies).energy_grad(include_prior=False)
     assert np.all(np.abs(got - e) <= tol)
+
+
+# 256 row blocks below the diagonal blocks of a launch, and more: one launch with the factor and two
+@pytest.mark.parametrize("copies", [127, 128, 129])
+def test_batched_step_at_its_line(copies):
+    x, y, _, e, tol = _problem(180)
+    got, _ = GPBatch([_gp()] * copies, [x] * copies, [y] * copies).energy_grad(include_prior=False)
+    assert np.all(np.abs(got - e) <= tol)
