@@ -224,6 +224,137 @@ static void gemm32_launch(hipStream_t s, int ta, int tb, int64_t M, int64_t N, i
 #undef GPL_G32
 }
 
+// The same product for launches of few tiles: a wave per 32x32 block of C (2 x 2 of them
+// a workgroup), operands straight from global memory to registers three chunks of 16 k
+// ahead, no LDS and no barrier.  A launch that does not fill the chip is bound by its k
+// loop, and the staged form takes a load latency and two barriers, about 1 us, for every
+// chunk: the updates (TB = 1) and inverse products of a batch of 128 problems of 64 ..
+// 2048 points took 9.9 and 13.7 us on average, here 7.5 and 10.  Where the chip is full the
+// loads are the bound instead (twice the operand bytes per product of a 64x64 tile in
+// LDS).  Sums run in the staged form's order (step s of a chunk takes k = s and 8 + s, folds
+// every 64 k), so both give the same bits.
+// M, N and K are multiples of 64.
+//
+// One 16-k chunk of a wave's 32 rows of an operand: lane (l32, h) takes k = 8h + s, s < 8.
+// KC: contiguous in k, 32 bytes per lane; else 128 bytes per k.
+template <bool KC>
+__device__ __forceinline__ void g32r_load(float (&f)[8], const float* p, int64_t ld) {
+    if (KC) {
+        const float4 a = reinterpret_cast<const float4*>(p)[0], b = reinterpret_cast<const float4*>(p)[1];
+        f[0] = a.x, f[1] = a.y, f[2] = a.z, f[3] = a.w;
+        f[4] = b.x, f[5] = b.y, f[6] = b.z, f[7] = b.w;
+    } else {
+#pragma unroll
+        for (int s = 0; s < 8; ++s) f[s] = p[s * ld];
+    }
+}
+
+template <int TA, int TB>
+__global__ __launch_bounds__(256) void k_gemm32_reg(int64_t M, int64_t K, float alpha, const float* A, int64_t lda,
+                                                    const float* B, int64_t ldb, float beta, float* C, int64_t ldc,
+                                                    int tiles, int64_t sA, int64_t sB, int64_t sC, int64_t sZ) {
+    constexpr bool KA = TA != 0, KB = TB == 0;  // contiguous in k
+    A += blockIdx.y * sA + blockIdx.z * sZ;
+    B += blockIdx.y * sB + blockIdx.z * sZ;
+    C += blockIdx.y * sC + blockIdx.z * sZ;
+    const int64_t bid = (tiles == 2 || tiles == 4) ? (int64_t)blockIdx.x : xcd_remap32(blockIdx.x, gridDim.x);
+    int64_t ti, tj;
+    if (tiles == 0 || tiles == 3 || tiles == 4) {
+        ti = bid % (M / 64);
+        tj = bid / (M / 64);
+        if (tiles == 3) ti = M / 64 - 1 - ti;  // the longest k ranges first
+    } else {
+        lower_tile32(bid, ti, tj);
+    }
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l32 = lane & 31, h = lane >> 5;
+    const int64_t row0 = ti * 64 + (w & 1) * 32, col0 = tj * 64 + (w >> 1) * 32;
+    const int64_t kbeg = (tiles == 2) ? ti * 64 : (tiles == 4) ? tj * 64 : 0;
+    const int64_t kend = (tiles == 3 && (ti + 1) * 64 < K) ? (ti + 1) * 64 : K;
+    const int nwin = kend > kbeg ? (int)((kend - kbeg) / 64) : 0;
+    const float* pa = KA ? A + (kbeg + 8 * h) + (row0 + l32) * lda : A + (row0 + l32) + (kbeg + 8 * h) * lda;
+    const float* pb = KB ? B + (kbeg + 8 * h) + (col0 + l32) * ldb : B + (col0 + l32) + (kbeg + 8 * h) * ldb;
+    const int64_t stepa = KA ? 16 : 16 * lda, stepb = KB ? 16 : 16 * ldb;
+    f16v acc;
+    double acc64[16];
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+        acc[v] = 0.f;
+        acc64[v] = 0.0;
+    }
+    float fa[4][8], fb[4][8];
+    auto load = [&](int st) {
+        g32r_load<KA>(fa[st], pa, lda);
+        g32r_load<KB>(fb[st], pb, ldb);
+        pa += stepa;
+        pb += stepb;
+    };
+    // the block is formed transposed: D lane (l32, h), item v holds column
+    // 8 (v / 4) + 4h + v % 4 of row l32
+    auto mult = [&](int st) {
+        if (st == 0)  // a new window of 64 k: the last one's sums to FP64
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                acc64[v] += (double)acc[v];
+                acc[v] = 0.f;
+            }
+#pragma unroll
+        for (int s = 0; s < 8; ++s) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(fb[st][s], fa[st][s], acc, 0, 0, 0);
+    };
+    if (nwin > 0) {
+        load(0);
+        load(1);
+        load(2);
+    }
+    for (int c = 0; c < nwin - 1; ++c)  // every load of the next window's start exists
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            load((q + 3) & 3);
+            mult(q);
+        }
+    if (nwin > 0) {
+        load(3);
+        mult(0);
+        mult(1);
+        mult(2);
+        mult(3);
+    }
+    // With beta != 0 every C value is loaded before the first store (a load placed
+    // after a store that may alias it waits for that store's round trip).
+    float* p = C + row0 + l32 + (col0 + 4 * h) * ldc;
+    float cv[16];
+    if (beta != 0.f) {
+#pragma unroll
+        for (int v = 0; v < 16; ++v) cv[v] = p[(8 * (v >> 2) + (v & 3)) * ldc];
+    }
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+        const double o = (double)alpha * (acc64[v] + (double)acc[v]);
+        p[(8 * (v >> 2) + (v & 3)) * ldc] = (float)((double)beta * (beta == 0.f ? 0.0 : (double)cv[v]) + o);
+    }
+}
+
+// 64x64 tiles that a tile mode forms
+static int64_t tiles64(int64_t M, int64_t N, int tiles) {
+    const int64_t tm = M / 64, tn = N / 64;
+    return (tiles == 0 || tiles == 3 || tiles == 4) ? tm * tn : tm * (tm + 1) / 2;
+}
+
+static void gemm32_reg_launch(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, float alpha,
+                              const float* A, int64_t lda, const float* B, int64_t ldb, float beta, float* C,
+                              int64_t ldc, int tiles, int batch, int64_t sA, int64_t sB, int64_t sC, int nz,
+                              int64_t sZ) {
+    dim3 grid((unsigned)tiles64(M, N, tiles), (unsigned)batch, (unsigned)nz), block(256);
+#define GPL_G32(TAv, TBv)                                                                                          \
+    hipLaunchKernelGGL((k_gemm32_reg<TAv, TBv>), grid, block, 0, s, M, K, alpha, A, lda, B, ldb, beta, C, ldc, tiles, \
+                       sA, sB, sC, sZ)
+    if (!ta && !tb) GPL_G32(0, 0);
+    else if (!ta && tb) GPL_G32(0, 1);
+    else if (ta && !tb) GPL_G32(1, 0);
+    else GPL_G32(1, 1);
+#undef GPL_G32
+}
+
 // fold != 0: FP32 sums folded into FP64 every 64 k; 128-wide tiles use eight
 // waves there (64x32 per wave keeps the FP64 accumulators at four waves/SIMD).
 // fold == 0: plain FP32 accumulation.  bm == 0 picks 128-wide tiles when the
@@ -236,6 +367,12 @@ void gemm_f32_batched2(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int6
         const int64_t tm = (M + 127) / 128, tn = (N + 127) / 128;
         const int64_t n128 = ((tiles == 0 || tiles == 3 || tiles == 4) ? tm * tn : tm * (tm + 1) / 2) * batch * nz;
         bm = (n128 >= 256) ? 128 : 64;
+    }
+    // up to a tile per CU (a batch of 128, 64 .. 2048 points: 20.4 ms with staged tiles only, 20.2 with
+    // a line at 32 tiles, 19.7 at 128 and 256, 19.9 at 400; one fit at n = 8192 9.5 ms up to 512, 9.7 at 4096)
+    if (fold && bm == 64 && tiles64(M, N, tiles) * batch * nz <= 256) {
+        gemm32_reg_launch(s, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tiles, batch, sA, sB, sC, nz, sZ);
+        return;
     }
 #define GPL_G32L(BMv, FOLDv, NWv)                                                                                     \
     gemm32_launch<BMv, FOLDv, NWv>(s, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tiles, batch, sA, sB, sC, \

@@ -61,3 +61,14 @@ def test_batched_step_at_its_line(copies):
     x, y, _, e, tol = _problem(180)
     got, _ = GPBatch([_gp()] * copies, [x] * copies, [y] * copies).energy_grad(include_prior=False)
     assert np.all(np.abs(got - e) <= tol)
+
+
+# 64x64 tiles of a launch, of one problem and of all, on both sides of the line between the two FP32 products
+@pytest.mark.parametrize("n,copies", [(64, 300), (130, 60), (500, 12), (1400, 2), (1500, 2)])
+def test_a_problem_alone_and_among_copies(n, copies):
+    x, y = _problem(n)[:2]
+    one = GPBatch([_gp()], [x], [y]).energy_grad(include_prior=False)
+    e, g = GPBatch([_gp()] * copies, [x] * copies, [y] * copies).energy_grad(include_prior=False)
+    # the factor and the inverses have one order of sums; alpha is refined to 1e-8 in any
+    np.testing.assert_allclose(e, np.full(copies, one[0][0]), rtol=1e-8)
+    np.testing.assert_allclose(g, np.tile(one[1][0], (copies, 1)), rtol=0, atol=1e-7 * np.abs(one[1]).max())
