@@ -184,7 +184,7 @@ __global__ __launch_bounds__(256) void k_gemm_reg(int64_t M, int64_t N, int64_t 
     for (int q = 0; q < PF - 1; ++q)
         if (q < nch) load(q);
     int c = 0;
-    for (; c + 2 * PF - 1 <= nch; c += PF)  // every load of this round exists
+    for (; c + 2 * PF - 1 <= nch; c += PF)  // every load of this pass exists
 #pragma unroll
         for (int q = 0; q < PF; ++q) {
             load((q + PF - 1) % PF);
