@@ -1749,7 +1749,7 @@ static size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 
 size_t gpl::pred_bufs_bytes(int64_t N, int64_t ncols, int64_t M) {
     return align256((size_t)M * std::max<int64_t>(ncols, 1) * 8) + align256((size_t)M * MAX_FEAT * 8) +
-           2 * align256((size_t)N * M * 8) + align256(((size_t)M * 4 + 16) * 8);
+           2 * align256((size_t)N * M * 8) + align256((size_t)M * 3 * 8);
 }
 
 PredBufs gpl::pred_bufs_carve(void* base, int64_t N, int64_t ncols, int64_t M) {
@@ -1812,14 +1812,17 @@ int gpl::pred_on(gpl_ctx* c, gpl_model* m, const double* xt, int64_t mt, int32_t
     double* xtd = pb ? pb->xt : (double*)c->buf(0, (size_t)mt * std::max<int64_t>(m->ncols, 1) * 8);
     double* Ft = pb ? pb->Ft : (double*)c->buf(1, (size_t)M * MAX_FEAT * 8);
     double* KtT = pb ? pb->KtT : (double*)c->buf(2, (size_t)N * M * 8);
-    double* vbuf = pb ? pb->v : (double*)c->buf(3, ((size_t)M * 4 + 16) * 8);
+    double* vbuf = pb ? pb->v : (double*)c->buf(3, (size_t)M * 3 * 8);
     if (!xtd || !Ft || !KtT || !vbuf) return fail(GPL_ERR_OOM, "device allocation failed");
-    // the result, mean[mt] var[mt] and the solve's status, in pinned memory if it fits; in vbuf
-    // else, and after it K_tt's diagonal and the variance reduction
+    // the solve's status, means and variances in pinned memory if they fit; the vectors in
+    // vbuf else, which also holds the variance reduction (the variances' place) and K_tt's diagonal
     const bool pinned = 2 * mt + 1 <= gpl_ctx::kStage;
-    double* const out = pinned ? c->stage : vbuf;
-    double* const kd = vbuf + 2 * M + 8;
-    double* const red = kd + M;
+    double* const status = c->stage;
+    double* const dmean = pinned ? c->stage + 1 : vbuf;
+    double* const dvar = pinned ? c->stage + 1 + mt : vbuf + M;
+    double* const red = vbuf + M;
+    double* const kd = vbuf + 2 * M;
+    *status = 0.0;
     if (mt * m->ncols > 0 && !(pb && pb->staged))
         HIP_TRY(hipMemcpyAsync(xtd, xt, mt * m->ncols * 8, hipMemcpyHostToDevice, s));
     launch_features(s, xtd, mt, mt, (int)m->ncols, pf, m->prog, Ft, M);
@@ -1827,14 +1830,13 @@ int gpl::pred_on(gpl_ctx* c, gpl_model* m, const double* xt, int64_t mt, int32_t
         Prof p(c, "pred_cross", 0, 8.0 * N * M);
         launch_build_cross(s, pd, *hp, m->d(B_F), N, n, N, Ft, M, mt, M, KtT, N);
     }
-    launch_pred_mean(s, pd, Ft, M, KtT, N, mt, m->d(B_ALPHA), out, want_var ? kd : nullptr);
+    launch_pred_mean(s, pd, Ft, M, KtT, N, mt, m->d(B_ALPHA), dmean, want_var ? kd : nullptr);
     if (want_var && m->split) {
         // var_reduction = K_t (K + V)^-1 K_t^T of the reference's C_lu branch (R/gp_pred.R:220-223)
         if (pb) return fail(GPL_ERR_UNSUPPORTED, "a fit with split sites (pseudo-variances <= 0) needs gpl_pred");
         int r = split_var_reduction(c, m, KtT, M, red);
         if (r) return r;
-        vec_axpby(s, mt, 1.0, kd, -1.0, red, out + mt);
-        fill_f64(s, out + 2 * mt, 1, 0.0);
+        vec_axpby(s, mt, 1.0, kd, -1.0, red, dvar);
     } else if (want_var) {
         // aux = C^-1 K_t^T = L^-1 (sv .* K_t^T)  (R/gp_pred.R:218)
         if (m->have_xinv) {
@@ -1851,20 +1853,17 @@ int gpl::pred_on(gpl_ctx* c, gpl_model* m, const double* xt, int64_t mt, int32_t
             Prof p(c, "pred_trsm", (double)N * N * M, 4.0 * N * N + 16.0 * N * M);
             trsm_forward(c, s, m->d(B_L), N, m->d(B_DINV), N, KtT, N, M, mt, m->d(B_SV), n, c->minfo);
         }
-        launch_pred_var(s, KtT, N, mt, kd, c->minfo, out + mt);
+        launch_pred_var(s, KtT, N, mt, kd, c->minfo, dvar, status);
     }
+    HIP_TRY(hipStreamSynchronize(s));
+    const double st = *status;
     if (pinned) {
-        HIP_TRY(hipStreamSynchronize(s));
-        memcpy(mean, out, mt * 8);
-        if (!want_var) return GPL_OK;
-        memcpy(var, out + mt, mt * 8);
-        return pred_status(c, out[2 * mt]);
+        memcpy(mean, dmean, mt * 8);
+        if (want_var) memcpy(var, dvar, mt * 8);
+    } else {
+        HIP_TRY(read_back(c, mean, dmean, mt * 8));
+        if (want_var) HIP_TRY(read_back(c, var, dvar, mt * 8));
     }
-    HIP_TRY(read_back(c, mean, out, mt * 8));
-    if (!want_var) return GPL_OK;
-    double st;
-    HIP_TRY(read_back(c, var, out + mt, mt * 8));
-    HIP_TRY(read_back(c, &st, out + 2 * mt, 8));
     return pred_status(c, st);
 }
 

@@ -461,7 +461,7 @@ void launch_pred_mean(hipStream_t s, const DevProg* prog, const double* Ft, int6
 
 __global__ __launch_bounds__(256) void k_pred_var(const double* __restrict__ Y, int64_t N, int64_t mt,
                                                   const double* __restrict__ kd, const int* __restrict__ info,
-                                                  double* __restrict__ out) {
+                                                  double* __restrict__ out, double* __restrict__ status) {
     const int lane = threadIdx.x & 63;
     const int64_t j = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (j >= mt) return;
@@ -475,13 +475,14 @@ __global__ __launch_bounds__(256) void k_pred_var(const double* __restrict__ Y, 
     s = wave_sum_xor(s);
     if (lane != 0) return;
     out[j] = kd[j] - s;
-    if (j == 0) out[mt] = (double)*info;
+    if (j == 0) *status = (double)*info;
 }
 
-// out: the variances, then the info word
+// out: the variances; status: the info word
 void launch_pred_var(hipStream_t s, const double* Y, int64_t N, int64_t mt, const double* kd, const int* info,
-                     double* out) {
-    hipLaunchKernelGGL(k_pred_var, dim3((unsigned)((mt + 3) / 4)), dim3(256), 0, s, Y, N, mt, kd, info, out);
+                     double* out, double* status) {
+    hipLaunchKernelGGL(k_pred_var, dim3((unsigned)((mt + 3) / 4)), dim3(256), 0, s, Y, N, mt, kd, info, out,
+                       status);
 }
 
 // ---------------------------------------------------------------------------

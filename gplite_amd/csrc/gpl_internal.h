@@ -63,7 +63,7 @@ void launch_build_diag(hipStream_t s, const DevProg* prog, const DevProg& hp, co
 void launch_pred_mean(hipStream_t s, const DevProg* prog, const double* Ft, int64_t ldf, const double* K, int64_t N,
                       int64_t mt, const double* alpha, double* mean, double* kd);
 void launch_pred_var(hipStream_t s, const double* Y, int64_t N, int64_t mt, const double* kd, const int* info,
-                     double* out);
+                     double* out, double* status);
 // y = (K + jitter I) v  (matrix-free FP64, recomputes K from F). part: N*nchunk scratch.
 void launch_kmatvec(hipStream_t s, const DevProg* prog, const DevProg& hp, const double* F,
                     int64_t n, int64_t N, double jitter, const double* v, double* y, double* part,
