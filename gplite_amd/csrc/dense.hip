@@ -326,6 +326,18 @@ void gemm_mixed_f32f64f64(hipStream_t s, int ta, int tb, int64_t M, int64_t N, i
     gemm_any(s, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tiles, 1, 0, 0, 0);
 }
 
+// A failing row + 1 into info, the lowest of all that are reported: the workgroups of
+// one launch that factor different diagonal blocks report in no fixed order, and past a
+// failing pivot every later block holds NaN and reports too.  A time-out stays.
+__device__ __forceinline__ void report_minor(int* info, int minor) {
+    int old = atomicCAS(info, 0, minor);
+    while (old > minor && old != kPanelWaitTimeout) {  // old only falls, or becomes the time-out
+        const int seen = atomicCAS(info, old, minor);
+        if (seen == old) return;
+        old = seen;
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Cholesky of a 64-column block held in LDS, FP64.  The block is a trapezoid
 // S[col][row] (64 columns, row stride kTP): rows 0..63 the diagonal block and,
@@ -513,7 +525,7 @@ __device__ __forceinline__ void put_shared(T* p, T v) {
 
 // After trapezoid_factor<4>: the factor of diagonal block k to global memory
 // (blk, leading dimension ld; the upper triangle as zeros), ldiag[64k + i] =
-// log L_ii, info = first failing row + 1, and the block's inverse to Dinv (FP64,
+// log L_ii, info = lowest failing row + 1, and the block's inverse to Dinv (FP64,
 // 64x64 column-major) by 16x16 blocks: DPP substitution inside the diagonal
 // blocks, f64 MFMA for the block rows.  The inverse is left in rows 64..127 of
 // S, S[c][64 + r] = X(r, c).  rinv, piv: 64 doubles of LDS each.  SH: other
@@ -534,7 +546,7 @@ __device__ __forceinline__ void diag_finish(T* __restrict__ blk, int64_t ld, int
     if (put && t < 64) {
         ldiag[k * 64 + t] = 0.5 * log(piv[t]);
         const unsigned long long bad = __ballot(!(piv[t] > 0.0));
-        if (t == 0 && bad) atomicCAS(info, 0, (int)(k * 64 + __ffsll((long long)bad)));
+        if (t == 0 && bad) report_minor(info, (int)(k * 64 + __ffsll((long long)bad)));
     }
     __syncthreads();
     // Inverse by 16x16 blocks.  (1) Each wave inverts its diagonal block by
@@ -2090,7 +2102,7 @@ void restore_factor_f64(hipStream_t s, double* L, int64_t n, int64_t N, const do
 // (what diag_finish does after the factorisation): Dinv + k*4096
 // receives L_kk^-1 (column-major, ld 64, zeros above the diagonal) and
 // ldiag[64k + i] = log L_ii.  Lane t forward-substitutes column t.  A pivot
-// that is not positive (or NaN) sets info to its 1-based index if info is 0.
+// that is not positive (or NaN) sets info to its 1-based index, the lowest of them.
 __global__ __launch_bounds__(64) void k_trtri_diag64(const double* __restrict__ L, int64_t ld,
                                                      double* __restrict__ Dinv, double* __restrict__ ldiag,
                                                      int* __restrict__ info) {
@@ -2116,7 +2128,7 @@ __global__ __launch_bounds__(64) void k_trtri_diag64(const double* __restrict__ 
     const double p = A[t][t];
     ldiag[k * 64 + t] = log(p);
     const unsigned long long bad = __ballot(!(p > 0.0));
-    if (t == 0 && bad) atomicCAS(info, 0, (int)(k * 64 + __ffsll((long long)bad)));
+    if (t == 0 && bad) report_minor(info, (int)(k * 64 + __ffsll((long long)bad)));
 }
 
 void trtri_diag64_f64(hipStream_t s, const double* L, int64_t ld, int64_t T, double* Dinv, double* ldiag, int* info) {
