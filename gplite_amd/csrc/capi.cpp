@@ -574,7 +574,7 @@ static void potrf_panel(gpl_ctx* c, hipStream_t st, double* L, int64_t N, int64_
         if (k1 < K0 + W) {
             Prof p(c, "syrk_update", 2.0 * (N - k1) * (K0 + W - k1) * w, 0, st);
             const double* Q = L + k1 + k0 * N;
-            gemm2_f64(st, 0, 1, N - k1, K0 + W - k1, w, -1.0, Q, N, Q, N, 1.0, L + k1 * (N + 1), N, 0);
+            gemm_sub_f64(st, N - k1, K0 + W - k1, w, Q, N, Q, N, L + k1 * (N + 1), N);
         }
     }
 }

@@ -50,6 +50,9 @@ __device__ __forceinline__ void lower_tile(int64_t t, int64_t& ti, int64_t& tj) 
 // whatever the tile.
 // M, N and K are multiples of 64, operand addresses of 16 bytes.
 //
+// SUB: C -= op(A) op(B) (alpha = -1, beta = 1), where every 64 k's products are summed on
+// their own and subtracted.
+//
 // INP: C is one of the operands (a solve against a 64x64 inverse).  A workgroup
 // of 64x64 then covers the whole contraction of its rows (A = C, N = 64) or
 // columns (B = C, M = 64), and stores only after all of its waves have read.
@@ -96,7 +99,7 @@ __device__ __forceinline__ void frag_load(T (&f)[NB][4], const T* p, int64_t ld)
 // C = beta*C + alpha*op(A) op(B); A, B and C may be stored as float or double.
 // KS: op(A) diag(ks) op(B), where the problems of the batch are consecutive ranges
 // of K of one contraction of length kall (the last may be shorter).
-template <int TA, int TB, int WT, int PF, bool INP, bool KS, typename TAs, typename TBs, typename TCs>
+template <int TA, int TB, int WT, int PF, bool INP, bool KS, bool SUB, typename TAs, typename TBs, typename TCs>
 __global__ __launch_bounds__(256) void k_gemm_reg(int64_t M, int64_t N, int64_t K, int64_t tilesM, double alpha,
                                                   const TAs* A, int64_t lda, const TBs* B, int64_t ldb, double beta,
                                                   TCs* C, int64_t ldc, int tiles, int64_t sA, int64_t sB, int64_t sC,
@@ -160,6 +163,39 @@ __global__ __launch_bounds__(256) void k_gemm_reg(int64_t M, int64_t N, int64_t 
         pa += stepa;
         pb += stepb;
     };
+    typedef typename vec2_of<TCs>::type C2;
+    constexpr bool PAIR = !KA && NB > 1;  // rows 2li, 2li + 1 of tiles i, i + 1
+    constexpr int RI = PAIR ? 2 : 1;
+    TCs cv[NB][NB][4];
+    auto addr = [&](int i, int j, int v) {
+        return C + (row0 + frag_row<KA, NB>(i, li)) + (col0 + frag_row<KB, NB>(j, g + 4 * v)) * ldc;
+    };
+    auto load_c = [&]() {
+#pragma unroll
+        for (int i = 0; i < NB; i += RI)
+#pragma unroll
+            for (int j = 0; j < NB; ++j)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    if (PAIR) {
+                        const C2 x = *reinterpret_cast<const C2*>(addr(i, j, v));
+                        cv[i][j][v] = x.x;
+                        cv[i + RI - 1][j][v] = x.y;
+                    } else {
+                        cv[i][j][v] = *addr(i, j, v);
+                    }
+                }
+    };
+    auto take = [&]() {
+#pragma unroll
+        for (int i = 0; i < NB; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j) {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) cv[i][j][v] -= (TCs)acc[i][j][v];
+                acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
+            }
+    };
     // the tiles are formed transposed: D lane (li, g) holds columns g + 4v of row li
     auto mult = [&](int st) {
         if (KS) {
@@ -184,45 +220,30 @@ __global__ __launch_bounds__(256) void k_gemm_reg(int64_t M, int64_t N, int64_t 
     for (int q = 0; q < PF - 1; ++q)
         if (q < nch) load(q);
     int c = 0;
-    for (; c + 2 * PF - 1 <= nch; c += PF)  // every load of this pass exists
+    if (SUB) load_c();
+    static_assert(!SUB || PF == 4, "a pass is the 64 k whose sum is subtracted");
+    for (; c + 2 * PF - 1 <= nch; c += PF) {  // every load of this pass exists
 #pragma unroll
         for (int q = 0; q < PF; ++q) {
             load((q + PF - 1) % PF);
             mult(q);
         }
-    for (; c < nch; c += PF)
+        if (SUB) take();
+    }
+    for (; c < nch; c += PF) {
 #pragma unroll
         for (int q = 0; q < PF; ++q) {
             if (c + q + PF - 1 < nch) load((q + PF - 1) % PF);
             if (c + q < nch) mult(q);
         }
+        if (SUB) take();
+    }
     // With beta != 0 every C value is loaded before the first store (a load placed
     // after a store that may alias it waits for that store's round trip).
-    typedef typename vec2_of<TCs>::type C2;
-    constexpr bool PAIR = !KA && NB > 1;  // rows 2li, 2li + 1 of tiles i, i + 1
-    constexpr int RI = PAIR ? 2 : 1;
-    TCs cv[NB][NB][4];
-    auto addr = [&](int i, int j, int v) {
-        return C + (row0 + frag_row<KA, NB>(i, li)) + (col0 + frag_row<KB, NB>(j, g + 4 * v)) * ldc;
-    };
-    if (beta != 0.0) {
-#pragma unroll
-        for (int i = 0; i < NB; i += RI)
-#pragma unroll
-            for (int j = 0; j < NB; ++j)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) {
-                    if (PAIR) {
-                        const C2 x = *reinterpret_cast<const C2*>(addr(i, j, v));
-                        cv[i][j][v] = x.x;
-                        cv[i + RI - 1][j][v] = x.y;
-                    } else {
-                        cv[i][j][v] = *addr(i, j, v);
-                    }
-                }
-    }
+    if (!SUB && beta != 0.0) load_c();
     if (INP) __syncthreads();
     auto out = [&](int i, int j, int v) {
+        if (SUB) return cv[i][j][v];
         const double o = alpha * acc[i][j][v];
         return (TCs)((beta == 0.0) ? o : beta * (double)cv[i][j][v] + o);
     };
@@ -252,7 +273,7 @@ static void gemm_reg_launch(hipStream_t s, int ta, int tb, int64_t M, int64_t N,
     const int64_t nblk = (tiles != 1 && tiles != 2) ? tm * tn : BM < 64 ? 4 * (t64 * (t64 + 1) / 2) : tm * (tm + 1) / 2;
     dim3 grid((unsigned)nblk, (unsigned)batch), block(256);
 #define GPL_GR(TAv, TBv)                                                                                           \
-    hipLaunchKernelGGL((k_gemm_reg<TAv, TBv, WT, PF, INP, false, TAs, TBs, TCs>), grid, block, 0, s, M, N, K, tm,    \
+    hipLaunchKernelGGL((k_gemm_reg<TAv, TBv, WT, PF, INP, false, false, TAs, TBs, TCs>), grid, block, 0, s, M, N, K, tm,    \
                        alpha, A, lda, B, ldb, beta, C, ldc, tiles, sA, sB, sC, (const double*)nullptr, (int64_t)0)
     if (!ta && !tb) GPL_GR(0, 0);
     else if (!ta && tb) GPL_GR(0, 1);
@@ -307,6 +328,22 @@ void gemm2_f64_batched(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int6
     gemm_any(s, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tiles, batch, sA, sB, sC);
 }
 
+// C -= A B^T (A: M x K, B: N x K), the sums of 64 k subtracted one by one: the update of
+// a panel's later columns by its earlier ones.  One sum of all 256 rounds each element at
+// the size of that sum 256 times; the solutions' error is then 1.15 to 1.45 times as large.
+void gemm_sub_f64(hipStream_t s, int64_t M, int64_t N, int64_t K, const double* A, int64_t lda, const double* B,
+                  int64_t ldb, double* C, int64_t ldc) {
+    if (M <= 0 || N <= 0) return;
+#define GPL_GS(WT)                                                                                                  \
+    hipLaunchKernelGGL((k_gemm_reg<0, 1, WT, 4, false, false, true, double, double, double>),                       \
+                       dim3((unsigned)(((M + 2 * WT - 1) / (2 * WT)) * ((N + 2 * WT - 1) / (2 * WT)))), dim3(256), 0, \
+                       s, M, N, K, (M + 2 * WT - 1) / (2 * WT), -1.0, A, lda, B, ldb, 1.0, C, ldc, 0, (int64_t)0,     \
+                       (int64_t)0, (int64_t)0, (const double*)nullptr, (int64_t)0)
+    if (M / 64 * (N / 64) < 128) GPL_GS(16);  // the line of gemm_any
+    else GPL_GS(32);
+#undef GPL_GS
+}
+
 // Lower 64x64 tiles of A diag(ks) A^T, A (M x K): `parts` partial products over kp
 // columns each, C + p * sC.  32-wide waves with three chunks in flight whatever the
 // size (M = 1024, K = 131072 in 64 parts: 2227 us, 64-wide 2330, 16-wide 5097;
@@ -314,7 +351,7 @@ void gemm2_f64_batched(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int6
 void gemm_gram_f64(hipStream_t s, int64_t M, int64_t K, const double* A, int64_t lda, const double* ks, int parts,
                    int64_t kp, double* C, int64_t ldc, int64_t sC) {
     const int64_t t = M / 64;
-    hipLaunchKernelGGL((k_gemm_reg<0, 1, 32, 4, false, true, double, double, double>),
+    hipLaunchKernelGGL((k_gemm_reg<0, 1, 32, 4, false, true, false, double, double, double>),
                        dim3((unsigned)(t * (t + 1) / 2), (unsigned)parts), dim3(256), 0, s, M, M, kp, t, 1.0, A, lda, A,
                        lda, 0.0, C, ldc, 1, kp * lda, kp * lda, sC, ks, K);
 }
@@ -962,29 +999,22 @@ __global__ __launch_bounds__(kPanelThreads) void k_potrf_panel(
             if (!kF64) __syncthreads();
         }
         if (rb < nc) panel_publish(&sync[P + P * rb + c], epoch);
-        // the own diagonal block: D -= L_{rb,c} L_{rb,c}^T, lower tiles (here and
-        // below FP32 storage sums the products first, as its results always were)
+        // the own diagonal block: D -= L_{rb,c} L_{rb,c}^T, lower tiles (here and below the
+        // products are summed before they are subtracted: one rounding at the block's size
+        // for 64, where accumulating into the block took the log-determinant's error to twice)
         auto diag_update = [&]() {
-            d4 old[2];
-#pragma unroll
-            for (int u = 0; u < 2; ++u) {
-                old[u] = dacc[u];
-                if (!kF64) dacc[u] = d4{0.0, 0.0, 0.0, 0.0};
-            }
+            d4 sum[2] = {d4{0.0, 0.0, 0.0, 0.0}, d4{0.0, 0.0, 0.0, 0.0}};
 #pragma unroll 8
             for (int k0 = 0; k0 < 64; k0 += 4) {
                 const double* Sk = &S[k0 + g][64 + li];
 #pragma unroll
                 for (int u = 0; u < 2; ++u)
-                    if (u < 1 || w < 2) {
-                        const double a = Sk[16 * diag_ct(w, u)];
-                        dacc[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(kF64 ? -a : a, Sk[16 * diag_rt(w, u)], dacc[u],
-                                                                       0, 0, 0);
-                    }
+                    if (u < 1 || w < 2)
+                        sum[u] = __builtin_amdgcn_mfma_f64_16x16x4f64(Sk[16 * diag_ct(w, u)], Sk[16 * diag_rt(w, u)],
+                                                                      sum[u], 0, 0, 0);
             }
-            if (!kF64)
 #pragma unroll
-                for (int u = 0; u < 2; ++u) dacc[u] = old[u] - dacc[u];
+            for (int u = 0; u < 2; ++u) dacc[u] -= sum[u];
         };
         if (rb == c + 1 && rb < nc) {
             // the next diagonal block: published before it is factored
@@ -1021,25 +1051,18 @@ __global__ __launch_bounds__(kPanelThreads) void k_potrf_panel(
                 for (int q = 0; q < 8; ++q) S[w + 8 * q][r64] = (double)lv[q];
                 __syncthreads();
                 if (i > 0) fetch(c2 - 1);
-                d4 acc[2];
-#pragma unroll
-                for (int j = 0; j < 2; ++j)
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) acc[j][v] = kF64 ? (double)own[i][j][v] : 0.0;
+                d4 acc[2] = {d4{0.0, 0.0, 0.0, 0.0}, d4{0.0, 0.0, 0.0, 0.0}};
 #pragma unroll 8
                 for (int k0 = 0; k0 < 64; k0 += 4) {
                     const double b = S[k0 + g][64 + r0];
 #pragma unroll
-                    for (int j = 0; j < 2; ++j) {
-                        const double a = S[k0 + g][q0 + 16 * j + li];
-                        acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(kF64 ? -a : a, b, acc[j], 0, 0, 0);
-                    }
+                    for (int j = 0; j < 2; ++j)
+                        acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(S[k0 + g][q0 + 16 * j + li], b, acc[j], 0, 0, 0);
                 }
 #pragma unroll
                 for (int j = 0; j < 2; ++j)
 #pragma unroll
-                    for (int v = 0; v < 4; ++v)
-                        own[i][j][v] = kF64 ? (T)acc[j][v] : (T)((double)own[i][j][v] - acc[j][v]);
+                    for (int v = 0; v < 4; ++v) own[i][j][v] = (T)((double)own[i][j][v] - acc[j][v]);
                 if (i > 0) __syncthreads();  // the operand is free
             }
         }

@@ -90,6 +90,8 @@ void gemm2_f64(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, d
 void gemm2_f64_batched(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha, const double* A,
                        int64_t lda, const double* B, int64_t ldb, double beta, double* C, int64_t ldc, int tiles,
                        int batch, int64_t sA, int64_t sB, int64_t sC);
+void gemm_sub_f64(hipStream_t s, int64_t M, int64_t N, int64_t K, const double* A, int64_t lda, const double* B,
+                  int64_t ldb, double* C, int64_t ldc);
 void gemm_gram_f64(hipStream_t s, int64_t M, int64_t K, const double* A, int64_t lda, const double* ks, int parts,
                    int64_t kp, double* C, int64_t ldc, int64_t sC);
 // FP64 MFMA on an FP32 A
