@@ -1291,6 +1291,11 @@ static int fit_ep(gpl_model* m) {
     const double tol = 1e-4, damping = m->opts.damping, dmin = m->opts.damping_min > 0 ? m->opts.damping_min : 0.1;
     double damp = damping, diff_old = INFINITY, diff_new = INFINITY;
     bool quad_ok = true;
+    // Whether the sites' flags are read before the factor (one more wait, 20 us), as a sweep
+    // with V <= 0 makes no use of it: the beta-binomial is the likelihood that is not
+    // log-concave, the others get there by the quadrature's error alone, and a fit that has
+    // split its sites once tends to do so in every sweep that follows.
+    bool ask = m->lik.kind == GPL_LIK_BETABINOM;
     int it;
     for (it = 1; it <= maxiter; ++it) {
         int* flags = m->b[B_INFO].as<int>();  // zero here: the finish kernel clears them
@@ -1301,25 +1306,31 @@ static int fit_ep(gpl_model* m) {
                      m->d(B_Y), tr, off, q, m->d(B_GH), m->d(B_GH) + 32, damp, m->d(B_Z), m->d(B_V), m->d(B_SV),
                      m->d(B_LOGZS), m->d(B_CAVM), m->d(B_CAVV), flags + 1, N, m->d(B_W1));
         }
-        {
-            Prof p(c, "form_B", 0, 16.0 * N * (N + 64) / 2);
-            form_B_f64(s, m->d(B_K), m->d(B_L), N, n, N, m->d(B_SV));
-        }
-        // X = L^-1 for the posterior variances: its front half beside the factor, no scratch
-        potrf_blocked(c, m->d(B_L), N, m->d(B_DINV), m->d(B_LDIAG), flags, m->d(B_XINV), nullptr, m->d(B_W1));
-        solve_alpha_back(c, m, gate);
-        {
-            Prof p(c, "symv", 2.0 * N * N, 8.0 * N * N / 2);
-            symv_lt_f64(s, m->d(B_K), N, m->d(B_ALPHA), m->d(B_FMEAN), m->d(B_KMV), kmatvec_chunks(N), 1, 0, 0, gate);
-        }
-        colsumsq_f64(s, m->d(B_XINV), N, N, n, m->d(B_W3), 1);
-        ep_finish(s, n, m->d(B_V), m->d(B_Z), m->d(B_W3), m->d(B_CAVM), m->d(B_CAVV), m->d(B_LOGZS), m->d(B_ALPHA),
-                  m->d(B_LDIAG), m->d(B_FMEAN), m->d(B_FVAR), m->d(B_FOLD), m->d(B_FVOLD), m->d(B_ZOLD), m->d(B_POLD),
-                  diff_old, flags, m->d(B_TERM), c->fin, c->stage);
         double h[4];
-        int fl[2];
-        int r = read_finish(c, h, fl);
-        if (r) return r;
+        int fl[2] = {0, 0}, r;
+        if (ask) HIP_TRY(read_back(c, fl, flags, 8));
+        if (fl[1] & 6) {
+            HIP_TRY(hipMemsetAsync(flags, 0, 8, s));
+        } else {
+            {
+                Prof p(c, "form_B", 0, 16.0 * N * (N + 64) / 2);
+                form_B_f64(s, m->d(B_K), m->d(B_L), N, n, N, m->d(B_SV));
+            }
+            // X = L^-1 for the posterior variances: its front half beside the factor, no scratch
+            potrf_blocked(c, m->d(B_L), N, m->d(B_DINV), m->d(B_LDIAG), flags, m->d(B_XINV), nullptr, m->d(B_W1));
+            solve_alpha_back(c, m, gate);
+            {
+                Prof p(c, "symv", 2.0 * N * N, 8.0 * N * N / 2);
+                symv_lt_f64(s, m->d(B_K), N, m->d(B_ALPHA), m->d(B_FMEAN), m->d(B_KMV), kmatvec_chunks(N), 1, 0, 0,
+                            gate);
+            }
+            colsumsq_f64(s, m->d(B_XINV), N, N, n, m->d(B_W3), 1);
+            ep_finish(s, n, m->d(B_V), m->d(B_Z), m->d(B_W3), m->d(B_CAVM), m->d(B_CAVV), m->d(B_LOGZS),
+                      m->d(B_ALPHA), m->d(B_LDIAG), m->d(B_FMEAN), m->d(B_FVAR), m->d(B_FOLD), m->d(B_FVOLD),
+                      m->d(B_ZOLD), m->d(B_POLD), diff_old, flags, m->d(B_TERM), c->fin, c->stage);
+            r = read_finish(c, h, fl);
+            if (r) return r;
+        }
         if (fl[1] & 2) {
             m->logZ = -INFINITY;
             m->iters = it;
@@ -1328,6 +1339,7 @@ static int fit_ep(gpl_model* m) {
         quad_ok = !(fl[1] & 1);  // the last sweep's flag decides (R/ep.R:326-328)
         if (fl[1] & 4) {
             // some site variance <= 0: the split sweep of R/ep.R:50-138
+            ask = true;
             double lz = 0;
             r = split_step(m, true, &lz);
             if (r) return r;
