@@ -7,6 +7,7 @@ front end.
 """
 
 from . import _lib
+from ._lib import release_memory  # noqa: F401
 from .api import (  # noqa: F401
     GP, approx_ep, approx_laplace, cf_const, cf_lin, cf_matern32, cf_matern52, cf_nn, cf_periodic, cf_prod,
     cf_sexp, eval_cf, get_param, gp_compare, gp_draw, gp_energy, gp_energy_grad, gp_fit, gp_init, gp_load, gp_loo, gp_optim,

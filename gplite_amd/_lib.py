@@ -64,6 +64,7 @@ def _sig(lib):
     sigs = {
         "gpl_ctx_create": (C.c_int, [i32, C.POINTER(_vp)]),
         "gpl_ctx_destroy": (None, [_vp]),
+        "gpl_release_memory": (None, []),
         "gpl_last_error": (C.c_char_p, []),
         "gpl_last_error_minor": (i64, []),
         "gpl_device_name": (C.c_int, [_vp, C.c_char_p, i32]),
@@ -193,6 +194,11 @@ def profile(enable=None, reset=False):
         nm = names.raw[32 * i:32 * i + 32].split(b"\0", 1)[0].decode()
         out[nm] = {"ms": ms[i], "launches": cnt[i], "flops": fl[i], "bytes": by[i]}
     return out
+
+
+def release_memory():
+    """Give the device blocks that freed models left for the next one back to the device."""
+    lib().gpl_release_memory()
 
 
 def device_name():

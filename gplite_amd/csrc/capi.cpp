@@ -10,6 +10,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 #include <cmath>
 #include <cstdio>
@@ -53,8 +54,9 @@ extern "C" int64_t gpl_last_error_minor(void) { return g_minor; }
 // ---------------------------------------------------------------------------
 static std::mutex g_pools_mu;
 static std::vector<BlockPool*> g_pools;
+static std::atomic<size_t> g_pool_bytes[kMaxDevices];  // in all pools of a device
 
-BlockPool::BlockPool(size_t cap_bytes) : cap(cap_bytes) {
+BlockPool::BlockPool(int dev, size_t cap_bytes) : device(dev), cap(cap_bytes) {
     std::lock_guard<std::mutex> lk(g_pools_mu);
     g_pools.push_back(this);
 }
@@ -75,9 +77,19 @@ void* BlockPool::take(size_t bytes, size_t* sz) {
     if (best < 0) return nullptr;
     void* p = blocks[best].p;
     *sz = blocks[best].sz;
-    total -= *sz;
+    g_pool_bytes[device] -= *sz;
     blocks.erase(blocks.begin() + best);
     return p;
+}
+bool BlockPool::reserve(size_t sz) {
+    if (g_pool_bytes[device].fetch_add(sz) + sz <= cap) return true;
+    g_pool_bytes[device] -= sz;
+    return false;
+}
+void BlockPool::drop(size_t i) {
+    g_pool_bytes[device] -= blocks[i].sz;
+    hipFree(blocks[i].p);
+    blocks.erase(blocks.begin() + i);
 }
 void BlockPool::put(void* p, size_t sz) {
     std::lock_guard<std::mutex> lk(mu);
@@ -85,36 +97,32 @@ void BlockPool::put(void* p, size_t sz) {
         hipFree(p);
         return;
     }
-    while (total + sz > cap) {  // the oldest first
-        total -= blocks.front().sz;
-        hipFree(blocks.front().p);
-        blocks.erase(blocks.begin());
+    while (!reserve(sz)) {
+        if (blocks.empty()) {  // the other contexts' blocks fill the room
+            hipFree(p);
+            return;
+        }
+        drop(0);  // the oldest first
     }
     blocks.push_back({p, sz, frees});
-    total += sz;
 }
 void BlockPool::age() {
     std::lock_guard<std::mutex> lk(mu);
     ++frees;
-    while (!blocks.empty() && frees - blocks.front().born > kKeep) {
-        total -= blocks.front().sz;
-        hipFree(blocks.front().p);
-        blocks.erase(blocks.begin());
-    }
+    while (!blocks.empty() && frees - blocks.front().born > kKeep) drop(0);
 }
 void BlockPool::clear() {
     std::lock_guard<std::mutex> lk(mu);
-    for (auto& b : blocks) hipFree(b.p);
-    blocks.clear();
-    total = 0;
+    while (!blocks.empty()) drop(blocks.size() - 1);
+}
+extern "C" void gpl_release_memory(void) {
+    std::lock_guard<std::mutex> lk(g_pools_mu);
+    for (auto* b : g_pools) b->clear();
 }
 hipError_t dev_malloc(void** p, size_t bytes) {
     hipError_t e = hipMalloc(p, bytes);
     if (e == hipSuccess) return e;
-    {
-        std::lock_guard<std::mutex> lk(g_pools_mu);
-        for (auto* b : g_pools) b->clear();
-    }
+    gpl_release_memory();
     (void)hipGetLastError();
     return hipMalloc(p, bytes);
 }
@@ -159,7 +167,7 @@ extern "C" int gpl_ctx_create(int32_t device, gpl_ctx** out) {
     if (e == hipSuccess) e = hipHostMalloc((void**)&c->up, gpl_ctx::kStage * sizeof(double));
     size_t mfree = 0, mtotal = 0;
     if (e == hipSuccess) e = hipMemGetInfo(&mfree, &mtotal);
-    if (e == hipSuccess) c->blocks = new BlockPool(t_ctx_for_server ? 0 : mtotal / 32);
+    if (e == hipSuccess) c->blocks = new BlockPool(device, t_ctx_for_server ? 0 : mtotal / 32);
     if (const char* pw = getenv("GPL_PANEL_WAIT_POLLS")) c->pwait = (unsigned)strtoul(pw, nullptr, 10);
     if (e != hipSuccess) {
         delete c;

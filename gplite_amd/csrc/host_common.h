@@ -102,11 +102,12 @@ struct ProfClass {
 // Device blocks above kMin bytes that freed models leave for the next one: such a
 // block costs 13 us to allocate and 15 us to free, 45 and 280 us from 256 MB up
 // (smaller ones come out of the runtime's own suballocator in under 1 us), which
-// was 1.5 of the 13.5 ms of a fit and gradient at n = 8192.  Bounded: at most
-// 1/32 of the device's memory, and a block that none of the last kKeep frees of a
-// model has led to a use of is given back.  A block enters only after its
-// streams were waited for.  Any allocation of the library that fails empties the
-// pools of all contexts of the process and is tried again.
+// was 1.5 of the 13.5 ms of a fit and gradient at n = 8192.  Bounded: the pools of
+// all contexts on a device hold at most 1/32 of its memory together, and a block that
+// none of the last kKeep frees of a model has led to a use of is given back.  A block
+// enters only after its streams were waited for.  Any allocation of the library that
+// fails empties the pools of all contexts of the process and is tried again; other
+// allocators' programs call gpl_release_memory.
 struct BlockPool {
     static constexpr size_t kMin = (size_t)1 << 20;
     static constexpr unsigned kKeep = 16;
@@ -117,15 +118,19 @@ struct BlockPool {
     };
     std::mutex mu;
     std::vector<Block> blocks;
-    size_t total = 0, cap = 0;
+    const int device;
+    const size_t cap;    // of the device's pools together (0: this one keeps nothing)
     unsigned frees = 0;  // models freed so far
-    explicit BlockPool(size_t cap_bytes);
+    BlockPool(int dev, size_t cap_bytes);
     ~BlockPool();
+    bool reserve(size_t sz);  // room for sz more bytes under the cap
+    void drop(size_t i);      // frees a block (mu is held)
     void* take(size_t bytes, size_t* sz);  // the smallest block of bytes .. 1.25 bytes, or nullptr
     void put(void* p, size_t sz);          // keeps or frees it
     void age();                            // a model was freed
     void clear();
 };
+constexpr int kMaxDevices = 64;
 hipError_t dev_malloc(void** p, size_t bytes);  // hipMalloc; when that fails, once more with empty pools
 
 struct gpl_ctx {

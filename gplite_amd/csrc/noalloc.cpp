@@ -25,7 +25,6 @@ namespace {
 constexpr size_t kScratchBytes = (size_t)GPL_NOALLOC_SCRATCH_MB << 20;
 __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
-constexpr int kMaxDevices = 64;
 std::mutex g_mu;                      // guards g_ptr
 void* g_ptr[kMaxDevices] = {};        // device address of `scratch` per device
 std::mutex g_call_mu[kMaxDevices];    // one gpl_pred_noalloc at a time per device

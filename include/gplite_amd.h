@@ -122,6 +122,10 @@ typedef struct gpl_model gpl_model;
 
 int gpl_ctx_create(int32_t device, gpl_ctx** out);
 void gpl_ctx_destroy(gpl_ctx* ctx);
+/* A context keeps device blocks of freed models for the next one (on a device at
+ * most 1/32 of its memory for all contexts together).  This gives them back, in
+ * every context of the process, for other libraries that allocate on the device. */
+void gpl_release_memory(void);
 const char* gpl_last_error(void);
 int64_t gpl_last_error_minor(void);
 int gpl_device_name(gpl_ctx* ctx, char* buf, int32_t len);
