@@ -715,14 +715,9 @@ static void potrf32_blocked(gpl_ctx* c, float* L, int64_t N, double* Dinv, doubl
     inv.finish();
 }
 
-void gpl::trsv_back(gpl_ctx* c, hipStream_t s, const double* L, int64_t ld, const double* Dinv, int64_t N, double* b,
-                    double* x, int* info, const double* scale, int64_t n, double* scaled, const int* gate) {
-    const int64_t T = N / 64;
-    if (T > kSolveMaxBlocks) {
-        trsv_lower_f64(s, L, ld, Dinv, N, b, x, 1);
-        if (scaled) vec_mul_pad(s, n, N, scale, x, scaled, gate);
-        return;
-    }
+void gpl::trsv_back(gpl_ctx* c, hipStream_t s, const double* L, int64_t ld, const double* Dinv, int64_t N,
+                    const double* b, double* x, int* info, const double* scale, int64_t n, double* scaled, const int* gate) {
+    const int64_t T = N / 64;  // <= kSolveMaxBlocks: a larger factor alone is 2^39 bytes
     double *pub, *reset;
     int64_t nreset;
     c->next_pub(T, &pub, &reset, &nreset);
@@ -1865,7 +1860,7 @@ int gpl::pred_on(gpl_ctx* c, gpl_model* m, const double* xt, int64_t mt, int32_t
             if (!A2) return fail(GPL_ERR_OOM, "device allocation failed");
             Prof p(c, "pred_trmm", (double)N * N * M, 8.0 * N * M * 2);
             if (m->opts.precision == GPL_PREC_MIXED)
-                gemm_mixed_f32f64f64(s, 0, 0, N, M, N, 1.0, m->b[B_XINV].as<float>(), N, KtT, N, 0.0, A2, N, 3);
+                gemm_mixed_f32f64f64(s, N, M, N, 1.0, m->b[B_XINV].as<float>(), N, KtT, N, 0.0, A2, N, 3);
             else
                 gemm2_f64(s, 0, 0, N, M, N, 1.0, m->d(B_XINV), N, KtT, N, 0.0, A2, N, 3);
             KtT = A2;
@@ -1932,7 +1927,7 @@ static int draw_on(gpl_ctx* c, gpl_model* m, const double* xt, int64_t mt, doubl
     if (m->have_xinv) {
         scale_rows_f64(s, KtT, N, n, M, m->d(B_SV));
         if (m->opts.precision == GPL_PREC_MIXED)
-            gemm_mixed_f32f64f64(s, 0, 0, N, M, N, 1.0, m->b[B_XINV].as<float>(), N, KtT, N, 0.0, A2, N, 3);
+            gemm_mixed_f32f64f64(s, N, M, N, 1.0, m->b[B_XINV].as<float>(), N, KtT, N, 0.0, A2, N, 3);
         else
             gemm2_f64(s, 0, 0, N, M, N, 1.0, m->d(B_XINV), N, KtT, N, 0.0, A2, N, 3);
     } else {

@@ -53,9 +53,9 @@ __device__ __forceinline__ void lower_tile(int64_t t, int64_t& ti, int64_t& tj) 
 // SUB: C -= op(A) op(B) (alpha = -1, beta = 1), where every 64 k's products are summed on
 // their own and subtracted.
 //
-// INP: C is one of the operands (a solve against a 64x64 inverse).  A workgroup
-// of 64x64 then covers the whole contraction of its rows (A = C, N = 64) or
-// columns (B = C, M = 64), and stores only after all of its waves have read.
+// INP: C is B (a solve against a 64x64 inverse, M = 64).  A workgroup of 64x64 then
+// covers the whole contraction of its columns, and stores only after all of its waves
+// have read.
 // ---------------------------------------------------------------------------
 template <typename T> struct vec2_of;
 template <> struct vec2_of<double> { typedef double2 type; };
@@ -275,7 +275,8 @@ static void gemm_reg_launch(hipStream_t s, int ta, int tb, int64_t M, int64_t N,
 #define GPL_GR(TAv, TBv)                                                                                           \
     hipLaunchKernelGGL((k_gemm_reg<TAv, TBv, WT, PF, INP, false, false, TAs, TBs, TCs>), grid, block, 0, s, M, N, K, tm,    \
                        alpha, A, lda, B, ldb, beta, C, ldc, tiles, sA, sB, sC, (const double*)nullptr, (int64_t)0)
-    if (!ta && !tb) GPL_GR(0, 0);
+    if constexpr (INP || sizeof(TAs) == 4) GPL_GR(0, 0);  // the only forms that are called
+    else if (!ta && !tb) GPL_GR(0, 0);
     else if (!ta && tb) GPL_GR(0, 1);
     else if (ta && !tb) GPL_GR(1, 0);
     else GPL_GR(1, 1);
@@ -303,9 +304,11 @@ static void gemm_any(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_
     if (M <= 0 || N <= 0 || batch <= 0) return;
 #define GPL_GA(WT, PF, INP) \
     gemm_reg_launch<WT, PF, INP>(s, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tiles, batch, sA, sB, sC)
-    if ((const void*)A == (const void*)C || (const void*)B == (const void*)C) {
-        GPL_GA(32, 3, true);
-        return;
+    if constexpr (sizeof(TAs) == 8) {
+        if (B == C) {
+            GPL_GA(32, 3, true);
+            return;
+        }
     }
     const bool low = tiles == 1 || tiles == 2;
     const int64_t m = M / 64, n = N / 64, m2 = (m + 1) / 2, n2 = (n + 1) / 2;
@@ -346,8 +349,8 @@ void gemm_sub_f64(hipStream_t s, int64_t M, int64_t N, int64_t K, const double* 
 
 // Lower 64x64 tiles of A diag(ks) A^T, A (M x K): `parts` partial products over kp
 // columns each, C + p * sC.  32-wide waves with three chunks in flight whatever the
-// size (M = 1024, K = 131072 in 64 parts: 2227 us, 64-wide 2330, 16-wide 5097;
-// M = 512 in 14 parts: 614, 1167, 1485).
+// size (the product alone, M = 1024, K = 131072 in 64 parts: 2227 us, 64-wide 2330,
+// 16-wide 5097; M = 512 in 14 parts: 614, 1167, 1485).
 void gemm_gram_f64(hipStream_t s, int64_t M, int64_t K, const double* A, int64_t lda, const double* ks, int parts,
                    int64_t kp, double* C, int64_t ldc, int64_t sC) {
     const int64_t t = M / 64;
@@ -357,10 +360,9 @@ void gemm_gram_f64(hipStream_t s, int64_t M, int64_t K, const double* A, int64_t
 }
 
 // FP64-compute GEMM on FP32 storage of A (prediction)
-void gemm_mixed_f32f64f64(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha,
-                          const float* A, int64_t lda, const double* B, int64_t ldb, double beta, double* C,
-                          int64_t ldc, int tiles) {
-    gemm_any(s, ta, tb, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tiles, 1, 0, 0, 0);
+void gemm_mixed_f32f64f64(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const float* A,
+                          int64_t lda, const double* B, int64_t ldb, double beta, double* C, int64_t ldc, int tiles) {
+    gemm_any(s, 0, 0, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, tiles, 1, 0, 0, 0);
 }
 
 // A failing row + 1 into info, the lowest of all that are reported: the workgroups of

@@ -402,27 +402,6 @@ void gemm_f32(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, fl
 // ---------------------------------------------------------------------------
 // FP32-matrix helpers with FP64 vectors
 // ---------------------------------------------------------------------------
-// A = I over all T x T tiles (the 128-wide triangular GEMM modes read the tile
-// just above each diagonal tile, so upper tiles must hold zeros)
-__global__ void k_set_identity32(float* __restrict__ A, int64_t ld, int64_t T, int64_t sA) {
-    A += blockIdx.y * sA;
-    const int64_t ti = blockIdx.x % T, tj = blockIdx.x / T;
-    const int t = threadIdx.x, i = t & 63;
-    for (int c = t >> 6; c < 64; c += 4) {
-        const int64_t gi = ti * 64 + i, gj = tj * 64 + c;
-        A[gi + gj * ld] = (gi == gj) ? 1.f : 0.f;
-    }
-}
-
-void set_identity_f32_batched(hipStream_t s, float* A, int64_t ld, int64_t N, int batch, int64_t sA) {
-    const int64_t T = N / 64;
-    hipLaunchKernelGGL(k_set_identity32, dim3((unsigned)(T * T), (unsigned)batch), dim3(256), 0, s, A, ld, T, sA);
-}
-
-void set_identity_f32(hipStream_t s, float* A, int64_t ld, int64_t N) {
-    set_identity_f32_batched(s, A, ld, N, 1, 0);
-}
-
 // Column j = c0 + blockIdx.x of X (FP32, N x N, ld N, batch stride sX): zero
 // above its 64x64 diagonal block, the block's column of Dinv (FP64, 64x64
 // column-major per block, zero above its diagonal, batch stride sD) rounded to

@@ -84,7 +84,7 @@ void launch_grad_tiles_f32(hipStream_t s, const DevProg* prog, const DevProg& hp
 // 3 = full grid and k stops after the row tile (C = X B with X lower triangular),
 // 4 = full grid and k starts at the column tile (C = A X with X lower triangular),
 // 5 = full grid and k starts at the row tile (C = X^T B with X lower triangular).
-// C may be A (N = 64) or B (M = 64), with tiles 0.
+// C may be B (M = 64, ta = tb = 0), with tiles 0.
 void gemm2_f64(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha, const double* A,
                int64_t lda, const double* B, int64_t ldb, double beta, double* C, int64_t ldc, int tiles);
 void gemm2_f64_batched(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha, const double* A,
@@ -95,14 +95,12 @@ void gemm_sub_f64(hipStream_t s, int64_t M, int64_t N, int64_t K, const double* 
 void gemm_gram_f64(hipStream_t s, int64_t M, int64_t K, const double* A, int64_t lda, const double* ks, int parts,
                    int64_t kp, double* C, int64_t ldc, int64_t sC);
 // FP64 MFMA on an FP32 A
-void gemm_mixed_f32f64f64(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, double alpha,
-                          const float* A, int64_t lda, const double* B, int64_t ldb, double beta, double* C,
-                          int64_t ldc, int tiles);
+void gemm_mixed_f32f64f64(hipStream_t s, int64_t M, int64_t N, int64_t K, double alpha, const float* A,
+                          int64_t lda, const double* B, int64_t ldb, double beta, double* C, int64_t ldc, int tiles);
 // FP32 storage and FP32 MFMA with FP32 accumulation (dense32.hip)
 void gemm_f32(hipStream_t s, int ta, int tb, int64_t M, int64_t N, int64_t K, float alpha, const float* A,
               int64_t lda, const float* B, int64_t ldb, float beta, float* C, int64_t ldc, int tiles, int bm,
               int fold = 1);
-void set_identity_f32(hipStream_t s, float* A, int64_t ld, int64_t N);
 void trmv_lower_f32(hipStream_t s, const float* X, int64_t ld, int64_t N, const double* b, double* y, int trans,
                     double* part, int nchunk);
 void colsumsq_f32(hipStream_t s, const float* A, int64_t ld, int64_t nrow, int64_t ncol, double* out, int lower);
@@ -251,8 +249,7 @@ void ep_post(hipStream_t s, int64_t n, const double* V, const double* z, const d
 void vec_axpby(hipStream_t s, int64_t n, double a, const double* x, double b, const double* y,
                double* out);
 void vec_mul(hipStream_t s, int64_t n, const double* a, const double* b, double* out);
-void vec_mul_pad(hipStream_t s, int64_t n, int64_t N, const double* a, const double* b, double* out,
-                 const int* gate = nullptr);
+void vec_mul_pad(hipStream_t s, int64_t n, int64_t N, const double* a, const double* b, double* out);
 void vec_recip(hipStream_t s, int64_t n, const double* a, double* out);
 
 // FITC (fitc.hip)
@@ -328,7 +325,6 @@ constexpr int kFoldInverse = 1;
 // multiplied by the inverse's transpose.
 void potrf_step_f32_batched(hipStream_t s, float* A, int64_t ld, int64_t k, int64_t M, double* Dinv, double* ldiag,
                             int* info, int batch, int64_t sA, int64_t sD, int64_t sL, const double* Dacc);
-void set_identity_f32_batched(hipStream_t s, float* A, int64_t ld, int64_t N, int batch, int64_t sA);
 void trmv_lower_f32_batched(hipStream_t s, const float* X, int64_t ld, int64_t N, const double* b, double* y,
                             int trans, int batch, int64_t sX, int64_t sv, double* part, int nchunk);
 void colsumsq_f32_batched(hipStream_t s, const float* A, int64_t ld, int64_t nrow, int64_t ncol, double* out,

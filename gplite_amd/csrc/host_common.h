@@ -36,12 +36,11 @@ int prepare_prog(const gpl_cf_term* terms, int32_t nterms, int64_t ncols, DevPro
 void potrf_blocked(gpl_ctx* c, double* L, int64_t N, double* Dinv, double* ldiag, int* info, double* X = nullptr,
                    double* Tm = nullptr, double* rhs = nullptr);
 void trtri_blocked(gpl_ctx* c, const double* L, const double* Dinv, int64_t N, double* X, double* T = nullptr);
-// L^T x = b with one vector (trsv_lower_f64's arguments, b left unchanged): one
-// launch when N / 64 <= kSolveMaxBlocks, else one per block.  info receives
-// kPanelWaitTimeout if a device wait times out.  With `scaled` also scaled =
+// L^T x = b with one vector in one launch (trsv_lower_f64's arguments, b left
+// unchanged).  info receives kPanelWaitTimeout if a device wait times out.  With `scaled` also scaled =
 // scale .* x (n entries, zero on the padding) unless *gate (if any) flags NaN or
 // V <= 0.
-void trsv_back(gpl_ctx* c, hipStream_t s, const double* L, int64_t ld, const double* Dinv, int64_t N, double* b,
+void trsv_back(gpl_ctx* c, hipStream_t s, const double* L, int64_t ld, const double* Dinv, int64_t N, const double* b,
                double* x, int* info, const double* scale = nullptr, int64_t n = 0, double* scaled = nullptr,
                const int* gate = nullptr);
 // L Y = diag(sv) B in place for M right-hand sides (of which the first mt are not padding) (sv: the first n rows, or null): the forward solve of a

@@ -374,16 +374,15 @@ void reduce_maxabsdiff(hipStream_t s, const double* a, const double* b, int64_t 
     hipLaunchKernelGGL(k_reduce<2>, dim3(1), dim3(1024), 0, s, a, b, n, out);
 }
 
-// out[i] = a[i] b[i] for i < n, 0 on the padding; nothing if the gate's flags say NaN or V <= 0
+// out[i] = a[i] b[i] for i < n, 0 on the padding
 __global__ void k_mul_pad(int64_t n, int64_t N, const double* __restrict__ a, const double* __restrict__ b,
-                          double* __restrict__ out, const int* __restrict__ gate) {
-    if (gate && (*gate & 6)) return;
+                          double* __restrict__ out) {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i < N) out[i] = i < n ? a[i] * b[i] : 0.0;
 }
 
-void vec_mul_pad(hipStream_t s, int64_t n, int64_t N, const double* a, const double* b, double* out, const int* gate) {
-    hipLaunchKernelGGL(k_mul_pad, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, s, n, N, a, b, out, gate);
+void vec_mul_pad(hipStream_t s, int64_t n, int64_t N, const double* a, const double* b, double* out) {
+    hipLaunchKernelGGL(k_mul_pad, dim3((unsigned)((N + 255) / 256)), dim3(256), 0, s, n, N, a, b, out);
 }
 
 // ---------------------------------------------------------------------------
