@@ -7,6 +7,7 @@
 #include "gpl_internal.h"
 
 #include <cmath>
+#include <type_traits>
 
 namespace gpl {
 
@@ -1421,9 +1422,8 @@ void trsv_persist_f64(hipStream_t s, const double* L, int64_t ld, const double* 
 // wait is on a block of a lower ticket; the order of the sums is fixed.
 //
 // Every 64-k block's product is summed on its own and subtracted as a whole: the
-// longest chain of roundings is then 64 + n / 64.  One sum over all k < 64 i made it n,
-// the variances' error 2.3 and 3.6 times as large (n = 640, 1500) and a prediction of
-// many points 3 % faster (1000 points on n = 4096 640 us, here 658).
+// longest chain of roundings is then 64 + n / 64.  One sum over all k < 64 i made it n
+// and the variances' error 2.3 and 3.6 times as large (n = 640, 1500).
 //
 // Bound by N/64 dependent blocks (a hand-over, one 64 x 64 x WN product and one
 // with the inverse each) for few columns, by its products for many.  In launches
@@ -1473,22 +1473,22 @@ __global__ __launch_bounds__(256) void k_trsm_persist(const double* __restrict__
 #pragma unroll
         for (int b = 0; b < NC; ++b) acc[0][a][b] = acc[1][a][b] = d4{0.0, 0.0, 0.0, 0.0};
     double fa[2][4][NR][4], fb[2][4][NC][4];  // two 64-k blocks of each operand, in 16-k chunks
-    auto load_a = [&](int st, int k) {  // L_{ik}; for k = i the inverse of the diagonal block
+    auto load_a = [&](int st, int k, int c) {  // L_{ik}; for k = i the inverse of the diagonal block
         const double* q = k < i ? pa + 64 * (int64_t)k * ld : pd;
         const int64_t l = k < i ? ld : 64;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) frag_load<false, NR>(fa[st][c], q + 16 * c * l, l);
+        frag_load<false, NR>(fa[st][c], q + 16 * c * l, l);
     };
-    auto load_b = [&](int st, int k) {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) frag_load<true, NC>(fb[st][c], pb + 64 * k + 16 * c, ldb);
-    };
+    auto load_b = [&](int st, int k, int c) { frag_load<true, NC>(fb[st][c], pb + 64 * k + 16 * c, ldb); };
     auto take = [&](int st, int a, int b) {
 #pragma unroll
         for (int v = 0; v < 4; ++v) bv[a][b][v] -= acc[st][a][b][v];
     };
-    // one block's product; the last one's is subtracted between the matrix instructions
-    auto mult = [&](int st, bool sub) {
+    // Block k's product.  Between its matrix instructions the last block's product is
+    // subtracted and the next block's operands are requested, a chunk's at a time: all of
+    // them in a row hold the wave up until the memory path has taken them (4096 points on
+    // n = 8192: 8.3 ms with all ahead of the product, 5.7 behind its first instruction,
+    // 5.0 here).
+    auto mult = [&](int st, int k, bool have, auto last) {  // last: the product with the inverse
 #pragma unroll
         for (int a = 0; a < NR; ++a)
 #pragma unroll
@@ -1503,10 +1503,17 @@ __global__ __launch_bounds__(256) void k_trsm_persist(const double* __restrict__
                     for (int b = 0; b < NC; ++b)
                         acc[st][a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(fb[st][c][b][s], fa[st][c][a][s],
                                                                              acc[st][a][b], 0, 0, 0);
-                if (sub && c == 1 && s < NR * NC) take(st ^ 1, s / NC, s % NC);
+                if (!last && s == 0) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    load_a(st ^ 1, k + 1, c);
+                    if (have) load_b(st ^ 1, k + 1, c);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                if (!last && c == 1 && s < NR * NC) take(st ^ 1, s / NC, s % NC);
             }
     };
-    load_a(0, 0);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) load_a(0, 0, c);
     int ready = 0;  // blocks below this one are published
     bool have = false;
     for (int k0 = 0; k0 < i; k0 += 2)
@@ -1536,11 +1543,11 @@ __global__ __launch_bounds__(256) void k_trsm_persist(const double* __restrict__
                 __syncthreads();
                 if (ready < 0) return;
             }
-            if (!have) load_b(u, k);
+            if (!have)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) load_b(u, k, c);
             have = k + 1 < ready;
-            if (have) load_b(u ^ 1, k + 1);
-            load_a(u ^ 1, k + 1);
-            mult(u, true);
+            mult(u, k, have, std::false_type());
         }
 #pragma unroll
     for (int a = 0; a < NR; ++a)
@@ -1571,7 +1578,7 @@ __global__ __launch_bounds__(256) void k_trsm_persist(const double* __restrict__
 #pragma unroll
                 for (int s = 0; s < 4; ++s) fa[0][c][a][s] = fa[1][c][a][s];
     }
-    mult(0, false);
+    mult(0, i, false, std::true_type());
 #pragma unroll
     for (int a = 0; a < NR; ++a)
 #pragma unroll
@@ -1684,12 +1691,14 @@ void trsm_few_f64(hipStream_t s, const double* L, int64_t ld, const double* Dinv
                        reset, nreset, ticket, base, info, maxpoll);
 }
 
-// 16 columns a workgroup while the chain of row blocks is what takes the time (4 us
-// a block against 8 with 64 columns), 64 once the products are (a quarter of the
-// reads of L).  A whole prediction with 16 / 64, us: n = 640 m = 4096 265 / 274;
-// n = 2048 m = 1000 351 / 428, m = 2000 543 / 448; n = 4096 m = 500 582 / 608,
-// m = 1000 903 / 686.
-int trsm_cols(int64_t N, int64_t M) { return N * M <= 3000000 ? 16 : 64; }
+// 16 columns a workgroup while the chain of row blocks is what takes the time, 64 once
+// the products are (a quarter of the reads of L).  A whole prediction with 16 / 64, us:
+// n = 640 m = 2000 161 / 182, m = 4096 220 / 217; n = 1000 m = 1400 189 / 211, m = 3000
+// 245 / 217; n = 2048 m = 1000 312 / 310, m = 1400 373 / 332; n = 4096 m = 500 532 / 540,
+// m = 700 641 / 563, m = 4096 2936 / 1518; n = 8192 m = 256 984 / 1021, m = 500 1593 /
+// 1084, m = 4096 11131 / 5320; n = 16384 m = 128 1924 / 2109, m = 256 3185 / 2157, m =
+// 4096 44191 / 20916.
+int trsm_cols(int64_t N, int64_t M) { return N * M <= 2400000 ? 16 : 64; }
 
 void trsm_persist_f64(hipStream_t s, const double* L, int64_t ld, const double* Dinv, int64_t N, double* B, int64_t ldb,
                       int64_t M, const double* sv, int64_t n, unsigned* sync, unsigned epoch, unsigned base, int* info,
