@@ -823,7 +823,6 @@ static int read_scalars(gpl_model* m, double* out, int k) {
     return GPL_OK;
 }
 
-// One Gaussian "Newton step" (exactly one: R/laplace.R:281-283).
 // What a finish kernel left in the context's pinned block: four scalars, two flags.
 static int read_finish(gpl_ctx* c, double* h, int* fl) {
     HIP_TRY(hipStreamSynchronize(c->stream));
@@ -833,6 +832,7 @@ static int read_finish(gpl_ctx* c, double* h, int* fl) {
     return GPL_OK;
 }
 
+// One Gaussian "Newton step" (exactly one: R/laplace.R:281-283).
 static int fit_gaussian(gpl_model* m) {
     gpl_ctx* c = m->ctx;
     hipStream_t s = c->stream;

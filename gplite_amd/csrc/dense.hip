@@ -349,9 +349,10 @@ void gemm_sub_f64(hipStream_t s, int64_t M, int64_t N, int64_t K, const double* 
 }
 
 // Lower 64x64 tiles of A diag(ks) A^T, A (M x K): `parts` partial products over kp
-// columns each, C + p * sC.  32-wide waves with three chunks in flight whatever the
-// size (the product alone, M = 1024, K = 131072 in 64 parts: 2227 us, 64-wide 2330,
-// 16-wide 5097; M = 512 in 14 parts: 614, 1167, 1485).
+// columns each, C + p * sC (fitc_part_cols chooses their number).  32-wide waves with
+// three chunks in flight whatever the size (16 / 32 / 64 wide, products and their sum, us:
+// K = 131072 with M = 1024 5454 / 2698 / 3568, M = 512 1563 / 762 / 1034, M = 128 137 / 90 /
+// 272; K = 32768 with M = 512 389 / 216 / 229).
 void gemm_gram_f64(hipStream_t s, int64_t M, int64_t K, const double* A, int64_t lda, const double* ks, int parts,
                    int64_t kp, double* C, int64_t ldc, int64_t sC) {
     const int64_t t = M / 64;

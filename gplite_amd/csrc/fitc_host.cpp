@@ -65,8 +65,9 @@ struct gpl_fitc {
 
 // Partial products of A S^-1 A^T over column ranges, summed in a fixed order: as
 // many as fill the chip with 64x64 output tiles four times over (2048 of them), at
-// least 256 columns each.  m = 1024, n = 131072: 7 / 15 / 30 parts 2.9 / 2.7 / 2.6 ms;
-// m = 128: 1 / 7 / 64 parts 4254 / 614 / 74 us.
+// least 256 columns each.  n = 131072, products and sum, in 7 / 15 / 30 / 64 parts, us:
+// m = 1024 2797 / 2668 / 2683 / 2723 (15 are taken), m = 512 749 / 964 / 843 / 736 (56:
+// 744), m = 128 630 / 306 / 165 / 90 (64).
 static int64_t fitc_part_cols(const gpl_fitc* f) {
     const int64_t T = f->Mz / 64, tiles = T * (T + 1) / 2;
     const int64_t P = std::max<int64_t>(1, std::min<int64_t>({2048 / tiles, 64, f->N / 256}));

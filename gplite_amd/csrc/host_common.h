@@ -29,10 +29,10 @@ void set_minor(int64_t minor);
 int prepare_prog(const gpl_cf_term* terms, int32_t nterms, int64_t ncols, DevProg& P);
 // Blocked FP64 Cholesky of the N x N lower tiles of L in place (Dinv: the 64x64
 // diagonal-block inverses, ldiag: log L_ii, info: first failing row + 1) and the
-// triangular inverse X = L^-1 (all tiles written; T: optional N x N scratch,
-// which selects the recursive-doubling form); potrf_blocked with X and Tm forms
-// both, the inverse's front half beside the factor's last panels, and with rhs
-// overwrites that vector (N rows) with L^-1 rhs
+// triangular inverse X = L^-1 by recursive doubling (all tiles written; T, Tm: N x N
+// scratch for its products, which otherwise lie above X's diagonal and are cleared
+// at the end); potrf_blocked with X forms both, the inverse's front half beside the
+// factor's last panels, and with rhs overwrites that vector (N rows) with L^-1 rhs
 void potrf_blocked(gpl_ctx* c, double* L, int64_t N, double* Dinv, double* ldiag, int* info, double* X = nullptr,
                    double* Tm = nullptr, double* rhs = nullptr);
 void trtri_blocked(gpl_ctx* c, const double* L, const double* Dinv, int64_t N, double* X, double* T = nullptr);
@@ -43,9 +43,10 @@ void trtri_blocked(gpl_ctx* c, const double* L, const double* Dinv, int64_t N, d
 void trsv_back(gpl_ctx* c, hipStream_t s, const double* L, int64_t ld, const double* Dinv, int64_t N, const double* b,
                double* x, int* info, const double* scale = nullptr, int64_t n = 0, double* scaled = nullptr,
                const int* gate = nullptr);
-// L Y = diag(sv) B in place for M right-hand sides (of which the first mt are not padding) (sv: the first n rows, or null): the forward solve of a
-// prediction, in launches of at most kTrsmFlags blocks.  info receives kPanelWaitTimeout if a device wait
-// times out.
+// L Y = diag(sv) B in place for M right-hand sides, of which the first mt are not
+// padding (sv: the first n rows, or null): the forward solve of a prediction, in
+// launches of at most kTrsmFlags blocks.  info receives kPanelWaitTimeout if a device
+// wait times out.
 void trsm_forward(gpl_ctx* c, hipStream_t s, const double* L, int64_t ld, const double* Dinv, int64_t N, double* B,
                 int64_t ldb, int64_t M, int64_t mt, const double* sv, int64_t n, int* info);
 // the error reported for an info word of kPanelWaitTimeout
